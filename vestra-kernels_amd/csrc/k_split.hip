@@ -1,0 +1,728 @@
+// Projection GEMMs on split rows (split_gemm.h): C[m][n] = sum_k X[m][k] W[n][k],
+// X the activation rows, W the weight rows, both k-contiguous.
+//
+// A workgroup owns a BM x BN tile; KG groups of WM x WN waves take every
+// KG-th k-slice of 32 and sum their tiles in group order through LDS.  A
+// slice (128 bytes per row) is copied straight into LDS (no registers, no
+// LDS stores) through a ring of three stages: while the products of slice t
+// run from registers, the fragments of slice t + 1 are read from LDS and
+// slices t + 2 and t + 3 are in flight from L2.  One barrier per slice.  The
+// granules of a row are XOR-swizzled by the row on the way in, so that a
+// fragment read (16 rows x 4 granules) touches every bank once per 256
+// bytes.  W is the A operand of the matrix instruction, so that a lane ends
+// with four consecutive columns of one row and stores 16 bytes.
+//
+// What bounds it: at 3460 x 2304 x 768 the f16 matrix cores, whose clock
+// drops to 1.7-1.9 GHz under this load (41 us, 890 TFLOP/s of f16 products; a
+// register-only loop of the same instruction reaches 1.9 PFLOP/s on random
+// data and 2.4 on zeros, an 8192^3 library product in f16 1.13 PFLOP/s); at 865
+// rows the one round of tiles and its start and end (13.6 us for N = 2304
+// against 28 on the fp32 matrix instructions, which are bound at 19.5).
+//
+// Error against float64 (2-norm, N(0, 1) rows times N(0, 0.02^2) weights):
+// 1.5e-7 to 2.0e-7 at K = 768 and 2.6e-7 to 3.6e-7 at K = 3072 (3.2e-7 and
+// 6.2e-7 on the 128 x 256 tile), against 2.5e-7 to 5.0e-7 and 5.8e-7 to
+// 9.9e-7 of the fp32 matrix instructions.
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+
+#include "common.h"
+#include "kernels.h"
+#include "split_gemm.h"
+
+namespace vh {
+namespace {
+
+struct SplitArgs {
+    const char *x, *w;      // split rows of X [M][Kp] and W [N][Kp]
+    const int *ex, *ew;     // row exponents (ex null: ex_c for every row)
+    int ex_c;
+    int M, N, slices;       // slices = Kp / 32
+    const float *xf, *wf;   // the f32 rows [M][K], [N][K] (non-finite rows)
+    int K, wf_n;            // wf_n: 0, or wf is [K][wf_n]
+    float *c;
+    const float *bias, *gamma;
+    float *q, *k, *v;
+    int tokens, heads;
+    const float *rot;
+    char *out_split;        // GeluSplit: split rows [M][N] of the output times out_scale
+    float out_scale;
+};
+
+enum class SEpi : int { Store, Gelu, Residual, Qkv, GeluSplit, Chw };
+
+// A product with a non-finite row, in floats: rare, so a plain loop.
+__device__ __attribute__((noinline)) float split_slow_dot(const float *x, const float *w, size_t step, int K) {
+    if (!x || !w) return __builtin_nanf("");
+    float s = 0.0f;
+    for (int k = 0; k < K; k++) s = fmaf(x[k], w[k * step], s);
+    return s;
+}
+
+template <int BM, int BN, int WM, int WN, int KG, int ST, SEpi EPI>
+__global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs ar) {
+    constexpr int NW = WM * WN, GT = NW * 64;
+    constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
+    constexpr int ROWS = BM + BN;
+    constexpr int CP = ROWS / 8;               // copies of 8 rows in a stage
+    constexpr int LD = (CP + NW - 1) / NW;     // per wave; past CP the last one again
+    constexpr int STAGE = ROWS * 128;
+    static_assert(BM % 8 == 0 && BN % 8 == 0, "whole copies");
+    static_assert(TM % 16 == 0 && TN % 16 == 0 && FM % KG == 0, "fragments");
+    static_assert(ST >= 3, "frag reads run a stage ahead of the products");
+    constexpr int FO = FM / KG;  // fragment rows (of 16 m) a K group finishes
+    static_assert(EPI != SEpi::Qkv || TN % 32 == 0, "whole 32-wide RoPE halves per wave");
+    extern __shared__ __attribute__((aligned(16))) char smem_c[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = KG == 1 ? 0 : wave / NW, gw = wave % NW;
+    const int wm = gw / WN, wn = gw % WN;
+    const int li = lane & 15, lh = lane >> 4;
+
+    // Workgroups go round-robin over the 8 XCDs; renumbered so that an XCD's
+    // share is a run of tiles that walks 8 row tiles column by column.
+    const int nx = (ar.N + BN - 1) / BN, ny = (ar.M + BM - 1) / BM;
+    int tm, tn;
+    {
+        const int total = nx * ny, bid = blockIdx.x;
+        const int q = total / 8, r = total % 8, xcd = bid % 8;
+        const int t = xcd * q + min(xcd, r) + bid / 8;
+        const int gm = min(8, ny), group = t / (gm * nx), first = group * gm;
+        const int rows = min(ny - first, gm), local = t - group * gm * nx;
+        tm = first + local % rows;
+        tn = local / rows;
+    }
+    const int m0 = tm * BM, n0 = tn * BN;
+    const size_t pitch = (size_t)ar.slices * 128;
+    const char *xb = ar.x + (size_t)m0 * pitch, *wb = ar.w + (size_t)n0 * pitch;
+
+    // Copy i of this wave moves rows 8 b .. 8 b + 7 (b = i * NW + gw) of the
+    // stage; LDS granule p of a row holds global granule p ^ (row % 8), so
+    // that the 16 rows of a fragment read spread over all banks.
+    uint32_t voff[LD];
+#pragma unroll
+    for (int i = 0; i < LD; i++) {
+        const int b = min(i * NW + gw, CP - 1), row = b * 8 + lane / 8;
+        const int r = row < BM ? min(row, ar.M - 1 - m0) : min(row - BM, ar.N - 1 - n0);
+        voff[i] = (uint32_t)(r * (int)pitch + (((lane & 7) ^ (lane >> 3)) << 4));
+    }
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem_c + kg * ST * STAGE;
+    auto copy_stage = [&](int slice, int buf) {
+        const size_t ko = (size_t)slice * 128;
+#pragma unroll
+        for (int i = 0; i < LD; i++) {
+            const int b = min(i * NW + gw, CP - 1);
+            const char *base = b * 8 < BM ? xb : wb;
+            copy16_to_lds(base + ko, voff[i], __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + b * 1024));
+        }
+    };
+
+    // The cross products hi.lo and lo.hi sum apart from hi.hi where there are
+    // registers for it: their sum is 2^-11 of the other's, so only a third
+    // of the additions round at full size (64 x 64 tiles,
+    // error against float64 at K = 768: 2.4e-7 -> 1.5e-7).
+    constexpr bool SEP = FM * FN <= 8;
+    f32x4 acc[FM][FN], cross[SEP ? FM : 1][SEP ? FN : 1];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (SEP) cross[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    auto low = [&](int i, int j) -> f32x4 & {
+        if constexpr (SEP) return cross[i][j];
+        else return acc[i][j];
+    };
+
+    // Fragment i of X: row wm*TM + 16 i + li, hi granule lh, lo granule 4 + lh.
+    const char *gs = smem_c + kg * ST * STAGE;
+    const int ohi = (lh ^ (li & 7)) << 4, olo = ((4 + lh) ^ (li & 7)) << 4;
+    f16x8 xh[2][FM], xl[2][FM], wh[2][FN], wl[2][FN];
+    auto fetch = [&](int set, int buf) {
+        const char *xs = gs + buf * STAGE + (wm * TM + li) * 128;
+        const char *ws = gs + buf * STAGE + (BM + wn * TN + li) * 128;
+#pragma unroll
+        for (int i = 0; i < FM; i++) xh[set][i] = *reinterpret_cast<const f16x8 *>(xs + i * 2048 + ohi);
+#pragma unroll
+        for (int j = 0; j < FN; j++) wh[set][j] = *reinterpret_cast<const f16x8 *>(ws + j * 2048 + ohi);
+#pragma unroll
+        for (int j = 0; j < FN; j++) wl[set][j] = *reinterpret_cast<const f16x8 *>(ws + j * 2048 + olo);
+#pragma unroll
+        for (int i = 0; i < FM; i++) xl[set][i] = *reinterpret_cast<const f16x8 *>(xs + i * 2048 + olo);
+    };
+    // W is the A operand: a lane ends with four consecutive n of one m.
+    auto products = [&](int set) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[i][j] = mfma16x16x32_f16(wh[set][j], xh[set][i], acc[i][j]);
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) low(i, j) = mfma16x16x32_f16(wl[set][j], xh[set][i], low(i, j));
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) low(i, j) = mfma16x16x32_f16(wh[set][j], xl[set][i], low(i, j));
+    };
+
+    // Group kg takes slices kg, kg + KG, ...; every group runs the same
+    // number of steps (barriers are workgroup-wide), one past its last slice
+    // reloads that slice and skips the products.
+    const int S = ar.slices;
+    const int steps = (S + KG - 1) / KG;
+    auto slice_of = [&](int t) { return min(kg + t * KG, S - 1); };
+    copy_stage(slice_of(0), 0);
+    copy_stage(slice_of(1), 1);
+    copy_stage(slice_of(2), 2);
+    split_wait<2 * LD>();
+    __builtin_amdgcn_s_barrier();
+    fetch(0, 0);
+    // Step t: products of slice t (fragments in registers) while the
+    // fragments of slice t + 1 are read; the buffer of slice t, whose reads
+    // ended before this step's barrier, takes slice t + 3.  Copies past the
+    // last slice reload it into a buffer that is not read again, so that
+    // every step is the same basic block.
+    auto step = [&](int t, auto setc, int buf) {
+        constexpr int set = decltype(setc)::value;
+        split_wait<LD>();  // slice t + 1 landed, slice t + 2 may be in flight
+        __builtin_amdgcn_s_barrier();
+        copy_stage(slice_of(t + 3), buf);
+        fetch(set ^ 1, buf == 2 ? 0 : buf + 1);
+        products(set);
+        // Issue order: a fragment read behind each of the first products.
+        constexpr int NR = 2 * (FM + FN), NM = 3 * FM * FN, PER = NM / NR < 1 ? 1 : (NM / NR > 2 ? 2 : NM / NR);
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+    };
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    // A group without a slice for the last step (S % KG) leaves it out.
+    const int mine = (S - kg + KG - 1) / KG;
+    int buf = 0, t = 0;
+    for (; t + 1 < mine; t += 2) {
+        step(t, P0{}, buf);
+        buf = buf == 2 ? 0 : buf + 1;
+        step(t + 1, P1{}, buf);
+        buf = buf == 2 ? 0 : buf + 1;
+    }
+    if (t < mine) {
+        step(t, P0{}, buf);
+        t++;
+    }
+    if (t < steps) __builtin_amdgcn_s_barrier();
+    split_wait<0>();
+    if constexpr (SEP) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) acc[i][j] += cross[i][j];
+    }
+
+    // The K groups' partial tiles are summed in group order through LDS:
+    // group g finishes fragment rows [g * FO, (g + 1) * FO), in accs[0 .. FO).
+    f32x4 fin[FO][FN];
+    if constexpr (KG > 1) {
+        __builtin_amdgcn_s_barrier();
+        f32x4 *xch = reinterpret_cast<f32x4 *>(smem_c);
+        const int gt = tid % GT;
+        // [source group][fragment][thread]; a group leaves out its own rows.
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+            if (i / FO != kg)
+#pragma unroll
+                for (int j = 0; j < FN; j++) xch[((kg * FM + i) * FN + j) * GT + gt] = acc[i][j];
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < KG; o++) {
+            if (o != kg) continue;
+#pragma unroll
+            for (int i = 0; i < FO; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) {
+                    const int row = o * FO + i;
+                    f32x4 sum = o == 0 ? acc[row][j] : xch[(row * FN + j) * GT + gt];
+#pragma unroll
+                    for (int g = 1; g < KG; g++) sum += g == o ? acc[row][j] : xch[((g * FM + row) * FN + j) * GT + gt];
+                    fin[i][j] = sum;
+                }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++) fin[i][j] = acc[i][j];
+    }
+
+    // Epilogue: lane (li, lh) holds C[m][n .. n + 3], m = mb + 16 i, n = nb + 16 j.
+    const int mb = m0 + wm * TM + kg * FO * 16 + li, nb = n0 + wn * TN + 4 * lh;
+    if (n0 + wn * TN >= ar.N) return;
+    const bool vec = (ar.N & 3) == 0;
+    int exr[FO], ewr[FN][4];
+    float bias[FN][4], gamma[FN][4];
+#pragma unroll
+    for (int i = 0; i < FO; i++) exr[i] = ar.ex ? ar.ex[min(mb + 16 * i, ar.M - 1)] : ar.ex_c;
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int cn = min(nb + 16 * j + r, ar.N - 1);
+            ewr[j][r] = ar.ew[cn];
+            bias[j][r] = load_or(ar.bias, reinterpret_cast<const float *>(ar.ew), cn, 0.0f);
+            gamma[j][r] = load_or(ar.gamma, reinterpret_cast<const float *>(ar.ew), cn, 1.0f);
+        }
+    f32x4 old[EPI == SEpi::Residual ? FO : 1][FN];
+    if constexpr (EPI == SEpi::Residual) {
+        if (vec) {
+#pragma unroll
+            for (int i = 0; i < FO; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++)
+                    old[i][j] = *reinterpret_cast<const f32x4 *>(
+                        ar.c + (size_t)min(mb + 16 * i, ar.M - 1) * ar.N + min(nb + 16 * j, ar.N - 4));
+        }
+    }
+    // Qkv: the wave's columns lie in one head of one of Q, K, V.
+    const int colw = n0 + wn * TN;
+    float *head_dst = nullptr;
+    bool rope = false;
+    if constexpr (EPI == SEpi::Qkv) {
+        const int per = ar.heads * 64, group = colw / per;
+        head_dst = group == 0 ? ar.q : (group == 1 ? ar.k : ar.v);
+        rope = ar.rot != nullptr && group < 2;
+    }
+#pragma unroll
+    for (int i = 0; i < FO; i++) {
+        const int m = mb + 16 * i;
+        if (m >= ar.M) continue;
+        float v[FN][4];
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float t = __builtin_ldexpf(fin[i][j][r], exr[i] + ewr[j][r]);
+                if (exr[i] == kSplitNonFinite || ewr[j][r] == kSplitNonFinite)
+                {
+                    const int n = min(nb + 16 * j + r, ar.N - 1);
+                    t = split_slow_dot(ar.xf ? ar.xf + (size_t)m * ar.K : nullptr,
+                                       ar.wf ? ar.wf + (ar.wf_n ? n : (size_t)n * ar.K) : nullptr,
+                                       ar.wf_n ? ar.wf_n : 1, ar.K);
+                }
+                if (ar.bias) t = add_rn(t, bias[j][r]);
+                if constexpr (EPI == SEpi::Store || EPI == SEpi::Residual || EPI == SEpi::Chw)
+                    if (ar.gamma) t = mul_rn(t, gamma[j][r]);
+                if constexpr (EPI == SEpi::Gelu || EPI == SEpi::GeluSplit) t = gelu_fast_form(t);
+                v[j][r] = t;
+            }
+        if constexpr (EPI == SEpi::Qkv) {
+            const int img = m / ar.tokens, tok = m - img * ar.tokens;
+#pragma unroll
+            for (int jp = 0; jp < FN; jp += 2) {
+                const int col = colw + jp * 16;       // a 32-wide half of a head
+                const int head = (col % (ar.heads * 64)) / 64, d0 = col % 64;
+                if (col >= ar.N) continue;
+                if (rope) {
+                    // rope::rotate_half (src/rope.rs:84-93): dims (d, d + 16) of
+                    // the half are fragments (jp, jp + 1) of this lane.
+                    const float *rp = ar.rot + (((size_t)tok * 2 + d0 / 32) * 16 + 4 * lh) * 2;
+                    const f32x4 r0 = *reinterpret_cast<const f32x4 *>(rp);
+                    const f32x4 r1 = *reinterpret_cast<const f32x4 *>(rp + 4);
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const float sn = r < 2 ? r0[2 * r] : r1[2 * r - 4], cs = r < 2 ? r0[2 * r + 1] : r1[2 * r - 3];
+                        const float a = v[jp][r], b = v[jp + 1][r];
+                        v[jp][r] = sub_rn(mul_rn(a, cs), mul_rn(b, sn));
+                        v[jp + 1][r] = add_rn(mul_rn(b, cs), mul_rn(a, sn));
+                    }
+                }
+                float *dst = head_dst + (((size_t)img * ar.heads + head) * ar.tokens + tok) * 64 + d0 + 4 * lh;
+                *reinterpret_cast<f32x4 *>(dst) = f32x4{v[jp][0], v[jp][1], v[jp][2], v[jp][3]};
+                *reinterpret_cast<f32x4 *>(dst + 16) =
+                    f32x4{v[jp + 1][0], v[jp + 1][1], v[jp + 1][2], v[jp + 1][3]};
+            }
+        } else if constexpr (EPI == SEpi::GeluSplit) {
+            // Split rows of the output, N % 32 == 0: one exponent for all.
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const int n = nb + 16 * j;
+                if (n >= ar.N) continue;
+                f16x4 hi, lo;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    _Float16 h, l;
+                    split_f16(v[j][r] * ar.out_scale, h, l);
+                    hi[r] = h;
+                    lo[r] = l;
+                }
+                char *dst = ar.out_split + ((size_t)m * (ar.N / 32) + n / 32) * 128 + (n % 32) * 2;
+                *reinterpret_cast<f16x4 *>(dst) = hi;
+                *reinterpret_cast<f16x4 *>(dst + 64) = lo;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const int n = nb + 16 * j;
+                if (n >= ar.N) continue;
+                if constexpr (EPI == SEpi::Chw) {
+                    // C^T: 16 lanes store 16 consecutive rows of one channel.
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (n + r < ar.N) ar.c[(size_t)(n + r) * ar.M + m] = v[j][r];
+                } else {
+                    float *dst = ar.c + (size_t)m * ar.N + n;
+                    if (vec) {
+                        f32x4 o{v[j][0], v[j][1], v[j][2], v[j][3]};
+                        if constexpr (EPI == SEpi::Residual)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) o[r] = add_rn(old[i][j][r], v[j][r]);
+                        *reinterpret_cast<f32x4 *>(dst) = o;
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            if (n + r < ar.N) dst[r] = EPI == SEpi::Residual ? add_rn(dst[r], v[j][r]) : v[j][r];
+                    }
+                }
+            }
+        }
+    }
+}
+
+// Split rows of 32-bit float rows, one wave per row.  The row maximum is
+// taken on the bit patterns (magnitude order, and a NaN sorts above every
+// number), then each value is scaled by its exact power of two and split.
+// Rows of up to 1024 values stay in registers between the two passes (the
+// row is read once: 865 x 768 in 2.4 us); longer rows are read again, from
+// the cache.
+__device__ __forceinline__ void store_split4(char *row, int k, f32x4 v, int e) {
+    f16x4 hi, lo;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        _Float16 h, l;
+        split_f16(__builtin_ldexpf(v[r], -e), h, l);
+        hi[r] = h;
+        lo[r] = l;
+    }
+    char *p = row + (k / 32) * 128 + (k % 32) * 2;
+    *reinterpret_cast<f16x4 *>(p) = hi;
+    *reinterpret_cast<f16x4 *>(p + 64) = lo;
+}
+
+__device__ __forceinline__ uint32_t absmax4(uint32_t mx, f32x4 v) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) mx = max(mx, __float_as_uint(v[r]) & 0x7fffffffu);
+    return mx;
+}
+
+__global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict__ in, char *__restrict__ out,
+                                                         int *__restrict__ ex, size_t rows, int K, int slices) {
+    const int lane = threadIdx.x & 63;
+    const size_t row = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const float *src = in + row * K;
+    char *dst = out + row * slices * 128;
+    const int Kp = slices * 32;
+    uint32_t mx = 0;
+    int e;
+    const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
+    if ((K & 3) == 0) {
+        const f32x4 *src4 = reinterpret_cast<const f32x4 *>(src);
+        const int n4 = K >> 2, np4 = Kp >> 2;
+        if (K <= 1024) {
+            f32x4 r[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) r[j] = lane + j * 64 < n4 ? src4[lane + j * 64] : zero;
+#pragma unroll
+            for (int j = 0; j < 4; j++) mx = absmax4(mx, r[j]);
+            e = split_exponent(wave_umax(mx));
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (lane + j * 64 < np4) store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
+        } else {
+            for (int c = lane; c < n4; c += 64) mx = absmax4(mx, src4[c]);
+            e = split_exponent(wave_umax(mx));
+            for (int c = lane; c < np4; c += 64)
+                store_split4(dst, 4 * c, c < n4 && e != kSplitNonFinite ? src4[c] : zero, e);
+        }
+    } else {
+        for (int k = lane; k < K; k += 64) mx = max(mx, __float_as_uint(src[k]) & 0x7fffffffu);
+        e = split_exponent(wave_umax(mx));
+        for (int c = lane; c < Kp >> 2; c += 64) {
+            f32x4 v = zero;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (4 * c + r < K && e != kSplitNonFinite) v[r] = src[4 * c + r];
+            store_split4(dst, 4 * c, v, e);
+        }
+    }
+    if (lane == 0) ex[row] = e;
+}
+
+// LayerNorm of each row straight into split rows (launch_layernorm's bits,
+// then split): cols % 32 == 0, cols <= 1024, one wave per row.  A row whose
+// normalised values hold a NaN (an infinity cannot arise without one in
+// the statistics) is stored as NaN with exponent 0.
+__global__ __launch_bounds__(256) void layernorm_split_kernel(const float *__restrict__ in,
+                                                              const float *__restrict__ gamma,
+                                                              const float *__restrict__ beta,
+                                                              char *__restrict__ out, int *__restrict__ ex,
+                                                              size_t rows, int cols, float eps) {
+    const int lane = threadIdx.x & 63;
+    const size_t row = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const f32x4 *x4 = reinterpret_cast<const f32x4 *>(in + row * cols);
+    const int n4 = cols >> 2;
+    f32x4 r[4], g[4], b[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int idx = lane + j * 64, ci = idx < n4 ? idx : 0;
+        r[j] = idx < n4 ? x4[idx] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        g[j] = reinterpret_cast<const f32x4 *>(gamma)[ci];
+        b[j] = reinterpret_cast<const f32x4 *>(beta)[ci];
+    }
+    float mean, inv;
+    ln_row_stats(r, lane, n4, cols, eps, mean, inv);
+    uint32_t mx = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (lane + j * 64 >= n4) continue;
+        r[j] = ln_apply(r[j], mean, inv, g[j], b[j]);
+        mx = absmax4(mx, r[j]);
+    }
+    mx = wave_umax(mx);
+    int e = split_exponent(mx);
+    if (e == kSplitNonFinite) {
+        e = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) r[j] = r[j] * __builtin_nanf("");
+    }
+    char *dst = out + row * (cols / 32) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (lane + j * 64 < n4) store_split4(dst, 4 * (lane + j * 64), r[j], e);
+    if (lane == 0) ex[row] = e;
+}
+
+// Upper bound of |LayerNorm(x) . w_n + b_n| over every x, per row n of
+// w [N][K]: |LN| without gamma has 2-norm at most sqrt(K), so the product
+// is at most sqrt(K) ||w_n g||_2 + sum |w_n beta| + |b_n|.  One wave per row.
+__global__ __launch_bounds__(256) void ln_output_bound_kernel(const float *__restrict__ w,
+                                                              const float *__restrict__ gamma,
+                                                              const float *__restrict__ beta,
+                                                              const float *__restrict__ bias,
+                                                              float *__restrict__ bound, int N, int K) {
+    const int lane = threadIdx.x & 63;
+    const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (n >= N) return;
+    float s2 = 0.0f, sb = 0.0f;
+    for (int k = lane; k < K; k += 64) {
+        const float v = w[(size_t)n * K + k], p = v * gamma[k];
+        s2 = fmaf(p, p, s2);
+        sb += fabsf(v * beta[k]);
+    }
+    s2 = wave_sum(s2);
+    sb = wave_sum(sb);
+    if (lane == 0) bound[n] = sqrtf((float)K) * sqrtf(s2) + sb + fabsf(bias[n]);
+}
+
+// Split rows of the columns of in [K][N] (row-major): 16 columns per
+// workgroup, 64 rows of them per pass.  The second pass reads the strip
+// again from the cache and stores a column's 32-value slice from 16 lanes'
+// halves through LDS.
+__global__ __launch_bounds__(1024) void split_columns_kernel(const float *__restrict__ in, char *__restrict__ out,
+                                                             int *__restrict__ ex, int K, int N, int slices) {
+    const int c = threadIdx.x & 15, kr = threadIdx.x >> 4;  // column, row of the pass
+    const int n = blockIdx.x * 16 + c, nc = min(n, N - 1);
+    __shared__ uint32_t red[16][17];
+    __shared__ float tile[64][17];
+    uint32_t mx = 0;
+    for (int k = kr; k < K; k += 64) mx = max(mx, __float_as_uint(in[(size_t)k * N + nc]) & 0x7fffffffu);
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 16, 64));
+    mx = max(mx, (uint32_t)__shfl_xor((int)mx, 32, 64));
+    if ((threadIdx.x & 63) < 16) red[threadIdx.x >> 6][c] = mx;
+    __syncthreads();
+    // Store role: column sc of the strip, values 4 sk .. 4 sk + 3 of a pass.
+    const int sc = threadIdx.x >> 4, sk = threadIdx.x & 15;
+    int e = 0;
+    if (sc < 16) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) m = max(m, red[w][sc]);
+        e = split_exponent(m);
+        if (sk == 0 && blockIdx.x * 16 + sc < N) ex[blockIdx.x * 16 + sc] = e;
+    }
+    for (int k0 = 0; k0 < slices * 32; k0 += 64) {
+        __syncthreads();
+        tile[kr][c] = k0 + kr < K ? in[(size_t)(k0 + kr) * N + nc] : 0.0f;
+        __syncthreads();
+        const int sn = blockIdx.x * 16 + sc, k = k0 + 4 * sk;
+        if (sc < 16 && sn < N && k < slices * 32) {
+            f32x4 v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = e == kSplitNonFinite ? 0.0f : tile[4 * sk + r][sc];
+            store_split4(out + (size_t)sn * slices * 128, k, v, e);
+        }
+    }
+}
+
+// The tiles, and what a k-slice of one costs a CU in microseconds when the
+// tile has it alone (slope between K = 768 and K = 3072 at 865 rows on
+// MI355X) with the cost of a launch that does not depend on K.
+struct SplitTile {
+    int bm, bn;
+    float slice_us, fixed_us;
+};
+constexpr SplitTile kSplitTiles[] = {
+    {128, 256, 0.858f, 5.0f},  // 2 x 4 waves
+    {128, 128, 0.480f, 5.9f},  // 2 x 4 waves
+    {128, 96, 0.378f, 5.0f},   // 4 x 2 waves (not Qkv: waves 48 columns wide)
+    {64, 128, 0.286f, 3.9f},   // 2 x 4 waves, two workgroups per CU
+    {64, 64, 0.211f, 3.0f},    // 2 x 2 waves, two K groups
+    {64, 32, 0.125f, 3.7f},    // 2 x 1 waves, two K groups, two workgroups per CU
+};
+
+// The tile with the lowest predicted time: every CU runs ceil(tiles / 256)
+// tiles of slices * slice_us, and a tile that has the CU alone (more than
+// half the LDS) adds about 2 us of prologue and epilogue per further round.
+// Of the 13 shapes swept on MI355X the prediction names the fastest of
+// these tiles in all but one, which it misses by 2% (865 x 3072 x 768: 18.1
+// us here, 20.5 for 64 x 128, 23.9 for 64 x 64; 3460 x 2304 x 768: 41.5 for
+// 128 x 256, 45.9 for 64 x 128; 97 x 2304 x 768: 6.2 for 64 x 32, 10.3 for
+// 64 x 128).
+int pick_split_tile(size_t m, size_t n, int slices, bool qkv) {
+    int best = 0;
+    float best_us = 0.0f;
+    for (int i = 0; i < 6; i++) {
+        if (qkv && i == 2) continue;
+        const SplitTile &t = kSplitTiles[i];
+        const size_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+        const float rounds = (float)((tiles + 255) / 256);
+        const bool alone = i != 3 && i != 5;
+        const float us = t.fixed_us + rounds * slices * t.slice_us + (alone ? 2.0f * (rounds - 1.0f) : 0.0f);
+        if (i == 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
+template <int BM, int BN, int WM, int WN, int KG, SEpi EPI>
+hipError_t launch_split_tile(hipStream_t s, const SplitArgs &ar) {
+    constexpr int ST = 3;
+    constexpr size_t stage = (size_t)KG * ST * (BM + BN) * 128;
+    constexpr size_t xch = KG > 1 ? (size_t)KG * BM * BN * 4 : 0;
+    constexpr size_t lds = stage > xch ? stage : xch;
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    auto kernel = gemm_split_kernel<BM, BN, WM, WN, KG, ST, EPI>;
+    static std::atomic<uint64_t> configured{0};
+    if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
+    const size_t tiles = (size_t)((ar.M + BM - 1) / BM) * (size_t)((ar.N + BN - 1) / BN);
+    if (tiles > (size_t)INT32_MAX / (WM * WN * KG * 64)) return hipErrorInvalidValue;
+    kernel<<<(unsigned)tiles, WM * WN * KG * 64, lds, s>>>(ar);
+    return hipGetLastError();
+}
+
+template <SEpi EPI>
+hipError_t launch_split_epi(hipStream_t s, const SplitArgs &ar) {
+    switch (pick_split_tile(ar.M, ar.N, ar.slices, EPI == SEpi::Qkv)) {
+        case 0: return launch_split_tile<128, 256, 2, 4, 1, EPI>(s, ar);
+        case 1: return launch_split_tile<128, 128, 2, 4, 1, EPI>(s, ar);
+        case 2:
+            if constexpr (EPI != SEpi::Qkv) return launch_split_tile<128, 96, 4, 2, 1, EPI>(s, ar);
+            return hipErrorInvalidValue;
+        case 3: return launch_split_tile<64, 128, 2, 4, 1, EPI>(s, ar);
+        case 4: return launch_split_tile<64, 64, 2, 2, 2, EPI>(s, ar);
+        default: return launch_split_tile<64, 32, 2, 1, 2, EPI>(s, ar);
+    }
+}
+
+}  // namespace
+
+bool split_gemm_fits(size_t m, size_t n, size_t k) {
+    // Row offsets inside a 256-row tile stay below 2^31 bytes, and the
+    // smallest tiles' grid below the launch limit.
+    return k > 0 && k <= ((size_t)1 << 21) - 32 && m <= INT32_MAX && n <= INT32_MAX &&
+           ((m + 63) / 64) * ((n + 31) / 32) <= (size_t)INT32_MAX / 512;
+}
+
+hipError_t launch_split_rows(hipStream_t s, const float *in, void *out, int *ex, size_t rows, size_t k) {
+    if (rows == 0) return hipSuccess;
+    const size_t wpb = rows <= 2048 ? 1 : 4;
+    split_rows_kernel<<<(unsigned)((rows + wpb - 1) / wpb), (unsigned)(64 * wpb), 0, s>>>(
+        in, static_cast<char *>(out), ex, rows, (int)k, (int)((k + 31) / 32));
+    return hipGetLastError();
+}
+
+hipError_t launch_split_columns(hipStream_t s, const float *in, void *out, int *ex, size_t k, size_t n) {
+    if (n == 0) return hipSuccess;
+    split_columns_kernel<<<(unsigned)((n + 15) / 16), 1024, 0, s>>>(in, static_cast<char *>(out), ex, (int)k, (int)n,
+                                                                   (int)((k + 31) / 32));
+    return hipGetLastError();
+}
+
+hipError_t launch_layernorm_split(hipStream_t s, const float *in, const float *gamma, const float *beta, void *out,
+                                  int *ex, size_t rows, size_t cols, float eps) {
+    if (rows == 0) return hipSuccess;
+    if (cols % 32 != 0 || cols == 0 || cols > 1024) return hipErrorInvalidValue;
+    const size_t wpb = rows <= 2048 ? 1 : 4;
+    layernorm_split_kernel<<<(unsigned)((rows + wpb - 1) / wpb), (unsigned)(64 * wpb), 0, s>>>(
+        in, gamma, beta, static_cast<char *>(out), ex, rows, (int)cols, eps);
+    return hipGetLastError();
+}
+
+hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *gamma, const float *beta,
+                                  const float *bias, float *bound, size_t n, size_t k) {
+    if (n == 0) return hipSuccess;
+    ln_output_bound_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(w, gamma, beta, bias, bound, (int)n, (int)k);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g) {
+    if (g.m == 0 || g.n == 0) return hipSuccess;
+    if (!split_gemm_fits(g.m, g.n, g.k)) return hipErrorInvalidValue;
+    SplitArgs ar{};
+    ar.x = static_cast<const char *>(g.x);
+    ar.w = static_cast<const char *>(g.w);
+    ar.ex = g.ex;
+    ar.ex_c = g.ex_c;
+    ar.ew = g.ew;
+    ar.M = (int)g.m;
+    ar.N = (int)g.n;
+    ar.K = (int)g.k;
+    ar.slices = (int)((g.k + 31) / 32);
+    ar.xf = g.xf;
+    ar.wf = g.wf;
+    ar.wf_n = g.wf_columns ? (int)g.n : 0;
+    ar.c = g.c;
+    ar.bias = g.bias;
+    ar.gamma = g.gamma;
+    ar.q = g.q;
+    ar.k = g.k_out;
+    ar.v = g.v;
+    ar.tokens = (int)g.tokens;
+    ar.heads = (int)g.heads;
+    ar.rot = g.rot;
+    ar.out_split = static_cast<char *>(g.out_split);
+    ar.out_scale = g.out_split ? __builtin_ldexpf(1.0f, -g.out_ex) : 0.0f;
+    if (g.out_split) {
+        if (g.epi != Epi::Gelu || g.n % 32 != 0 || g.out_ex > 100 || g.out_ex < -100) return hipErrorInvalidValue;
+        return launch_split_epi<SEpi::GeluSplit>(s, ar);
+    }
+    if (g.chw) return g.epi == Epi::Store ? launch_split_epi<SEpi::Chw>(s, ar) : hipErrorInvalidValue;
+    switch (g.epi) {
+        case Epi::Store: return launch_split_epi<SEpi::Store>(s, ar);
+        case Epi::Gelu: return launch_split_epi<SEpi::Gelu>(s, ar);
+        case Epi::Residual: return launch_split_epi<SEpi::Residual>(s, ar);
+        case Epi::Qkv: return g.n == 3 * g.heads * 64 ? launch_split_epi<SEpi::Qkv>(s, ar) : hipErrorInvalidValue;
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace vh

@@ -195,6 +195,50 @@ constexpr size_t kTailTiles = 512;
 constexpr size_t kTailFloats = kTailTiles * 4 * 64 * 64;
 constexpr size_t kTailStatFloats = kTailTiles * 4 * 4 * 256;
 
+// ---- GEMM on split rows (k_split.hip) -------------------------------------------
+// Split rows (split_gemm.h): each float row as two halves per value and one
+// power-of-two exponent, rows * ceil(k / 32) * 128 bytes and one int per row.
+// Exponent of a row that holds an infinity or NaN: its halves are zeros and
+// the GEMM recomputes its products from the floats.
+constexpr int kSplitNonFinite = INT32_MIN / 4;
+// Shapes launch_gemm_split takes.
+bool split_gemm_fits(size_t m, size_t n, size_t k);
+constexpr size_t split_bytes(size_t rows, size_t k) { return rows * ((k + 31) / 32) * 128; }
+hipError_t launch_split_rows(hipStream_t s, const float *in, void *out, int *ex, size_t rows, size_t k);
+// Split rows [n][k] of the columns of in [k][n].
+hipError_t launch_split_columns(hipStream_t s, const float *in, void *out, int *ex, size_t k, size_t n);
+// LayerNorm of each row into split rows (cols % 32 == 0, cols <= 1024).
+hipError_t launch_layernorm_split(hipStream_t s, const float *in, const float *gamma, const float *beta,
+                                  void *out, int *ex, size_t rows, size_t cols, float eps);
+// bound[n] >= |LayerNorm(x) . w_n + bias_n| for every x (w [n][k]).
+hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *gamma, const float *beta,
+                                  const float *bias, float *bound, size_t n, size_t k);
+struct SplitGemm {
+    const void *x;          // split rows [m][k]
+    const int *ex;          // their exponents, or null: ex_c for all
+    int ex_c;
+    const void *w;          // split rows [n][k]
+    const int *ew;
+    // The float rows, read for rows that hold an inf or NaN (null: such
+    // products are NaN).
+    const float *xf, *wf;
+    bool wf_columns;        // wf is [k][n]
+    size_t m, n, k;
+    Epi epi;
+    bool chw;               // Store only: c is [n][m]
+    float *c;
+    const float *bias;      // [n] or null
+    const float *gamma;     // [n] or null (Store, Residual)
+    float *q, *k_out, *v;   // Qkv, as GemmArgs
+    size_t tokens, heads;
+    const float *rot;
+    // Gelu only: the output as split rows [m][n] (n % 32 == 0) with the one
+    // exponent out_ex instead of c; |output| <= 2^(15 + out_ex).
+    void *out_split;
+    int out_ex;
+};
+hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g);
+
 // ---- Q8_0 (k_q8.hip) --------------------------------------------------------
 // x [rows][k] -> block-major Q8_0: qs [k/32][rows][32] int8, d [k/32][rows] f16 bits
 hipError_t launch_quantize_q8_0(hipStream_t s, const float *x, int8_t *qs, uint16_t *d,

@@ -91,6 +91,8 @@ struct RtState {
     size_t fcnt_n = 0;
     char *aq = nullptr;                         // grow-only Q8_0 activation blocks
     size_t aq_bytes = 0;
+    char *sx = nullptr;                         // grow-only split rows of a projection's input
+    size_t sx_bytes = 0;
     float *tw = nullptr;                        // balanced-tail GEMM partials
     unsigned *tcnt = nullptr;                   // and arrival counters (zeroed once)
     float *scratch = nullptr;                   // this device's copy of `scratch` (below)
@@ -110,6 +112,7 @@ struct RtState {
         if (fw) hipFree(fw);
         if (fcnt) hipFree(fcnt);
         if (aq) hipFree(aq);
+        if (sx) hipFree(sx);
         if (tw) hipFree(tw);
         if (tcnt) hipFree(tcnt);
 
@@ -150,10 +153,17 @@ struct Lin {
     float *wt = nullptr;  // [N][K]
     float *bias = nullptr;
     float *gamma = nullptr;  // null = unit LayerScale
-    // Set for a projection that takes a LayerNorm of its input folded in
-    // (prepare_lin_ln): wt = W diag(ln gamma), bias = b + W . ln beta and
-    // ln_c[n] = sum_k wt[n][k].
-    float *ln_c = nullptr;
+    // Split rows of wt for the f16 matrix cores (split_gemm.h), or null where
+    // the fp32 kernel serves (split_k_fits) and for weights with an inf or NaN.
+    char *sw = nullptr;
+    int *sew = nullptr;
+    void release(hipStream_t s) {
+        for (float *p : {wt, bias, gamma})
+            if (p) hipFreeAsync(p, s);
+        if (sw) hipFreeAsync(sw, s);
+        if (sew) hipFreeAsync(sew, s);
+        *this = Lin{};
+    }
 };
 
 // A projection with Q8_0 weights: W^T [N][K] as block-major blocks,
@@ -181,8 +191,7 @@ struct vh_linear {
     ~vh_linear() {
         if (!rt) return;
         hipSetDevice(rt->device);
-        for (float *p : {L.wt, L.bias, L.gamma})
-            if (p) hipFreeAsync(p, rt->stream);
+        L.release(rt->stream);
     }
 };
 
@@ -212,6 +221,10 @@ struct vh_linear_q8 {
 struct vh_block {
     Rt rt;
     Lin qkv, proj, fc1, fc2;
+    // f32 blocks: all four projections hold split rows, and |GELU(fc1)| of
+    // every input is at most 2^(15 + fc1_ex) (the exponent of its split rows).
+    bool split = false;
+    int fc1_ex = 0;
     bool q8 = false;  // projections in Q8_0 (qqkv..qfc2) instead of f32
     Q8Lin qqkv, qproj, qfc1, qfc2;
     float *ln1_g = nullptr, *ln1_b = nullptr, *ln2_g = nullptr, *ln2_b = nullptr;
@@ -219,9 +232,7 @@ struct vh_block {
     ~vh_block() {
         if (!rt) return;
         hipSetDevice(rt->device);
-        for (Lin *l : {&qkv, &proj, &fc1, &fc2})
-            for (float *p : {l->wt, l->bias, l->gamma, l->ln_c})
-                if (p) hipFreeAsync(p, rt->stream);
+        for (Lin *l : {&qkv, &proj, &fc1, &fc2}) l->release(rt->stream);
         for (Q8Lin *l : {&qqkv, &qproj, &qfc1, &qfc2}) l->release(rt->stream);
         for (float *p : {ln1_g, ln1_b, ln2_g, ln2_b, qn_g, qn_b, kn_g, kn_b})
             if (p) hipFreeAsync(p, rt->stream);
@@ -454,6 +465,53 @@ vh_status flash(RtState &s, const float *q, const float *k, const float *v, floa
     });
 }
 
+// Products of fewer than kSplitMinK terms stay on the fp32 matrix instructions:
+// the split keeps 23 of a float's 24 significand bits, which shows where a
+// sum has few roundings of its own.  2-norm error against float64 at 1000 x
+// 2304, N(0, 1) operands, fp32 and split: K = 64 1.45e-7 and 0.95e-7, K = 256
+// 2.8e-7 and 1.3e-7, K = 768 4.8e-7 and 2.0e-7, K = 3072 9.9e-7 and 3.6e-7; the
+// representation alone costs 0.9e-7, which the fp32 ones pass at K = 32.
+constexpr size_t kSplitMinK = 64;
+bool split_k_fits(size_t m, size_t n, size_t k) { return k >= kSplitMinK && vh::split_gemm_fits(m, n, k); }
+// VESTRA_HIP_GEMM_TAIL and VESTRA_HIP_GEMM_KGROUP choose between forms of the
+// fp32 GEMM (A/B studies and tests, read per call): set, they ask for that
+// GEMM.
+bool fp32_gemm_asked() {
+    for (const char *name : {"VESTRA_HIP_GEMM_TAIL", "VESTRA_HIP_GEMM_KGROUP"}) {
+        const char *e = std::getenv(name);
+        if (e && *e) return true;
+    }
+    return false;
+}
+
+// Adds the split rows of L's weight (left out where split_k_fits says so or a
+// row holds an inf or NaN).
+vh_status split_weight(RtState &s, Lin *L) {
+    if (L->N == 0 || !split_k_fits(1, L->N, L->K)) return VH_OK;
+    vh_status st = dalloc(s, vh::split_bytes(L->N, L->K), &L->sw, "split weight allocation");
+    if (!st) st = dalloc(s, L->N, &L->sew, "split weight allocation");
+    if (!st)
+        st = launch(s, "split_weight", [&] {
+            return vh::launch_split_rows(s.stream, L->wt, L->sw, L->sew, L->N, L->K);
+        });
+    std::vector<int> ex(L->N);
+    if (!st) {
+        hipError_t e = hipMemcpyAsync(ex.data(), L->sew, L->N * sizeof(int), hipMemcpyDeviceToHost, s.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
+        if (e != hipSuccess) st = fail(VH_ERR_UPLOAD, hip_msg("split weight exponents", e));
+    }
+    if (st) return st;
+    for (int e : ex)
+        if (e == vh::kSplitNonFinite) {
+            hipFreeAsync(L->sw, s.stream);
+            hipFreeAsync(L->sew, s.stream);
+            L->sw = nullptr;
+            L->sew = nullptr;
+            break;
+        }
+    return VH_OK;
+}
+
 vh_status prepare_lin(RtState &s, size_t K, size_t N, const float *w, const float *bias,
                       const float *gamma, Lin *L) {
     float *tmp = nullptr;
@@ -466,9 +524,7 @@ vh_status prepare_lin(RtState &s, size_t K, size_t N, const float *w, const floa
     if (!st) st = upload_array(s, bias, N, &L->bias, "linear bias upload");
     if (!st && gamma) st = upload_array(s, gamma, N, &L->gamma, "linear gamma upload");
     if (st) {
-        for (float *p : {L->wt, L->bias, L->gamma})
-            if (p) hipFreeAsync(p, s.stream);
-        *L = Lin{};
+        L->release(s.stream);
         return st;
     }
     L->K = K;
@@ -476,60 +532,116 @@ vh_status prepare_lin(RtState &s, size_t K, size_t N, const float *w, const floa
     return VH_OK;
 }
 
-// A projection of LayerNorm(x) (gamma g, beta be) prepared for the folded
-// form LayerNorm(x) . W^T + b = rstd * (x . W'^T - mean * c) + b' (see
-// GemmArgs::ln_fold_c): W'[n][k] = W[k][n] * g[k] (w is [K][N], in x out),
-// c[n] = sum_k W'[n][k] and b'[n] = b[n] + sum_k W[k][n] * be[k], both sums in
-// double over the rounded W' and the given W.
-vh_status prepare_lin_ln(RtState &s, size_t K, size_t N, const float *w, const float *bias,
-                         const float *ln_g, const float *ln_b, Lin *L) {
-    if (!w || !bias || !ln_g || !ln_b) return null_arg("prepare_lin_ln");
-    std::vector<float> wt(K * N), c(N), bp(N);
-    for (size_t n = 0; n < N; n++) {
-        double cs = 0.0, bs = (double)bias[n];
-        for (size_t k = 0; k < K; k++) {
-            const float wv = w[k * N + n];
-            const float f = wv * ln_g[k];
-            wt[n * K + k] = f;
-            cs += (double)f;
-            bs += (double)wv * (double)ln_b[k];
+vh_status prepare_split_lin(RtState &s, size_t K, size_t N, const float *w, const float *bias,
+                            const float *gamma, Lin *L) {
+    TRY(prepare_lin(s, K, N, w, bias, gamma, L));
+    vh_status st = split_weight(s, L);
+    if (st) L->release(s.stream);
+    return st;
+}
+
+// The exponent e for which every |LayerNorm(x) . w_n + b_n| of the projection
+// is at most 2^(15 + e), for LayerNorm parameters g, be on the device; false
+// if there is none within the range of a split output.
+vh_status ln_output_exponent(RtState &s, const Lin &L, const float *g, const float *be, int *e, bool *ok) {
+    float *bound = nullptr;
+    TRY(dalloc(s, L.N, &bound, "bound allocation"));
+    vh_status st = launch(s, "ln_output_bound", [&] {
+        return vh::launch_ln_output_bound(s.stream, L.wt, g, be, L.bias, bound, L.N, L.K);
+    });
+    std::vector<float> h(L.N);
+    if (!st) {
+        hipError_t he = hipMemcpyAsync(h.data(), bound, L.N * sizeof(float), hipMemcpyDeviceToHost, s.stream);
+        if (he == hipSuccess) he = hipStreamSynchronize(s.stream);
+        if (he != hipSuccess) st = fail(VH_ERR_UPLOAD, hip_msg("bound download", he));
+    }
+    hipFreeAsync(bound, s.stream);
+    if (st) return st;
+    float mx = 0.0f;
+    *ok = true;
+    for (float v : h) {
+        if (!(v <= 1e30f)) *ok = false;  // NaN and overflow too
+        mx = std::max(mx, v);
+    }
+    *e = 0;
+    if (*ok && mx > 0.0f) {
+        int x = 0;
+        frexpf(mx * 1.01f, &x);  // the bound's own rounding; mx * 1.01 <= 2^x
+        *e = x - 15;
+    }
+    if (*e > 90 || *e < -90) *ok = false;
+    return VH_OK;
+}
+
+// Split rows of `in` [rows][k] in the runtime's workspace, or null pointers
+// where there is no memory for them (the caller then takes the fp32 kernel).
+struct SplitRows {
+    char *x = nullptr;
+    int *ex = nullptr;
+};
+vh_status split_input(RtState &s, const float *in, size_t rows, size_t k, SplitRows *out) {
+    const size_t bytes = vh::split_bytes(rows, k), need = bytes + rows * sizeof(int);
+    if (s.sx_bytes < need) {
+        hipStreamSynchronize(s.stream);
+        if (s.sx) hipFree(s.sx);
+        s.sx = nullptr;
+        s.sx_bytes = 0;
+        if (hipMalloc(&s.sx, need) != hipSuccess) {
+            hipGetLastError();
+            s.sx = nullptr;
+            return VH_OK;
         }
-        c[n] = (float)cs;
-        bp[n] = (float)bs;
+        s.sx_bytes = need;
     }
-    vh_status st = upload_array(s, wt.data(), K * N, &L->wt, "linear weight upload");
-    if (!st) st = upload_array(s, bp.data(), N, &L->bias, "linear bias upload");
-    if (!st) st = upload_array(s, c.data(), N, &L->ln_c, "linear LayerNorm fold upload");
-    if (st) {
-        for (float *p : {L->wt, L->bias, L->ln_c})
-            if (p) hipFreeAsync(p, s.stream);
-        *L = Lin{};
-        return st;
-    }
-    L->K = K;
-    L->N = N;
-    return VH_OK;
+    out->x = s.sx;
+    out->ex = reinterpret_cast<int *>(s.sx + bytes);
+    return launch(s, "split_rows", [&] { return vh::launch_split_rows(s.stream, in, out->x, out->ex, rows, k); });
 }
 
-// LayerNorm applied to the rows a Residual GEMM has just updated.
+// LayerNorm parameters of a normalised input.
 struct RowNorm {
     const float *gamma, *beta;
     float *out;
     float eps;
 };
 
-// Row statistics passed between a Residual GEMM and the LayerNorm-folded
-// GEMM after it: (mean, M2) per column chunk of each row (GemmArgs).
-struct ChunkStats {
-    const float *in = nullptr;     // the input rows' statistics, or null
-    size_t in_chunks = 0;          // chunks per row of in
-    float *out = nullptr;          // where a Residual GEMM writes them, or null
-    int *out_chunks = nullptr;     // chunks per row written to out (0: none)
-};
+// The operands of c = epilogue(in . W^T) that both matrix paths share.
+vh::SplitGemm split_gemm_args(const Lin &L, const float *in, size_t rows, vh::Epi epi, float *c) {
+    vh::SplitGemm g{};
+    g.w = L.sw;
+    g.ew = L.sew;
+    g.xf = in;
+    g.wf = L.wt;
+    g.m = rows;
+    g.n = L.N;
+    g.k = L.K;
+    g.epi = epi;
+    g.c = c;
+    g.bias = L.bias;
+    g.gamma = epi == vh::Epi::Store || epi == vh::Epi::Residual ? L.gamma : nullptr;
+    return g;
+}
+
+// Runs g on split rows of its float input g.xf where L holds split weights;
+// *done is false where the fp32 kernel has to run instead.
+vh_status try_split(RtState &s, const Lin &L, vh::SplitGemm g, const char *name, bool *done) {
+    *done = false;
+    if (!L.sw || g.m == 0 || !split_k_fits(g.m, g.n, g.k) || fp32_gemm_asked()) return VH_OK;
+    SplitRows x;
+    TRY(split_input(s, g.xf, g.m, g.k, &x));
+    if (!x.x) return VH_OK;
+    g.x = x.x;
+    g.ex = x.ex;
+    *done = true;
+    return launch(s, name, [&] { return vh::launch_gemm_split(s.stream, g); });
+}
 
 vh_status run_lin(RtState &s, const Lin &L, const float *in, size_t rows, vh::Epi epi, float *c,
-                  const char *name, const RowNorm *norm = nullptr, float fold_eps = 0.0f,
-                  const ChunkStats &cs = ChunkStats{}) {
+                  const char *name) {
+    const vh::SplitGemm sg = split_gemm_args(L, in, rows, epi, c);
+    bool done = false;
+    TRY(try_split(s, L, sg, name, &done));
+    if (done) return VH_OK;
     vh::GemmArgs g{};
     g.a = in;
     g.bt = L.wt;
@@ -539,41 +651,29 @@ vh_status run_lin(RtState &s, const Lin &L, const float *in, size_t rows, vh::Ep
     g.epi = epi;
     g.c = c;
     g.bias = L.bias;
-    g.gamma = epi == vh::Epi::Gelu ? nullptr : L.gamma;
-    if (norm) {
-        g.ln_gamma = norm->gamma;
-        g.ln_beta = norm->beta;
-        g.ln_out = norm->out;
-        g.ln_eps = norm->eps;
-    }
-    g.ln_fold_c = L.ln_c;
-    g.ln_fold_eps = fold_eps;
-    if (cs.in && cs.in_chunks) {
-        g.stats_in = cs.in;
-        g.stats_in_chunks = cs.in_chunks;
-    }
-    if (cs.out) {
-        g.stats_out = cs.out;
-        g.stats_out_chunks = cs.out_chunks;
-    }
+    g.gamma = sg.gamma;
     TRY(splitk_workspace(s, rows, L.N, &g.ws, &g.ws_floats));
     TRY(tail_workspace(s, g));
     return launch(s, name, [&] { return vh::launch_gemm(s.stream, g); });
 }
 
 vh_status run_qkv(RtState &s, const Lin &L, const float *in, size_t images, size_t tokens,
-                  size_t heads, const float *rot, float *q, float *k, float *v, float fold_eps = 0.0f,
-                  const float *stats_in = nullptr, size_t stats_in_chunks = 0) {
+                  size_t heads, const float *rot, float *q, float *k, float *v) {
+    const size_t rows = images * tokens;
+    vh::SplitGemm sg = split_gemm_args(L, in, rows, vh::Epi::Qkv, nullptr);
+    sg.q = q;
+    sg.k_out = k;
+    sg.v = v;
+    sg.tokens = tokens;
+    sg.heads = heads;
+    sg.rot = rot;
+    bool done = false;
+    TRY(try_split(s, L, sg, "gemm_qkv_rope", &done));
+    if (done) return VH_OK;
     vh::GemmArgs g{};
-    g.ln_fold_c = L.ln_c;
-    g.ln_fold_eps = fold_eps;
-    if (stats_in && stats_in_chunks) {
-        g.stats_in = stats_in;
-        g.stats_in_chunks = stats_in_chunks;
-    }
     g.a = in;
     g.bt = L.wt;
-    g.m = images * tokens;
+    g.m = rows;
     g.n = L.N;
     g.k = L.K;
     g.epi = vh::Epi::Qkv;
@@ -985,6 +1085,42 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
     TRY(set_device(s));
     vh_tensor *t = nullptr;
     TRY(new_tensor(rt->s, mn, &t, "GEMM output allocation"));
+    // Split rows of A and of B's columns, then the f16 matrix cores.
+    if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked()) {
+        char *w = nullptr;
+        int *ew = nullptr;
+        SplitRows x;
+        vh_status st = split_input(s, a->ptr, m, k, &x);
+        const size_t wbytes = vh::split_bytes(n, k);
+        if (!st && x.x) st = dalloc(s, wbytes + n * sizeof(int), &w, "GEMM operand allocation");
+        if (!st && x.x) {
+            ew = reinterpret_cast<int *>(w + wbytes);
+            st = launch(s, "split_columns", [&] { return vh::launch_split_columns(s.stream, b->ptr, w, ew, k, n); });
+            vh::SplitGemm g{};
+            g.x = x.x;
+            g.ex = x.ex;
+            g.w = w;
+            g.ew = ew;
+            g.xf = a->ptr;
+            g.wf = b->ptr;
+            g.wf_columns = true;
+            g.m = m;
+            g.n = n;
+            g.k = k;
+            g.epi = vh::Epi::Store;
+            g.c = t->ptr;
+            if (!st) st = launch(s, "gemm", [&] { return vh::launch_gemm_split(s.stream, g); });
+        }
+        if (w) hipFreeAsync(w, s.stream);
+        if (st) {
+            delete t;
+            return st;
+        }
+        if (x.x) {
+            *out = t;
+            return VH_OK;
+        }
+    }
     // B read in place, K-major: the direct convolution's loader as a 1 x 1
     // tap over a one-row "image" of n pixels and k channels, whose
     // channel-major output is row-major C; no transposed copy of B.  Its
@@ -1519,7 +1655,7 @@ extern "C" vh_status vh_prepare_linear_f32(const vh_runtime *rt, size_t input_fe
     TRY(set_device(s));
     vh_linear *l = new vh_linear;
     l->rt = rt->s;
-    vh_status st = prepare_lin(s, input_features, output_features, weight, bias, gamma, &l->L);
+    vh_status st = prepare_split_lin(s, input_features, output_features, weight, bias, gamma, &l->L);
     if (st) {
         delete l;
         return st;
@@ -1579,7 +1715,15 @@ extern "C" vh_status vh_linear_run_chw(const vh_linear *linear, const vh_tensor 
     const Lin &L = linear->L;
     vh_tensor *t = nullptr;
     vh_status st = new_tensor(linear->rt, len, &t, "DPT CHW allocation");
-    if (!st && !L.gamma && !L.ln_c && L.K % 32 == 0 && rows <= (size_t)INT32_MAX) {
+    // Channel-major stores of the split product: no token-major copy.
+    bool done = false;
+    if (!st) {
+        vh::SplitGemm sg = split_gemm_args(L, input->ptr, rows, vh::Epi::Store, t->ptr);
+        sg.chw = true;
+        st = try_split(s, L, sg, "gemm_bias_chw", &done);
+    }
+    if (done) {
+    } else if (!st && !L.gamma && L.K % 32 == 0 && rows <= (size_t)INT32_MAX) {
         // The transposed product in one GEMM: the weight rows [N][K] as A and
         // the input rows as Bt, stored channel-major with the bias per
         // channel by the implicit convolution's epilogue (a 1 x 1 tap over
@@ -2030,20 +2174,16 @@ vh_status upload_small(RtState &s, const float *h, size_t n, float **out, const 
     return upload_array(s, h, n, out, what);
 }
 
-// One pre-norm block, in place on x.  x_chunks (encoder runs): on entry,
-// the chunks per row of x's row statistics in the block workspace (the
-// previous f32 block's fc2 wrote them; 0: none); on return, those this
-// block's fc2 wrote.
+// One pre-norm block, in place on x.
 vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size_t tokens,
-                    const int64_t *pos, float freq, float eps, int *x_chunks = nullptr) {
+                    const int64_t *pos, float freq, float eps) {
     const size_t M = images * tokens;
     const size_t D = kDim;
     float *ws = nullptr;
-    TRY(workspace(s, M * (4 * D + kMlp + 2 * (D / 16)), &ws));
+    TRY(workspace(s, M * (5 * D + kMlp + 1), &ws));
     float *q = ws, *k = q + M * D, *v = k + M * D, *att = v + M * D, *f = att + M * D;
-    float *rs = f + M * kMlp;  // row statistics [M][chunks <= D / 16][mean, M2]
-    const int in_chunks = x_chunks ? *x_chunks : 0;
-    if (x_chunks) *x_chunks = 0;
+    float *h = f + M * kMlp;  // a projection's input: LayerNorm rows, as floats or split rows
+    int *hex = reinterpret_cast<int *>(h + M * D);  // the split rows' exponents
     const float *rot = nullptr;
     if (pos) {
         TRY(rope_table(s, pos, tokens, 64, freq, &rot));
@@ -2102,32 +2242,73 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
                                         vh::Epi::Residual, b.qfc2.bias, b.qfc2.gamma);
         });
     }
-    // f32 projections: LayerNorm 1 and 2 are folded into the QKV and fc1
-    // GEMMs (prepare_lin_ln), which read the residual stream x itself and
-    // take its row statistics from the Residual GEMM before them when that
-    // one wrote them (the out-projection for fc1, the previous block's fc2
-    // for QKV), else from their own A slices.
-    const float *qkv_stats = in_chunks ? rs : nullptr;
-    if (b.qn_g) {
-        // Late block: QKV with bias only, then LayerNorm of every 64-wide Q
-        // and K head row fused with the RoPE (src/specialized.rs:278-316).
-        TRY(run_qkv(s, b.qkv, x, images, tokens, kHeads, nullptr, q, k, v, eps, qkv_stats, in_chunks));
+    if (!b.split) {
+        // Weights with an inf or NaN: the fp32 matrix instructions.
+        auto norm = [&](const float *g, const float *be) {
+            return launch(s, "layernorm", [&] { return vh::launch_layernorm(s.stream, x, g, be, h, M, D, eps); });
+        };
+        TRY(norm(b.ln1_g, b.ln1_b));
+        TRY(run_qkv(s, b.qkv, h, images, tokens, kHeads, b.qn_g ? nullptr : rot, q, k, v));
+        if (b.qn_g)
+            TRY(launch(s, "qk_norm_rope", [&] {
+                return vh::launch_qk_norm_rope(s.stream, q, k, b.qn_g, b.qn_b, b.kn_g, b.kn_b, rot,
+                                               M * kHeads, tokens, eps);
+            }));
+        TRY(flash(s, q, k, v, att, images * kHeads, tokens, kHeads, true));
+        TRY(run_lin(s, b.proj, att, M, vh::Epi::Residual, x, "gemm_proj_residual"));
+        TRY(norm(b.ln2_g, b.ln2_b));
+        TRY(run_lin(s, b.fc1, h, M, vh::Epi::Gelu, f, "gemm_fc1_gelu"));
+        return run_lin(s, b.fc2, f, M, vh::Epi::Residual, x, "gemm_fc2_residual");
+    }
+    // Split projections: each GEMM takes split rows, so the LayerNorms and
+    // fc1's GELU write them directly (fc1's with the exponent that bounds
+    // every input, block_prepare).
+    auto norm = [&](const float *g, const float *be) {
+        return launch(s, "layernorm_split", [&] {
+            return vh::launch_layernorm_split(s.stream, x, g, be, h, hex, M, D, eps);
+        });
+    };
+    TRY(norm(b.ln1_g, b.ln1_b));
+    {
+        vh::SplitGemm g = split_gemm_args(b.qkv, nullptr, M, vh::Epi::Qkv, nullptr);
+        g.x = h;
+        g.ex = hex;
+        g.q = q;
+        g.k_out = k;
+        g.v = v;
+        g.tokens = tokens;
+        g.heads = kHeads;
+        g.rot = b.qn_g ? nullptr : rot;
+        TRY(launch(s, "gemm_qkv_rope", [&] { return vh::launch_gemm_split(s.stream, g); }));
+    }
+    if (b.qn_g)
+        // Late block: LayerNorm of every 64-wide Q and K head row fused with
+        // the RoPE (src/specialized.rs:278-316).
         TRY(launch(s, "qk_norm_rope", [&] {
             return vh::launch_qk_norm_rope(s.stream, q, k, b.qn_g, b.qn_b, b.kn_g, b.kn_b, rot,
                                            M * kHeads, tokens, eps);
         }));
-    } else {
-        TRY(run_qkv(s, b.qkv, x, images, tokens, kHeads, rot, q, k, v, eps, qkv_stats, in_chunks));
-    }
     TRY(flash(s, q, k, v, att, images * kHeads, tokens, kHeads, true));
-    int proj_chunks = 0;
-    TRY(run_lin(s, b.proj, att, M, vh::Epi::Residual, x, "gemm_proj_residual", nullptr, 0.0f,
-                ChunkStats{nullptr, 0, rs, &proj_chunks}));
-    TRY(run_lin(s, b.fc1, x, M, vh::Epi::Gelu, f, "gemm_fc1_gelu", nullptr, eps,
-                ChunkStats{proj_chunks ? rs : nullptr, (size_t)proj_chunks, nullptr, nullptr}));
-    if (!x_chunks) return run_lin(s, b.fc2, f, M, vh::Epi::Residual, x, "gemm_fc2_residual");
-    return run_lin(s, b.fc2, f, M, vh::Epi::Residual, x, "gemm_fc2_residual", nullptr, 0.0f,
-                   ChunkStats{nullptr, 0, rs, x_chunks});
+    TRY(launch(s, "split_rows", [&] { return vh::launch_split_rows(s.stream, att, h, hex, M, D); }));
+    {
+        vh::SplitGemm g = split_gemm_args(b.proj, att, M, vh::Epi::Residual, x);
+        g.x = h;
+        g.ex = hex;
+        TRY(launch(s, "gemm_proj_residual", [&] { return vh::launch_gemm_split(s.stream, g); }));
+    }
+    TRY(norm(b.ln2_g, b.ln2_b));
+    {
+        vh::SplitGemm g = split_gemm_args(b.fc1, nullptr, M, vh::Epi::Gelu, nullptr);
+        g.x = h;
+        g.ex = hex;
+        g.out_split = f;
+        g.out_ex = b.fc1_ex;
+        TRY(launch(s, "gemm_fc1_gelu", [&] { return vh::launch_gemm_split(s.stream, g); }));
+    }
+    vh::SplitGemm g = split_gemm_args(b.fc2, nullptr, M, vh::Epi::Residual, x);
+    g.x = f;
+    g.ex_c = b.fc1_ex;
+    return launch(s, "gemm_fc2_residual", [&] { return vh::launch_gemm_split(s.stream, g); });
 }
 
 vh_status check_block_x(const vh_tensor *x, size_t images, size_t tokens) {
@@ -2167,15 +2348,25 @@ static vh_status block_prepare(const vh_runtime *rt, const vh_block_params *p, b
         if (!st) st = prepare_q8_from_f32(s, kDim, kMlp, p->w_fc1, p->b_fc1, nullptr, &b->qfc1);
         if (!st) st = prepare_q8_from_f32(s, kMlp, kDim, p->w_fc2, p->b_fc2, p->ls2, &b->qfc2);
     } else {
-        st = prepare_lin_ln(s, kDim, 3 * kDim, p->w_qkv, p->b_qkv, p->ln1_gamma, p->ln1_beta, &b->qkv);
-        if (!st) st = prepare_lin(s, kDim, kDim, p->w_proj, p->b_proj, p->ls1, &b->proj);
-        if (!st) st = prepare_lin_ln(s, kDim, kMlp, p->w_fc1, p->b_fc1, p->ln2_gamma, p->ln2_beta, &b->fc1);
-        if (!st) st = prepare_lin(s, kMlp, kDim, p->w_fc2, p->b_fc2, p->ls2, &b->fc2);
+        st = prepare_split_lin(s, kDim, 3 * kDim, p->w_qkv, p->b_qkv, nullptr, &b->qkv);
+        if (!st) st = prepare_split_lin(s, kDim, kDim, p->w_proj, p->b_proj, p->ls1, &b->proj);
+        if (!st) st = prepare_split_lin(s, kDim, kMlp, p->w_fc1, p->b_fc1, nullptr, &b->fc1);
+        if (!st) st = prepare_split_lin(s, kMlp, kDim, p->w_fc2, p->b_fc2, p->ls2, &b->fc2);
     }
     if (!st) st = upload_small(s, p->ln1_gamma, kDim, &b->ln1_g, "ln1 gamma");
     if (!st) st = upload_small(s, p->ln1_beta, kDim, &b->ln1_b, "ln1 beta");
     if (!st) st = upload_small(s, p->ln2_gamma, kDim, &b->ln2_g, "ln2 gamma");
     if (!st) st = upload_small(s, p->ln2_beta, kDim, &b->ln2_b, "ln2 beta");
+    if (!st && !q8) {
+        bool ok = false;
+        st = ln_output_exponent(s, b->fc1, b->ln2_g, b->ln2_b, &b->fc1_ex, &ok);
+        b->split = ok && b->qkv.sw && b->proj.sw && b->fc1.sw && b->fc2.sw;
+        if (b->split)
+            for (Lin *l : {&b->qkv, &b->fc1, &b->fc2}) {  // their inputs hold no inf without a NaN
+                hipFreeAsync(l->wt, s.stream);
+                l->wt = nullptr;
+            }
+    }
     if (qk_norm) {
         if (!st) st = upload_small(s, p->q_norm_gamma, 64, &b->qn_g, "q norm gamma");
         if (!st) st = upload_small(s, p->q_norm_beta, 64, &b->qn_b, "q norm beta");
@@ -2233,14 +2424,8 @@ extern "C" vh_status vh_encoder_run(const vh_runtime *rt, const vh_block *const 
     RtState &s = *rt->s;
     TRY(set_device(s));
     if (images * tokens == 0) return VH_OK;
-    // Each f32 block's fc2 leaves the row statistics of its output for the
-    // next block's QKV (a Q8_0 block normalises its own input).
-    int x_chunks = 0;
-    for (size_t i = 0; i < layers; i++) {
-        if (blocks[i]->q8) x_chunks = 0;
-        TRY(block_run(s, *blocks[i], x->ptr, images, tokens, pos_yx, rope_frequency, epsilon,
-                      blocks[i]->q8 ? nullptr : &x_chunks));
-    }
+    for (size_t i = 0; i < layers; i++)
+        TRY(block_run(s, *blocks[i], x->ptr, images, tokens, pos_yx, rope_frequency, epsilon));
     return VH_OK;
     GUARD_END
 }
