@@ -94,3 +94,58 @@ def test_split_gemm_inf_and_nan(rt, where):
         assert np.array_equal(np.isnan(got), np.isnan(ref))
         assert np.array_equal(got[~fine & ~np.isnan(ref)], ref[~fine & ~np.isnan(ref)].astype(np.float32))
         assert np.all(np.abs(got[fine] - clean[fine]) <= 2 * bound[fine])
+
+
+def _attention64(q, k, v):
+    s = q.astype(np.float64) @ k.astype(np.float64).transpose(0, 2, 1) / np.sqrt(q.shape[2])
+    p = np.exp(s - s.max(-1, keepdims=True))
+    return (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
+
+
+# One key, one panel and one more (32 keys), one step and one more (128), the
+# second and third step, the one-launch split's last length (1024) and the
+# first past it, head dims that fill no granule; scores up to 3 x the usual.
+@pytest.mark.parametrize("heads, tokens, hd, scale", [
+    (1, 1, 64, 1.0), (3, 32, 64, 1.0), (2, 33, 64, 1.0), (13, 128, 64, 1.0), (2, 129, 64, 3.0), (1, 257, 40, 1.0),
+    (2, 385, 7, 1.0), (1, 1024, 64, 3.0), (1, 1025, 64, 1.0), (5, 1700, 33, 1.0)])
+def test_split_attention_vs_float64(rt, heads, tokens, hd, scale):
+    """Relative to the largest |v| of the head: each weight p is off by the
+    rounding of its exponent (2^-24 of up to 32, twice), the exponential (2^-23)
+    and the score (2^-21 of sum |q k| / sqrt(hd), as a projection's), and the
+    average of V by 2^-21 and one addition per eight keys in each stream."""
+    n = heads * tokens * hd
+    q, k, v = (seeded.normal(s + tokens, n).reshape(heads, tokens, hd) for s in (9900, 9910, 9920))
+    q = q * np.float32(scale)
+    q[0, 0] *= np.float32(1e-3)
+    exp = _attention64(q, k, v)
+    t = [rt.upload_f32(a) for a in (q, k, v)]
+    score = 2.0 ** -21 * (np.abs(q).astype(np.float64) @ np.abs(k).transpose(0, 2, 1)).max() / np.sqrt(hd)
+    tol = (2 * (score + 2.0 ** -18 + 2.0 ** -23) + 2.0 ** -21 + tokens / 32 * 2.0 ** -23) * np.abs(v).max()
+    got = rt.download_f32(rt.attention_online_f32(*t, heads, tokens, hd)).reshape(exp.shape)
+    assert np.abs(got - exp).max() <= tol
+    if hd == 64:
+        tm = rt.download_f32(rt.flash_attention_f32_da3_base(*t, heads, tokens, True))
+        assert np.array_equal(tm.reshape(tokens, heads, hd).transpose(1, 0, 2), got)
+
+
+def test_split_attention_head_scales_and_non_finite(rt):
+    """Heads of different magnitude, and heads with a NaN or an infinity,
+    which fall back to floats: the NaN reaches what the float attention lets
+    it reach, and no other head."""
+    H, T, hd = 5, 70, 64
+    q, k, v = (seeded.normal(s, H * T * hd).reshape(H, T, hd) for s in (9930, 9940, 9950))
+    k[1] *= np.float32(1e-20)
+    v[1] *= np.float32(1e20)
+    q[2] *= np.float32(1e-38)
+    clean = _attention64(q, k, v)
+    q[3, 5, 7] = np.nan           # one query
+    v[4, 9, 3] = np.inf           # one output column
+    got = rt.download_f32(rt.attention_online_f32(*(rt.upload_f32(a) for a in (q, k, v)), H, T, hd)).reshape(H, T, hd)
+    vmax = np.abs(v[:3]).max(axis=(1, 2))[:, None, None]
+    assert np.all(np.abs(got[:3] - clean[:3]) <= 2e-5 * vmax)
+    assert np.isnan(got[3, 5]).all()
+    rest = np.delete(np.arange(T), 5)
+    assert np.abs(got[3, rest] - clean[3, rest]).max() <= 2e-5 * 5
+    assert np.isposinf(got[4, :, 3]).all()
+    cols = np.delete(np.arange(hd), 3)
+    assert np.abs(got[4][:, cols] - clean[4][:, cols]).max() <= 2e-5 * 5

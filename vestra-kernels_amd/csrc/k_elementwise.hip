@@ -8,6 +8,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "split_gemm.h"
 
 namespace vh {
 
@@ -356,10 +357,13 @@ __global__ __launch_bounds__(256) void rope2d_hd64_kernel(float *__restrict__ x,
 // qk_norm_rope (src/specialized.rs:412-454): 16 lanes per 64-wide row, lane j
 // holds dims 4j..4j+3; the rotation partner (dim + 16) lives in lane j ^ 4.
 // LayerNorm sums use a 16-lane tree (tolerance-checked against the CPU order).
+// SPLIT: the row is written back as its split row, times q_scale or k_scale
+// (the 16 lanes of a row have all read it by then).
+template <bool SPLIT>
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
     float *__restrict__ q, float *__restrict__ k, const float *__restrict__ qg,
     const float *__restrict__ qb, const float *__restrict__ kg, const float *__restrict__ kb,
-    const float *__restrict__ rot, size_t rows, size_t tokens, float eps) {
+    const float *__restrict__ rot, size_t rows, size_t tokens, float eps, float q_scale, float k_scale) {
     size_t gid = (size_t)blockIdx.x * 16 + (threadIdx.x >> 4);  // row over [q rows | k rows]
     const int j = threadIdx.x & 15;
     bool valid = gid < 2 * rows;
@@ -403,7 +407,22 @@ __global__ __launch_bounds__(256) void qk_norm_rope_kernel(
         outv[c] = first ? sub_rn(mul_rn(mine, cs), mul_rn(part, sn))
                         : add_rn(mul_rn(mine, cs), mul_rn(part, sn));
     }
-    reinterpret_cast<f32x4 *>(data)[j] = outv;
+    if constexpr (SPLIT) {
+        const float scale = gid < rows ? q_scale : k_scale;
+        f16x4 hi, lo;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            _Float16 a, b;
+            split_f16(outv[c] * scale, a, b);
+            hi[c] = a;
+            lo[c] = b;
+        }
+        char *p = reinterpret_cast<char *>(data) + axis * 128 + (j & 7) * 8;
+        *reinterpret_cast<f16x4 *>(p) = hi;
+        *reinterpret_cast<f16x4 *>(p + 64) = lo;
+    } else {
+        reinterpret_cast<f32x4 *>(data)[j] = outv;
+    }
 }
 
 // Rotation table from device positions (f32 [tokens][2]) with the device
@@ -573,8 +592,20 @@ hipError_t launch_qk_norm_rope(hipStream_t s, float *q, float *k, const float *q
                                const float *rot, size_t rows, size_t tokens, float eps) {
     if (rows == 0) return hipSuccess;
     size_t blocks = (2 * rows + 15) / 16;
-    qk_norm_rope_kernel<<<(unsigned)blocks, 256, 0, s>>>(q, k, qg, qb, kg, kb, rot, rows, tokens,
-                                                         eps);
+    qk_norm_rope_kernel<false><<<(unsigned)blocks, 256, 0, s>>>(q, k, qg, qb, kg, kb, rot, rows,
+                                                                tokens, eps, 0.0f, 0.0f);
+    return hipGetLastError();
+}
+
+hipError_t launch_qk_norm_rope_split(hipStream_t s, float *q, float *k, const float *qg,
+                                     const float *qb, const float *kg, const float *kb,
+                                     const float *rot, size_t rows, size_t tokens, float eps, int eq,
+                                     int ek) {
+    if (rows == 0) return hipSuccess;
+    size_t blocks = (2 * rows + 15) / 16;
+    qk_norm_rope_kernel<true><<<(unsigned)blocks, 256, 0, s>>>(
+        q, k, qg, qb, kg, kb, rot, rows, tokens, eps, __builtin_ldexpf(1.0f, -eq),
+        __builtin_ldexpf(1.0f, -ek));
     return hipGetLastError();
 }
 

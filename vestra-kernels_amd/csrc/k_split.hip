@@ -44,6 +44,7 @@ struct SplitArgs {
     float *c;
     const float *bias, *gamma;
     float *q, *k, *v;
+    float qkv_scale[3];     // Qkv: 0 for floats, or split rows of the values times this
     int tokens, heads;
     const float *rot;
     char *out_split;        // GeluSplit: split rows [M][N] of the output times out_scale
@@ -292,10 +293,12 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     // Qkv: the wave's columns lie in one head of one of Q, K, V.
     const int colw = n0 + wn * TN;
     float *head_dst = nullptr;
+    float head_scale = 0.0f;
     bool rope = false;
     if constexpr (EPI == SEpi::Qkv) {
         const int per = ar.heads * 64, group = colw / per;
         head_dst = group == 0 ? ar.q : (group == 1 ? ar.k : ar.v);
+        head_scale = group == 0 ? ar.qkv_scale[0] : (group == 1 ? ar.qkv_scale[1] : ar.qkv_scale[2]);
         rope = ar.rot != nullptr && group < 2;
     }
 #pragma unroll
@@ -342,7 +345,26 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
                         v[jp + 1][r] = add_rn(mul_rn(b, cs), mul_rn(a, sn));
                     }
                 }
-                float *dst = head_dst + (((size_t)img * ar.heads + head) * ar.tokens + tok) * 64 + d0 + 4 * lh;
+                float *row = head_dst + (((size_t)img * ar.heads + head) * ar.tokens + tok) * 64;
+                if (head_scale != 0.0f) {
+                    // Split row of 256 bytes: slice d0 / 32, hi then lo.
+                    char *sd = reinterpret_cast<char *>(row) + d0 * 4 + lh * 8;
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        f16x4 hi, lo;
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            _Float16 a, b;
+                            split_f16(v[jp + h][r] * head_scale, a, b);
+                            hi[r] = a;
+                            lo[r] = b;
+                        }
+                        *reinterpret_cast<f16x4 *>(sd + 32 * h) = hi;
+                        *reinterpret_cast<f16x4 *>(sd + 32 * h + 64) = lo;
+                    }
+                    continue;
+                }
+                float *dst = row + d0 + 4 * lh;
                 *reinterpret_cast<f32x4 *>(dst) = f32x4{v[jp][0], v[jp][1], v[jp][2], v[jp][3]};
                 *reinterpret_cast<f32x4 *>(dst + 16) =
                     f32x4{v[jp + 1][0], v[jp + 1][1], v[jp + 1][2], v[jp + 1][3]};
@@ -412,12 +434,6 @@ __device__ __forceinline__ void store_split4(char *row, int k, f32x4 v, int e) {
     char *p = row + (k / 32) * 128 + (k % 32) * 2;
     *reinterpret_cast<f16x4 *>(p) = hi;
     *reinterpret_cast<f16x4 *>(p + 64) = lo;
-}
-
-__device__ __forceinline__ uint32_t absmax4(uint32_t mx, f32x4 v) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) mx = max(mx, __float_as_uint(v[r]) & 0x7fffffffu);
-    return mx;
 }
 
 __global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict__ in, char *__restrict__ out,
@@ -709,6 +725,8 @@ hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g) {
     ar.tokens = (int)g.tokens;
     ar.heads = (int)g.heads;
     ar.rot = g.rot;
+    for (int i = 0; i < 3; i++)
+        ar.qkv_scale[i] = g.qkv_split[i] ? __builtin_ldexpf(1.0f, -g.qkv_ex[i]) : 0.0f;
     ar.out_split = static_cast<char *>(g.out_split);
     ar.out_scale = g.out_split ? __builtin_ldexpf(1.0f, -g.out_ex) : 0.0f;
     if (g.out_split) {

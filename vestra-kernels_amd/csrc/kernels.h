@@ -37,6 +37,12 @@ hipError_t launch_rope2d(hipStream_t s, float *x, size_t heads, size_t n, size_t
 hipError_t launch_qk_norm_rope(hipStream_t s, float *q, float *k, const float *qg,
                                const float *qb, const float *kg, const float *kb,
                                const float *rot, size_t rows, size_t tokens, float eps);
+// The same, each row replaced by its split row of 256 bytes (split_gemm.h) with
+// the exponents eq and ek.
+hipError_t launch_qk_norm_rope_split(hipStream_t s, float *q, float *k, const float *qg,
+                                     const float *qb, const float *kg, const float *kb,
+                                     const float *rot, size_t rows, size_t tokens, float eps, int eq,
+                                     int ek);
 // Table for qk_norm_rope from device f32 positions [tokens][2].
 hipError_t launch_rope_table_device(hipStream_t s, const float *pos, size_t tokens, float freq,
                                     float *rot);
@@ -230,6 +236,10 @@ struct SplitGemm {
     const float *bias;      // [n] or null
     const float *gamma;     // [n] or null (Store, Residual)
     float *q, *k_out, *v;   // Qkv, as GemmArgs
+    // Qkv: write this one as split rows [img][head][token][64] of exponent
+    // qkv_ex (|value| <= 2^(15 + qkv_ex)) instead of floats.
+    bool qkv_split[3];
+    int qkv_ex[3];
     size_t tokens, heads;
     const float *rot;
     // Gelu only: the output as split rows [m][n] (n % 32 == 0) with the one
@@ -238,6 +248,26 @@ struct SplitGemm {
     int out_ex;
 };
 hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g);
+
+// ---- attention on split rows (k_attn_split.hip) ---------------------------------
+bool attn_split_fits(size_t bh, size_t tokens);
+// Workspace of launch_attn_split_f32.
+size_t attn_split_bytes(size_t bh, size_t tokens);
+// q/k/v [bh][tokens][hd] f32, hd <= 64; out head-major, or token-major
+// [img][tokens][heads * hd].
+hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, const float *v, float *out,
+                                 size_t bh, size_t tokens, size_t heads, size_t hd, bool token_major,
+                                 float softmax_scale, void *ws);
+// Q, K and V as split rows [bh][tokens][64] with one exponent each (finite
+// or NaN values), head_dim 64, scale 1/8; out_split: split rows
+// [img * tokens][heads * 64] with exponent ev (an output is an average of V
+// rows, so V's exponent bounds it).
+struct SplitQkv {
+    void *q, *k, *v;
+    int eq, ek, ev;
+};
+hipError_t launch_attn_split(hipStream_t s, const SplitQkv &p, void *out_split, size_t bh, size_t tokens,
+                             size_t heads);
 
 // ---- Q8_0 (k_q8.hip) --------------------------------------------------------
 // x [rows][k] -> block-major Q8_0: qs [k/32][rows][32] int8, d [k/32][rows] f16 bits

@@ -221,10 +221,11 @@ struct vh_linear_q8 {
 struct vh_block {
     Rt rt;
     Lin qkv, proj, fc1, fc2;
-    // f32 blocks: all four projections hold split rows, and |GELU(fc1)| of
-    // every input is at most 2^(15 + fc1_ex) (the exponent of its split rows).
+    // f32 blocks: all four projections hold split rows, and for every input
+    // Q, K and V (after their norm and RoPE) and GELU(fc1) are at most 2^(15 +
+    // e) for these exponents, which their split rows then have.
     bool split = false;
-    int fc1_ex = 0;
+    int qkv_ex[3] = {}, fc1_ex = 0;
     bool q8 = false;  // projections in Q8_0 (qqkv..qfc2) instead of f32
     Q8Lin qqkv, qproj, qfc1, qfc2;
     float *ln1_g = nullptr, *ln1_b = nullptr, *ln2_g = nullptr, *ln2_b = nullptr;
@@ -425,9 +426,48 @@ bool flash_grid_fits(size_t heads, size_t tokens) {
            items <= (size_t)UINT32_MAX / 256 / vh::kMaxFlashSplits;
 }
 
+// VESTRA_HIP_FLASH_* choose between forms of the fp32 flash kernels (A/B
+// studies and tests, read per call): set, they ask for those kernels.
+bool fp32_flash_asked() {
+    for (const char *name : {"VESTRA_HIP_FLASH_SPLITS", "VESTRA_HIP_FLASH_STREAMS", "VESTRA_HIP_FLASH_DIRECT",
+                             "VESTRA_HIP_FLASH_FUSED", "VESTRA_HIP_FLASH_XCD"}) {
+        const char *e = std::getenv(name);
+        if (e && *e) return true;
+    }
+    return false;
+}
+
+// Attention of bh heads of `tokens` rows of hd <= 64 floats on the f16
+// matrix cores; *done is false where the fp32 kernels have to run instead.
+vh_status try_attn_split(RtState &s, const float *q, const float *k, const float *v, float *out, size_t bh,
+                         size_t tokens, size_t heads, size_t hd, bool token_major, float scale, bool *done) {
+    *done = false;
+    if (!vh::attn_split_fits(bh, tokens) || fp32_flash_asked()) return VH_OK;
+    const size_t need = (vh::attn_split_bytes(bh, tokens) + sizeof(float) - 1) / sizeof(float);
+    if (s.fw_floats < need) {
+        hipStreamSynchronize(s.stream);
+        if (s.fw) hipFree(s.fw);
+        s.fw = nullptr;
+        s.fw_floats = 0;
+        if (hipMalloc(&s.fw, need * sizeof(float)) != hipSuccess) {
+            hipGetLastError();
+            s.fw = nullptr;
+            return VH_OK;
+        }
+        s.fw_floats = need;
+    }
+    *done = true;
+    return launch(s, "flash_attention", [&] {
+        return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, s.fw);
+    });
+}
+
 vh_status flash(RtState &s, const float *q, const float *k, const float *v, float *out,
                 size_t bh, size_t tokens, size_t heads, bool token_major, int8_t *q8_qs = nullptr,
                 uint16_t *q8_d = nullptr, bool *quantized = nullptr, float scale = 0.125f) {
+    bool done = false;
+    TRY(try_attn_split(s, q, k, v, out, bh, tokens, heads, 64, token_major, scale, &done));
+    if (done) return VH_OK;
     // Partials of the key splits (room for either layout: the merge launch's
     // or the in-kernel merge's); without them the kernel runs unsplit.
     const size_t need =
@@ -540,37 +580,39 @@ vh_status prepare_split_lin(RtState &s, size_t K, size_t N, const float *w, cons
     return st;
 }
 
-// The exponent e for which every |LayerNorm(x) . w_n + b_n| of the projection
-// is at most 2^(15 + e), for LayerNorm parameters g, be on the device; false
-// if there is none within the range of a split output.
-vh_status ln_output_exponent(RtState &s, const Lin &L, const float *g, const float *be, int *e, bool *ok) {
+// Upper bounds of |LayerNorm(x) . w_n + b_n| over every x, per output n, for
+// LayerNorm parameters g, be on the device.
+vh_status ln_output_bounds(RtState &s, const Lin &L, const float *g, const float *be, std::vector<float> *h) {
     float *bound = nullptr;
     TRY(dalloc(s, L.N, &bound, "bound allocation"));
     vh_status st = launch(s, "ln_output_bound", [&] {
         return vh::launch_ln_output_bound(s.stream, L.wt, g, be, L.bias, bound, L.N, L.K);
     });
-    std::vector<float> h(L.N);
+    h->resize(L.N);
     if (!st) {
-        hipError_t he = hipMemcpyAsync(h.data(), bound, L.N * sizeof(float), hipMemcpyDeviceToHost, s.stream);
+        hipError_t he = hipMemcpyAsync(h->data(), bound, L.N * sizeof(float), hipMemcpyDeviceToHost, s.stream);
         if (he == hipSuccess) he = hipStreamSynchronize(s.stream);
         if (he != hipSuccess) st = fail(VH_ERR_UPLOAD, hip_msg("bound download", he));
     }
     hipFreeAsync(bound, s.stream);
-    if (st) return st;
+    return st;
+}
+
+// The exponent e with every v[i] <= 2^(15 + e); false if there is none within
+// the range of a split output (or a bound is NaN).
+bool bound_exponent(const float *v, size_t n, int *e) {
     float mx = 0.0f;
-    *ok = true;
-    for (float v : h) {
-        if (!(v <= 1e30f)) *ok = false;  // NaN and overflow too
-        mx = std::max(mx, v);
+    for (size_t i = 0; i < n; i++) {
+        if (!(v[i] <= 1e30f)) return false;
+        mx = std::max(mx, v[i]);
     }
     *e = 0;
-    if (*ok && mx > 0.0f) {
+    if (mx > 0.0f) {
         int x = 0;
         frexpf(mx * 1.01f, &x);  // the bound's own rounding; mx * 1.01 <= 2^x
         *e = x - 15;
     }
-    if (*e > 90 || *e < -90) *ok = false;
-    return VH_OK;
+    return *e <= 90 && *e >= -90;
 }
 
 // Split rows of `in` [rows][k] in the runtime's workspace, or null pointers
@@ -1290,10 +1332,14 @@ extern "C" vh_status vh_attention_online_f32(const vh_runtime *rt, const vh_tens
     } else {
         // Rows zero-padded to 64 dims run through the flash kernel with the
         // 1/sqrt(head_dim) scale; the output keeps the first head_dim columns.
+        // (On split rows the padding is part of the split.)
         const size_t padded = ht * 64;
         float *pad = nullptr;
-        st = dalloc(s, 4 * padded, &pad, "attention padding allocation");
-        if (!st) {
+        bool done = false;
+        st = try_attn_split(s, q->ptr, k->ptr, v->ptr, t->ptr, heads, tokens, heads, head_dim, false,
+                            1.0f / sqrtf((float)head_dim), &done);
+        if (!st && !done) st = dalloc(s, 4 * padded, &pad, "attention padding allocation");
+        if (!st && !done) {
             float *pq = pad, *pk = pad + padded, *pv = pad + 2 * padded, *po = pad + 3 * padded;
             st = launch(s, "attention_pad", [&] {
                 return vh::launch_pad_rows64(s.stream, q->ptr, k->ptr, v->ptr, pq, pk, pv, ht,
@@ -1390,8 +1436,15 @@ extern "C" vh_status vh_flash_attention_f32_da3_base_into(const vh_runtime *rt,
     const bool order = capture == hipStreamCaptureStatusNone;
     if (order && (e = hipStreamWaitEvent(s.stream, done, 0)) != hipSuccess)
         return fail(VH_ERR_KERNEL, hip_msg(what, e));
-    e = vh::launch_flash_attention(s.stream, q->ptr, k->ptr, v->ptr, out->ptr, heads, tokens, heads,
-                                   token_major != 0, s.scratch, kScratchFloats);
+    // The allocating entry point's choice of kernel, so the same bits; the
+    // array holds the split rows of every shape accepted above.
+    if (vh::attn_split_fits(heads, tokens) && !fp32_flash_asked() &&
+        vh::attn_split_bytes(heads, tokens) <= kScratchBytes)
+        e = vh::launch_attn_split_f32(s.stream, q->ptr, k->ptr, v->ptr, out->ptr, heads, tokens, heads, 64,
+                                      token_major != 0, 0.125f, s.scratch);
+    else
+        e = vh::launch_flash_attention(s.stream, q->ptr, k->ptr, v->ptr, out->ptr, heads, tokens, heads,
+                                       token_major != 0, s.scratch, kScratchFloats);
     if (e != hipSuccess) return fail(VH_ERR_KERNEL, hip_msg(what, e));
     if (order && (e = hipEventRecord(done, s.stream)) != hipSuccess)
         return fail(VH_ERR_KERNEL, hip_msg(what, e));
@@ -2242,7 +2295,7 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
                                         vh::Epi::Residual, b.qfc2.bias, b.qfc2.gamma);
         });
     }
-    if (!b.split) {
+    if (!b.split || !vh::attn_split_fits(images * kHeads, tokens)) {
         // Weights with an inf or NaN: the fp32 matrix instructions.
         auto norm = [&](const float *g, const float *be) {
             return launch(s, "layernorm", [&] { return vh::launch_layernorm(s.stream, x, g, be, h, M, D, eps); });
@@ -2279,21 +2332,27 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
         g.tokens = tokens;
         g.heads = kHeads;
         g.rot = b.qn_g ? nullptr : rot;
+        for (int i = 0; i < 3; i++) {
+            g.qkv_split[i] = !b.qn_g || i == 2;
+            g.qkv_ex[i] = b.qkv_ex[i];
+        }
         TRY(launch(s, "gemm_qkv_rope", [&] { return vh::launch_gemm_split(s.stream, g); }));
     }
     if (b.qn_g)
         // Late block: LayerNorm of every 64-wide Q and K head row fused with
         // the RoPE (src/specialized.rs:278-316).
         TRY(launch(s, "qk_norm_rope", [&] {
-            return vh::launch_qk_norm_rope(s.stream, q, k, b.qn_g, b.qn_b, b.kn_g, b.kn_b, rot,
-                                           M * kHeads, tokens, eps);
+            return vh::launch_qk_norm_rope_split(s.stream, q, k, b.qn_g, b.qn_b, b.kn_g, b.kn_b, rot,
+                                                 M * kHeads, tokens, eps, b.qkv_ex[0], b.qkv_ex[1]);
         }));
-    TRY(flash(s, q, k, v, att, images * kHeads, tokens, kHeads, true));
-    TRY(launch(s, "split_rows", [&] { return vh::launch_split_rows(s.stream, att, h, hex, M, D); }));
+    TRY(launch(s, "flash_attention", [&] {
+        return vh::launch_attn_split(s.stream, vh::SplitQkv{q, k, v, b.qkv_ex[0], b.qkv_ex[1], b.qkv_ex[2]}, att,
+                                     images * kHeads, tokens, kHeads);
+    }));
     {
-        vh::SplitGemm g = split_gemm_args(b.proj, att, M, vh::Epi::Residual, x);
-        g.x = h;
-        g.ex = hex;
+        vh::SplitGemm g = split_gemm_args(b.proj, nullptr, M, vh::Epi::Residual, x);
+        g.x = att;
+        g.ex_c = b.qkv_ex[2];
         TRY(launch(s, "gemm_proj_residual", [&] { return vh::launch_gemm_split(s.stream, g); }));
     }
     TRY(norm(b.ln2_g, b.ln2_b));
@@ -2358,11 +2417,26 @@ static vh_status block_prepare(const vh_runtime *rt, const vh_block_params *p, b
     if (!st) st = upload_small(s, p->ln2_gamma, kDim, &b->ln2_g, "ln2 gamma");
     if (!st) st = upload_small(s, p->ln2_beta, kDim, &b->ln2_b, "ln2 beta");
     if (!st && !q8) {
-        bool ok = false;
-        st = ln_output_exponent(s, b->fc1, b->ln2_g, b->ln2_b, &b->fc1_ex, &ok);
-        b->split = ok && b->qkv.sw && b->proj.sw && b->fc1.sw && b->fc2.sw;
+        std::vector<float> h;
+        st = ln_output_bounds(s, b->fc1, b->ln2_g, b->ln2_b, &h);
+        b->split = b->qkv.sw && b->proj.sw && b->fc1.sw && b->fc2.sw && bound_exponent(h.data(), kMlp, &b->fc1_ex);
+        if (!st) st = ln_output_bounds(s, b->qkv, b->ln1_g, b->ln1_b, &h);
+        if (!st) {
+            // The RoPE rotates pairs: at most sqrt(2) of the larger.
+            for (size_t i = 0; i < 2 * kDim; i++) h[i] *= 1.4143f;
+            if (qk_norm) {
+                // LayerNorm of a 64-wide row: at most sqrt(64) |gamma| + |beta|.
+                const float *nq[] = {p->q_norm_gamma, p->q_norm_beta, p->k_norm_gamma, p->k_norm_beta};
+                for (size_t i = 0; i < 2 * kDim; i++) {
+                    const float *const *np = nq + 2 * (i / kDim);
+                    h[i] = (8.0f * fabsf(np[0][i % 64]) + fabsf(np[1][i % 64])) * 1.4143f;
+                }
+            }
+            for (int i = 0; i < 3; i++)
+                b->split = b->split && bound_exponent(h.data() + i * kDim, kDim, &b->qkv_ex[i]);
+        }
         if (b->split)
-            for (Lin *l : {&b->qkv, &b->fc1, &b->fc2}) {  // their inputs hold no inf without a NaN
+            for (Lin *l : {&b->qkv, &b->proj, &b->fc1, &b->fc2}) {  // no input holds an inf
                 hipFreeAsync(l->wt, s.stream);
                 l->wt = nullptr;
             }

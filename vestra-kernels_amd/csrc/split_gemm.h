@@ -56,6 +56,13 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     return v;
 }
 
+// Running maximum of magnitudes as bit patterns (a NaN sorts above every number).
+__device__ __forceinline__ uint32_t absmax4(uint32_t mx, f32x4 v) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) mx = max(mx, __float_as_uint(v[r]) & 0x7fffffffu);
+    return mx;
+}
+
 // One asynchronous copy of 16 bytes per lane, global base + voff to LDS
 // lds + 16 * lane (global_load_lds_dwordx4; lds is wave-uniform).  In asm,
 // because the compiler orders LDS reads behind every builtin copy in flight
