@@ -24,6 +24,7 @@
 // 6.2e-7 on the 128 x 256 tile), against 2.5e-7 to 5.0e-7 and 5.8e-7 to
 // 9.9e-7 of the fp32 matrix instructions.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -436,13 +437,9 @@ __device__ __forceinline__ void store_split4(char *row, int k, f32x4 v, int e) {
     *reinterpret_cast<f16x4 *>(p + 64) = lo;
 }
 
-__global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict__ in, char *__restrict__ out,
-                                                         int *__restrict__ ex, size_t rows, int K, int slices) {
-    const int lane = threadIdx.x & 63;
-    const size_t row = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const float *src = in + row * K;
-    char *dst = out + row * slices * 128;
+// One row of K floats to its split row, by one wave.
+__device__ __forceinline__ void split_row(const float *__restrict__ src, char *__restrict__ dst, int *__restrict__ ex,
+                                          int K, int slices, int lane) {
     const int Kp = slices * 32;
     uint32_t mx = 0;
     int e;
@@ -461,23 +458,51 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict
             for (int j = 0; j < 4; j++)
                 if (lane + j * 64 < np4) store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
         } else {
-            for (int c = lane; c < n4; c += 64) mx = absmax4(mx, src4[c]);
+            int c = lane;
+            for (; c + 192 < n4; c += 256)
+                mx = absmax4(absmax4(absmax4(absmax4(mx, src4[c]), src4[c + 64]), src4[c + 128]), src4[c + 192]);
+            for (; c < n4; c += 64) mx = absmax4(mx, src4[c]);
             e = split_exponent(wave_umax(mx));
-            for (int c = lane; c < np4; c += 64)
+#pragma unroll 4
+            for (c = lane; c < np4; c += 64)
                 store_split4(dst, 4 * c, c < n4 && e != kSplitNonFinite ? src4[c] : zero, e);
         }
     } else {
-        for (int k = lane; k < K; k += 64) mx = max(mx, __float_as_uint(src[k]) & 0x7fffffffu);
-        e = split_exponent(wave_umax(mx));
-        for (int c = lane; c < Kp >> 2; c += 64) {
-            f32x4 v = zero;
+        // Rows that are not 16-byte aligned: lane-consecutive floats, sixteen
+        // loads in flight, in registers when the row has at most 1024.
+        auto store1 = [&](int k, float v) {
+            _Float16 h, l;
+            split_f16(__builtin_ldexpf(v, -e), h, l);
+            _Float16 *p = reinterpret_cast<_Float16 *>(dst + (k / 32) * 128) + k % 32;
+            p[0] = h;
+            p[32] = l;
+        };
+        float r[16];
+        for (int k0 = 0; k0 < K; k0 += 1024) {
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (4 * c + r < K && e != kSplitNonFinite) v[r] = src[4 * c + r];
-            store_split4(dst, 4 * c, v, e);
+            for (int j = 0; j < 16; j++) r[j] = k0 + lane + 64 * j < K ? src[k0 + lane + 64 * j] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 16; j++) mx = max(mx, __float_as_uint(r[j]) & 0x7fffffffu);
+        }
+        e = split_exponent(wave_umax(mx));
+        for (int k0 = 0; k0 < Kp; k0 += 1024) {
+            if (K > 1024) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) r[j] = k0 + lane + 64 * j < K ? src[k0 + lane + 64 * j] : 0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+                if (k0 + lane + 64 * j < Kp) store1(k0 + lane + 64 * j, e == kSplitNonFinite ? 0.0f : r[j]);
         }
     }
-    if (lane == 0) ex[row] = e;
+    if (lane == 0) *ex = e;
+}
+
+__global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict__ in, char *__restrict__ out,
+                                                         int *__restrict__ ex, size_t rows, int K, int slices) {
+    const size_t row = (size_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    split_row(in + row * K, out + row * slices * 128, ex + row, K, slices, threadIdx.x & 63);
 }
 
 // LayerNorm of each row straight into split rows (launch_layernorm's bits,
@@ -547,42 +572,70 @@ __global__ __launch_bounds__(256) void ln_output_bound_kernel(const float *__res
     if (lane == 0) bound[n] = sqrtf((float)K) * sqrtf(s2) + sb + fabsf(bias[n]);
 }
 
-// Split rows of the columns of in [K][N] (row-major): 16 columns per
-// workgroup, 64 rows of them per pass.  The second pass reads the strip
-// again from the cache and stores a column's 32-value slice from 16 lanes'
-// halves through LDS.
-__global__ __launch_bounds__(1024) void split_columns_kernel(const float *__restrict__ in, char *__restrict__ out,
-                                                             int *__restrict__ ex, int K, int N, int slices) {
+// Both operands of a row-major product a [M][K] . b [K][N] in one launch:
+// workgroups [0, col_wgs) split 16 columns of b each, the rest 16 rows of a
+// each, one per wave.  A column strip is read twice, the second time from
+// the cache (strips of at most 1024 rows stay in registers): for the largest
+// magnitudes, then 256 rows at a time through LDS, so that a column's slice
+// is stored from consecutive lanes (1153 x 1003 x 771: both operands SPLIT_OPS us, against 28 in
+// two launches with 64 rows at a time).
+__global__ __launch_bounds__(1024) void split_operands_kernel(const float *__restrict__ a, char *__restrict__ as,
+                                                              int *__restrict__ ea, int M, const float *__restrict__ b,
+                                                              char *__restrict__ bs, int *__restrict__ eb, int K,
+                                                              int N, int slices, int col_wgs) {
+    if ((int)blockIdx.x >= col_wgs) {
+        const size_t row = (size_t)(blockIdx.x - col_wgs) * 16 + (threadIdx.x >> 6);
+        if (row < (size_t)M)
+            split_row(a + row * K, as + row * slices * 128, ea + row, K, slices, threadIdx.x & 63);
+        return;
+    }
     const int c = threadIdx.x & 15, kr = threadIdx.x >> 4;  // column, row of the pass
-    const int n = blockIdx.x * 16 + c, nc = min(n, N - 1);
+    const int n0 = blockIdx.x * 16, nc = min(n0 + c, N - 1);
     __shared__ uint32_t red[16][17];
-    __shared__ float tile[64][17];
+    __shared__ float tile[256][17];
+    // Sixteen loads in flight: 1024 rows of the strip, which stay in registers
+    // when there are no more.
+    float r[16];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int kk = k0 + kr + 64 * j;
+            r[j] = kk < K ? b[(size_t)kk * N + nc] : 0.0f;
+        }
+    };
     uint32_t mx = 0;
-    for (int k = kr; k < K; k += 64) mx = max(mx, __float_as_uint(in[(size_t)k * N + nc]) & 0x7fffffffu);
+    for (int k0 = 0; k0 < K; k0 += 1024) {
+        load(k0);
+#pragma unroll
+        for (int j = 0; j < 16; j++) mx = max(mx, __float_as_uint(r[j]) & 0x7fffffffu);
+    }
     mx = max(mx, (uint32_t)__shfl_xor((int)mx, 16, 64));
     mx = max(mx, (uint32_t)__shfl_xor((int)mx, 32, 64));
     if ((threadIdx.x & 63) < 16) red[threadIdx.x >> 6][c] = mx;
     __syncthreads();
-    // Store role: column sc of the strip, values 4 sk .. 4 sk + 3 of a pass.
-    const int sc = threadIdx.x >> 4, sk = threadIdx.x & 15;
-    int e = 0;
-    if (sc < 16) {
-        uint32_t m = 0;
+    // Store role: column sc of the strip, rows 4 sk .. 4 sk + 3 of a tile.
+    const int sc = threadIdx.x >> 6, sk = threadIdx.x & 63;
+    uint32_t m = 0;
 #pragma unroll
-        for (int w = 0; w < 16; w++) m = max(m, red[w][sc]);
-        e = split_exponent(m);
-        if (sk == 0 && blockIdx.x * 16 + sc < N) ex[blockIdx.x * 16 + sc] = e;
-    }
-    for (int k0 = 0; k0 < slices * 32; k0 += 64) {
-        __syncthreads();
-        tile[kr][c] = k0 + kr < K ? in[(size_t)(k0 + kr) * N + nc] : 0.0f;
-        __syncthreads();
-        const int sn = blockIdx.x * 16 + sc, k = k0 + 4 * sk;
-        if (sc < 16 && sn < N && k < slices * 32) {
-            f32x4 v;
+    for (int w = 0; w < 16; w++) m = max(m, red[w][sc]);
+    const int e = split_exponent(m), sn = n0 + sc;
+    if (sk == 0 && sn < N) eb[sn] = e;
+    for (int k0 = 0; k0 < slices * 32; k0 += 1024) {
+        if (K > 1024) load(k0);
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = e == kSplitNonFinite ? 0.0f : tile[4 * sk + r][sc];
-            store_split4(out + (size_t)sn * slices * 128, k, v, e);
+        for (int q = 0; q < 4; q++) {
+            if (k0 + 256 * q >= slices * 32) break;
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 4; j++) tile[kr + 64 * j][c] = r[4 * q + j];
+            __syncthreads();
+            const int ks = k0 + 256 * q + 4 * sk;
+            if (sn < N && ks < slices * 32) {
+                f32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = e == kSplitNonFinite ? 0.0f : tile[4 * sk + j][sc];
+                store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
+            }
         }
     }
 }
@@ -611,7 +664,7 @@ constexpr SplitTile kSplitTiles[] = {
 // us here, 20.5 for 64 x 128, 23.9 for 64 x 64; 3460 x 2304 x 768: 41.5 for
 // 128 x 256, 45.9 for 64 x 128; 97 x 2304 x 768: 6.2 for 64 x 32, 10.3 for
 // 64 x 128).
-int pick_split_tile(size_t m, size_t n, int slices, bool qkv) {
+int pick_split_tile(size_t m, size_t n, int slices, bool qkv, float *predicted_us = nullptr) {
     int best = 0;
     float best_us = 0.0f;
     for (int i = 0; i < 6; i++) {
@@ -626,6 +679,7 @@ int pick_split_tile(size_t m, size_t n, int slices, bool qkv) {
             best_us = us;
         }
     }
+    if (predicted_us) *predicted_us = best_us;
     return best;
 }
 
@@ -668,6 +722,28 @@ bool split_gemm_fits(size_t m, size_t n, size_t k) {
            ((m + 63) / 64) * ((n + 31) / 32) <= (size_t)INT32_MAX / 512;
 }
 
+// Splitting reads and writes four bytes per value at about 3 TB/s, in a launch
+// of 2.5 us.  The fp32 GEMM runs 64 x 64 tiles at 0.55 us per k-slice of 32,
+// the K of a grid below half the CUs in two parts at once, a partial last round
+// as K pieces (0.3 of a round), and takes twice as long where K is no
+// multiple of 32 (its masked loads).  Fitted to 12 shapes on MI355X (fp32 and
+// split, us): 16 x 768 x 768 12.7 and 8.9, 64 x 588 x 96 20.8 and 8.4, 256 x 768
+// x 768 13.0 and 10.2, 865 x 768 x 768 14.0 and 12; the fp32 GEMM keeps 300 x 96
+// x 200 (4.9 and 7.5), 3460 x 64 x 768 (8.8 and 12.6) and 3460 x 768 x 96 (13.0
+// and 16.5).  whole_tiles: the fp32 route is the channel-major one, which
+// splits no K (865 x 768 x 96 19.3 and 11).
+bool split_gemm_pays(size_t m, size_t n, size_t k, size_t split_values, bool whole_tiles) {
+    const int slices = (int)((k + 31) / 32);
+    float gemm_us;
+    pick_split_tile(m, n, slices, false, &gemm_us);
+    const float split_us = 2.5f + (float)split_values * 8.0f / 3e6f + gemm_us;
+    const float tiles = (float)((m + 63) / 64) * (float)((n + 63) / 64);
+    float rounds = tiles > 256.0f ? tiles / 256.0f + 0.3f : (tiles > 128.0f ? tiles / 256.0f : 0.5f);
+    if (whole_tiles) rounds = ceilf(tiles / 256.0f);
+    const float fp32_us = (4.0f + rounds * slices * 0.55f) * (k % 32 == 0 ? 1.0f : 2.0f);
+    return split_us < fp32_us;
+}
+
 hipError_t launch_split_rows(hipStream_t s, const float *in, void *out, int *ex, size_t rows, size_t k) {
     if (rows == 0) return hipSuccess;
     const size_t wpb = rows <= 2048 ? 1 : 4;
@@ -676,10 +752,13 @@ hipError_t launch_split_rows(hipStream_t s, const float *in, void *out, int *ex,
     return hipGetLastError();
 }
 
-hipError_t launch_split_columns(hipStream_t s, const float *in, void *out, int *ex, size_t k, size_t n) {
-    if (n == 0) return hipSuccess;
-    split_columns_kernel<<<(unsigned)((n + 15) / 16), 1024, 0, s>>>(in, static_cast<char *>(out), ex, (int)k, (int)n,
-                                                                   (int)((k + 31) / 32));
+hipError_t launch_split_operands(hipStream_t s, const float *a, void *as, int *ea, size_t m, const float *b, void *bs,
+                                 int *eb, size_t k, size_t n) {
+    if (m == 0 || n == 0) return hipSuccess;
+    const size_t cols = (n + 15) / 16, rows = (m + 15) / 16;
+    split_operands_kernel<<<(unsigned)(cols + rows), 1024, 0, s>>>(a, static_cast<char *>(as), ea, (int)m, b,
+                                                                   static_cast<char *>(bs), eb, (int)k, (int)n,
+                                                                   (int)((k + 31) / 32), (int)cols);
     return hipGetLastError();
 }
 

@@ -209,10 +209,14 @@ constexpr size_t kTailStatFloats = kTailTiles * 4 * 4 * 256;
 constexpr int kSplitNonFinite = INT32_MIN / 4;
 // Shapes launch_gemm_split takes.
 bool split_gemm_fits(size_t m, size_t n, size_t k);
+// Whether splitting split_values floats and multiplying them is predicted to
+// take less time than the fp32 GEMM of the shape.
+bool split_gemm_pays(size_t m, size_t n, size_t k, size_t split_values, bool whole_tiles = false);
 constexpr size_t split_bytes(size_t rows, size_t k) { return rows * ((k + 31) / 32) * 128; }
 hipError_t launch_split_rows(hipStream_t s, const float *in, void *out, int *ex, size_t rows, size_t k);
-// Split rows [n][k] of the columns of in [k][n].
-hipError_t launch_split_columns(hipStream_t s, const float *in, void *out, int *ex, size_t k, size_t n);
+// Split rows of a [m][k] and, as [n][k], of the columns of b [k][n].
+hipError_t launch_split_operands(hipStream_t s, const float *a, void *as, int *ea, size_t m, const float *b, void *bs,
+                                 int *eb, size_t k, size_t n);
 // LayerNorm of each row into split rows (cols % 32 == 0, cols <= 1024).
 hipError_t launch_layernorm_split(hipStream_t s, const float *in, const float *gamma, const float *beta,
                                   void *out, int *ex, size_t rows, size_t cols, float eps);

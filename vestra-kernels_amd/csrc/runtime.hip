@@ -20,6 +20,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "kernels.h"
@@ -76,9 +77,59 @@ struct ProfileRec {
     hipEvent_t a, b;
 };
 
+// Device blocks of freed tensors, kept for the next tensor of the same size:
+// hipMallocAsync and hipFreeAsync cost a call about 10 us of host time between
+// them on MI355X (vh_linear_run at 16 x 768 x 768 18.3 us a call, 8.7 with
+// the pool), a lookup here none that shows.  A block only ever serves its runtime's one stream, whose
+// order makes the reuse safe exactly as hipFreeAsync's would; the blocks held
+// are bounded (larger ones, and those past the bound, go back at once), are
+// given back when an allocation fails and when the runtime ends, and are left
+// alone while the stream is captured, where allocations become the graph's.
+struct TensorPool {
+    static constexpr size_t kMaxBlock = (size_t)128 << 20, kMaxHeld = (size_t)512 << 20, kGrain = 512;
+    std::mutex mu;  // tensors may be freed from any host thread
+    std::unordered_map<size_t, std::vector<void *>> blocks;
+    size_t held = 0;
+    static size_t rounded(size_t bytes) { return (bytes + kGrain - 1) / kGrain * kGrain; }
+    void *take(size_t bytes) {
+        std::lock_guard<std::mutex> lock(mu);
+        auto it = blocks.find(bytes);
+        if (it == blocks.end() || it->second.empty()) return nullptr;
+        void *p = it->second.back();
+        it->second.pop_back();
+        held -= bytes;
+        return p;
+    }
+    bool keep(void *p, size_t bytes) noexcept {
+        if (bytes > kMaxBlock) return false;
+        std::lock_guard<std::mutex> lock(mu);
+        if (held + bytes > kMaxHeld) return false;
+        try {
+            blocks[bytes].push_back(p);
+        } catch (...) {
+            return false;
+        }
+        held += bytes;
+        return true;
+    }
+    void give_back(hipStream_t stream) {
+        std::lock_guard<std::mutex> lock(mu);
+        for (auto &kv : blocks)
+            for (void *p : kv.second) hipFreeAsync(p, stream);
+        blocks.clear();
+        held = 0;
+    }
+};
+
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 struct RtState {
     int device = 0;
     hipStream_t stream = nullptr;
+    TensorPool pool;
     std::mutex mu;
     std::map<std::string, float *> rope_cache;  // host-built sin/cos tables
     float *ws = nullptr;                        // grow-only block workspace
@@ -105,6 +156,7 @@ struct RtState {
     ~RtState() {
         if (!stream) return;
         hipSetDevice(device);
+        pool.give_back(stream);
         hipStreamSynchronize(stream);
         for (auto &kv : rope_cache) hipFree(kv.second);
         if (ws) hipFree(ws);
@@ -138,11 +190,12 @@ struct vh_tensor {
     Rt rt;
     float *ptr = nullptr;
     size_t len = 0;
+    size_t block = 0;  // bytes of the block, a TensorPool size; 0: a captured allocation
     ~vh_tensor() {
-        if (ptr && rt) {
-            hipSetDevice(rt->device);
-            hipFreeAsync(ptr, rt->stream);
-        }
+        if (!ptr || !rt) return;
+        if (block && !capturing(rt->stream) && rt->pool.keep(ptr, block)) return;
+        hipSetDevice(rt->device);
+        hipFreeAsync(ptr, rt->stream);
     }
 };
 
@@ -280,17 +333,28 @@ vh_status upload_array(RtState &s, const float *host, size_t n, float **out, con
 }
 
 vh_status new_tensor(const Rt &rt, size_t len, vh_tensor **out, const char *what) {
-    float *p = nullptr;
-    vh_status st = dalloc(*rt, len, &p, what);
-    if (st) return st;
     vh_tensor *t = new (std::nothrow) vh_tensor;
-    if (!t) {
-        hipFreeAsync(p, rt->stream);
-        return fail(VH_ERR_UPLOAD, std::string(what) + ": host allocation failed");
+    if (!t) return fail(VH_ERR_UPLOAD, std::string(what) + ": host allocation failed");
+    const size_t bytes = len <= (SIZE_MAX >> 3) ? TensorPool::rounded((len ? len : 1) * sizeof(float)) : SIZE_MAX;
+    const bool captured = capturing(rt->stream);
+    void *p = captured ? nullptr : rt->pool.take(bytes);
+    if (!p) {
+        hipError_t e = hipMallocAsync(&p, bytes, rt->stream);
+        if (e != hipSuccess && !captured) {
+            hipGetLastError();
+            rt->pool.give_back(rt->stream);
+            p = nullptr;
+            e = hipMallocAsync(&p, bytes, rt->stream);
+        }
+        if (e != hipSuccess) {
+            delete t;
+            return fail(VH_ERR_UPLOAD, hip_msg(what, e));
+        }
     }
     t->rt = rt;
-    t->ptr = p;
+    t->ptr = static_cast<float *>(p);
     t->len = len;
+    t->block = captured ? 0 : bytes;
     *out = t;
     return VH_OK;
 }
@@ -621,22 +685,29 @@ struct SplitRows {
     char *x = nullptr;
     int *ex = nullptr;
 };
-vh_status split_input(RtState &s, const float *in, size_t rows, size_t k, SplitRows *out) {
-    const size_t bytes = vh::split_bytes(rows, k), need = bytes + rows * sizeof(int);
-    if (s.sx_bytes < need) {
+vh_status split_space(RtState &s, size_t bytes, char **out) {
+    *out = nullptr;
+    if (s.sx_bytes < bytes) {
         hipStreamSynchronize(s.stream);
         if (s.sx) hipFree(s.sx);
         s.sx = nullptr;
         s.sx_bytes = 0;
-        if (hipMalloc(&s.sx, need) != hipSuccess) {
+        if (hipMalloc(&s.sx, bytes) != hipSuccess) {
             hipGetLastError();
             s.sx = nullptr;
             return VH_OK;
         }
-        s.sx_bytes = need;
+        s.sx_bytes = bytes;
     }
-    out->x = s.sx;
-    out->ex = reinterpret_cast<int *>(s.sx + bytes);
+    *out = s.sx;
+    return VH_OK;
+}
+
+vh_status split_input(RtState &s, const float *in, size_t rows, size_t k, SplitRows *out) {
+    const size_t bytes = vh::split_bytes(rows, k);
+    TRY(split_space(s, bytes + rows * sizeof(int), &out->x));
+    if (!out->x) return VH_OK;
+    out->ex = reinterpret_cast<int *>(out->x + bytes);
     return launch(s, "split_rows", [&] { return vh::launch_split_rows(s.stream, in, out->x, out->ex, rows, k); });
 }
 
@@ -668,7 +739,9 @@ vh::SplitGemm split_gemm_args(const Lin &L, const float *in, size_t rows, vh::Ep
 // *done is false where the fp32 kernel has to run instead.
 vh_status try_split(RtState &s, const Lin &L, vh::SplitGemm g, const char *name, bool *done) {
     *done = false;
-    if (!L.sw || g.m == 0 || !split_k_fits(g.m, g.n, g.k) || fp32_gemm_asked()) return VH_OK;
+    if (!L.sw || g.m == 0 || !split_k_fits(g.m, g.n, g.k) || fp32_gemm_asked() ||
+        !vh::split_gemm_pays(g.m, g.n, g.k, g.m * g.k, g.chw))
+        return VH_OK;
     SplitRows x;
     TRY(split_input(s, g.xf, g.m, g.k, &x));
     if (!x.x) return VH_OK;
@@ -1128,19 +1201,16 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
     vh_tensor *t = nullptr;
     TRY(new_tensor(rt->s, mn, &t, "GEMM output allocation"));
     // Split rows of A and of B's columns, then the f16 matrix cores.
-    if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked()) {
-        char *w = nullptr;
-        int *ew = nullptr;
-        SplitRows x;
-        vh_status st = split_input(s, a->ptr, m, k, &x);
-        const size_t wbytes = vh::split_bytes(n, k);
-        if (!st && x.x) st = dalloc(s, wbytes + n * sizeof(int), &w, "GEMM operand allocation");
-        if (!st && x.x) {
-            ew = reinterpret_cast<int *>(w + wbytes);
-            st = launch(s, "split_columns", [&] { return vh::launch_split_columns(s.stream, b->ptr, w, ew, k, n); });
+    if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked() && vh::split_gemm_pays(m, n, k, mk + kn)) {
+        const size_t abytes = vh::split_bytes(m, k), bbytes = vh::split_bytes(n, k);
+        char *x = nullptr;
+        vh_status st = split_space(s, abytes + bbytes + (m + n) * sizeof(int), &x);
+        if (!st && x) {
             vh::SplitGemm g{};
-            g.x = x.x;
-            g.ex = x.ex;
+            char *w = x + abytes;
+            int *ex = reinterpret_cast<int *>(w + bbytes), *ew = ex + m;
+            g.x = x;
+            g.ex = ex;
             g.w = w;
             g.ew = ew;
             g.xf = a->ptr;
@@ -1151,14 +1221,16 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
             g.k = k;
             g.epi = vh::Epi::Store;
             g.c = t->ptr;
+            st = launch(s, "split_operands", [&] {
+                return vh::launch_split_operands(s.stream, a->ptr, x, ex, m, b->ptr, w, ew, k, n);
+            });
             if (!st) st = launch(s, "gemm", [&] { return vh::launch_gemm_split(s.stream, g); });
         }
-        if (w) hipFreeAsync(w, s.stream);
         if (st) {
             delete t;
             return st;
         }
-        if (x.x) {
+        if (x) {
             *out = t;
             return VH_OK;
         }
