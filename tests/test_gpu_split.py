@@ -149,3 +149,47 @@ def test_split_attention_head_scales_and_non_finite(rt):
     assert np.isposinf(got[4, :, 3]).all()
     cols = np.delete(np.arange(hd), 3)
     assert np.abs(got[4][:, cols] - clean[4][:, cols]).max() <= 2e-5 * 5
+
+
+# Grids of at least 128 64 x 64 tiles: ragged rows and widths, one and five
+# channel slices, 1 x 1, 3 x 3 and 5 x 5 taps with and without padding, output
+# channels that fill no tile.
+@pytest.mark.parametrize("in_c, out_c, ih, iw, k, p, relu", [
+    (32, 64, 97, 91, 3, 1, False), (160, 70, 71, 65, 3, 1, True), (256, 33, 96, 93, 1, 0, False),
+    (64, 128, 70, 67, 5, 2, False), (96, 130, 61, 50, 3, 0, True)])
+def test_split_convolution_vs_float64(rt, in_c, out_c, ih, iw, k, p, relu):
+    x = seeded.normal(10000 + ih, in_c * ih * iw).reshape(in_c, ih, iw)
+    w = seeded.normal(10100 + k, out_c * in_c * k * k, 0.05).reshape(out_c, in_c, k, k)
+    b = seeded.normal(10200, out_c)
+    conv = rt.prepare_conv2d_f32(in_c, out_c, k, k, 1, p, w, b)
+    oh, ow = ih + 2 * p - k + 1, iw + 2 * p - k + 1
+
+    def direct(img, wt):
+        z = np.pad(img.astype(np.float64), ((0, 0), (p, p), (p, p)))
+        out = np.zeros((out_c, oh, ow))
+        for ky in range(k):
+            for kx in range(k):
+                out += np.einsum("oc,cyx->oyx", wt[:, :, ky, kx].astype(np.float64),
+                                 z[:, ky:ky + oh, kx:kx + ow], optimize=True)
+        return out
+
+    xin = np.maximum(x, 0) if relu else x
+    exp = direct(xin, w) + b[:, None, None]
+    n = in_c * k * k
+    bound = ((2.0 ** -21 + n / 4 * 2.0 ** -23) * direct(np.abs(xin), np.abs(w)) + 2.0 ** -23 * np.abs(exp) +
+             2.0 ** -39 * np.abs(x).max() * np.abs(w).sum(axis=(1, 2, 3))[:, None, None])
+    run = conv.run_relu_input if relu else conv.run
+    got = rt.download_f32(run(rt.upload_f32(x), ih, iw)).reshape(exp.shape)
+    assert np.all(np.abs(got - exp) <= bound)
+    # An infinity and a NaN reach what they reach in floats, and no more.
+    x[1, 3, 5], x[0, ih - 1, 0] = np.inf, np.nan
+    with np.errstate(invalid="ignore"):
+        odd = direct(np.maximum(x, 0) if relu else x, w) + b[:, None, None]
+    if relu:  # the crate's max(x, 0) of a NaN is 0
+        x[0, ih - 1, 0] = 0.0
+        odd = direct(np.maximum(x, 0), w) + b[:, None, None]
+    got = rt.download_f32(run(rt.upload_f32(x), ih, iw)).reshape(exp.shape)
+    fine = np.isfinite(odd)
+    assert np.array_equal(np.isnan(got), np.isnan(odd))
+    assert np.array_equal(got[~fine & ~np.isnan(odd)], odd[~fine & ~np.isnan(odd)].astype(np.float32))
+    assert np.all(np.abs(got[fine] - odd[fine]) <= bound[fine])

@@ -610,7 +610,7 @@ hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, 
     const size_t head_floats = tokens * hd;
     // Heads of up to 64 K floats (1024 tokens): one launch whose workgroups
     // each read the whole head for its largest magnitude, from the cache past
-    // the first (12 x 865 x 64: 7 us; two launches 13.4).  Longer heads take
+    // the first (12 x 865 x 64: 10 us; two launches 13.4).  Longer heads take
     // it in a launch of its own.
     if (head_floats <= 65536) {
         const unsigned wgs = (unsigned)std::min<size_t>((tokens + 63) / 64, 4);

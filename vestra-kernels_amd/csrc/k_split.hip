@@ -48,17 +48,43 @@ struct SplitArgs {
     float qkv_scale[3];     // Qkv: 0 for floats, or split rows of the values times this
     int tokens, heads;
     const float *rot;
+    // Conv: X is a zero-padded channel-last image of split rows, one per
+    // pixel of its grid of width conv_wp, with the one exponent ex[0]; the
+    // slices of W walk the taps (ky, kx), conv_cs channel slices each, and
+    // row m of the product reads image row m + ky * conv_wp + kx.  C^T goes to
+    // c[n][y][x] for x < conv_ow (m = y * conv_wp + x), conv_plane floats a
+    // channel.  xf is the CHW image [conv_cs * 32][conv_ih][conv_iw] and wf
+    // [N][taps][channels], for the outputs an inf or NaN reaches.
+    int conv_cs, conv_kw, conv_wp, conv_ow, conv_ih, conv_iw, conv_pad, conv_relu;
+    size_t conv_plane;
     char *out_split;        // GeluSplit: split rows [M][N] of the output times out_scale
     float out_scale;
 };
 
-enum class SEpi : int { Store, Gelu, Residual, Qkv, GeluSplit, Chw };
+enum class SEpi : int { Store, Gelu, Residual, Qkv, GeluSplit, Chw, Conv };
 
 // A product with a non-finite row, in floats: rare, so a plain loop.
 __device__ __attribute__((noinline)) float split_slow_dot(const float *x, const float *w, size_t step, int K) {
     if (!x || !w) return __builtin_nanf("");
     float s = 0.0f;
     for (int k = 0; k < K; k++) s = fmaf(x[k], w[k * step], s);
+    return s;
+}
+
+// One output of a convolution in floats, for an image or weight with an inf or
+// NaN: taps outside the image are zeros that are still multiplied.
+__device__ __attribute__((noinline)) float split_slow_conv(const float *img, const float *w, int taps, int kw, int ic,
+                                                           int ih, int iw, int pad, int relu, int y, int x) {
+    float s = 0.0f;
+    for (int t = 0; t < taps; t++) {
+        const int yy = y + t / kw - pad, xx = x + t % kw - pad;
+        const bool in = yy >= 0 && yy < ih && xx >= 0 && xx < iw;
+        for (int c = 0; c < ic; c++) {
+            float v = in ? img[((size_t)c * ih + yy) * iw + xx] : 0.0f;
+            if (relu) v = fmaxf(v, 0.0f);
+            s = fmaf(v, w[(size_t)t * ic + c], s);
+        }
+    }
     return s;
 }
 
@@ -72,7 +98,7 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     constexpr int STAGE = ROWS * 128;
     static_assert(BM % 8 == 0 && BN % 8 == 0, "whole copies");
     static_assert(TM % 16 == 0 && TN % 16 == 0 && FM % KG == 0, "fragments");
-    static_assert(ST >= 3, "frag reads run a stage ahead of the products");
+    static_assert(ST == 2 || ST == 3, "a stage being filled besides the one being read");
     constexpr int FO = FM / KG;  // fragment rows (of 16 m) a K group finishes
     static_assert(EPI != SEpi::Qkv || TN % 32 == 0, "whole 32-wide RoPE halves per wave");
     extern __shared__ __attribute__((aligned(16))) char smem_c[];
@@ -98,7 +124,8 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     }
     const int m0 = tm * BM, n0 = tn * BN;
     const size_t pitch = (size_t)ar.slices * 128;
-    const char *xb = ar.x + (size_t)m0 * pitch, *wb = ar.w + (size_t)n0 * pitch;
+    const size_t xpitch = EPI == SEpi::Conv ? (size_t)ar.conv_cs * 128 : pitch;
+    const char *xb = ar.x + (size_t)m0 * xpitch, *wb = ar.w + (size_t)n0 * pitch;
 
     // Copy i of this wave moves rows 8 b .. 8 b + 7 (b = i * NW + gw) of the
     // stage; LDS granule p of a row holds global granule p ^ (row % 8), so
@@ -108,16 +135,35 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     for (int i = 0; i < LD; i++) {
         const int b = min(i * NW + gw, CP - 1), row = b * 8 + lane / 8;
         const int r = row < BM ? min(row, ar.M - 1 - m0) : min(row - BM, ar.N - 1 - n0);
-        voff[i] = (uint32_t)(r * (int)pitch + (((lane & 7) ^ (lane >> 3)) << 4));
+        voff[i] = (uint32_t)(r * (int)(row < BM ? xpitch : pitch) + (((lane & 7) ^ (lane >> 3)) << 4));
     }
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)smem_c + kg * ST * STAGE;
+    int conv_at = 0, conv_kin = 0, conv_kx = 0;  // Conv: the slice last copied and its place
+    size_t conv_off = 0;
     auto copy_stage = [&](int slice, int buf) {
         const size_t ko = (size_t)slice * 128;
+        size_t xo = ko;
+        if constexpr (EPI == SEpi::Conv) {
+            // Stages are copied in slice order: step to this one.
+            while (conv_at < slice) {
+                conv_at++;
+                conv_off += 128;
+                if (++conv_kin == ar.conv_cs) {
+                    // conv_off now holds the next pixel: the next tap of the row.
+                    conv_kin = 0;
+                    if (++conv_kx == ar.conv_kw) {
+                        conv_kx = 0;
+                        conv_off += (size_t)(ar.conv_wp - ar.conv_kw) * xpitch;
+                    }
+                }
+            }
+            xo = conv_off;
+        }
 #pragma unroll
         for (int i = 0; i < LD; i++) {
             const int b = min(i * NW + gw, CP - 1);
-            const char *base = b * 8 < BM ? xb : wb;
-            copy16_to_lds(base + ko, voff[i], __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + b * 1024));
+            const char *base = b * 8 < BM ? xb + xo : wb + ko;
+            copy16_to_lds(base, voff[i], __builtin_amdgcn_readfirstlane(lds0 + buf * STAGE + b * 1024));
         }
     };
 
@@ -171,29 +217,27 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
             for (int j = 0; j < FN; j++) low(i, j) = mfma16x16x32_f16(wh[set][j], xl[set][i], low(i, j));
     };
 
-    // Group kg takes slices kg, kg + KG, ...; every group runs the same
-    // number of steps (barriers are workgroup-wide), one past its last slice
-    // reloads that slice and skips the products.
-    const int S = ar.slices;
-    const int steps = (S + KG - 1) / KG;
+    // Group kg takes slices kg, kg + KG, ...; every group runs the same number
+    // of steps (barriers are workgroup-wide).
+    const int S = ar.slices, steps = (S + KG - 1) / KG;
     auto slice_of = [&](int t) { return min(kg + t * KG, S - 1); };
     copy_stage(slice_of(0), 0);
     copy_stage(slice_of(1), 1);
-    copy_stage(slice_of(2), 2);
-    split_wait<2 * LD>();
+    if constexpr (ST == 3) copy_stage(slice_of(2), 2);
+    split_wait<(ST - 1) * LD>();
     __builtin_amdgcn_s_barrier();
     fetch(0, 0);
     // Step t: products of slice t (fragments in registers) while the
     // fragments of slice t + 1 are read; the buffer of slice t, whose reads
-    // ended before this step's barrier, takes slice t + 3.  Copies past the
+    // ended before this step's barrier, takes slice t + ST.  Copies past the
     // last slice reload it into a buffer that is not read again, so that
     // every step is the same basic block.
     auto step = [&](int t, auto setc, int buf) {
         constexpr int set = decltype(setc)::value;
-        split_wait<LD>();  // slice t + 1 landed, slice t + 2 may be in flight
+        split_wait<(ST - 2) * LD>();  // slice t + 1 landed; of three, t + 2 may be in flight
         __builtin_amdgcn_s_barrier();
-        copy_stage(slice_of(t + 3), buf);
-        fetch(set ^ 1, buf == 2 ? 0 : buf + 1);
+        copy_stage(slice_of(t + ST), buf);
+        fetch(set ^ 1, buf == ST - 1 ? 0 : buf + 1);
         products(set);
         // Issue order: a fragment read behind each of the first products.
         constexpr int NR = 2 * (FM + FN), NM = 3 * FM * FN, PER = NM / NR < 1 ? 1 : (NM / NR > 2 ? 2 : NM / NR);
@@ -211,9 +255,9 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     int buf = 0, t = 0;
     for (; t + 1 < mine; t += 2) {
         step(t, P0{}, buf);
-        buf = buf == 2 ? 0 : buf + 1;
+        buf = buf == ST - 1 ? 0 : buf + 1;
         step(t + 1, P1{}, buf);
-        buf = buf == 2 ? 0 : buf + 1;
+        buf = buf == ST - 1 ? 0 : buf + 1;
     }
     if (t < mine) {
         step(t, P0{}, buf);
@@ -270,7 +314,8 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     int exr[FO], ewr[FN][4];
     float bias[FN][4], gamma[FN][4];
 #pragma unroll
-    for (int i = 0; i < FO; i++) exr[i] = ar.ex ? ar.ex[min(mb + 16 * i, ar.M - 1)] : ar.ex_c;
+    for (int i = 0; i < FO; i++)
+        exr[i] = ar.ex ? ar.ex[EPI == SEpi::Conv ? 0 : min(mb + 16 * i, ar.M - 1)] : ar.ex_c;
 #pragma unroll
     for (int j = 0; j < FN; j++)
 #pragma unroll
@@ -312,8 +357,16 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 float t = __builtin_ldexpf(fin[i][j][r], exr[i] + ewr[j][r]);
-                if (exr[i] == kSplitNonFinite || ewr[j][r] == kSplitNonFinite)
-                {
+                if constexpr (EPI == SEpi::Conv) {
+                    // The image's inf and NaN are in its halves: what they
+                    // reach is a NaN here.
+                    if (t != t || ewr[j][r] == kSplitNonFinite) {
+                        const int n = min(nb + 16 * j + r, ar.N - 1), y = m / ar.conv_wp;
+                        t = split_slow_conv(ar.xf, ar.wf + (size_t)n * ar.K, ar.slices / ar.conv_cs, ar.conv_kw,
+                                            ar.conv_cs * 32, ar.conv_ih, ar.conv_iw, ar.conv_pad, ar.conv_relu, y,
+                                            m - y * ar.conv_wp);
+                    }
+                } else if (exr[i] == kSplitNonFinite || ewr[j][r] == kSplitNonFinite) {
                     const int n = min(nb + 16 * j + r, ar.N - 1);
                     t = split_slow_dot(ar.xf ? ar.xf + (size_t)m * ar.K : nullptr,
                                        ar.wf ? ar.wf + (ar.wf_n ? n : (size_t)n * ar.K) : nullptr,
@@ -393,7 +446,14 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
             for (int j = 0; j < FN; j++) {
                 const int n = nb + 16 * j;
                 if (n >= ar.N) continue;
-                if constexpr (EPI == SEpi::Chw) {
+                if constexpr (EPI == SEpi::Conv) {
+                    const int y = m / ar.conv_wp, x = m - y * ar.conv_wp;
+                    if (x >= ar.conv_ow) continue;
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (n + r < ar.N)
+                            ar.c[(size_t)(n + r) * ar.conv_plane + (size_t)y * ar.conv_ow + x] = v[j][r];
+                } else if constexpr (EPI == SEpi::Chw) {
                     // C^T: 16 lanes store 16 consecutive rows of one channel.
 #pragma unroll
                     for (int r = 0; r < 4; r++)
@@ -577,7 +637,7 @@ __global__ __launch_bounds__(256) void ln_output_bound_kernel(const float *__res
 // each, one per wave.  A column strip is read twice, the second time from
 // the cache (strips of at most 1024 rows stay in registers): for the largest
 // magnitudes, then 256 rows at a time through LDS, so that a column's slice
-// is stored from consecutive lanes (1153 x 1003 x 771: both operands SPLIT_OPS us, against 28 in
+// is stored from consecutive lanes (1153 x 1003 x 771: both operands 12.4 us, against 28 in
 // two launches with 64 rows at a time).
 __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__restrict__ a, char *__restrict__ as,
                                                               int *__restrict__ ea, int M, const float *__restrict__ b,
@@ -637,6 +697,91 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
                 store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
             }
         }
+    }
+}
+
+// Largest finite magnitude (as bits) of each chunk of n floats, with ReLU
+// applied first when relu: kConvChunks workgroups, part [kConvChunks].
+constexpr int kConvChunks = 256;
+__global__ __launch_bounds__(256) void conv_absmax_kernel(const float *__restrict__ in, uint32_t *__restrict__ part,
+                                                          size_t n, int relu) {
+    uint32_t mx = 0;
+    auto take = [&](float v) {
+        if (relu) v = fmaxf(v, 0.0f);
+        const uint32_t b = __float_as_uint(v) & 0x7fffffffu;
+        mx = b < 0x7f800000u ? max(mx, b) : mx;
+    };
+    const f32x4 *in4 = reinterpret_cast<const f32x4 *>(in);
+    const size_t n4 = n / 4, stride = (size_t)gridDim.x * 256;
+    size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (; i + 3 * stride < n4; i += 4 * stride) {
+        const f32x4 a = in4[i], b = in4[i + stride], c = in4[i + 2 * stride], d = in4[i + 3 * stride];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            take(a[e]);
+            take(b[e]);
+            take(c[e]);
+            take(d[e]);
+        }
+    }
+    for (; i < n4; i += stride) {
+        const f32x4 a = in4[i];
+#pragma unroll
+        for (int e = 0; e < 4; e++) take(a[e]);
+    }
+    if (blockIdx.x == 0 && threadIdx.x < n - 4 * n4) take(in[4 * n4 + threadIdx.x]);
+    mx = wave_umax(mx);
+    __shared__ uint32_t red[4];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
+}
+
+// The CHW image [cs * 32][ih][iw] as split rows, one per pixel of the grid
+// padded by `pad` (zeros; also the rows past the grid), with one exponent:
+// grid (positions / 64, cs), a workgroup moving 64 positions of 32 channels
+// through LDS (64 consecutive pixels per load, 8 bytes per store).
+__global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__restrict__ in,
+                                                               const uint32_t *__restrict__ part,
+                                                               char *__restrict__ out, int *__restrict__ ex, int cs,
+                                                               int ih, int iw, int pad, int rows, int relu) {
+    __shared__ uint32_t red[4];
+    __shared__ float tile[32][65];
+    uint32_t mx = wave_umax(part[threadIdx.x]);
+    static_assert(kConvChunks == 256, "one chunk per thread");
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    const int wp = iw + 2 * pad, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane, y = p / wp - pad, x = p % wp - pad;
+    const bool inside = p < rows && y >= 0 && y < ih && x >= 0 && x < iw;
+    const float *src = in + ((size_t)(blockIdx.y * 32 + wv * 8) * ih + (inside ? y : 0)) * iw + (inside ? x : 0);
+    const size_t plane = (size_t)ih * iw;
+    float v[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) v[c] = src[c * plane];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        if (relu) v[c] = fmaxf(v[c], 0.0f);
+        tile[wv * 8 + c][lane] = inside ? v[c] : 0.0f;
+    }
+    __syncthreads();
+    const int e = split_exponent(max(max(red[0], red[1]), max(red[2], red[3])));
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ex[0] = e;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int pos = i * 32 + (threadIdx.x >> 3), c4 = 4 * (threadIdx.x & 7), q = blockIdx.x * 64 + pos;
+        if (q >= rows) continue;
+        f16x4 hi, lo;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            _Float16 h, l;
+            const float t = __builtin_ldexpf(tile[c4 + r][pos], -e);
+            split_f16(t, h, l);
+            hi[r] = h;
+            lo[r] = __builtin_isfinite(t) ? l : (_Float16)0.0f;
+        }
+        char *dst = out + ((size_t)q * cs + blockIdx.y) * 128 + c4 * 2;
+        *reinterpret_cast<f16x4 *>(dst) = hi;
+        *reinterpret_cast<f16x4 *>(dst + 64) = lo;
     }
 }
 
@@ -777,6 +922,59 @@ hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *ga
     if (n == 0) return hipSuccess;
     ln_output_bound_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(w, gamma, beta, bias, bound, (int)n, (int)k);
     return hipGetLastError();
+}
+
+size_t conv_split_bytes(const SplitConv &c) {
+    const size_t wp = c.iw + 2 * c.pad, rows = (c.ih + 2 * c.pad) * wp + c.kw - 1;
+    return rows * c.in_c * 4 + (kConvChunks + 1) * sizeof(int);
+}
+
+bool conv_split_fits(const SplitConv &c) {
+    if (c.in_c % 32 != 0 || c.in_c == 0) return false;
+    const size_t wp = c.iw + 2 * c.pad, hp = c.ih + 2 * c.pad;
+    const size_t oh = hp - c.kh + 1, ow = wp - c.kw + 1;
+    // Whole 64 x 64 tiles of the fp32 kernel for half the CUs: below that its
+    // K split over idle CUs is as fast (384 -> 128 on 24 x 36: 28 us against
+    // about 25, 768 -> 128 on 12 x 18: 18), and the staging launches here are not.
+    const size_t tiles = ((c.out_c + 63) / 64) * ((oh * ow + 63) / 64);
+    return tiles >= 128 && c.kh * c.kw * c.in_c >= 256 && hp * wp + c.kw <= (size_t)INT32_MAX / 512 &&
+           c.in_c / 32 <= 65535 && split_gemm_fits(oh * wp, c.out_c, c.kh * c.kw * c.in_c);
+}
+
+hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws) {
+    const int cs = (int)(c.in_c / 32), wp = (int)(c.iw + 2 * c.pad), hp = (int)(c.ih + 2 * c.pad);
+    const int rows = hp * wp + (int)c.kw - 1, oh = hp - (int)c.kh + 1, ow = wp - (int)c.kw + 1;
+    char *img = static_cast<char *>(ws);
+    uint32_t *part = reinterpret_cast<uint32_t *>(img + (size_t)rows * c.in_c * 4);
+    int *ex = reinterpret_cast<int *>(part + kConvChunks);
+    conv_absmax_kernel<<<kConvChunks, 256, 0, s>>>(c.in, part, c.in_c * c.ih * c.iw, c.relu ? 1 : 0);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    conv_split_image_kernel<<<dim3((rows + 63) / 64, cs), 256, 0, s>>>(
+        c.in, part, img, ex, cs, (int)c.ih, (int)c.iw, (int)c.pad, rows, c.relu ? 1 : 0);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    SplitArgs ar{};
+    ar.x = img;
+    ar.w = static_cast<const char *>(c.w);
+    ar.ex = ex;
+    ar.ew = c.ew;
+    ar.M = oh * wp;
+    ar.N = (int)c.out_c;
+    ar.K = (int)(c.kh * c.kw * c.in_c);
+    ar.slices = ar.K / 32;
+    ar.xf = c.in;
+    ar.wf = c.wf;
+    ar.c = c.out;
+    ar.bias = c.bias;
+    ar.conv_cs = cs;
+    ar.conv_kw = (int)c.kw;
+    ar.conv_wp = wp;
+    ar.conv_ow = ow;
+    ar.conv_ih = (int)c.ih;
+    ar.conv_iw = (int)c.iw;
+    ar.conv_pad = (int)c.pad;
+    ar.conv_relu = c.relu ? 1 : 0;
+    ar.conv_plane = (size_t)oh * ow;
+    return launch_split_epi<SEpi::Conv>(s, ar);
 }
 
 hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g) {

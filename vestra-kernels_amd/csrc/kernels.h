@@ -253,6 +253,24 @@ struct SplitGemm {
 };
 hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g);
 
+// Stride-1 convolution of a CHW image on split rows: the image is split
+// channel-last on its padded grid with one exponent for all of it (values
+// below 2^-18 of its largest are held to 2^-40 of that), then multiplied tap by
+// tap.
+struct SplitConv {
+    const float *in;        // [in_c][ih][iw]
+    size_t in_c, ih, iw, out_c, kh, kw, pad;
+    bool relu;              // ReLU on the image
+    const void *w;          // split rows [out_c][kh * kw * in_c], k = (ky, kx, ic)
+    const int *ew;
+    const float *wf;        // the float weight, the same order
+    const float *bias;      // [out_c] or null
+    float *out;             // [out_c][oh][ow]
+};
+bool conv_split_fits(const SplitConv &c);
+size_t conv_split_bytes(const SplitConv &c);
+hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws);
+
 // ---- attention on split rows (k_attn_split.hip) ---------------------------------
 bool attn_split_fits(size_t bh, size_t tokens);
 // Workspace of launch_attn_split_f32.

@@ -2588,11 +2588,16 @@ struct vh_conv2d {
     bool hwc = false;
     float *w = nullptr;
     float *bias = nullptr;  // [out_c] or null
+    // Stride 1, in_c % 32 == 0: split rows of w and their exponents.
+    char *sw = nullptr;
+    int *sew = nullptr;
     ~vh_conv2d() {
         if (!rt) return;
         hipSetDevice(rt->device);
         for (float *p : {w, bias})
             if (p) hipFreeAsync(p, rt->stream);
+        if (sw) hipFreeAsync(sw, rt->stream);
+        if (sew) hipFreeAsync(sew, rt->stream);
     }
 };
 
@@ -2646,6 +2651,20 @@ vh_status conv_run(RtState &s, const vh_conv2d &c, const float *in, size_t ih, s
     const bool plain = c.kh == 1 && c.kw == 1 && c.stride == 1 && c.pad == 0 && !relu;
     float *xh = nullptr, *col = nullptr, *tmp = nullptr;
     vh_status st = VH_OK;
+    const char *direct_env = std::getenv("VESTRA_HIP_CONV_DIRECT");
+    // On split rows and the f16 matrix cores: three launches, but 3 to 4 times
+    // the fp32 form's rate (128 -> 128 on 96 x 144: 21 + 6.5 + 3.9 us
+    // against 69).  VESTRA_HIP_CONV_DIRECT and the GEMM overrides ask for the
+    // fp32 forms.
+    if (c.sw && !direct_env && !fp32_gemm_asked()) {
+        const vh::SplitConv sc{in,     c.in_c, ih,   iw,    c.out_c, c.kh, c.kw,
+                               c.pad,  relu,   c.sw, c.sew, c.w,     c.bias, out};
+        if (vh::conv_split_fits(sc)) {
+            char *ws = nullptr;
+            TRY(split_space(s, vh::conv_split_bytes(sc), &ws));
+            if (ws) return launch(s, "conv_gemm", [&] { return vh::launch_conv_split(s.stream, sc, ws); });
+        }
+    }
     // The direct form reads the image with eight 4-byte loads per thread and
     // k-slice where the staged GEMM issues two 16-byte ones, but saves the
     // staging launches and copies, and its balanced tail splits the K of
@@ -2656,7 +2675,6 @@ vh_status conv_run(RtState &s, const vh_conv2d &c, const float *in, size_t ih, s
     // 169.2 vs 173.3; only stride-1 convolutions with K >= 1152 and more than
     // 4 M outputs stay staged (128 -> 128 on 192 x 288: 168.7 vs 160.4).
     // VESTRA_HIP_CONV_DIRECT=0|1 forces either form (A/B runs).
-    const char *direct_env = std::getenv("VESTRA_HIP_CONV_DIRECT");
     const bool direct_default =
         !(c.stride == 1 && K >= 1152 && npix * c.out_c > ((size_t)4 << 20));
     const bool direct_ok = direct_env ? std::atoi(direct_env) != 0 : direct_default;
@@ -2802,6 +2820,15 @@ vh_status prepare_conv(const vh_runtime *rt, size_t in_c, size_t out_c, size_t k
         st = upload_array(s, weight, n, &c->w, "conv2d weight upload");
     }
     if (!st && bias) st = upload_array(s, bias, out_c, &c->bias, "conv2d bias upload");
+    const size_t K = in_c * kh * kw;
+    if (!st && stride == 1 && in_c % 32 == 0 && split_k_fits(1, out_c, K)) {
+        st = dalloc(s, vh::split_bytes(out_c, K), &c->sw, "split weight allocation");
+        if (!st) st = dalloc(s, out_c, &c->sew, "split weight allocation");
+        if (!st)
+            st = launch(s, "split_weight", [&] {
+                return vh::launch_split_rows(s.stream, c->w, c->sw, c->sew, out_c, K);
+            });
+    }
     if (st) {
         delete c;
         return st;
