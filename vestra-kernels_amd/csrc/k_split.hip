@@ -6,14 +6,15 @@
 // slice (128 bytes per row) is copied straight into LDS (no registers, no
 // LDS stores) through a ring of three stages: while the products of slice t
 // run from registers, the fragments of slice t + 1 are read from LDS and
-// slices t + 2 and t + 3 are in flight from L2.  One barrier per slice.  The
-// granules of a row are XOR-swizzled by the row on the way in, so that a
-// fragment read (16 rows x 4 granules) touches every bank once per 256
-// bytes.  W is the A operand of the matrix instruction, so that a lane ends
-// with four consecutive columns of one row and stores 16 bytes.
+// slices t + 2 and t + 3 are in flight from L2 (t + 2 alone on the largest
+// tile, whose ring is two stages).  One barrier per slice.  The granules of a
+// row are XOR-swizzled by the row on the way in, so that a fragment read (16
+// rows x 4 granules) touches every bank once per 256 bytes.  W is the A
+// operand of the matrix instruction, so that a lane ends with four
+// consecutive columns of one row and stores 16 bytes.
 //
 // What bounds it: at 3460 x 2304 x 768 the f16 matrix cores, whose clock
-// drops to 1.7-1.9 GHz under this load (41 us, 890 TFLOP/s of f16 products; a
+// drops to 1.7-1.9 GHz under this load (40.4 us, 910 TFLOP/s of f16 products; a
 // register-only loop of the same instruction reaches 1.9 PFLOP/s on random
 // data and 2.4 on zeros, an 8192^3 library product in f16 1.13 PFLOP/s); at 865
 // rows the one round of tiles and its start and end (13.6 us for N = 2304
@@ -791,35 +792,37 @@ __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__re
 struct SplitTile {
     int bm, bn;
     float slice_us, fixed_us;
+    bool qkv;    // waves a whole number of 32-wide RoPE halves across
+    bool alone;  // takes more than half the LDS
 };
 constexpr SplitTile kSplitTiles[] = {
-    {128, 256, 0.858f, 5.0f},  // 2 x 4 waves
-    {128, 128, 0.480f, 5.9f},  // 2 x 4 waves
-    {128, 96, 0.378f, 5.0f},   // 4 x 2 waves (not Qkv: waves 48 columns wide)
-    {64, 128, 0.286f, 3.9f},   // 2 x 4 waves, two workgroups per CU
-    {64, 64, 0.211f, 3.0f},    // 2 x 2 waves, two K groups
-    {64, 32, 0.125f, 3.7f},    // 2 x 1 waves, two K groups, two workgroups per CU
+    {128, 256, 0.858f, 5.0f, true, true},   // 2 x 4 waves
+    {128, 192, 0.646f, 6.0f, false, true},  // 2 x 4 waves
+    {128, 128, 0.480f, 5.9f, true, true},   // 2 x 4 waves
+    {128, 96, 0.378f, 5.0f, false, true},   // 4 x 2 waves
+    {64, 128, 0.286f, 3.9f, true, false},   // 2 x 4 waves, two workgroups per CU
+    {64, 64, 0.211f, 3.0f, true, true},     // 2 x 2 waves, two K groups
+    {64, 32, 0.125f, 3.7f, true, false},    // 2 x 1 waves, two K groups, two workgroups per CU
 };
 
 // The tile with the lowest predicted time: every CU runs ceil(tiles / 256)
-// tiles of slices * slice_us, and a tile that has the CU alone (more than
-// half the LDS) adds about 2 us of prologue and epilogue per further round.
-// Of the 13 shapes swept on MI355X the prediction names the fastest of
-// these tiles in all but one, which it misses by 2% (865 x 3072 x 768: 18.1
-// us here, 20.5 for 64 x 128, 23.9 for 64 x 64; 3460 x 2304 x 768: 41.5 for
-// 128 x 256, 45.9 for 64 x 128; 97 x 2304 x 768: 6.2 for 64 x 32, 10.3 for
-// 64 x 128).
+// tiles of slices * slice_us, and a tile that has the CU alone adds about 2 us
+// of prologue and epilogue per further round.  Of the 14 shapes swept on
+// MI355X the prediction names the fastest of these tiles in all but one, which
+// it misses by 2% (865 x 3072 x 768: 18.1 us here, 20.5 for 64 x 128, 23.9 for
+// 64 x 64; 3460 x 2304 x 768: 40.4 for 128 x 256, 45.9 for 64 x 128; 3460 x
+// 3072 x 768: 57.2 for 128 x 192, 63.9 for 128 x 128 and 65.2 for 128 x 256; 97
+// x 2304 x 768: 6.2 for 64 x 32, 10.3 for 64 x 128).
 int pick_split_tile(size_t m, size_t n, int slices, bool qkv, float *predicted_us = nullptr) {
     int best = 0;
-    float best_us = 0.0f;
-    for (int i = 0; i < 6; i++) {
-        if (qkv && i == 2) continue;
+    float best_us = INFINITY;
+    for (int i = 0; i < (int)(sizeof(kSplitTiles) / sizeof(kSplitTiles[0])); i++) {
         const SplitTile &t = kSplitTiles[i];
+        if (qkv && !t.qkv) continue;
         const size_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
         const float rounds = (float)((tiles + 255) / 256);
-        const bool alone = i != 3 && i != 5;
-        const float us = t.fixed_us + rounds * slices * t.slice_us + (alone ? 2.0f * (rounds - 1.0f) : 0.0f);
-        if (i == 0 || us < best_us) {
+        const float us = t.fixed_us + rounds * slices * t.slice_us + (t.alone ? 2.0f * (rounds - 1.0f) : 0.0f);
+        if (us < best_us) {
             best = i;
             best_us = us;
         }
@@ -830,7 +833,9 @@ int pick_split_tile(size_t m, size_t n, int slices, bool qkv, float *predicted_u
 
 template <int BM, int BN, int WM, int WN, int KG, SEpi EPI>
 hipError_t launch_split_tile(hipStream_t s, const SplitArgs &ar) {
-    constexpr int ST = 3;
+    // The largest tile's step is long enough for one stage in flight (40.4 us
+    // against 42.5 for three stages at 3460 x 2304 x 768).
+    constexpr int ST = BM * BN >= 128 * 256 ? 2 : 3;
     constexpr size_t stage = (size_t)KG * ST * (BM + BN) * 128;
     constexpr size_t xch = KG > 1 ? (size_t)KG * BM * BN * 4 : 0;
     constexpr size_t lds = stage > xch ? stage : xch;
@@ -846,14 +851,18 @@ hipError_t launch_split_tile(hipStream_t s, const SplitArgs &ar) {
 
 template <SEpi EPI>
 hipError_t launch_split_epi(hipStream_t s, const SplitArgs &ar) {
-    switch (pick_split_tile(ar.M, ar.N, ar.slices, EPI == SEpi::Qkv)) {
+    constexpr bool Q = EPI == SEpi::Qkv;
+    switch (pick_split_tile(ar.M, ar.N, ar.slices, Q)) {
         case 0: return launch_split_tile<128, 256, 2, 4, 1, EPI>(s, ar);
-        case 1: return launch_split_tile<128, 128, 2, 4, 1, EPI>(s, ar);
-        case 2:
-            if constexpr (EPI != SEpi::Qkv) return launch_split_tile<128, 96, 4, 2, 1, EPI>(s, ar);
+        case 1:
+            if constexpr (!Q) return launch_split_tile<128, 192, 2, 4, 1, EPI>(s, ar);
             return hipErrorInvalidValue;
-        case 3: return launch_split_tile<64, 128, 2, 4, 1, EPI>(s, ar);
-        case 4: return launch_split_tile<64, 64, 2, 2, 2, EPI>(s, ar);
+        case 2: return launch_split_tile<128, 128, 2, 4, 1, EPI>(s, ar);
+        case 3:
+            if constexpr (!Q) return launch_split_tile<128, 96, 4, 2, 1, EPI>(s, ar);
+            return hipErrorInvalidValue;
+        case 4: return launch_split_tile<64, 128, 2, 4, 1, EPI>(s, ar);
+        case 5: return launch_split_tile<64, 64, 2, 2, 2, EPI>(s, ar);
         default: return launch_split_tile<64, 32, 2, 1, 2, EPI>(s, ar);
     }
 }
