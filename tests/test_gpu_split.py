@@ -23,10 +23,12 @@ def _bound(x, w):
 
 
 # One row; ragged rows, columns and K on every tile (64 x 32, 64 x 64, 64 x
-# 128, 128 x 96, 128 x 128, 128 x 192, 128 x 256), K of 2, 3 and an odd count of slices.
+# 128, 128 x 96, 128 x 128, 128 x 192, 128 x 256), K of 2, 3 and an odd count of
+# slices, and K shared out over 2, 3 and 4 workgroups.
 SHAPES = [(1, 64, 1), (65, 64, 33), (63, 70, 95), (97, 96, 770), (257, 101, 771), (500, 768, 768),
           (865, 768, 2304), (865, 100, 3074), (1153, 1003, 771), (1800, 416, 1500), (1500, 330, 3301),
-          (3460, 768, 2307)]
+          (3460, 768, 2307), (97, 2563, 70), (257, 3072, 768), (300, 2402, 500),
+          (400, 3000, 400)]
 
 
 @pytest.mark.parametrize("m, k, n", SHAPES)

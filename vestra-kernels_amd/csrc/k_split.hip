@@ -41,6 +41,13 @@ struct SplitArgs {
     const int *ex, *ew;     // row exponents (ex null: ex_c for every row)
     int ex_c;
     int M, N, slices;       // slices = Kp / 32
+    // K pieces: a tile's slices are shared out over `pieces` workgroups, whose
+    // tiles (in `partial`, [tile][piece][value][thread]) the last to finish
+    // sums in piece order; piece_cnt counts a tile's arrivals, zero between
+    // launches.
+    int pieces;
+    float *partial;  // null: whole tiles only
+    unsigned *piece_cnt;
     const float *xf, *wf;   // the f32 rows [M][K], [N][K] (non-finite rows)
     int K, wf_n;            // wf_n: 0, or wf is [K][wf_n]
     float *c;
@@ -61,6 +68,8 @@ struct SplitArgs {
     char *out_split;        // GeluSplit: split rows [M][N] of the output times out_scale
     float out_scale;
 };
+
+constexpr int kSplitMaxPieces = 4;
 
 enum class SEpi : int { Store, Gelu, Residual, Qkv, GeluSplit, Chw, Conv };
 
@@ -89,7 +98,7 @@ __device__ __attribute__((noinline)) float split_slow_conv(const float *img, con
     return s;
 }
 
-template <int BM, int BN, int WM, int WN, int KG, int ST, SEpi EPI>
+template <int BM, int BN, int WM, int WN, int KG, int ST, SEpi EPI, bool PIECES>
 __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs ar) {
     constexpr int NW = WM * WN, GT = NW * 64;
     constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 16, FN = TN / 16;
@@ -113,11 +122,16 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     // Workgroups go round-robin over the 8 XCDs; renumbered so that an XCD's
     // share is a run of tiles that walks 8 row tiles column by column.
     const int nx = (ar.N + BN - 1) / BN, ny = (ar.M + BM - 1) / BM;
-    int tm, tn;
+    int tm, tn, piece = 0, tile;
     {
-        const int total = nx * ny, bid = blockIdx.x;
+        const int total = nx * ny * (PIECES ? ar.pieces : 1), bid = blockIdx.x;
         const int q = total / 8, r = total % 8, xcd = bid % 8;
-        const int t = xcd * q + min(xcd, r) + bid / 8;
+        int t = xcd * q + min(xcd, r) + bid / 8;
+        if constexpr (PIECES) {
+            piece = t % ar.pieces;
+            t /= ar.pieces;
+        }
+        tile = t;
         const int gm = min(8, ny), group = t / (gm * nx), first = group * gm;
         const int rows = min(ny - first, gm), local = t - group * gm * nx;
         tm = first + local % rows;
@@ -218,10 +232,16 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
             for (int j = 0; j < FN; j++) low(i, j) = mfma16x16x32_f16(wh[set][j], xl[set][i], low(i, j));
     };
 
-    // Group kg takes slices kg, kg + KG, ...; every group runs the same number
-    // of steps (barriers are workgroup-wide).
-    const int S = ar.slices, steps = (S + KG - 1) / KG;
-    auto slice_of = [&](int t) { return min(kg + t * KG, S - 1); };
+    // Of the piece's slices [beg, beg + S) group kg takes every KG-th; every
+    // group runs the same number of steps (barriers are workgroup-wide).
+    int beg = 0, S = ar.slices;
+    if constexpr (PIECES) {
+        const int each = (ar.slices + ar.pieces - 1) / ar.pieces;
+        beg = piece * each;
+        S = min(each, ar.slices - beg);
+    }
+    const int steps = (S + KG - 1) / KG;
+    auto slice_of = [&](int t) { return beg + min(kg + t * KG, S - 1); };
     copy_stage(slice_of(0), 0);
     copy_stage(slice_of(1), 1);
     if constexpr (ST == 3) copy_stage(slice_of(2), 2);
@@ -306,6 +326,59 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
         for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int j = 0; j < FN; j++) fin[i][j] = acc[i][j];
+    }
+
+    if constexpr (PIECES) {
+        // Publish, count in, and go on only as the last of the tile.  The
+        // partials are agent-scope atomic stores, which write through the
+        // XCD's L2 to where every XCD reads; each thread waits for its own to
+        // be acknowledged (vmcnt counts stores; the asm's memory clobber keeps
+        // them before it), the barrier orders those waits before thread 0's
+        // increment, and the last piece reads with agent-scope atomic loads
+        // after it.  No piece waits for another, so the grid drains at any
+        // residency.
+        constexpr int NT = NW * KG * 64, PER = FO * FN * 4;
+        __shared__ int last_piece;
+        float *base = ar.partial + (size_t)tile * ar.pieces * PER * NT + tid;
+        float *mine = base + (size_t)piece * PER * NT;
+#pragma unroll
+        for (int i = 0; i < FO; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    __hip_atomic_store(mine + ((i * FN + j) * 4 + r) * NT, fin[i][j][r], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0)
+            last_piece = __hip_atomic_fetch_add(ar.piece_cnt + tile, 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(ar.pieces - 1);
+        __syncthreads();
+        if (!last_piece) return;
+        if (tid == 0) __hip_atomic_store(ar.piece_cnt + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // Every load before the first sum, under a uniform branch per piece.
+        float pv[kSplitMaxPieces][PER];
+#pragma unroll
+        for (int p = 0; p < kSplitMaxPieces; p++)
+#pragma unroll
+            for (int e = 0; e < PER; e++)
+                pv[p][e] = p < ar.pieces ? __hip_atomic_load(base + ((size_t)p * PER + e) * NT, __ATOMIC_RELAXED,
+                                                             __HIP_MEMORY_SCOPE_AGENT)
+                                         : 0.0f;
+#pragma unroll
+        for (int i = 0; i < FO; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int e = (i * FN + j) * 4 + r;
+                    float v = pv[0][e];
+#pragma unroll
+                    for (int p = 1; p < kSplitMaxPieces; p++)
+                        if (p < ar.pieces) v += pv[p][e];
+                    fin[i][j][r] = v;
+                }
     }
 
     // Epilogue: lane (li, lh) holds C[m][n .. n + 3], m = mb + 16 i, n = nb + 16 j.
@@ -794,44 +867,56 @@ struct SplitTile {
     float slice_us, fixed_us;
     bool qkv;    // waves a whole number of 32-wide RoPE halves across
     bool alone;  // takes more than half the LDS
+    bool pieces;
 };
 constexpr SplitTile kSplitTiles[] = {
-    {128, 256, 0.858f, 5.0f, true, true},   // 2 x 4 waves
-    {128, 192, 0.646f, 6.0f, false, true},  // 2 x 4 waves
-    {128, 128, 0.480f, 5.9f, true, true},   // 2 x 4 waves
-    {128, 96, 0.378f, 5.0f, false, true},   // 4 x 2 waves
-    {64, 128, 0.286f, 3.9f, true, false},   // 2 x 4 waves, two workgroups per CU
-    {64, 64, 0.211f, 3.0f, true, true},     // 2 x 2 waves, two K groups
-    {64, 32, 0.125f, 3.7f, true, false},    // 2 x 1 waves, two K groups, two workgroups per CU
+    {128, 256, 0.858f, 5.0f, true, true, false},   // 2 x 4 waves
+    {128, 192, 0.646f, 6.0f, false, true, false},  // 2 x 4 waves
+    {128, 128, 0.480f, 5.9f, true, true, false},   // 2 x 4 waves
+    {128, 96, 0.378f, 5.0f, false, true, false},   // 4 x 2 waves
+    {64, 128, 0.286f, 3.9f, true, false, false},   // 2 x 4 waves, two workgroups per CU
+    {64, 64, 0.211f, 3.0f, true, true, true},      // 2 x 2 waves, two K groups
+    {64, 32, 0.125f, 3.7f, true, false, true},     // 2 x 1 waves, two K groups, two workgroups per CU
+};
+
+struct SplitPlan {
+    int tile, pieces;
+    float us;
 };
 
 // The tile with the lowest predicted time: every CU runs ceil(tiles / 256)
-// tiles of slices * slice_us, and a tile that has the CU alone adds about 2 us
-// of prologue and epilogue per further round.  Of the 14 shapes swept on
-// MI355X the prediction names the fastest of these tiles in all but one, which
-// it misses by 2% (865 x 3072 x 768: 18.1 us here, 20.5 for 64 x 128, 23.9 for
-// 64 x 64; 3460 x 2304 x 768: 40.4 for 128 x 256, 45.9 for 64 x 128; 3460 x
-// 3072 x 768: 57.2 for 128 x 192, 63.9 for 128 x 128 and 65.2 for 128 x 256; 97
-// x 2304 x 768: 6.2 for 64 x 32, 10.3 for 64 x 128).
-int pick_split_tile(size_t m, size_t n, int slices, bool qkv, float *predicted_us = nullptr) {
-    int best = 0;
-    float best_us = INFINITY;
+// tiles of slices * slice_us, and a tile that has the CU alone (more than
+// half the LDS) adds about 2 us of prologue and epilogue per further round.
+// Grids of at most half the CUs may share a tile's K out over 2 to 4
+// workgroups of at least 8 slices: the partials, which go past the L2 both
+// ways, take 1.5 us and 1.8 TB/s.  So it pays for few rows only (97 x 768 x
+// 3072 10.0 us in 4 pieces, 14.9 whole; 865 x 768 x 3072 22.2 in 3 pieces of 64 x
+// 128, 22.0 whole on 64 x 64).  The prediction names the fastest or comes
+// within 3% of it on the shapes swept on MI355X (865 x 3072 x 768: 18.1 us
+// here, 20.5 for 64 x 128, 23.9 for 64 x 64; 3460 x 2304 x 768: 40.4 for 128 x
+// 256, 45.9 for 64 x 128; 3460 x 3072 x 768: 57.2 for 128 x 192, 63.9 for 128 x
+// 128 and 65.2 for 128 x 256; 97 x 2304 x 768: 6.2 for 64 x 32, 10.3 for 64 x
+// 128).
+SplitPlan plan_split(size_t m, size_t n, int slices, bool qkv, bool pieces_ok) {
+    SplitPlan best{0, 1, INFINITY};
     for (int i = 0; i < (int)(sizeof(kSplitTiles) / sizeof(kSplitTiles[0])); i++) {
         const SplitTile &t = kSplitTiles[i];
         if (qkv && !t.qkv) continue;
         const size_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
         const float rounds = (float)((tiles + 255) / 256);
-        const float us = t.fixed_us + rounds * slices * t.slice_us + (t.alone ? 2.0f * (rounds - 1.0f) : 0.0f);
-        if (us < best_us) {
-            best = i;
-            best_us = us;
+        const float whole = t.fixed_us + rounds * slices * t.slice_us + (t.alone ? 2.0f * (rounds - 1.0f) : 0.0f);
+        if (whole < best.us) best = SplitPlan{i, 1, whole};
+        for (int p = 2; pieces_ok && t.pieces && p <= kSplitMaxPieces; p++) {
+            const int each = (slices + p - 1) / p;
+            if (tiles * p > 256 || each < 8 || each * (p - 1) >= slices) continue;
+            const float us = t.fixed_us + each * t.slice_us + 1.5f + (float)m * (float)n * (float)(8 * p) / 1.8e6f;
+            if (us < best.us) best = SplitPlan{i, p, us};
         }
     }
-    if (predicted_us) *predicted_us = best_us;
     return best;
 }
 
-template <int BM, int BN, int WM, int WN, int KG, SEpi EPI>
+template <int BM, int BN, int WM, int WN, int KG, SEpi EPI, bool PIECES = false>
 hipError_t launch_split_tile(hipStream_t s, const SplitArgs &ar) {
     // The largest tile's step is long enough for one stage in flight (40.4 us
     // against 42.5 for three stages at 3460 x 2304 x 768).
@@ -840,19 +925,21 @@ hipError_t launch_split_tile(hipStream_t s, const SplitArgs &ar) {
     constexpr size_t xch = KG > 1 ? (size_t)KG * BM * BN * 4 : 0;
     constexpr size_t lds = stage > xch ? stage : xch;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    auto kernel = gemm_split_kernel<BM, BN, WM, WN, KG, ST, EPI>;
+    auto kernel = gemm_split_kernel<BM, BN, WM, WN, KG, ST, EPI, PIECES>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
-    const size_t tiles = (size_t)((ar.M + BM - 1) / BM) * (size_t)((ar.N + BN - 1) / BN);
+    const size_t tiles = (size_t)((ar.M + BM - 1) / BM) * (size_t)((ar.N + BN - 1) / BN) * (size_t)ar.pieces;
     if (tiles > (size_t)INT32_MAX / (WM * WN * KG * 64)) return hipErrorInvalidValue;
     kernel<<<(unsigned)tiles, WM * WN * KG * 64, lds, s>>>(ar);
     return hipGetLastError();
 }
 
 template <SEpi EPI>
-hipError_t launch_split_epi(hipStream_t s, const SplitArgs &ar) {
+hipError_t launch_split_epi(hipStream_t s, SplitArgs ar) {
+    const SplitPlan p = plan_split(ar.M, ar.N, ar.slices, EPI == SEpi::Qkv, ar.partial != nullptr);
+    ar.pieces = p.pieces;
     constexpr bool Q = EPI == SEpi::Qkv;
-    switch (pick_split_tile(ar.M, ar.N, ar.slices, Q)) {
+    switch (p.tile) {
         case 0: return launch_split_tile<128, 256, 2, 4, 1, EPI>(s, ar);
         case 1:
             if constexpr (!Q) return launch_split_tile<128, 192, 2, 4, 1, EPI>(s, ar);
@@ -862,8 +949,12 @@ hipError_t launch_split_epi(hipStream_t s, const SplitArgs &ar) {
             if constexpr (!Q) return launch_split_tile<128, 96, 4, 2, 1, EPI>(s, ar);
             return hipErrorInvalidValue;
         case 4: return launch_split_tile<64, 128, 2, 4, 1, EPI>(s, ar);
-        case 5: return launch_split_tile<64, 64, 2, 2, 2, EPI>(s, ar);
-        default: return launch_split_tile<64, 32, 2, 1, 2, EPI>(s, ar);
+        case 5:
+            return p.pieces > 1 ? launch_split_tile<64, 64, 2, 2, 2, EPI, true>(s, ar)
+                                : launch_split_tile<64, 64, 2, 2, 2, EPI>(s, ar);
+        default:
+            return p.pieces > 1 ? launch_split_tile<64, 32, 2, 1, 2, EPI, true>(s, ar)
+                                : launch_split_tile<64, 32, 2, 1, 2, EPI>(s, ar);
     }
 }
 
@@ -888,8 +979,7 @@ bool split_gemm_fits(size_t m, size_t n, size_t k) {
 // splits no K (865 x 768 x 96 19.3 and 11).
 bool split_gemm_pays(size_t m, size_t n, size_t k, size_t split_values, bool whole_tiles) {
     const int slices = (int)((k + 31) / 32);
-    float gemm_us;
-    pick_split_tile(m, n, slices, false, &gemm_us);
+    const float gemm_us = plan_split(m, n, slices, false, true).us;
     const float split_us = 2.5f + (float)split_values * 8.0f / 3e6f + gemm_us;
     const float tiles = (float)((m + 63) / 64) * (float)((n + 63) / 64);
     float rounds = tiles > 256.0f ? tiles / 256.0f + 0.3f : (tiles > 128.0f ? tiles / 256.0f : 0.5f);
@@ -1013,6 +1103,10 @@ hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g) {
     ar.rot = g.rot;
     for (int i = 0; i < 3; i++)
         ar.qkv_scale[i] = g.qkv_split[i] ? __builtin_ldexpf(1.0f, -g.qkv_ex[i]) : 0.0f;
+    if (g.piece_cnt && g.piece_cnt_n >= 256 && g.partial_floats >= kSplitPieceFloats) {
+        ar.partial = g.partial;
+        ar.piece_cnt = g.piece_cnt;
+    }
     ar.out_split = static_cast<char *>(g.out_split);
     ar.out_scale = g.out_split ? __builtin_ldexpf(1.0f, -g.out_ex) : 0.0f;
     if (g.out_split) {

@@ -246,11 +246,19 @@ struct SplitGemm {
     int qkv_ex[3];
     size_t tokens, heads;
     const float *rot;
+    // Room for K pieces of the tiles of small grids (kSplitPieceFloats floats
+    // and 256 counters, zero on entry and on return), or null.  Launches
+    // sharing them must not overlap in time.
+    float *partial;
+    size_t partial_floats;
+    unsigned *piece_cnt;
+    size_t piece_cnt_n;
     // Gelu only: the output as split rows [m][n] (n % 32 == 0) with the one
     // exponent out_ex instead of c; |output| <= 2^(15 + out_ex).
     void *out_split;
     int out_ex;
 };
+constexpr size_t kSplitPieceFloats = (size_t)256 * 64 * 64;
 hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g);
 
 // Stride-1 convolution of a CHW image on split rows: the image is split

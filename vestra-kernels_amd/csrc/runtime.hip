@@ -481,6 +481,19 @@ vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
     return VH_OK;
 }
 
+// The same room for the K pieces of a split GEMM (both run on the runtime's one
+// stream, so never at once).  Without it a grid runs whole tiles: under
+// capture nothing is allocated.
+void piece_workspace(RtState &s, vh::SplitGemm &g) {
+    static_assert(vh::kSplitPieceFloats <= vh::kTailFloats && vh::kTailTiles >= 256, "the tail workspace fits");
+    vh::GemmArgs t{};
+    if ((!s.tw && capturing(s.stream)) || tail_workspace(s, t) != VH_OK) return;
+    g.partial = t.tail_ws;
+    g.partial_floats = t.tail_ws_floats;
+    g.piece_cnt = t.tail_cnt;
+    g.piece_cnt_n = t.tail_cnt_n;
+}
+
 // The flash grid holds heads * ceil(tokens/64) * splits workgroups of 256
 // threads; its thread count must fit the 32-bit launch limit.
 bool flash_grid_fits(size_t heads, size_t tokens) {
@@ -747,6 +760,7 @@ vh_status try_split(RtState &s, const Lin &L, vh::SplitGemm g, const char *name,
     if (!x.x) return VH_OK;
     g.x = x.x;
     g.ex = x.ex;
+    piece_workspace(s, g);
     *done = true;
     return launch(s, name, [&] { return vh::launch_gemm_split(s.stream, g); });
 }
@@ -1221,6 +1235,7 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
             g.k = k;
             g.epi = vh::Epi::Store;
             g.c = t->ptr;
+            piece_workspace(s, g);
             st = launch(s, "split_operands", [&] {
                 return vh::launch_split_operands(s.stream, a->ptr, x, ex, m, b->ptr, w, ew, k, n);
             });
@@ -2408,6 +2423,7 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
             g.qkv_split[i] = !b.qn_g || i == 2;
             g.qkv_ex[i] = b.qkv_ex[i];
         }
+        piece_workspace(s, g);
         TRY(launch(s, "gemm_qkv_rope", [&] { return vh::launch_gemm_split(s.stream, g); }));
     }
     if (b.qn_g)
@@ -2425,6 +2441,7 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
         vh::SplitGemm g = split_gemm_args(b.proj, nullptr, M, vh::Epi::Residual, x);
         g.x = att;
         g.ex_c = b.qkv_ex[2];
+        piece_workspace(s, g);
         TRY(launch(s, "gemm_proj_residual", [&] { return vh::launch_gemm_split(s.stream, g); }));
     }
     TRY(norm(b.ln2_g, b.ln2_b));
@@ -2434,11 +2451,13 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
         g.ex = hex;
         g.out_split = f;
         g.out_ex = b.fc1_ex;
+        piece_workspace(s, g);
         TRY(launch(s, "gemm_fc1_gelu", [&] { return vh::launch_gemm_split(s.stream, g); }));
     }
     vh::SplitGemm g = split_gemm_args(b.fc2, nullptr, M, vh::Epi::Residual, x);
     g.x = f;
     g.ex_c = b.fc1_ex;
+    piece_workspace(s, g);
     return launch(s, "gemm_fc2_residual", [&] { return vh::launch_gemm_split(s.stream, g); });
 }
 
