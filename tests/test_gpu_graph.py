@@ -91,3 +91,30 @@ def test_encoder_graph_replays_equal_eager(rt, layers, q8):
     finally:
         hip.hipGraphExecDestroy(exe)
         hip.hipGraphDestroy(graph)
+
+
+def test_graph_keeps_its_workspace_when_a_later_run_needs_a_larger_one(rt):
+    """The workspace a capture was given outlives the graph's use of it: an
+    eager run of more rows gets a larger one and the replays stay right."""
+    hip = _hip()
+    stream = ctypes.c_void_p(rt.stream())
+    k = n = 768
+    lin = rt.prepare_linear_f32(k, n, seeded.normal(9500, k * n, 0.02), seeded.normal(9501, n))
+    x = rt.upload_f32(seeded.normal(9502, 865 * k))
+    r0 = seeded.normal(9503, 865 * n)
+    res, ref = rt.upload_f32(r0), rt.upload_f32(r0)
+    lin.run_residual(x, 865, ref)
+    rt.synchronize()
+    exp = rt.download_f32(ref)
+    graph, exe = _capture(hip, stream, lambda: lin.run_residual(x, 865, res))
+    try:
+        many = 40000
+        big, acc = rt.upload_f32(seeded.normal(9504, many * k)), rt.upload_f32(np.zeros(many * n, np.float32))
+        lin.run_residual(big, many, acc)
+        rt.synchronize()
+        assert hip.hipGraphLaunch(exe, stream) == 0
+        assert hip.hipStreamSynchronize(stream) == 0
+        assert_bits_equal(rt.download_f32(res), exp, "replay after the growth")
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)

@@ -144,6 +144,8 @@ struct RtState {
     size_t aq_bytes = 0;
     char *sx = nullptr;                         // grow-only split rows of a projection's input
     size_t sx_bytes = 0;
+    bool fw_recorded = false, sx_recorded = false;  // fw, sx: a captured graph may hold the block
+    std::vector<void *> recorded;                   // outgrown blocks of that kind
     float *tw = nullptr;                        // balanced-tail GEMM partials
     unsigned *tcnt = nullptr;                   // and arrival counters (zeroed once)
     float *scratch = nullptr;                   // this device's copy of `scratch` (below)
@@ -165,6 +167,7 @@ struct RtState {
         if (fcnt) hipFree(fcnt);
         if (aq) hipFree(aq);
         if (sx) hipFree(sx);
+        for (void *p : recorded) hipFree(p);
         if (tw) hipFree(tw);
         if (tcnt) hipFree(tcnt);
 
@@ -177,6 +180,19 @@ struct RtState {
         hipStreamDestroy(stream);
     }
 };
+
+// Device memory of the runtime's own, with the tensor pool's blocks given back
+// if it takes them.
+hipError_t device_malloc(RtState &s, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    hipGetLastError();
+    s.pool.give_back(s.stream);
+    hipStreamSynchronize(s.stream);
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
 
 using Rt = std::shared_ptr<RtState>;
 
@@ -308,6 +324,11 @@ vh_status dalloc(RtState &s, size_t count, T **out, const char *what) {
     size_t bytes = (count ? count : 1) * sizeof(T);
     void *p = nullptr;
     hipError_t e = hipMallocAsync(&p, bytes, s.stream);
+    if (e != hipSuccess && !capturing(s.stream)) {
+        hipGetLastError();
+        s.pool.give_back(s.stream);
+        e = hipMallocAsync(&p, bytes, s.stream);
+    }
     if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg(what, e));
     *out = static_cast<T *>(p);
     return VH_OK;
@@ -425,7 +446,7 @@ vh_status workspace(RtState &s, size_t floats, float **out) {
         if (s.ws) hipFree(s.ws);
         s.ws = nullptr;
         s.ws_floats = 0;
-        hipError_t e = hipMalloc(&s.ws, floats * sizeof(float));
+        hipError_t e = device_malloc(s, (void **)&s.ws, floats * sizeof(float));
         if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("block workspace allocation", e));
         s.ws_floats = floats;
     }
@@ -446,7 +467,7 @@ vh_status splitk_workspace(RtState &s, size_t m, size_t n, float **out, size_t *
         if (s.sk) hipFree(s.sk);
         s.sk = nullptr;
         s.sk_floats = 0;
-        hipError_t e = hipMalloc(&s.sk, need * sizeof(float));
+        hipError_t e = device_malloc(s, (void **)&s.sk, need * sizeof(float));
         if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("split-K workspace allocation", e));
         s.sk_floats = need;
     }
@@ -462,7 +483,7 @@ vh_status splitk_workspace(RtState &s, size_t m, size_t n, float **out, size_t *
 vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
     if (!s.tw) {
         hipStreamSynchronize(s.stream);
-        hipError_t e = hipMalloc(&s.tw, (vh::kTailFloats + vh::kTailStatFloats) * sizeof(float));
+        hipError_t e = device_malloc(s, (void **)&s.tw, (vh::kTailFloats + vh::kTailStatFloats) * sizeof(float));
         if (e == hipSuccess) e = hipMalloc(&s.tcnt, vh::kTailTiles * sizeof(unsigned));
         if (e == hipSuccess) e = hipMemsetAsync(s.tcnt, 0, vh::kTailTiles * sizeof(unsigned), s.stream);
         if (e != hipSuccess) {
@@ -503,6 +524,33 @@ bool flash_grid_fits(size_t heads, size_t tokens) {
            items <= (size_t)UINT32_MAX / 256 / vh::kMaxFlashSplits;
 }
 
+// Grows the workspace *p of *have units to `need` units of `unit` bytes; false
+// where it stays too small: no memory, or the stream is being captured, where
+// nothing can be allocated.  A block that a capture was given may be in a graph
+// that is yet to be replayed, so growth keeps it until the runtime ends.
+template <typename T>
+bool grow_workspace(RtState &s, T **p, size_t *have, size_t need, bool *in_graph) {
+    if (capturing(s.stream)) {
+        if (*have >= need) *in_graph = true;
+        return *have >= need;
+    }
+    if (*have >= need) return true;
+    hipStreamSynchronize(s.stream);
+    if (*p && *in_graph) s.recorded.push_back(*p);
+    else if (*p) hipFree(*p);
+    *p = nullptr;
+    *have = 0;
+    *in_graph = false;
+    void *fresh = nullptr;
+    if (device_malloc(s, &fresh, need * sizeof(T)) != hipSuccess) {
+        hipGetLastError();
+        return false;
+    }
+    *p = static_cast<T *>(fresh);
+    *have = need;
+    return true;
+}
+
 // VESTRA_HIP_FLASH_* choose between forms of the fp32 flash kernels (A/B
 // studies and tests, read per call): set, they ask for those kernels.
 bool fp32_flash_asked() {
@@ -521,18 +569,7 @@ vh_status try_attn_split(RtState &s, const float *q, const float *k, const float
     *done = false;
     if (!vh::attn_split_fits(bh, tokens) || fp32_flash_asked()) return VH_OK;
     const size_t need = (vh::attn_split_bytes(bh, tokens) + sizeof(float) - 1) / sizeof(float);
-    if (s.fw_floats < need) {
-        hipStreamSynchronize(s.stream);
-        if (s.fw) hipFree(s.fw);
-        s.fw = nullptr;
-        s.fw_floats = 0;
-        if (hipMalloc(&s.fw, need * sizeof(float)) != hipSuccess) {
-            hipGetLastError();
-            s.fw = nullptr;
-            return VH_OK;
-        }
-        s.fw_floats = need;
-    }
+    if (!grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded)) return VH_OK;
     *done = true;
     return launch(s, "flash_attention", [&] {
         return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, s.fw);
@@ -549,14 +586,7 @@ vh_status flash(RtState &s, const float *q, const float *k, const float *v, floa
     // or the in-kernel merge's); without them the kernel runs unsplit.
     const size_t need =
         std::max(vh::flash_workspace_floats(bh, tokens), vh::flash_fused_workspace_floats(bh, tokens));
-    if (s.fw_floats < need) {
-        hipStreamSynchronize(s.stream);
-        if (s.fw) hipFree(s.fw);
-        s.fw = nullptr;
-        s.fw_floats = 0;
-        if (hipMalloc(&s.fw, need * sizeof(float)) == hipSuccess) s.fw_floats = need;
-        else hipGetLastError();
-    }
+    grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded);
     // Arrival counters of the in-kernel merge, zeroed once here (outside any
     // stream capture: the first run of a shape allocates); every run leaves
     // them zero.  Without them the merge runs as its own launch.
@@ -601,16 +631,25 @@ bool fp32_gemm_asked() {
     return false;
 }
 
+// Split rows of the weight w [n][k] for the f16 matrix cores.  Where there is
+// no memory for them *sw and *sew stay null and the fp32 kernels serve.
+vh_status split_weight_rows(RtState &s, const float *w, size_t n, size_t k, char **sw, int **sew) {
+    if (dalloc(s, vh::split_bytes(n, k), sw, "split weight allocation") != VH_OK ||
+        dalloc(s, n, sew, "split weight allocation") != VH_OK) {
+        hipGetLastError();
+        if (*sw) hipFreeAsync(*sw, s.stream);
+        *sw = nullptr;
+        return VH_OK;
+    }
+    return launch(s, "split_weight", [&] { return vh::launch_split_rows(s.stream, w, *sw, *sew, n, k); });
+}
+
 // Adds the split rows of L's weight (left out where split_k_fits says so or a
 // row holds an inf or NaN).
 vh_status split_weight(RtState &s, Lin *L) {
     if (L->N == 0 || !split_k_fits(1, L->N, L->K)) return VH_OK;
-    vh_status st = dalloc(s, vh::split_bytes(L->N, L->K), &L->sw, "split weight allocation");
-    if (!st) st = dalloc(s, L->N, &L->sew, "split weight allocation");
-    if (!st)
-        st = launch(s, "split_weight", [&] {
-            return vh::launch_split_rows(s.stream, L->wt, L->sw, L->sew, L->N, L->K);
-        });
+    vh_status st = split_weight_rows(s, L->wt, L->N, L->K, &L->sw, &L->sew);
+    if (!st && !L->sw) return VH_OK;
     std::vector<int> ex(L->N);
     if (!st) {
         hipError_t e = hipMemcpyAsync(ex.data(), L->sew, L->N * sizeof(int), hipMemcpyDeviceToHost, s.stream);
@@ -700,19 +739,7 @@ struct SplitRows {
 };
 vh_status split_space(RtState &s, size_t bytes, char **out) {
     *out = nullptr;
-    if (s.sx_bytes < bytes) {
-        hipStreamSynchronize(s.stream);
-        if (s.sx) hipFree(s.sx);
-        s.sx = nullptr;
-        s.sx_bytes = 0;
-        if (hipMalloc(&s.sx, bytes) != hipSuccess) {
-            hipGetLastError();
-            s.sx = nullptr;
-            return VH_OK;
-        }
-        s.sx_bytes = bytes;
-    }
-    *out = s.sx;
+    *out = grow_workspace(s, &s.sx, &s.sx_bytes, bytes, &s.sx_recorded) ? s.sx : nullptr;
     return VH_OK;
 }
 
@@ -827,7 +854,7 @@ vh_status q8_workspace(RtState &s, size_t rows, size_t k, int8_t **qs, uint16_t 
         if (s.aq) hipFree(s.aq);
         s.aq = nullptr;
         s.aq_bytes = 0;
-        hipError_t e = hipMalloc(&s.aq, need);
+        hipError_t e = device_malloc(s, (void **)&s.aq, need);
         if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("Q8_0 activation workspace allocation", e));
         s.aq_bytes = need;
     }
@@ -2840,14 +2867,8 @@ vh_status prepare_conv(const vh_runtime *rt, size_t in_c, size_t out_c, size_t k
     }
     if (!st && bias) st = upload_array(s, bias, out_c, &c->bias, "conv2d bias upload");
     const size_t K = in_c * kh * kw;
-    if (!st && stride == 1 && in_c % 32 == 0 && split_k_fits(1, out_c, K)) {
-        st = dalloc(s, vh::split_bytes(out_c, K), &c->sw, "split weight allocation");
-        if (!st) st = dalloc(s, out_c, &c->sew, "split weight allocation");
-        if (!st)
-            st = launch(s, "split_weight", [&] {
-                return vh::launch_split_rows(s.stream, c->w, c->sw, c->sew, out_c, K);
-            });
-    }
+    if (!st && stride == 1 && in_c % 32 == 0 && split_k_fits(1, out_c, K))
+        st = split_weight_rows(s, c->w, out_c, K, &c->sw, &c->sew);
     if (st) {
         delete c;
         return st;
