@@ -27,24 +27,6 @@
 //              Kernels::gelu on the hardware reciprocal and exp2, gelu_fast_form)
 //   Residual : c = c + (acc + bias) * gamma      (out-proj / fc2 + residual)
 //   Qkv      : head-major Q/K/V with bias and the 2-D RoPE rotation of Q, K
-//
-// LayerNorm fold (LNF, Gelu and Qkv): the GEMM of a pre-norm sub-layer,
-// LayerNorm(x) . W^T + b with LayerNorm gamma g and beta be, is computed as
-//     rstd * (x . W'^T - mean * c) + b',   W' = W diag(g),
-//     c[n] = sum_k W'[n][k],               b' = b + W . be,
-// on the raw rows x (W', c and b' prepared once).  Every workgroup sees
-// whole rows of A (K is not split), so the row statistics come either from
-// the producer of x (LNF == 2: per-chunk mean and M2, merged with Chan's
-// formula) or from the A slices as they pass through registers on their way
-// to LDS (LNF == 1): each thread sums (x - s) and (x - s)^2 over its chunks,
-// with s the mean of the row's first slice, and the threads of a row reduce
-// once after the slice loop.  Balanced-tail pieces publish their sums beside
-// their partial tiles; the last piece adds them in piece order.  The GEMM
-// term x . W'^T - mean * c cancels in proportion to |mean| / std, as the
-// crate's own float32 LayerNorm sums do (scalar::layernorm sums the raw row
-// in float32 too); staging x - s instead costs fc1 about 1 us per block on
-// gfx950, because the subtraction pulls the wait for the next slice's loads
-// ahead of the slice's last MFMAs.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
@@ -87,17 +69,6 @@ struct EpiArgs {
     // between launches (the last piece resets it).
     int tail_full, tail_splits, tail_count, tail_kps;
     unsigned *tail_cnt;
-    // LayerNorm fold (LNF kernels): per-row sums of the tail pieces
-    // ([tail tile][piece][2 * ACH][threads]), c[n] = sum_k Bt[n][k] and eps.
-    float *tail_stats;
-    const float *ln_c;
-    float ln_eps;
-    // Row statistics per 32-column chunk, (mean, M2) pairs [M][stats_chunks]:
-    // written by a Residual epilogue (stats_out, wave tiles 32 columns wide)
-    // for the next pre-norm GEMM, read by LNF == 2 kernels (stats_in).
-    float2 *stats_out;
-    const float2 *stats_in;
-    int stats_chunks;
 };
 
 // Applies a Store / Gelu / Residual epilogue to one output element.
@@ -218,7 +189,7 @@ constexpr size_t gemm_lds_bytes() {
 // zeroed when the slice is stored to LDS (after the MFMAs), and the output
 // is the channel-major tile itself, i.e. CHW.
 template <int BM, int BN, int BK, int WM, int WN, Epi EPI, bool SPLIT, bool EXACT, int CONV = 0,
-          bool TAIL = false, int LNF = 0>
+          bool TAIL = false>
 __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__restrict__ A,
                                                               const float *__restrict__ Bt,
                                                               int M, int N, int K,
@@ -280,44 +251,10 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         cd_x = x * ep.cd_stride - ep.cd_pad;
     }
 
-    // A registers of the slice in flight.  LNF keeps two sets, by slice
-    // parity, so that the LayerNorm sums of a slice read registers that no
-    // load is writing (and need no wait of their own); otherwise one set.
-    constexpr bool LN_LOOP = LNF == 1;  // row sums taken from the A slices
-    constexpr bool LN_ANY = LNF != 0;
-    // LayerNorm fold, statistics from the A slices (LNF == 1): this thread's
-    // A chunks c = tid + i * NT all lie in row c / CPR of the tile (NT is a
-    // multiple of CPR); ln_s1 / ln_s2 sum x - s and (x - s)^2 over the chunks
-    // it sees, with s = ln_sh[i] the mean of the row's first BK elements.
-    // Then (s - mean)^2 <= M2 / BK, so S2 = M2 + K (s - mean)^2 stays within
-    // (1 + K / BK) M2 whatever the row holds, and S2 / K - (S1 / K)^2 does not
-    // cancel (a shift by one element does: x[row][0] far from the mean).
-    // The CPR threads of a row hold those BK elements between them (chunk
-    // tid % CPR of slice 0), loaded here and summed after the first slice is
-    // stored.  Every piece of a balanced-tail tile derives the same shift
-    // from the same loads, so their partial sums add.
-    constexpr int LA = LN_LOOP ? ACH : 1;
-    float ln_sh[LA], ln_s1[LA], ln_s2[LA];
-    f32x4 ln_first[LA];
-    if constexpr (LN_ANY) {
-        static_assert(EXACT && !SPLIT && CONV == 0 && (EPI == Epi::Gelu || EPI == Epi::Qkv),
-                      "LayerNorm fold: whole-slice Gelu / Qkv GEMMs");
-        static_assert(NT % CPR == 0, "a thread's chunks share one row");
-    }
-    if constexpr (LN_LOOP) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            ln_first[i] = *reinterpret_cast<const f32x4 *>(A + (size_t)min(m0 + (tid + i * NT) / CPR, M - 1) * K +
-                                                            (tid % CPR) * 4);
-            ln_s1[i] = 0.0f;
-            ln_s2[i] = 0.0f;
-        }
-    }
-    f32x4 ra_sets[LN_LOOP ? 2 : 1][ACH], rb[BCH];
+    f32x4 ra[ACH], rb[BCH];
     using P0 = std::integral_constant<int, 0>;
     using P1 = std::integral_constant<int, 1>;
-    auto gload = [&](int k0, auto par) {
-        f32x4 *ra = ra_sets[LN_LOOP ? decltype(par)::value : 0];
+    auto gload = [&](int k0) {
         if constexpr (EXACT) {
 #pragma unroll
             for (int i = 0; i < ACH; i++) {
@@ -387,8 +324,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
             }
         }
     };
-    auto lstore = [&](int buf, auto par) {
-        const f32x4 *ra = ra_sets[LN_LOOP ? decltype(par)::value : 0];
+    auto lstore = [&](int buf) {
         float *as = smem + buf * STAGE;
         float *bs = as + BM * BK;
 #pragma unroll
@@ -418,35 +354,6 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         }
     };
 
-    // LNF == 2: the producer's statistics of this tile's rows, one (mean,
-    // M2) per 32-column chunk of the row (stats_chunks per row), prefetched
-    // before the slice loop: TPR threads per row, ln_cpt chunks each (host:
-    // stats_chunks == ln_cpt * TPR, ln_cpt <= LCP).  The loads are clamped,
-    // not selected, so that nothing waits for them before the loop.
-    constexpr int TPR = NT / BM, LCP = 8;
-    float2 ln_ch[LNF == 2 ? LCP : 1];
-    int ln_cpt = 0;
-    if constexpr (LNF == 2) {
-        static_assert(NT % BM == 0 && TPR >= 2 && TPR <= 16, "row statistics: 2-16 threads per row");
-        ln_cpt = ep.stats_chunks / TPR;
-        const float2 *src = ep.stats_in + (size_t)min(m0 + tid / TPR, M - 1) * ep.stats_chunks +
-                            (tid % TPR) * ln_cpt;
-#pragma unroll
-        for (int c = 0; c < LCP; c++) ln_ch[c] = src[min(c, ln_cpt - 1)];
-    }
-    auto ln_acc = [&](auto par) {
-        if constexpr (LN_LOOP) {
-            const f32x4 *ra = ra_sets[decltype(par)::value];
-#pragma unroll
-            for (int i = 0; i < ACH; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float d = ra[i][e] - ln_sh[i];
-                    ln_s1[i] += d;
-                    ln_s2[i] = fmaf(d, d, ln_s2[i]);
-                }
-        }
-    };
 
     f32x4 acc[FM][FN];
 #pragma unroll
@@ -491,17 +398,9 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
     };
 
     const int ktiles = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-    gload(kbeg, P0{});
-    lstore(0, P0{});
+    gload(kbeg);
+    lstore(0);
     __syncthreads();
-    if constexpr (LN_LOOP) {
-        // After the first slice's stores, so that they do not wait for it.
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            const float part = (ln_first[i][0] + ln_first[i][1]) + (ln_first[i][2] + ln_first[i][3]);
-            ln_sh[i] = group_sum<CPR>(part) * (1.0f / BK);
-        }
-    }
     if constexpr (EXACT) {
         // Branch-free slice loop: the last iteration reloads its own slice
         // into the idle buffer (never read again), so each iteration is one
@@ -511,17 +410,11 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         // next slice go out first.  Unrolled by two, so that the buffer of
         // each slice is a constant and every LDS address is a loop-invariant
         // register plus an immediate.
-        // LNF: slice t's own elements (register set t % 2, loaded during
-        // slice t - 1 and already waited for by its LDS stores) go into the
-        // LayerNorm sums while this slice's loads fill the other set; the
-        // sums are free to sit anywhere in the slice.
         auto slice = [&](int t, auto curc) {
             constexpr int cur = decltype(curc)::value;
-            using Next = std::integral_constant<int, cur ^ 1>;
-            gload(kbeg + min(t + 1, ktiles - 1) * BK, Next{});
-            ln_acc(curc);
+            gload(kbeg + min(t + 1, ktiles - 1) * BK);
             compute(cur);
-            lstore(cur ^ 1, Next{});
+            lstore(cur ^ 1);
             constexpr int NR = FM + FN, NM = 4 * FM * FN, NL = ACH + BCH;
             __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);  // k-step 0 fragments
             __builtin_amdgcn_sched_group_barrier(0x020, NL, 0);  // next slice, global
@@ -554,9 +447,9 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         for (int t = 0; t < ktiles; t++) {
             const int cur = t & 1;
             const bool next = t + 1 < ktiles;
-            if (next) gload(kbeg + (t + 1) * BK, P0{});
+            if (next) gload(kbeg + (t + 1) * BK);
             compute(cur);
-            if (next) lstore(cur ^ 1, P0{});
+            if (next) lstore(cur ^ 1);
             __syncthreads();
         }
     }
@@ -595,18 +488,6 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
                     for (int r = 0; r < 4; r++)
                         __hip_atomic_store(mine + ((i * FN + j) * 4 + r) * NT + tid, acc[i][j][r],
                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            constexpr int LS = 2 * LA;  // LayerNorm sums per thread and piece
-            const size_t stats_base = (size_t)tail_u * ep.tail_splits * LS * NT;
-            if constexpr (LN_LOOP) {
-                float *st = ep.tail_stats + stats_base + (size_t)piece * LS * NT;
-#pragma unroll
-                for (int i = 0; i < LA; i++) {
-                    __hip_atomic_store(st + (2 * i) * NT + tid, ln_s1[i], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(st + (2 * i + 1) * NT + tid, ln_s2[i], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             if (tid == 0)
@@ -621,7 +502,6 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
             constexpr int MAXS = 4;  // tail_splits <= 4 (tail_plan)
             const float *parts = ep.partial + tile_base;
             float pv[MAXS][PER];
-            float ps[MAXS][LN_LOOP ? LS : 1];
 #pragma unroll
             for (int p = 0; p < MAXS; p++) {
                 if (p < ep.tail_splits) {
@@ -629,33 +509,9 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
                     for (int e = 0; e < PER; e++)
                         pv[p][e] = __hip_atomic_load(parts + (size_t)(p * PER + e) * NT + tid, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT);
-                    if constexpr (LN_LOOP) {
-#pragma unroll
-                        for (int e = 0; e < LS; e++)
-                            ps[p][e] = __hip_atomic_load(ep.tail_stats + stats_base + (size_t)(p * LS + e) * NT + tid,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    }
                 } else {
 #pragma unroll
                     for (int e = 0; e < PER; e++) pv[p][e] = 0.0f;
-                    if constexpr (LN_LOOP) {
-#pragma unroll
-                        for (int e = 0; e < LS; e++) ps[p][e] = 0.0f;
-                    }
-                }
-            }
-            if constexpr (LN_LOOP) {
-#pragma unroll
-                for (int i = 0; i < LA; i++) {
-                    float s1 = ps[0][2 * i], s2 = ps[0][2 * i + 1];
-#pragma unroll
-                    for (int p = 1; p < MAXS; p++)
-                        if (p < ep.tail_splits) {
-                            s1 += ps[p][2 * i];
-                            s2 += ps[p][2 * i + 1];
-                        }
-                    ln_s1[i] = s1;
-                    ln_s2[i] = s2;
                 }
             }
 #pragma unroll
@@ -674,52 +530,6 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
             if (tid == 0) __hip_atomic_store(ep.tail_cnt + tail_u, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-
-    // LayerNorm fold: each row's sums are spread over CPR consecutive lanes;
-    // after the reduction one lane per row writes (mean, rstd) to LDS for the
-    // epilogue.  LDS is free: every slice ends with a barrier, after the
-    // last fragment reads.  mean = s + S1/K, var = S2/K - (S1/K)^2 about the
-    // shift s.
-    if constexpr (LN_LOOP) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-            ln_s1[i] = group_sum<CPR>(ln_s1[i]);
-            ln_s2[i] = group_sum<CPR>(ln_s2[i]);
-        }
-        float2 *lns = reinterpret_cast<float2 *>(smem);
-        if (tid % CPR == 0) {
-            const float kf = (float)K;
-#pragma unroll
-            for (int i = 0; i < ACH; i++) {
-                const float m1 = ln_s1[i] / kf;
-                const float var = fmaxf(ln_s2[i] / kf - m1 * m1, 0.0f);
-                lns[(tid + i * NT) / CPR] = float2{ln_sh[i] + m1, 1.0f / sqrtf(var + ep.ln_eps)};
-            }
-        }
-        __syncthreads();
-    } else if constexpr (LNF == 2) {
-        // Chan's merge of equal-width chunks: mean = mean of the chunk
-        // means, M2 = sum of (M2_c + w * (mean_c - mean)^2).
-        const float w = (float)(K / ep.stats_chunks);
-        float msum = 0.0f;
-#pragma unroll
-        for (int c = 0; c < LCP; c++)
-            if (c < ln_cpt) msum += ln_ch[c].x;
-        const float mean = group_sum<TPR>(msum) / (float)ep.stats_chunks;
-        float q = 0.0f;
-#pragma unroll
-        for (int c = 0; c < LCP; c++)
-            if (c < ln_cpt) {
-                const float d = ln_ch[c].x - mean;
-                q += fmaf(w * d, d, ln_ch[c].y);
-            }
-        q = group_sum<TPR>(q);
-        if (tid % TPR == 0)
-            reinterpret_cast<float2 *>(smem)[tid / TPR] = float2{mean, 1.0f / sqrtf(q / (float)K + ep.ln_eps)};
-        __syncthreads();
-    }
-    // (mean, rstd) of tile row r (LNF only).
-    auto ln_row = [&](int r) { return reinterpret_cast<const float2 *>(smem)[r]; };
 
     // C fragment layout: register r of lane l holds row 4*(l/16)+r, column l%16.
     const int rbase = m0 + wm * TM + 4 * lh;
@@ -819,12 +629,9 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         const int d0 = colw % 64;       // 0 or 32 (32-wide tile) / 0 (64-wide)
         float *dst = group == 0 ? ep.q : (group == 1 ? ep.k : ep.v);
         const bool rope = ep.rot != nullptr && group < 2;
-        float bias[FN], lc[FN];
+        float bias[FN];
 #pragma unroll
-        for (int j = 0; j < FN; j++) {
-            bias[j] = ep.bias[colw + j * 16 + li];
-            if constexpr (LN_ANY) lc[j] = ep.ln_c[colw + j * 16 + li];
-        }
+        for (int j = 0; j < FN; j++) bias[j] = ep.bias[colw + j * 16 + li];
         // Rotation (sin, cos) of every row this lane stores, read before any
         // store from clamped rows so that the reads overlap.
         float2 rot[FM][4][FN / 2];
@@ -851,14 +658,8 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
                 if (row >= M) continue;
                 const int img = row / ep.tokens, t = row % ep.tokens;
                 float vals[FN];
-                if constexpr (LN_ANY) {
-                    const float2 st = ln_row(row - m0);
 #pragma unroll
-                    for (int j = 0; j < FN; j++) vals[j] = fmaf(st.y, fmaf(-st.x, lc[j], acc[i][j][r]), bias[j]);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < FN; j++) vals[j] = add_rn(acc[i][j][r], bias[j]);
-                }
+                for (int j = 0; j < FN; j++) vals[j] = add_rn(acc[i][j][r], bias[j]);
                 if (rope) {
                     // rope::rotate_half (src/rope.rs:84-93): dims (i, i+16) of
                     // each 32-wide axis half sit in fragments (2h, 2h+1).
@@ -880,23 +681,14 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
         // store, so the reads overlap instead of each waiting behind the
         // bounds branch of its element.
         const int cbase = n0 + wn * TN + li;
-        float bias[FN], gamma[FN], lc[FN];
+        float bias[FN], gamma[FN];
 #pragma unroll
         for (int j = 0; j < FN; j++) {
             const int col = min(cbase + j * 16, N - 1);
             bias[j] = load_or(ep.bias, (const float *)ep.c, col, 0.0f);
             gamma[j] = load_or(ep.gamma, (const float *)ep.c, col, 1.0f);
-            if constexpr (LN_ANY) lc[j] = ep.ln_c[col];
-        }
-        float2 lnst[LN_ANY ? FM : 1][4];
-        if constexpr (LN_ANY) {
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) lnst[i][r] = ln_row(wm * TM + 4 * lh + i * 16 + r);
         }
         float resid[EPI == Epi::Residual ? FM : 1][FN][4];
-        float outv[EPI == Epi::Residual ? FM : 1][FN][4];
         if constexpr (EPI == Epi::Residual) {
 #pragma unroll
             for (int i = 0; i < FM; i++)
@@ -926,10 +718,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
                         if (!WHOLE && row >= M) continue;
                         const size_t idx = (size_t)row * N + col;
                         float v = acc[i][j][r];
-                        if constexpr (LN_ANY)
-                            v = fmaf(lnst[i][r].y, fmaf(-lnst[i][r].x, lc[j], v), bias[j]);
-                        else if (ep.bias)
-                            v = add_rn(v, bias[j]);
+                        if (ep.bias) v = add_rn(v, bias[j]);
                         if constexpr (EPI == Epi::Store) {
                             if (ep.gamma) v = mul_rn(v, gamma[j]);
                             stream_store(ep.c + idx, v);
@@ -937,9 +726,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
                             stream_store(ep.c + idx, gelu_fast_form(v));
                         } else {
                             if (ep.gamma) v = mul_rn(v, gamma[j]);
-                            const float o = add_rn(resid[i][j][r], v);
-                            stream_store(ep.c + idx, o);
-                            if constexpr (EPI == Epi::Residual) outv[i][j][r] = o;
+                            stream_store(ep.c + idx, add_rn(resid[i][j][r], v));
                         }
                     }
             }
@@ -949,26 +736,6 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
             store_all(std::true_type{});
         else
             store_all(std::false_type{});
-        // Row statistics of the updated rows for the next sub-layer's
-        // LayerNorm fold: a wave's 32 columns are one chunk; the 16 lanes of
-        // a lane group hold a row's 32 values (two per lane), so the chunk's
-        // mean and M2 take two 16-lane sums (two passes, no cancellation).
-        if constexpr (EPI == Epi::Residual && TN == 32) {
-            if (ep.stats_out && n0 + wn * TN < N) {
-                const int chunk = (n0 + wn * TN) / 32;
-#pragma unroll
-                for (int i = 0; i < FM; i++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float mean = group_sum<16>(outv[i][0][r] + outv[i][1][r]) * (1.0f / 32.0f);
-                        const float d0 = outv[i][0][r] - mean, d1 = outv[i][1][r] - mean;
-                        const float m2 = group_sum<16>(fmaf(d0, d0, d1 * d1));
-                        const int row = rbase + i * 16 + r;
-                        if (li == 0 && row < M)
-                            ep.stats_out[(size_t)row * ep.stats_chunks + chunk] = float2{mean, m2};
-                    }
-            }
-        }
     }
 }
 
@@ -983,8 +750,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const float *__res
 // epilogue: c = c + (acc + bias) * gamma.  With 32 x 96 tiles, 2 x 2 waves
 // and two K groups the 865-row projection is 224 workgroups of 8 waves, one
 // per CU, two waves per SIMD, with no partial tiles leaving the CU and no
-// second launch.  With ep.stats_out, group 0 also writes each row's (mean,
-// M2) over each wave's TN columns: one chunk per wave column.
+// second launch.
 template <int BM, int BN, int BK, int WM, int WN, int KG, Epi EPI = Epi::Residual>
 __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_kgroup_kernel(const float *__restrict__ A,
                                                                       const float *__restrict__ Bt,
@@ -1159,7 +925,6 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_kgroup_kernel(const floa
 
     // Residual epilogue (gemm_nt_kernel's), reads issued before any store.
     epi_loads();
-    float outv[FM][FN][4];
     wait_vmem_all();
 #pragma unroll
     for (int j = 0; j < FN; j++)
@@ -1171,35 +936,9 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_kgroup_kernel(const floa
                 if (ep.bias) v = add_rn(v, bias[j]);
                 if (ep.gamma) v = mul_rn(v, gamma[j]);
                 const float o = EPI == Epi::Residual ? add_rn(resid[i][j][r], v) : v;
-                outv[i][j][r] = o;
                 const int row = rbase + i * 16 + r, col = cbase + j * 16;
                 if (row < M && col < N) stream_store(ep.c + (size_t)row * N + col, o);
             }
-    {
-        // The 16 lanes of a lane group hold a row's TN values of this wave
-        // (FN per lane): mean and M2 over them by two 16-lane sums.
-        if (EPI == Epi::Residual && ep.stats_out) {
-            const int chunk = (n0 + wn * TN) / TN;
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    float sum = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < FN; j++) sum += outv[i][j][r];
-                    const float mean = group_sum<16>(sum) / (float)TN;
-                    float m2 = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < FN; j++) {
-                        const float d = outv[i][j][r] - mean;
-                        m2 = fmaf(d, d, m2);
-                    }
-                    m2 = group_sum<16>(m2);
-                    const int row = rbase + i * 16 + r;
-                    if (li == 0 && row < M) ep.stats_out[(size_t)row * ep.stats_chunks + chunk] = float2{mean, m2};
-                }
-        }
-    }
 }
 
 // Sums the split-K partials in split order, then applies the epilogue; four
@@ -1308,69 +1047,6 @@ __global__ __launch_bounds__(256) void splitk_reduce4_kernel(int M, int N, EpiAr
     *c4 = o;
 }
 
-// Split-K reduction fused with the residual update and the LayerNorm of the
-// updated rows: one wave per row (N % 4 == 0, N <= 1024).  Each element is
-// computed exactly as by splitk_reduce_kernel<Residual>, and each row is
-// normalised exactly as by layernorm_kernel, in one pass over the row.  All
-// reads of a lane are issued before any arithmetic (chunks past the row end
-// read chunk 0 and are dropped), so they are in flight together.
-template <int SPLITS>
-__global__ __launch_bounds__(256) void splitk_residual_ln_kernel(int M, int N, EpiArgs ep,
-                                                                 const float *__restrict__ ln_g,
-                                                                 const float *__restrict__ ln_b,
-                                                                 float *__restrict__ ln_out,
-                                                                 float eps) {
-    const int lane = threadIdx.x & 63;
-    const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    if (row >= M) return;
-    const int n4 = N >> 2;
-    const size_t mn4 = (size_t)M * n4;
-    const f32x4 *part = reinterpret_cast<const f32x4 *>(ep.partial);
-    f32x4 *c4 = reinterpret_cast<f32x4 *>(ep.c + (size_t)row * N);
-    const f32x4 *bias4 = reinterpret_cast<const f32x4 *>(ep.bias);
-    const f32x4 *gamma4 = reinterpret_cast<const f32x4 *>(ep.gamma);
-    f32x4 p[4][SPLITS], x[4], b[4], g[4], lg[4], lb[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int idx = lane + j * 64 < n4 ? lane + j * 64 : 0;
-        const size_t i4 = (size_t)row * n4 + idx;
-#pragma unroll
-        for (int sp = 0; sp < SPLITS; sp++) p[j][sp] = part[(size_t)sp * mn4 + i4];
-        x[j] = c4[idx];
-        b[j] = load_or(bias4, (const f32x4 *)c4, idx, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-        g[j] = load_or(gamma4, (const f32x4 *)c4, idx, f32x4{1.0f, 1.0f, 1.0f, 1.0f});
-        lg[j] = reinterpret_cast<const f32x4 *>(ln_g)[idx];
-        lb[j] = reinterpret_cast<const f32x4 *>(ln_b)[idx];
-    }
-    wait_vmem_all();  // one wait for all of them; the stores below then need none
-    f32x4 r[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const bool live = lane + j * 64 < n4;
-        f32x4 v = p[j][0];
-#pragma unroll
-        for (int sp = 1; sp < SPLITS; sp++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = add_rn(v[e], p[j][sp][e]);
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            if (ep.bias) v[e] = add_rn(v[e], b[j][e]);
-            if (ep.gamma) v[e] = mul_rn(v[e], g[j][e]);
-            x[j][e] = add_rn(x[j][e], v[e]);
-        }
-        r[j] = live ? x[j] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (live) c4[lane + j * 64] = x[j];
-    }
-    float mean, inv;
-    ln_row_stats(r, lane, n4, N, eps, mean, inv);
-    f32x4 *y4 = reinterpret_cast<f32x4 *>(ln_out + (size_t)row * N);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int idx = lane + j * 64;
-        if (idx < n4) y4[idx] = ln_apply(r[j], mean, inv, lg[j], lb[j]);
-    }
-}
-
 struct Tile {
     int bm, bn, bk, wm, wn;
 };
@@ -1395,11 +1071,10 @@ int use_xcd_order(const GemmArgs &g) {
     return g.m > 1024 || g.k >= 2048;
 }
 
-template <int BM, int BN, int BK, int WM, int WN, Epi EPI, bool SPLIT, bool EXACT, int CONV = 0,
-          int LNF = 0>
+template <int BM, int BN, int BK, int WM, int WN, Epi EPI, bool SPLIT, bool EXACT, int CONV = 0>
 hipError_t launch_tile(hipStream_t s, const GemmArgs &g, const EpiArgs &ep, int splits, int kps) {
     constexpr size_t lds = gemm_lds_bytes<BM, BN, BK>();
-    auto kernel = gemm_nt_kernel<BM, BN, BK, WM, WN, EPI, SPLIT, EXACT, CONV, false, LNF>;
+    auto kernel = gemm_nt_kernel<BM, BN, BK, WM, WN, EPI, SPLIT, EXACT, CONV, false>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
     dim3 grid((unsigned)((g.n + BN - 1) / BN), (unsigned)((g.m + BM - 1) / BM), (unsigned)splits);
@@ -1546,15 +1221,14 @@ bool tail_plan(const GemmArgs &g, const Tile &t, TailPlan *plan, int only_splits
     return true;
 }
 
-template <Epi EPI, int LNF = 0, int CONV = 0>
+template <Epi EPI, int CONV = 0>
 hipError_t launch_tail(hipStream_t s, const GemmArgs &g, EpiArgs ep, const TailPlan &p) {
     constexpr int BM = 64, BN = 64, BK = 32, WM = 2, WN = 2;
     constexpr size_t lds = gemm_lds_bytes<BM, BN, BK>();
-    auto kernel = gemm_nt_kernel<BM, BN, BK, WM, WN, EPI, false, true, CONV, true, LNF>;
+    auto kernel = gemm_nt_kernel<BM, BN, BK, WM, WN, EPI, false, true, CONV, true>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
     ep.partial = g.tail_ws;
-    ep.tail_stats = g.tail_stats;
     ep.tail_cnt = g.tail_cnt;
     ep.tail_full = p.full;
     ep.tail_splits = p.splits;
@@ -1593,11 +1267,6 @@ hipError_t launch_kgroup_t(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
     auto kernel = gemm_kgroup_kernel<BM, BN, BK, WM, WN, KG, EPI>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
-    if (EPI == Epi::Residual && g.stats_out) {
-        ep.stats_out = reinterpret_cast<float2 *>(g.stats_out);
-        ep.stats_chunks = (int)(g.n / (BN / WN));
-        if (g.stats_out_chunks) *g.stats_out_chunks = ep.stats_chunks;
-    }
     dim3 grid((unsigned)(g.n / BN), (unsigned)((g.m + BM - 1) / BM));
     kernel<<<grid, WM * WN * KG * 64, lds, s>>>(g.a, g.bt, (int)g.m, (int)g.n, (int)g.k, ep);
     return hipGetLastError();
@@ -1609,50 +1278,8 @@ hipError_t launch_kgroup(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
     return launch_kgroup_t<EPI, 32, 96, 32, 2, 2, 2>(s, g, ep);
 }
 
-// LayerNorm-folded Gelu / Qkv GEMM (ln_fold_c set): whole slices and no K
-// split, on the 64x128x64 tile where the per-shape table picks it and the
-// 64x64x32 tile otherwise (with the balanced tail for Gelu when tail_plan
-// takes it).  The row statistics come from the producer's chunk statistics
-// (stats_in) when given in a shape the tile takes, else from the A slices.
-template <Epi EPI, int LNF>
-hipError_t launch_lnf(hipStream_t s, const GemmArgs &g, const EpiArgs &ep, bool wide) {
-    if constexpr (EPI == Epi::Gelu) {
-        TailPlan p;
-        if (!wide && g.tail_stats && tail_plan(g, Tile{64, 64, 32, 2, 2}, &p))
-            return launch_tail<EPI, LNF>(s, g, ep, p);
-    }
-    if (wide) return launch_tile<64, 128, 64, 2, 4, EPI, false, true, 0, LNF>(s, g, ep, 1, (int)g.k);
-    return launch_tile<64, 64, 32, 2, 2, EPI, false, true, 0, LNF>(s, g, ep, 1, (int)g.k);
-}
-
-template <Epi EPI>
-hipError_t dispatch_lnf(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
-    Tile t;
-    int splits;
-    if (!tile_override(&t, &splits)) default_tile(g, &t, &splits);
-    const bool wide = t.bm == 64 && t.bn == 128 && t.bk == 64 && t.wm == 2 && t.wn == 4;
-    const int bk = wide ? 64 : 32;
-    if (g.k == 0 || g.k % bk != 0 || !g.bias) return hipErrorInvalidValue;
-    const size_t tpr = wide ? 8 : 4;  // threads per tile row (NT / BM)
-    const size_t ch = g.stats_in_chunks;
-    // VESTRA_HIP_LN_STATS=0 ignores the producer's statistics (A/B studies
-    // and tests of both forms; read per call).
-    const char *env = std::getenv("VESTRA_HIP_LN_STATS");
-    const bool use_in = !(env && env[0] == '0');
-    if (use_in && g.stats_in && ch && g.k % ch == 0 && ch % tpr == 0 && ch / tpr <= 8) {
-        ep.stats_in = reinterpret_cast<const float2 *>(g.stats_in);
-        ep.stats_chunks = (int)ch;
-        return launch_lnf<EPI, 2>(s, g, ep, wide);
-    }
-    return launch_lnf<EPI, 1>(s, g, ep, wide);
-}
-
 template <Epi EPI>
 hipError_t dispatch(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
-    if (g.ln_fold_c) {
-        if constexpr (EPI == Epi::Gelu || EPI == Epi::Qkv) return dispatch_lnf<EPI>(s, g, ep);
-        return hipErrorInvalidValue;
-    }
     Tile t;
     int splits;
     const bool overridden = tile_override(&t, &splits);
@@ -1660,18 +1287,6 @@ hipError_t dispatch(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
     if (EPI == Epi::Qkv) splits = 1;
     const int table_splits = !overridden && splits > 1 ? splits : 0;
     if (splits > 1 && (g.ws == nullptr || g.ws_floats < (size_t)splits * g.m * g.n)) splits = 1;
-    // Residual with stats_out: the 64-wide tiles of the tail and of the
-    // unsplit 64 x 64 x 32 launch (32-column wave tiles) also write the row
-    // statistics of the updated rows (chunks per row in stats_out_chunks).
-    auto with_stats = [&](EpiArgs e) {
-        if (EPI == Epi::Residual && g.stats_out && g.n % 32 == 0) {
-            e.stats_out = reinterpret_cast<float2 *>(g.stats_out);
-            e.stats_chunks = (int)(g.n / 32);
-            if (g.stats_out_chunks) *g.stats_out_chunks = e.stats_chunks;
-        }
-        return e;
-    };
-    if (g.stats_out_chunks) *g.stats_out_chunks = 0;
     if constexpr (EPI == Epi::Residual) {
         if (!overridden && use_kgroup(g)) return launch_kgroup<EPI>(s, g, ep);
     } else if constexpr (EPI == Epi::Store) {
@@ -1685,24 +1300,21 @@ hipError_t dispatch(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
         // Store, GELU and Residual: the last piece of a tail tile runs the
         // epilogue once (a Residual tile adds its residual exactly once).
         TailPlan p;
-        if (splits == 1 && tail_plan(g, t, &p)) return launch_tail<EPI>(s, g, with_stats(ep), p);
+        if (splits == 1 && tail_plan(g, t, &p)) return launch_tail<EPI>(s, g, ep, p);
         // A long-K launch that the table splits, whose 64 x 64 grid has
         // fewer tiles than CUs (fc2 at 865 tokens: 168 tiles): every tile as
         // K pieces, the last piece of each summing them in order and running
         // the epilogue, saves the separate reduction launch (fc2 41.3 against
         // 42.1 us for split-K 3 of 64 x 128 tiles plus the reduction).  The
         // pieces are the table's K ranges, so each output is the same sum of
-        // the same partials as split-K with its reduction (the encoder's
-        // fused fc2 reduction and LayerNorm still splits K that way).
+        // the same partials as split-K with its reduction.
         if (table_splits && g.k % ((size_t)table_splits * t.bk) == 0 &&
             tail_plan(g, Tile{64, 64, 32, 2, 2}, &p, table_splits) && p.full == 0)
-            return launch_tail<EPI>(s, g, with_stats(ep), p);
+            return launch_tail<EPI>(s, g, ep, p);
     }
     if (splits == 1) {
-        const bool narrow_wave = t.bm == 64 && t.bn == 64 && t.bk == 32 && t.wm == 2 && t.wn == 2;
-        hipError_t e = run_cfg<EPI, false>(s, g, narrow_wave ? with_stats(ep) : ep, t, 1);
+        hipError_t e = run_cfg<EPI, false>(s, g, ep, t, 1);
         if (e == hipErrorInvalidValue) {
-            if (g.stats_out_chunks) *g.stats_out_chunks = 0;
             default_tile(g, &t, &splits);
             e = run_cfg<EPI, false>(s, g, ep, t, 1);
         }
@@ -1784,7 +1396,7 @@ hipError_t dispatch_conv_direct(hipStream_t s, const GemmArgs &g, const EpiArgs 
         }
     }
     TailPlan p;
-    if (tail_plan(g, Tile{64, 64, 32, 2, 2}, &p)) return launch_tail<Epi::Store, 0, 3>(s, g, ep, p);
+    if (tail_plan(g, Tile{64, 64, 32, 2, 2}, &p)) return launch_tail<Epi::Store, 3>(s, g, ep, p);
     return launch_tile<64, 64, 32, 2, 2, Epi::Store, false, true, 3>(s, g, ep, 1, (int)g.k);
 }
 
@@ -1798,51 +1410,6 @@ hipError_t dispatch_scatter(hipStream_t s, const GemmArgs &g, const EpiArgs &ep)
 
 }  // namespace
 
-// Residual GEMM followed by the LayerNorm of the updated rows: split K and
-// fuse the reduction with the normalisation when the shape allows, else run
-// the GEMM and a separate LayerNorm.
-static hipError_t residual_ln(hipStream_t s, const GemmArgs &g, EpiArgs ep) {
-    Tile t;
-    int splits;
-    if (!tile_override(&t, &splits)) {
-        default_tile(g, &t, &splits);
-        // The out-projection shape (K <= 1024) splits K at M <= 1024, where its
-        // 168 tiles would leave CUs idle (865 tokens: 20.4 us fused against
-        // 25.4 unsplit plus LayerNorm); past 1024 rows the tiles fill the GPU
-        // and the unsplit GEMM plus a LayerNorm launch is faster (4 x 865
-        // tokens: 47.9 against 53.5 us).
-        if (splits < 2 && g.m <= 1024) {
-            t = Tile{64, 64, 32, 2, 2};
-            splits = 3;
-        }
-    }
-    const bool fused = splits >= 2 && splits <= 4 && g.k >= 64 * (size_t)splits && g.n % 4 == 0 && g.n <= 1024 &&
-                       g.ws != nullptr && g.ws_floats >= (size_t)splits * g.m * g.n;
-    if (!fused) {
-        hipError_t e = dispatch<Epi::Residual>(s, g, ep);
-        if (e != hipSuccess) return e;
-        return launch_layernorm(s, g.c, g.ln_gamma, g.ln_beta, g.ln_out, g.m, g.n, g.ln_eps);
-    }
-    ep.partial = g.ws;
-    hipError_t e = run_cfg<Epi::Residual, true>(s, g, ep, t, splits);
-    if (e == hipErrorInvalidValue) {
-        t = Tile{64, 64, 32, 2, 2};
-        e = run_cfg<Epi::Residual, true>(s, g, ep, t, splits);
-    }
-    if (e != hipSuccess) return e;
-    // One wave per row; up to 2048 rows, one row per workgroup spreads the
-    // rows over every CU.
-    const unsigned wpb = g.m <= 2048 ? 1 : 4;
-    const dim3 grid((unsigned)((g.m + wpb - 1) / wpb));
-    const int m = (int)g.m, n = (int)g.n, nt = (int)(64 * wpb);
-    switch (splits) {
-        case 2: splitk_residual_ln_kernel<2><<<grid, nt, 0, s>>>(m, n, ep, g.ln_gamma, g.ln_beta, g.ln_out, g.ln_eps); break;
-        case 3: splitk_residual_ln_kernel<3><<<grid, nt, 0, s>>>(m, n, ep, g.ln_gamma, g.ln_beta, g.ln_out, g.ln_eps); break;
-        default: splitk_residual_ln_kernel<4><<<grid, nt, 0, s>>>(m, n, ep, g.ln_gamma, g.ln_beta, g.ln_out, g.ln_eps); break;
-    }
-    return hipGetLastError();
-}
-
 hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
     if (g.m == 0 || g.n == 0) return hipSuccess;
     EpiArgs ep{};
@@ -1855,8 +1422,6 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
     ep.tokens = (int)g.tokens;
     ep.heads = (int)g.heads;
     ep.rot = g.rot;
-    ep.ln_c = g.ln_fold_c;
-    ep.ln_eps = g.ln_fold_eps;
     if (g.conv_in_c && g.conv_ih) {
         if (g.epi != Epi::Store || g.conv_kw == 0 || g.conv_ow == 0 || g.conv_iw == 0 ||
             g.conv_stride == 0 || g.n % g.conv_ow != 0 || g.k % (g.conv_in_c * g.conv_kw) != 0)
@@ -1907,8 +1472,7 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
     switch (g.epi) {
         case Epi::Store: return dispatch<Epi::Store>(s, g, ep);
         case Epi::Gelu: return dispatch<Epi::Gelu>(s, g, ep);
-        case Epi::Residual:
-            return g.ln_out ? residual_ln(s, g, ep) : dispatch<Epi::Residual>(s, g, ep);
+        case Epi::Residual: return dispatch<Epi::Residual>(s, g, ep);
         case Epi::Qkv: return dispatch<Epi::Qkv>(s, g, ep);
     }
     return hipErrorInvalidValue;

@@ -144,31 +144,6 @@ struct GemmArgs {
     size_t tail_ws_floats = 0;
     unsigned *tail_cnt = nullptr;
     size_t tail_cnt_n = 0;
-    // Per-row LayerNorm sums of LayerNorm-folded tail pieces (kTailStatFloats).
-    float *tail_stats = nullptr;
-    // Gelu / Qkv only: a is the raw input of a pre-norm sub-layer and the
-    // GEMM computes LayerNorm(a) . W^T + b as rstd * (a . bt^T - mean * c) +
-    // bias, with bt = W diag(ln gamma), ln_fold_c = c[n] = sum_k bt[n][k] and
-    // bias = b + W . ln beta prepared by the caller; the row statistics are
-    // taken inside the GEMM (epsilon ln_fold_eps).  K % 64 == 0.
-    const float *ln_fold_c = nullptr;
-    float ln_fold_eps = 0.0f;
-    // Row statistics per chunk of equal-width column ranges, (mean, M2)
-    // float pairs [m][chunks]: a Residual GEMM with stats_out (room for
-    // m * n / 16 pairs) writes them for the rows it updates when its tile
-    // allows, and reports the chunks per row in *stats_out_chunks (0: none
-    // written); a LayerNorm-folded GEMM with stats_in (stats_in_chunks per
-    // row, k a multiple of it) takes its row statistics from them instead of
-    // from its A slices.
-    float *stats_out = nullptr;
-    int *stats_out_chunks = nullptr;
-    const float *stats_in = nullptr;
-    size_t stats_in_chunks = 0;
-    // Residual only: also write LayerNorm(c) row by row to ln_out (the next
-    // sub-layer's input), fused into the split-K reduction when possible.
-    const float *ln_gamma = nullptr, *ln_beta = nullptr;
-    float *ln_out = nullptr;
-    float ln_eps = 0.0f;
     // Implicit stride-1 convolution (Store only): a is the weight
     // [out_c][kh][kw][conv_in_c] (m = out_c, k = tap * conv_in_c + ic, tap =
     // ky * conv_kw + kx), bt is a zero-padded channel-last image
@@ -199,7 +174,6 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g);
 // Sizes of the balanced-tail workspace (GemmArgs::tail_ws / tail_cnt).
 constexpr size_t kTailTiles = 512;
 constexpr size_t kTailFloats = kTailTiles * 4 * 64 * 64;
-constexpr size_t kTailStatFloats = kTailTiles * 4 * 4 * 256;
 
 // ---- GEMM on split rows (k_split.hip) -------------------------------------------
 // Split rows (split_gemm.h): each float row as two halves per value and one

@@ -483,7 +483,7 @@ vh_status splitk_workspace(RtState &s, size_t m, size_t n, float **out, size_t *
 vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
     if (!s.tw) {
         hipStreamSynchronize(s.stream);
-        hipError_t e = device_malloc(s, (void **)&s.tw, (vh::kTailFloats + vh::kTailStatFloats) * sizeof(float));
+        hipError_t e = device_malloc(s, (void **)&s.tw, vh::kTailFloats * sizeof(float));
         if (e == hipSuccess) e = hipMalloc(&s.tcnt, vh::kTailTiles * sizeof(unsigned));
         if (e == hipSuccess) e = hipMemsetAsync(s.tcnt, 0, vh::kTailTiles * sizeof(unsigned), s.stream);
         if (e != hipSuccess) {
@@ -496,7 +496,6 @@ vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
     }
     g.tail_ws = s.tw;
     g.tail_ws_floats = vh::kTailFloats;
-    g.tail_stats = s.tw + vh::kTailFloats;
     g.tail_cnt = s.tcnt;
     g.tail_cnt_n = vh::kTailTiles;
     return VH_OK;
