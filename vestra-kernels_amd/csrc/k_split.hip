@@ -962,9 +962,14 @@ hipError_t launch_split_epi(hipStream_t s, SplitArgs ar) {
 
 bool split_gemm_fits(size_t m, size_t n, size_t k) {
     // Row offsets inside a 256-row tile stay below 2^31 bytes, and the
-    // smallest tiles' grid below the launch limit.
-    return k > 0 && k <= ((size_t)1 << 21) - 32 && m <= INT32_MAX && n <= INT32_MAX &&
-           ((m + 63) / 64) * ((n + 31) / 32) <= (size_t)INT32_MAX / 512;
+    // chosen tile's grid (with or without Qkv's choice) below the launch limit.
+    if (k == 0 || k > ((size_t)1 << 21) - 32 || m > INT32_MAX || n > INT32_MAX) return false;
+    if (m == 0 || n == 0) return true;
+    for (bool qkv : {false, true}) {
+        const SplitTile &t = kSplitTiles[plan_split(m, n, (int)((k + 31) / 32), qkv, false).tile];
+        if ((m + t.bm - 1) / t.bm > (size_t)INT32_MAX / 512 / ((n + t.bn - 1) / t.bn)) return false;
+    }
+    return true;
 }
 
 // Splitting reads and writes four bytes per value at about 3 TB/s, in a launch

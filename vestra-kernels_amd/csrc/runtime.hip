@@ -2408,7 +2408,7 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
                                         vh::Epi::Residual, b.qfc2.bias, b.qfc2.gamma);
         });
     }
-    if (!b.split || !vh::attn_split_fits(images * kHeads, tokens)) {
+    if (!b.split) {
         // Weights with an inf or NaN: the fp32 matrix instructions.
         auto norm = [&](const float *g, const float *be) {
             return launch(s, "layernorm", [&] { return vh::launch_layernorm(s.stream, x, g, be, h, M, D, eps); });
