@@ -10,7 +10,8 @@ is held to 2^-40 of that instead.
 import numpy as np
 import pytest
 
-from vestra_hip import seeded
+from q8_compose import q8_block
+from vestra_hip import da3, seeded
 
 pytestmark = pytest.mark.gpu
 
@@ -196,3 +197,25 @@ def test_split_convolution_vs_float64(rt, in_c, out_c, ih, iw, k, p, relu):
     assert np.array_equal(np.isnan(got), np.isnan(odd))
     assert np.array_equal(got[~fine & ~np.isnan(odd)], odd[~fine & ~np.isnan(odd)].astype(np.float32))
     assert np.all(np.abs(got[fine] - odd[fine]) <= bound[fine])
+
+
+@pytest.mark.parametrize("T, inf", [(1, None), (65, "v"), (130, "q"), (200, None)])
+def test_q8_block_attention_writes_q8_rows(rt, T, inf):
+    """The Q8_0 rows that the attention writes are quantize_row_q8_0 of its
+    float output, bit for bit: ragged query tiles, and heads with an inf."""
+    w = da3.block_weights(seed=42, layerscale=1.0)
+    if inf:
+        w["b_qkv"][{"q": 5, "v": 2 * 768 + 70}[inf]] = np.inf
+    x = seeded.normal(9960 + T, T * 768)
+
+    def attention(q, k, v, heads, tokens, hd):
+        return rt.download_f32(rt.flash_attention_f32_da3_base(rt.upload_f32(q), rt.upload_f32(k), rt.upload_f32(v),
+                                                               heads, tokens))
+
+    def layernorm(a, rows, cols, g, b, eps):
+        return rt.download_f32(rt.layernorm_f32(rt.upload_f32(a), rt.upload_f32(g), rt.upload_f32(b), rows, cols, eps))
+
+    exp = q8_block(x, w, T, None, attention=attention, layernorm=layernorm)
+    xt = rt.upload_f32(x)
+    rt.vit_block_run(rt.prepare_block(w, q8_0=True), xt, 1, T)
+    assert np.array_equal(rt.download_f32(xt), exp, equal_nan=True)

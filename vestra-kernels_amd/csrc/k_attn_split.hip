@@ -23,10 +23,15 @@
 // least); the running maximum is only raised when a score passes it by 2^8
 // (still inside the half's range), so most panels need no correction.
 //
+// The output is floats, split rows (the next projection's input), or Q8_0 rows
+// (the Q8_0 block's: two streams finish a block of 32 dims and exchange their
+// largest magnitudes), which saves the launch that quantised the floats
+// (4.8 us at 865 tokens).
+//
 // Error against float64 at 12 x 865 x 64, N(0, 1): 2.5e-7, against 4.3e-7 of the
 // fp32 matrix instructions.  Time on split rows (kernel trace): 12 x 865 18 us
 // against 28 (fp32 matrix instructions), 48 x 865 54 against 100, 12 x 3457
-// 165 against 343.  Products alone would take a third of that: the softmax's
+// 157 against 343.  Products alone would take a third of that: the softmax's
 // VALU work and the products share the SIMD's issue (a product holds it
 // for 8 of its 16 cycles, measured), and taking out the copies, the LDS reads or
 // the exponentials one at a time saves 14%, 4% and 6% at 12 x 3457.  Single K and
@@ -56,9 +61,17 @@ struct AttnArgs {
     float *out;                   // f32: token-major [img][T][heads*hd] or [bh][T][hd]
     int token_major;
     char *out_split;              // split rows [img*T][heads*64] with exponent ev
+    int8_t *q8_qs;                // Q8: blocks [heads*2][img*T][32] of the token-major
+    uint16_t *q8_d;               // output and their scales (hd = 64)
 };
 
-enum class AOut : int { F32, Split };
+enum class AOut : int { F32, Split, Q8 };
+
+// quantize_row_q8_0's value (src/q8_0_dot.rs:38-44): half away from zero, NaN to 0.
+__device__ __forceinline__ int q8_value(float v, float inv) {
+    const float q = roundf(mul_rn(v, inv));
+    return isnan(q) ? 0 : (int)fminf(fmaxf(q, -127.0f), 127.0f);
+}
 
 // Two floats to two halves (one v_cvt_pk_f16_f32; the empty asm keeps the
 // compiler from converting each again where a half is used), and what the
@@ -112,10 +125,9 @@ __device__ __forceinline__ f16x4 read_tr(const char *p) {
 }
 
 // A head with an infinity or NaN, in floats, one query per wave at a time:
-// rare, so plain.  64 keys per step, one per lane.
-__device__ __attribute__((noinline)) void attention_floats(const float *q, const float *k, const float *v, int T,
-                                                           int hd, float scale_log2, int query, float *orow,
-                                                           int lane) {
+// rare, so plain.  64 keys per step, one per lane; output dim `lane` (< hd).
+__device__ __attribute__((noinline)) float attention_floats(const float *q, const float *k, const float *v, int T,
+                                                            int hd, float scale_log2, int query, int lane) {
     float m = -INFINITY, l = 0.0f, o = 0.0f;
     for (int k0 = 0; k0 < T; k0 += 64) {
         const int key = k0 + lane;
@@ -135,7 +147,7 @@ __device__ __attribute__((noinline)) void attention_floats(const float *q, const
             if (lane < hd) o = fmaf(pj, v[(size_t)(k0 + j) * hd + lane], o);
         }
     }
-    if (lane < hd) orow[lane] = o / l;
+    return o / l;
 }
 
 template <int QG, AOut OUT>
@@ -159,14 +171,27 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
     const int ev = fa.ex ? fa.ex[2 * fa.bh + bh] : fa.ev;
     const int img = bh / fa.heads, head = bh - img * fa.heads;
 
-    if constexpr (OUT == AOut::F32) {
+    if constexpr (OUT != AOut::Split) {
         if (eq == kSplitNonFinite || ek == kSplitNonFinite || ev == kSplitNonFinite) {
             const size_t off = (size_t)bh * T * fa.hd;
             for (int i = wave; i < QG * 32 && q0 + i < T; i += 8) {
-                float *orow = fa.token_major
-                                  ? fa.out + (((size_t)img * T + q0 + i) * fa.heads + head) * fa.hd
-                                  : fa.out + off + (size_t)(q0 + i) * fa.hd;
-                attention_floats(fa.qf + off, fa.kf + off, fa.vf + off, T, fa.hd, fa.scale_log2, q0 + i, orow, lane);
+                const float o =
+                    attention_floats(fa.qf + off, fa.kf + off, fa.vf + off, T, fa.hd, fa.scale_log2, q0 + i, lane);
+                if constexpr (OUT == AOut::Q8) {
+                    float amax = q8_absmax(0.0f, o), d, inv;
+#pragma unroll
+                    for (int x = 1; x < 32; x *= 2) amax = q8_absmax(amax, __shfl_xor(amax, x, kWave));
+                    q8_scale(amax, d, inv);
+                    const size_t rows = (size_t)(fa.bh / fa.heads) * T;
+                    const size_t slot = (size_t)(head * 2 + lane / 32) * rows + (size_t)img * T + q0 + i;
+                    fa.q8_qs[slot * 32 + lane % 32] = (int8_t)q8_value(o, inv);
+                    if (lane % 32 == 0) fa.q8_d[slot] = __builtin_bit_cast(uint16_t, (_Float16)d);
+                } else {
+                    float *orow = fa.token_major
+                                      ? fa.out + (((size_t)img * T + q0 + i) * fa.heads + head) * fa.hd
+                                      : fa.out + off + (size_t)(q0 + i) * fa.hd;
+                    if (lane < fa.hd) orow[lane] = o;
+                }
             }
             return;
         }
@@ -416,6 +441,11 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
     xm[wave * 64 + lane] = make_float4(m[0], m[1], l[0], l[1]);
     __syncthreads();
     constexpr int DF = 4 / KS;
+    // Q8: a block of 32 dims is finished by two streams (16 dims each); their
+    // largest magnitudes meet in LDS.
+    static_assert(OUT != AOut::Q8 || DF == 1, "two streams per Q8_0 block");
+    float *xq = reinterpret_cast<float *>(smem_c + 8 * 8 * 64 * 16 + 8 * 64 * 16);  // [wave][2][16]
+    f32x4 q8v[2];
     float ms[KS][2], ls[KS][2];
 #pragma unroll
     for (int z = 0; z < KS; z++) {
@@ -459,6 +489,16 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
                 *reinterpret_cast<f16x4 *>(dst) = __builtin_shufflevector(h0, h1, 0, 1, 2, 3);
                 *reinterpret_cast<f16x4 *>(dst + 64) = __builtin_shufflevector(l0, l1, 0, 1, 2, 3);
             }
+        } else if constexpr (OUT == AOut::Q8) {
+            float amax = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                q8v[u][e] = __builtin_ldexpf(r[0][e], ev);
+                amax = q8_absmax(amax, q8v[u][e]);
+            }
+            amax = q8_absmax(amax, __shfl_xor(amax, 16, kWave));
+            amax = q8_absmax(amax, __shfl_xor(amax, 32, kWave));
+            if (lh == 0) xq[(wave * 2 + u) * 16 + li] = amax;
         } else {
             if (query >= T) continue;
 #pragma unroll
@@ -478,6 +518,24 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
                         if (d + e < fa.hd) dst[e] = v[e];
                 }
             }
+        }
+    }
+    if constexpr (OUT == AOut::Q8) {
+        __syncthreads();
+        const size_t rows = (size_t)(fa.bh / fa.heads) * T;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int query = q0 + qg * 32 + 16 * u + li;
+            const int other = (stream ^ 1) * QG + qg;
+            float d, inv;
+            q8_scale(fmaxf(xq[(wave * 2 + u) * 16 + li], xq[(other * 2 + u) * 16 + li]), d, inv);
+            if (query >= T) continue;
+            uint32_t w = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) w |= (uint32_t)(q8_value(q8v[u][e], inv) & 0xff) << (8 * e);
+            const size_t slot = (size_t)(head * 2 + stream / 2) * rows + (size_t)img * T + query;
+            *reinterpret_cast<uint32_t *>(fa.q8_qs + slot * 32 + (stream & 1) * 16 + 4 * lh) = w;
+            if (lh == 0 && (stream & 1) == 0) fa.q8_d[slot] = __builtin_bit_cast(uint16_t, (_Float16)d);
         }
     }
 }
@@ -569,7 +627,7 @@ __global__ __launch_bounds__(NT) void attn_split_rows_kernel(const float *__rest
 template <int QG, AOut OUT>
 hipError_t run_attn(hipStream_t s, AttnArgs fa) {
     constexpr size_t lds = 4 * 128 * 256;  // two steps of K and of V panels
-    static_assert(lds >= 8 * 8 * 64 * 16 + 8 * 64 * 16, "the merge fits the panels' LDS");
+    static_assert(lds >= 8 * 8 * 64 * 16 + 8 * 64 * 16 + 8 * 2 * 16 * 4, "the merge fits the panels' LDS");
     auto kernel = attn_split_kernel<QG, OUT>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
@@ -600,9 +658,10 @@ size_t attn_split_bytes(size_t bh, size_t tokens) {
 
 hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, const float *v, float *out,
                                  size_t bh, size_t tokens, size_t heads, size_t hd, bool token_major,
-                                 float softmax_scale, void *ws) {
+                                 float softmax_scale, void *ws, int8_t *q8_qs, uint16_t *q8_d) {
     if (bh == 0 || tokens == 0) return hipSuccess;
     if (!attn_split_fits(bh, tokens) || hd == 0 || hd > 64) return hipErrorInvalidValue;
+    if (q8_qs && (hd != 64 || !q8_d || heads == 0 || bh % heads != 0)) return hipErrorInvalidValue;
     char *planes = static_cast<char *>(ws);
     const size_t each = bh * tokens * 256;
     int *ex = reinterpret_cast<int *>(planes + 3 * each);
@@ -639,7 +698,9 @@ hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, 
     fa.scale_log2 = softmax_scale * kLog2e;
     fa.out = out;
     fa.token_major = token_major ? 1 : 0;
-    return dispatch_attn<AOut::F32>(s, fa);
+    fa.q8_qs = q8_qs;
+    fa.q8_d = q8_d;
+    return q8_qs ? dispatch_attn<AOut::Q8>(s, fa) : dispatch_attn<AOut::F32>(s, fa);
 }
 
 hipError_t launch_attn_split(hipStream_t s, const SplitQkv &p, void *out_split, size_t bh, size_t tokens,

@@ -255,13 +255,15 @@ hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws);
 
 // ---- attention on split rows (k_attn_split.hip) ---------------------------------
 bool attn_split_fits(size_t bh, size_t tokens);
-// Workspace of launch_attn_split_f32.
+// Workspace of launch_attn_split_f32.  With q8_qs and q8_d (head_dim 64) the
+// token-major output is written as Q8_0 blocks instead of to `out`.
 size_t attn_split_bytes(size_t bh, size_t tokens);
 // q/k/v [bh][tokens][hd] f32, hd <= 64; out head-major, or token-major
 // [img][tokens][heads * hd].
 hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, const float *v, float *out,
                                  size_t bh, size_t tokens, size_t heads, size_t hd, bool token_major,
-                                 float softmax_scale, void *ws);
+                                 float softmax_scale, void *ws, int8_t *q8_qs = nullptr,
+                                 uint16_t *q8_d = nullptr);
 // Q, K and V as split rows [bh][tokens][64] with one exponent each (finite
 // or NaN values), head_dim 64, scale 1/8; out_split: split rows
 // [img * tokens][heads * 64] with exponent ev (an output is an average of V

@@ -564,14 +564,16 @@ bool fp32_flash_asked() {
 // Attention of bh heads of `tokens` rows of hd <= 64 floats on the f16
 // matrix cores; *done is false where the fp32 kernels have to run instead.
 vh_status try_attn_split(RtState &s, const float *q, const float *k, const float *v, float *out, size_t bh,
-                         size_t tokens, size_t heads, size_t hd, bool token_major, float scale, bool *done) {
+                         size_t tokens, size_t heads, size_t hd, bool token_major, float scale, bool *done,
+                         int8_t *q8_qs = nullptr, uint16_t *q8_d = nullptr) {
     *done = false;
     if (!vh::attn_split_fits(bh, tokens) || fp32_flash_asked()) return VH_OK;
     const size_t need = (vh::attn_split_bytes(bh, tokens) + sizeof(float) - 1) / sizeof(float);
     if (!grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded)) return VH_OK;
     *done = true;
     return launch(s, "flash_attention", [&] {
-        return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, s.fw);
+        return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, s.fw,
+                                         q8_qs, q8_d);
     });
 }
 
@@ -579,8 +581,11 @@ vh_status flash(RtState &s, const float *q, const float *k, const float *v, floa
                 size_t bh, size_t tokens, size_t heads, bool token_major, int8_t *q8_qs = nullptr,
                 uint16_t *q8_d = nullptr, bool *quantized = nullptr, float scale = 0.125f) {
     bool done = false;
-    TRY(try_attn_split(s, q, k, v, out, bh, tokens, heads, 64, token_major, scale, &done));
-    if (done) return VH_OK;
+    TRY(try_attn_split(s, q, k, v, out, bh, tokens, heads, 64, token_major, scale, &done, q8_qs, q8_d));
+    if (done) {
+        if (quantized) *quantized = q8_qs != nullptr;
+        return VH_OK;
+    }
     // Partials of the key splits (room for either layout: the merge launch's
     // or the in-kernel merge's); without them the kernel runs unsplit.
     const size_t need =
@@ -2374,8 +2379,9 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
         } else {
             TRY(run_q8_qkv(s, b.qqkv, qin, images, tokens, rot, q, k, v, n1));
         }
-        // The attention merge writes Q8_0 rows directly when the keys are
-        // split; otherwise the f32 output is quantised.
+        // The attention writes Q8_0 rows directly (2.66 MB of floats less each
+        // way, and the 4.8 us launch that quantised them, at 865 tokens); the fp32
+        // kernels do so when the keys are split, else their output is quantised.
         Q8Rows a;
         TRY(q8_workspace(s, M, D, &a.qs, &a.d));
         bool quantized = false;
