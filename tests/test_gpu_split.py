@@ -159,7 +159,7 @@ def test_split_attention_head_scales_and_non_finite(rt):
 # channel slices, 1 x 1, 3 x 3 and 5 x 5 taps with and without padding, output
 # channels that fill no tile.
 @pytest.mark.parametrize("in_c, out_c, ih, iw, k, p, relu", [
-    (32, 64, 97, 91, 3, 1, False), (160, 70, 71, 65, 3, 1, True), (256, 33, 96, 93, 1, 0, False),
+    (32, 130, 97, 143, 3, 1, False), (160, 70, 71, 65, 3, 1, True), (256, 257, 96, 93, 1, 0, False),
     (64, 128, 70, 67, 5, 2, False), (96, 130, 61, 50, 3, 0, True)])
 def test_split_convolution_vs_float64(rt, in_c, out_c, ih, iw, k, p, relu):
     x = seeded.normal(10000 + ih, in_c * ih * iw).reshape(in_c, ih, iw)

@@ -1035,14 +1035,28 @@ size_t conv_split_bytes(const SplitConv &c) {
 
 bool conv_split_fits(const SplitConv &c) {
     if (c.in_c % 32 != 0 || c.in_c == 0) return false;
-    const size_t wp = c.iw + 2 * c.pad, hp = c.ih + 2 * c.pad;
+    const size_t wp = c.iw + 2 * c.pad, hp = c.ih + 2 * c.pad, K = c.kh * c.kw * c.in_c;
     const size_t oh = hp - c.kh + 1, ow = wp - c.kw + 1;
-    // Whole 64 x 64 tiles of the fp32 kernel for half the CUs: below that its
-    // K split over idle CUs is as fast (384 -> 128 on 24 x 36: 28 us against
-    // about 25, 768 -> 128 on 12 x 18: 18), and the staging launches here are not.
+    if (K < 256 || hp * wp + c.kw > (size_t)INT32_MAX / 512 || c.in_c / 32 > 65535 ||
+        !split_gemm_fits(oh * wp, c.out_c, K))
+        return false;
+    // Below half the CUs in 64 x 64 tiles the fp32 kernel splits K over the idle
+    // ones, and the staging launches here are no gain (384 -> 128 on 24 x 36: 18
+    // us against about 25).
     const size_t tiles = ((c.out_c + 63) / 64) * ((oh * ow + 63) / 64);
-    return tiles >= 128 && c.kh * c.kw * c.in_c >= 256 && hp * wp + c.kw <= (size_t)INT32_MAX / 512 &&
-           c.in_c / 32 <= 65535 && split_gemm_fits(oh * wp, c.out_c, c.kh * c.kw * c.in_c);
+    if (tiles < 128) return false;
+    // Otherwise by the time of two staging launches at 1.5 TB/s of image and the
+    // product, against 0.75 us per tile and k-slice of the fp32 kernel, a
+    // partial last round as K pieces.  Per call on MI355X, split and fp32 (us):
+    // 128 -> 128 on 96 x 144 30.7 and 53.6, 64 -> 32 on 384 x 576 89 and 171,
+    // 32 -> 128 on 96 x 144 15.3 and 18.1, 1 x 1 256 -> 256 there 25.8 and
+    // 27.9; the fp32 form keeps 32 -> 64 on 97 x 91 (12.1 and 10.8) and 1 x 1
+    // with few outputs (256 -> 33 on 96 x 144 19.1 and 10.0).
+    const int slices = (int)(K / 32);
+    const float split_us =
+        7.0f + (float)(c.in_c * c.ih * c.iw) * 4.0f / 1.5e6f + plan_split(oh * wp, c.out_c, slices, false, false).us;
+    const float rounds = tiles > 256 ? (float)tiles / 256.0f + 0.3f : 1.0f;
+    return split_us < 5.0f + rounds * (float)slices * 0.75f;
 }
 
 hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws) {
