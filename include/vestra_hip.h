@@ -101,7 +101,9 @@ vh_status vh_add_f32_in_place(const vh_runtime *rt, vh_tensor *destination,
 
 /* ---- GEMM and epilogues --------------------------------------------------- */
 /* src/cuda.rs:661-704 gemm_row_major_f32: C[m,n] = A[m,k] x B[k,n], row-major.
- * fp32 MFMA kernel (replaces cublasSgemm). */
+ * Replaces cublasSgemm: f32 in and out, on split rows and the f16 matrix
+ * cores where that is faster (closer to the exact product than the fp32
+ * matrix instructions), else on those. */
 vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor *a, const vh_tensor *b,
                                 size_t m, size_t k, size_t n, vh_tensor **out);
 /* src/cuda.rs:708-742 bias_scale_f32_in_place: v = (v + bias[c]) * gamma[c]. */
@@ -130,7 +132,7 @@ vh_status vh_attention_online_f32(const vh_runtime *rt, const vh_tensor *q, cons
                                   const vh_tensor *v, size_t heads, size_t tokens,
                                   size_t head_dim, vh_tensor **out);
 /* flash_attention_f32_da3_base (src/lib.rs:82-91, src/specialized.rs:730-765):
- * head_dim 64, scale 1/8, fp32-MFMA online softmax.  Any token count is
+ * head_dim 64, scale 1/8, online softmax, split products.  Any token count is
  * accepted (the reference's tokens % 865 gate is a CPU-kernel limit).
  * token_major = 0 writes head-major [heads,tokens,64]; 1 writes token-major
  * [tokens, heads*64] (the fused hnd_to_token of src/cuda.rs:984-1036). */
@@ -141,7 +143,7 @@ vh_status vh_flash_attention_f32_da3_base(const vh_runtime *rt, const vh_tensor 
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): it calls no
  * allocator.  The caller passes `out` (heads*tokens*64 floats, layout as
- * above).  The key-split partials live in a 64 MiB device array of the
+ * above).  The split rows of Q, K and V live in a 64 MiB device array of the
  * library, one per GPU, reserved until the process ends; heads*tokens above
  * 63550 is rejected with VH_ERR_KERNEL before any launch.  Every call on a
  * GPU shares that GPU's array, and the library orders the calls in the order
@@ -325,7 +327,7 @@ vh_status vh_encoder_run(const vh_runtime *rt, const vh_block *const *blocks, si
 
 /* ---- DPT head: convolution, transposed convolution, resize ----------------- */
 /* Batch-1 CHW tensors as in src/conv.rs and src/resample.rs.  Convolutions run
- * as fp32-MFMA GEMMs (direct convolution: the crate's 3x3 stride-1 pad-1
+ * as GEMMs (direct convolution: the crate's 3x3 stride-1 pad-1
  * Winograd F(2x2,3x3) path is tested against the same direct definition,
  * src/conv.rs:1438-1477); results agree with conv2d_naive (src/conv.rs:950-
  * 998) within f32 accumulation error.  The resizes are bit-exact. */
