@@ -7,6 +7,8 @@ inside and between the matrix instructions rounds or truncates by at most
 2^-23 of the running sum of |x w|; a value below 2^-18 of its row's largest
 is held to 2^-40 of that instead.
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -98,6 +100,73 @@ def test_split_gemm_inf_and_nan(rt, where):
         assert np.array_equal(np.isnan(got), np.isnan(ref))
         assert np.array_equal(got[~fine & ~np.isnan(ref)], ref[~fine & ~np.isnan(ref)].astype(np.float32))
         assert np.all(np.abs(got[fine] - clean[fine]) <= 2 * bound[fine])
+
+
+def _launches(rt, run):
+    """The names of the launches that run() makes."""
+    rt.profile_reset()
+    rt.profile_enable(True)
+    try:
+        run()
+        return set(rt.profile_report())
+    finally:
+        rt.profile_enable(False)
+
+
+def _wide_operands(kind, m, k, n):
+    """Finite operands whose large entries meet zeros or small ones."""
+    x = seeded.normal(10300 + m, m * k).reshape(m, k)
+    w = seeded.normal(10400 + n, k * n).reshape(k, n)
+    u = seeded.uniform01(10500, m * k).reshape(m, k)
+    if kind == "outlier":         # one entry of each row, of rising size, has no weight
+        x[:, 7] = np.float32(10.0) ** np.linspace(4, 37, m, dtype=np.float32)
+        w[7] = 0.0
+    elif kind == "weight":        # the same of the columns
+        w[9] = np.float32(10.0) ** np.linspace(-37, 37, n, dtype=np.float32)
+        x[:, 9] = 0.0
+    elif kind == "bands":         # half of the columns see the small half of each row alone
+        x[:, ::2] *= np.float32(2.0 ** 45)
+        w[::2, : n // 2] = 0.0
+    elif kind == "spread":        # log-uniform over 2^80
+        x *= np.exp2(80.0 * u - 40.0).astype(np.float32)
+        w *= np.exp2(80.0 * seeded.uniform01(10600, k * n).reshape(k, n) - 40.0).astype(np.float32)
+    elif kind == "one_hot":       # single entries, some of them tiny
+        w[:] = 0.0
+        w[(np.arange(n) * 7) % k, np.arange(n)] = 1.0
+        x[u < 0.01] *= np.float32(1e-9)
+    elif kind == "gelu":          # a GELU's tail: a tenth of the row far below its largest
+        x = (3 * x * 0.5 * (1 + np.vectorize(math.erf)(3 * x / np.sqrt(2.0)))).astype(np.float32)
+    return x, w
+
+
+@pytest.mark.parametrize("kind", ["outlier", "weight", "bands", "spread", "one_hot", "gelu"])
+@pytest.mark.parametrize("m, k, n", [(65, 101, 770), (97, 2563, 70), (865, 100, 3074), (1153, 1003, 768)])
+def test_split_gemm_of_wide_ranges(rt, kind, m, k, n):
+    """Each output is right to the rounding of its own terms |x w|, whatever
+    else its row and column hold: no term for the range of either."""
+    x, w = _wide_operands(kind, m, k, n)
+    xt, wt = rt.upload_f32(x), rt.upload_f32(w)
+    lin = rt.prepare_linear_f32(k, n, w, np.zeros(n, np.float32))
+    ref = x.astype(np.float64) @ w.astype(np.float64)
+    bound = (2.0 ** -21 + k / 4 * 2.0 ** -23) * (np.abs(x).astype(np.float64) @ np.abs(w)) + 2.0 ** -148
+    res = rt.upload_f32(np.zeros(m * n, np.float32))
+    out = {}
+
+    def run():
+        out["row_major"] = rt.download_f32(rt.gemm_row_major_f32(xt, wt, m, k, n)).reshape(m, n)
+        out["linear"] = rt.download_f32(lin.run(xt, m)).reshape(m, n)
+        out["chw"] = rt.download_f32(lin.run_chw(xt, m)).reshape(n, m).T
+        lin.run_residual(xt, m, res)
+        out["residual"] = rt.download_f32(res).reshape(m, n)
+        if n % 192 == 0:
+            q, kk, v = lin.run_qkv_hnd(xt, 1, m, n // 192)
+            out["qkv"] = np.concatenate([rt.download_f32(t).reshape(n // 192, m, 64).transpose(1, 0, 2).reshape(m, -1)
+                                         for t in (q, kk, v)], axis=1)
+
+    assert {"split_operands", "split_rows"} <= _launches(rt, run)
+    for name, got in out.items():
+        over = np.abs(got - ref) / bound
+        assert np.all(over <= 1.0), (name, float(over.max()), int((over > 1).sum()))
 
 
 def _attention64(q, k, v):

@@ -38,7 +38,7 @@ namespace {
 
 struct SplitArgs {
     const char *x, *w;      // split rows of X [M][Kp] and W [N][Kp]
-    const int *ex, *ew;     // row exponents (ex null: ex_c for every row)
+    const int *ex, *ew;     // row codes (ex null: exponent ex_c for every row)
     int ex_c;
     int M, N, slices;       // slices = Kp / 32
     // K pieces: a tile's slices are shared out over `pieces` workgroups, whose
@@ -48,7 +48,7 @@ struct SplitArgs {
     int pieces;
     float *partial;  // null: whole tiles only
     unsigned *piece_cnt;
-    const float *xf, *wf;   // the f32 rows [M][K], [N][K] (non-finite rows)
+    const float *xf, *wf;   // the f32 rows [M][K], [N][K], or null
     int K, wf_n;            // wf_n: 0, or wf is [K][wf_n]
     float *c;
     const float *bias, *gamma;
@@ -73,29 +73,97 @@ constexpr int kSplitMaxPieces = 4;
 
 enum class SEpi : int { Store, Gelu, Residual, Qkv, GeluSplit, Chw, Conv };
 
-// A product with a non-finite row, in floats: rare, so a plain loop.
-__device__ __attribute__((noinline)) float split_slow_dot(const float *x, const float *w, size_t step, int K) {
-    if (!x || !w) return __builtin_nanf("");
-    float s = 0.0f;
-    for (int k = 0; k < K; k++) s = fmaf(x[k], w[k * step], s);
-    return s;
+// ---- outputs recomputed in floats -------------------------------------------------
+// The halves of a value below 2^-3 of the scaled row (a "small" one, at most 2^-17
+// of the row's largest) are off by up to 2^-25, so n_x of them in a row of X and
+// n_w in a row of W leave an error of at most (n_x + n_w) 2^-25 2^15 in a
+// scaled product of the rows.  Where the product is at least 2^22 times
+// that, it is right to the halves' own 2^-22; where it is less (the large
+// values cancelled, or met zeros), it is formed again from the floats.
+// Rows of ordinary data hold a small value once in a hundred (N(0, 1), K =
+// 768), and then one product in 10^5 or so is that small.
+constexpr float kSmallBound = 0x1p12f;
+// Up to this many outputs of a wave's tile one at a time (2 us each), else the
+// tile on the fp32 matrix instructions, at about their rate in the fp32 GEMM.
+constexpr int kFewOutputs = 12;
+
+// Convolution: float (tap, channel) k of output m's window, 0 outside the image.
+__device__ __forceinline__ float conv_value(const SplitArgs &ar, int m, int k) {
+    const int cin = ar.conv_cs * 32, t = k / cin, c = k - t * cin, y = m / ar.conv_wp;
+    const int yy = y + t / ar.conv_kw - ar.conv_pad, xx = m - y * ar.conv_wp + t % ar.conv_kw - ar.conv_pad;
+    if (yy < 0 || yy >= ar.conv_ih || xx < 0 || xx >= ar.conv_iw) return 0.0f;
+    const float v = ar.xf[((size_t)c * ar.conv_ih + yy) * ar.conv_iw + xx];
+    return ar.conv_relu ? fmaxf(v, 0.0f) : v;
 }
 
-// One output of a convolution in floats, for an image or weight with an inf or
-// NaN: taps outside the image are zeros that are still multiplied.
-__device__ __attribute__((noinline)) float split_slow_conv(const float *img, const float *w, int taps, int kw, int ic,
-                                                           int ih, int iw, int pad, int relu, int y, int x) {
+// Output (m, n) by a whole wave (the same m and n in every lane).
+template <bool CONV>
+__device__ __forceinline__ float float_dot(const SplitArgs &ar, int m, int n, int lane) {
+    const float *w = ar.wf + (ar.wf_n ? (size_t)n : (size_t)n * ar.K);
+    const size_t step = ar.wf_n ? (size_t)ar.wf_n : 1;
     float s = 0.0f;
-    for (int t = 0; t < taps; t++) {
-        const int yy = y + t / kw - pad, xx = x + t % kw - pad;
-        const bool in = yy >= 0 && yy < ih && xx >= 0 && xx < iw;
-        for (int c = 0; c < ic; c++) {
-            float v = in ? img[((size_t)c * ih + yy) * iw + xx] : 0.0f;
-            if (relu) v = fmaxf(v, 0.0f);
-            s = fmaf(v, w[(size_t)t * ic + c], s);
-        }
+#pragma unroll 8
+    for (int k = lane; k < ar.K; k += 64) {
+        const float x = CONV ? conv_value(ar, m, k) : ar.xf[(size_t)m * ar.K + k];
+        s = fmaf(x, w[k * step], s);
     }
-    return s;
+    return wave_sum(s);
+}
+
+// A wave's tile, FO x FN fragments of 16 x 16 in the layout of the split
+// products: rows m = mb + 16 i (mb with the lane's row), columns from nb on.
+// The 16 values of a step go to the lanes as k = k0 + 4 (lane / 16) + 0 .. 3.
+template <int FO, int FN, bool CONV>
+__device__ __forceinline__ void float_tile(const SplitArgs &ar, int mb, int nb, int lane, f32x4 (&out)[FO][FN]) {
+    const int li = lane & 15, lh = lane >> 4;
+    constexpr int D = 12 / (FO + FN) < 1 ? 1 : 12 / (FO + FN);  // steps loaded at once
+    const bool vec = (ar.K & 3) == 0, xvec = vec && !CONV, wvec = vec && !ar.wf_n;
+    auto four = [&](const float *p, size_t step, bool v16, int k) {
+        f32x4 v{0.0f, 0.0f, 0.0f, 0.0f};
+        if (v16) {
+            if (k < ar.K) v = *reinterpret_cast<const f32x4 *>(p + k);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (k + e < ar.K) v[e] = p[(size_t)(k + e) * step];
+        }
+        return v;
+    };
+#pragma unroll
+    for (int i = 0; i < FO; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) out[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k0 = 0; k0 < ar.K; k0 += 16 * D) {
+        f32x4 xv[D][FO], wv[D][FN];
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int k = k0 + 16 * d + 4 * lh;
+#pragma unroll
+            for (int i = 0; i < FO; i++) {
+                const int m = min(mb + 16 * i, ar.M - 1);
+                if constexpr (CONV) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) xv[d][i][e] = k < ar.K ? conv_value(ar, m, k + e) : 0.0f;
+                } else {
+                    xv[d][i] = four(ar.xf + (size_t)m * ar.K, 1, xvec, k);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < FN; j++) {
+                const size_t n = min(nb + 16 * j + li, ar.N - 1);
+                wv[d][j] = four(ar.wf + (ar.wf_n ? n : n * ar.K), ar.wf_n ? ar.wf_n : 1, wvec, k);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int i = 0; i < FO; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+                        out[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[d][j][e], xv[d][i][e], out[i][j], 0, 0, 0);
+    }
 }
 
 template <int BM, int BN, int WM, int WN, int KG, int ST, SEpi EPI, bool PIECES>
@@ -385,31 +453,36 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     const int mb = m0 + wm * TM + kg * FO * 16 + li, nb = n0 + wn * TN + 4 * lh;
     if (n0 + wn * TN >= ar.N) return;
     const bool vec = (ar.N & 3) == 0;
-    int exr[FO], ewr[FN][4];
+    int xcode[FO], wcode[FN][4];
     float bias[FN][4], gamma[FN][4];
 #pragma unroll
     for (int i = 0; i < FO; i++)
-        exr[i] = ar.ex ? ar.ex[EPI == SEpi::Conv ? 0 : min(mb + 16 * i, ar.M - 1)] : ar.ex_c;
+        xcode[i] = ar.ex ? ar.ex[EPI == SEpi::Conv ? 0 : min(mb + 16 * i, ar.M - 1)] : split_code(ar.ex_c, 0);
 #pragma unroll
     for (int j = 0; j < FN; j++)
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int cn = min(nb + 16 * j + r, ar.N - 1);
-            ewr[j][r] = ar.ew[cn];
+            wcode[j][r] = ar.ew[cn];
             bias[j][r] = load_or(ar.bias, reinterpret_cast<const float *>(ar.ew), cn, 0.0f);
             gamma[j][r] = load_or(ar.gamma, reinterpret_cast<const float *>(ar.ew), cn, 1.0f);
         }
     f32x4 old[EPI == SEpi::Residual ? FO : 1][FN];
-    if constexpr (EPI == SEpi::Residual) {
-        if (vec) {
+    auto load_old = [&] {
+        if constexpr (EPI == SEpi::Residual) {
+            if (vec) {
 #pragma unroll
-            for (int i = 0; i < FO; i++)
+                for (int i = 0; i < FO; i++)
 #pragma unroll
-                for (int j = 0; j < FN; j++)
-                    old[i][j] = *reinterpret_cast<const f32x4 *>(
-                        ar.c + (size_t)min(mb + 16 * i, ar.M - 1) * ar.N + min(nb + 16 * j, ar.N - 4));
+                    for (int j = 0; j < FN; j++)
+                        old[i][j] = *reinterpret_cast<const f32x4 *>(
+                            ar.c + (size_t)min(mb + 16 * i, ar.M - 1) * ar.N + min(nb + 16 * j, ar.N - 4));
+            }
         }
-    }
+    };
+    // Early, behind what follows; on the largest tile its registers are needed.
+    constexpr bool EARLY = FO * FN < 16;
+    if constexpr (EARLY) load_old();
     // Qkv: the wave's columns lie in one head of one of Q, K, V.
     const int colw = n0 + wn * TN;
     float *head_dst = nullptr;
@@ -421,6 +494,83 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
         head_scale = group == 0 ? ar.qkv_scale[0] : (group == 1 ? ar.qkv_scale[1] : ar.qkv_scale[2]);
         rope = ar.rot != nullptr && group < 2;
     }
+    // The products in their own scale, and from the floats where small values
+    // may show (kSmallBound) or a value is not finite.
+    auto too_small = [&](int i, int j, int r) {
+        const float n = (float)(split_code_small(xcode[i]) + split_code_small(wcode[j][r]));
+        return !(__builtin_fabsf(fin[i][j][r]) >= n * kSmallBound);
+    };
+    // First the lane's least product against its largest counts (a product of
+    // finite rows is no NaN; a convolution's may be), then each of them.
+    bool spoilt = false;
+    if (ar.xf && ar.wf) {
+        float least = INFINITY;
+        int nx = 0, nw = 0;
+#pragma unroll
+        for (int i = 0; i < FO; i++) nx = max(nx, split_code_small(xcode[i]));
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                nw = max(nw, split_code_small(wcode[j][r]));
+#pragma unroll
+                for (int i = 0; i < FO; i++) {
+                    const float p = __builtin_fabsf(fin[i][j][r]);
+                    if constexpr (EPI == SEpi::Conv) spoilt |= p != p;
+                    least = fminf(least, p);
+                }
+            }
+        spoilt |= least < (float)(nx + nw) * kSmallBound;
+    }
+    uint64_t bad = 0;  // of this lane, bit (i * FN + j) * 4 + r
+    static_assert(FO * FN * 4 <= 64, "one bit per output");
+    spoilt = __any(spoilt);
+    if (spoilt) {
+#pragma unroll
+        for (int i = 0; i < FO; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = mb + 16 * i, n = nb + 16 * j + r;
+                    const bool real = m < ar.M && n < ar.N && (EPI != SEpi::Conv || m % ar.conv_wp < ar.conv_ow);
+                    if (real && too_small(i, j, r)) bad |= (uint64_t)1 << ((i * FN + j) * 4 + r);
+                }
+    }
+#pragma unroll
+    for (int j = 0; j < FN; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int i = 0; i < FO; i++)
+                fin[i][j][r] = __builtin_ldexpf(fin[i][j][r], split_code_exponent(xcode[i]) + split_code_exponent(wcode[j][r]));
+    if (spoilt) {
+        // The arguments are read again here, so that the loop above need not
+        // hold those of this rare path, nor the registers of `old`.
+        const auto *again = (const __attribute__((address_space(4))) SplitArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(again));
+        SplitArgs late;
+        __builtin_memcpy(&late, (const void *)again, sizeof(late));
+        if (wave_sum((float)__popcll(bad)) > (float)kFewOutputs) {
+            float_tile<FO, FN, EPI == SEpi::Conv>(late, mb, nb - 4 * lh, lane, fin);
+        } else {
+            for (uint64_t lanes = __ballot(bad != 0); lanes; lanes = __ballot(bad != 0)) {
+                const int src = (int)__ffsll((unsigned long long)lanes) - 1;
+                const int bit = __shfl((int)__ffsll((unsigned long long)bad) - 1, src, 64);
+                const int i = bit / (4 * FN), j = bit / 4 % FN, r = bit % 4;
+                const float s = float_dot<EPI == SEpi::Conv>(late, __shfl(mb, src, 64) + 16 * i,
+                                                             __shfl(nb, src, 64) + 16 * j + r, lane);
+                if (lane == src) {
+                    bad &= bad - 1;
+#pragma unroll
+                    for (int e = 0; e < FO * FN * 4; e++)
+                        if (e == bit) fin[e / (4 * FN)][e / 4 % FN][e % 4] = s;
+                }
+            }
+        }
+        if constexpr (EARLY) load_old();
+    }
+    if constexpr (!EARLY) load_old();
 #pragma unroll
     for (int i = 0; i < FO; i++) {
         const int m = mb + 16 * i;
@@ -430,22 +580,7 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
         for (int j = 0; j < FN; j++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                float t = __builtin_ldexpf(fin[i][j][r], exr[i] + ewr[j][r]);
-                if constexpr (EPI == SEpi::Conv) {
-                    // The image's inf and NaN are in its halves: what they
-                    // reach is a NaN here.
-                    if (t != t || ewr[j][r] == kSplitNonFinite) {
-                        const int n = min(nb + 16 * j + r, ar.N - 1), y = m / ar.conv_wp;
-                        t = split_slow_conv(ar.xf, ar.wf + (size_t)n * ar.K, ar.slices / ar.conv_cs, ar.conv_kw,
-                                            ar.conv_cs * 32, ar.conv_ih, ar.conv_iw, ar.conv_pad, ar.conv_relu, y,
-                                            m - y * ar.conv_wp);
-                    }
-                } else if (exr[i] == kSplitNonFinite || ewr[j][r] == kSplitNonFinite) {
-                    const int n = min(nb + 16 * j + r, ar.N - 1);
-                    t = split_slow_dot(ar.xf ? ar.xf + (size_t)m * ar.K : nullptr,
-                                       ar.wf ? ar.wf + (ar.wf_n ? n : (size_t)n * ar.K) : nullptr,
-                                       ar.wf_n ? ar.wf_n : 1, ar.K);
-                }
+                float t = fin[i][j][r];
                 if (ar.bias) t = add_rn(t, bias[j][r]);
                 if constexpr (EPI == SEpi::Store || EPI == SEpi::Residual || EPI == SEpi::Chw)
                     if (ar.gamma) t = mul_rn(t, gamma[j][r]);
@@ -557,18 +692,28 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
 // Rows of up to 1024 values stay in registers between the two passes (the
 // row is read once: 865 x 768 in 2.4 us); longer rows are read again, from
 // the cache.
-__device__ __forceinline__ void store_split4(char *row, int k, f32x4 v, int e) {
+__device__ __forceinline__ int store_split4(char *row, int k, f32x4 v, int e) {
     f16x4 hi, lo;
+    int small = 0;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         _Float16 h, l;
-        split_f16(__builtin_ldexpf(v[r], -e), h, l);
+        const float t = __builtin_ldexpf(v[r], -e);
+        split_f16(t, h, l);
         hi[r] = h;
         lo[r] = l;
+        small += split_small(v[r], t);
     }
     char *p = row + (k / 32) * 128 + (k % 32) * 2;
     *reinterpret_cast<f16x4 *>(p) = hi;
     *reinterpret_cast<f16x4 *>(p + 64) = lo;
+    return small;
+}
+
+// A wave's count of small values and its exponent to the row's code.
+__device__ __forceinline__ int wave_split_code(int e, int small) {
+    const float n = wave_sum((float)small);
+    return e == kSplitNonFinite ? kSplitNonFinite : split_code(e, (int)n);
 }
 
 // One row of K floats to its split row, by one wave.
@@ -576,7 +721,7 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
                                           int K, int slices, int lane) {
     const int Kp = slices * 32;
     uint32_t mx = 0;
-    int e;
+    int e, small = 0;
     const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
     if ((K & 3) == 0) {
         const f32x4 *src4 = reinterpret_cast<const f32x4 *>(src);
@@ -590,7 +735,8 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
             e = split_exponent(wave_umax(mx));
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (lane + j * 64 < np4) store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
+                if (lane + j * 64 < np4)
+                    small += store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
         } else {
             int c = lane;
             for (; c + 192 < n4; c += 256)
@@ -599,14 +745,16 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
             e = split_exponent(wave_umax(mx));
 #pragma unroll 4
             for (c = lane; c < np4; c += 64)
-                store_split4(dst, 4 * c, c < n4 && e != kSplitNonFinite ? src4[c] : zero, e);
+                small += store_split4(dst, 4 * c, c < n4 && e != kSplitNonFinite ? src4[c] : zero, e);
         }
     } else {
         // Rows that are not 16-byte aligned: lane-consecutive floats, sixteen
         // loads in flight, in registers when the row has at most 1024.
         auto store1 = [&](int k, float v) {
             _Float16 h, l;
-            split_f16(__builtin_ldexpf(v, -e), h, l);
+            const float t = __builtin_ldexpf(v, -e);
+            split_f16(t, h, l);
+            small += split_small(v, t);
             _Float16 *p = reinterpret_cast<_Float16 *>(dst + (k / 32) * 128) + k % 32;
             p[0] = h;
             p[32] = l;
@@ -629,7 +777,8 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
                 if (k0 + lane + 64 * j < Kp) store1(k0 + lane + 64 * j, e == kSplitNonFinite ? 0.0f : r[j]);
         }
     }
-    if (lane == 0) *ex = e;
+    const int code = wave_split_code(e, small);
+    if (lane == 0) *ex = code;
 }
 
 __global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict__ in, char *__restrict__ out,
@@ -642,7 +791,8 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float *__restrict
 // LayerNorm of each row straight into split rows (launch_layernorm's bits,
 // then split): cols % 32 == 0, cols <= 1024, one wave per row.  A row whose
 // normalised values hold a NaN (an infinity cannot arise without one in
-// the statistics) is stored as NaN with exponent 0.
+// the statistics) is stored as NaN with exponent 0.  Small values are not
+// counted: its products take no float rows.
 __global__ __launch_bounds__(256) void layernorm_split_kernel(const float *__restrict__ in,
                                                               const float *__restrict__ gamma,
                                                               const float *__restrict__ beta,
@@ -681,7 +831,7 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float *__res
 #pragma unroll
     for (int j = 0; j < 4; j++)
         if (lane + j * 64 < n4) store_split4(dst, 4 * (lane + j * 64), r[j], e);
-    if (lane == 0) ex[row] = e;
+    if (lane == 0) ex[row] = split_code(e, 0);
 }
 
 // Upper bound of |LayerNorm(x) . w_n + b_n| over every x, per row n of
@@ -753,7 +903,7 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
 #pragma unroll
     for (int w = 0; w < 16; w++) m = max(m, red[w][sc]);
     const int e = split_exponent(m), sn = n0 + sc;
-    if (sk == 0 && sn < N) eb[sn] = e;
+    int small = 0;
     for (int k0 = 0; k0 < slices * 32; k0 += 1024) {
         if (K > 1024) load(k0);
 #pragma unroll
@@ -768,10 +918,12 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
                 f32x4 v;
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = e == kSplitNonFinite ? 0.0f : tile[4 * sk + j][sc];
-                store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
+                small += store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
             }
         }
     }
+    const int code = wave_split_code(e, small);  // a column's tiles are stored by one wave
+    if (sk == 0 && sn < N) eb[sn] = code;
 }
 
 // Largest finite magnitude (as bits) of each chunk of n floats, with ReLU
@@ -839,7 +991,7 @@ __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__re
     }
     __syncthreads();
     const int e = split_exponent(max(max(red[0], red[1]), max(red[2], red[3])));
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ex[0] = e;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ex[0] = split_code(e, 0);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const int pos = i * 32 + (threadIdx.x >> 3), c4 = 4 * (threadIdx.x & 7), q = blockIdx.x * 64 + pos;

@@ -177,10 +177,16 @@ constexpr size_t kTailFloats = kTailTiles * 4 * 64 * 64;
 
 // ---- GEMM on split rows (k_split.hip) -------------------------------------------
 // Split rows (split_gemm.h): each float row as two halves per value and one
-// power-of-two exponent, rows * ceil(k / 32) * 128 bytes and one int per row.
-// Exponent of a row that holds an infinity or NaN: its halves are zeros and
-// the GEMM recomputes its products from the floats.
-constexpr int kSplitNonFinite = INT32_MIN / 4;
+// power-of-two exponent, rows * ceil(k / 32) * 128 bytes and one code per row:
+// the exponent, and how many of its values are small (nonzero and below 2^-3
+// once scaled: held to 2^-25 there, larger ones to 2^-22 of themselves).  The
+// GEMM recomputes from the floats the outputs that small values may have
+// spoilt, and those of a row that holds an infinity or NaN (its halves are
+// zeros).
+constexpr int kSplitNonFinite = INT32_MAX;
+constexpr int split_code(int exponent, int small) { return (small << 10) | (exponent + 512); }
+constexpr int split_code_exponent(int code) { return (code & 1023) - 512; }
+constexpr int split_code_small(int code) { return code >> 10; }
 // Shapes launch_gemm_split takes.
 bool split_gemm_fits(size_t m, size_t n, size_t k);
 // Whether splitting split_values floats and multiplying them is predicted to
@@ -199,12 +205,11 @@ hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *ga
                                   const float *bias, float *bound, size_t n, size_t k);
 struct SplitGemm {
     const void *x;          // split rows [m][k]
-    const int *ex;          // their exponents, or null: ex_c for all
+    const int *ex;          // their codes, or null: exponent ex_c for all
     int ex_c;
     const void *w;          // split rows [n][k]
     const int *ew;
-    // The float rows, read for rows that hold an inf or NaN (null: such
-    // products are NaN).
+    // The float rows, read for the outputs recomputed in floats (null: none is).
     const float *xf, *wf;
     bool wf_columns;        // wf is [k][n]
     size_t m, n, k;

@@ -3,8 +3,11 @@
 // A float row is scaled by a power of two so that its largest magnitude lies
 // in [2^14, 2^15), and each scaled value v is held as two halves, hi = f16(v)
 // and lo = f16(v - hi): 22 significand bits and lo's sign, about 23 in all,
-// for every value within 2^-18 of the row's largest (smaller ones keep an
-// absolute error of 2^-40 of it).  A product of two such rows is
+// for every value within 2^-18 of the row's largest.  Smaller ones keep an
+// absolute error of 2^-40 of it, which shows where the large values of a row
+// meet zeros or small values: a row's code counts them, and what they may have
+// spoilt is recomputed in floats (gemm_split_kernel).  A product of two such
+// rows is
 //     sum hi.hi + hi.lo + lo.hi      (lo.lo, below 2^-22 of hi.hi, dropped)
 // accumulated in f32 by v_mfma_f32_16x16x32_f16: three instructions of 16
 // cycles for 32 k-values against eight v_mfma_f32_16x16x4_f32 of 32 cycles.
@@ -54,6 +57,11 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
         v = w > v ? w : v;
     }
     return v;
+}
+
+// A value that the halves hold to less than 2^-22 of itself (v, scaled to t).
+__device__ __forceinline__ int split_small(float v, float t) {
+    return v != 0.0f && !(__builtin_fabsf(t) >= 0.125f);
 }
 
 // Running maximum of magnitudes as bit patterns (a NaN sorts above every number).
