@@ -224,6 +224,50 @@ def test_split_attention_head_scales_and_non_finite(rt):
     assert np.abs(got[4][:, cols] - clean[4][:, cols]).max() <= 2e-5 * 5
 
 
+def _conv64(x, w, p):
+    out_c, _, kh, kw = w.shape
+    z = np.pad(x.astype(np.float64), ((0, 0), (p, p), (p, p)))
+    oh, ow = z.shape[1] - kh + 1, z.shape[2] - kw + 1
+    out = np.zeros((out_c, oh, ow))
+    for ky in range(kh):
+        for kx in range(kw):
+            tap = z[:, ky:ky + oh, kx:kx + ow].reshape(z.shape[0], -1)
+            out += (w[:, :, ky, kx].astype(np.float64) @ tap).reshape(out.shape)
+    return out
+
+
+@pytest.mark.parametrize("kind", ["pixel", "lowest", "channel", "region", "weight", "tiny"])
+@pytest.mark.parametrize("in_c, out_c, ih, iw, k, p, relu", [
+    (32, 130, 97, 143, 3, 1, False), (160, 70, 71, 65, 3, 1, True), (256, 257, 96, 93, 1, 0, False),
+    (96, 130, 61, 50, 3, 0, False)])
+def test_split_convolution_of_wide_ranges(rt, kind, in_c, out_c, ih, iw, k, p, relu):
+    """Each output is right to the rounding of the terms in its own window,
+    whatever else the image and the weight hold."""
+    x = seeded.normal(10700 + ih, in_c * ih * iw).reshape(in_c, ih, iw)
+    w = seeded.normal(10800 + k, out_c * in_c * k * k, 0.05).reshape(out_c, in_c, k, k)
+    if kind == "pixel":       # one far pixel, each size in its own channel
+        x[:, ih // 2, iw // 3] = np.float32(10.0) ** np.linspace(3, 30, in_c, dtype=np.float32)
+    elif kind == "lowest":    # a mask of the type's lowest value, weightless channels under it
+        x[0, :, : iw // 4] = np.finfo(np.float32).min
+        w[:, 0] = 0.0
+    elif kind == "channel":   # a large channel that half of the outputs do not see
+        x[5] *= np.float32(1e12)
+        w[: out_c // 2, 5] = 0.0
+    elif kind == "region":    # a dark region
+        x[:, : ih // 2] *= np.float32(1e-11)
+    elif kind == "weight":    # large weights on empty channels
+        w[:, 3] = np.float32(1e15)
+        x[3] = 0.0
+    elif kind == "tiny":      # values of every size down to a subnormal
+        x *= np.exp2(-120.0 * seeded.uniform01(10900, x.size)).astype(np.float32).reshape(x.shape)
+    xin = np.maximum(x, 0) if relu else x
+    exp, mag = _conv64(xin, w, p), _conv64(np.abs(xin), np.abs(w), p)
+    conv = rt.prepare_conv2d_f32(in_c, out_c, k, k, 1, p, w, np.zeros(out_c, np.float32))
+    got = rt.download_f32((conv.run_relu_input if relu else conv.run)(rt.upload_f32(x), ih, iw)).reshape(exp.shape)
+    over = np.abs(got - exp) / ((2.0 ** -21 + in_c * k * k / 4 * 2.0 ** -23) * mag + 2.0 ** -148)
+    assert np.all(over <= 1.0), (float(over.max()), int((over > 1).sum()))
+
+
 # Grids of at least 128 64 x 64 tiles: ragged rows and widths, one and five
 # channel slices, 1 x 1, 3 x 3 and 5 x 5 taps with and without padding, output
 # channels that fill no tile.

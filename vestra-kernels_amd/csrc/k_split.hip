@@ -62,7 +62,9 @@ struct SplitArgs {
     // row m of the product reads image row m + ky * conv_wp + kx.  C^T goes to
     // c[n][y][x] for x < conv_ow (m = y * conv_wp + x), conv_plane floats a
     // channel.  xf is the CHW image [conv_cs * 32][conv_ih][conv_iw] and wf
-    // [N][taps][channels], for the outputs an inf or NaN reaches.
+    // [N][taps][channels], and conv_small [M] the small values of each
+    // output's window.
+    const int *conv_small;
     int conv_cs, conv_kw, conv_wp, conv_ow, conv_ih, conv_iw, conv_pad, conv_relu;
     size_t conv_plane;
     char *out_split;        // GeluSplit: split rows [M][N] of the output times out_scale
@@ -87,13 +89,18 @@ constexpr float kSmallBound = 0x1p12f;
 // tile on the fp32 matrix instructions, at about their rate in the fp32 GEMM.
 constexpr int kFewOutputs = 12;
 
-// Convolution: float (tap, channel) k of output m's window, 0 outside the image.
-__device__ __forceinline__ float conv_value(const SplitArgs &ar, int m, int k) {
+// Convolution: the floats (tap, channel) k and on, N of one tap, of output m's
+// window; 0 outside the image.
+template <int N>
+__device__ __forceinline__ void conv_values(const SplitArgs &ar, int m, int k, float (&v)[N]) {
     const int cin = ar.conv_cs * 32, t = k / cin, c = k - t * cin, y = m / ar.conv_wp;
     const int yy = y + t / ar.conv_kw - ar.conv_pad, xx = m - y * ar.conv_wp + t % ar.conv_kw - ar.conv_pad;
-    if (yy < 0 || yy >= ar.conv_ih || xx < 0 || xx >= ar.conv_iw) return 0.0f;
-    const float v = ar.xf[((size_t)c * ar.conv_ih + yy) * ar.conv_iw + xx];
-    return ar.conv_relu ? fmaxf(v, 0.0f) : v;
+    const bool in = yy >= 0 && yy < ar.conv_ih && xx >= 0 && xx < ar.conv_iw;
+#pragma unroll
+    for (int e = 0; e < N; e++) {
+        v[e] = in ? ar.xf[((size_t)(c + e) * ar.conv_ih + yy) * ar.conv_iw + xx] : 0.0f;
+        if (ar.conv_relu) v[e] = fmaxf(v[e], 0.0f);
+    }
 }
 
 // Output (m, n) by a whole wave (the same m and n in every lane).
@@ -104,8 +111,10 @@ __device__ __forceinline__ float float_dot(const SplitArgs &ar, int m, int n, in
     float s = 0.0f;
 #pragma unroll 8
     for (int k = lane; k < ar.K; k += 64) {
-        const float x = CONV ? conv_value(ar, m, k) : ar.xf[(size_t)m * ar.K + k];
-        s = fmaf(x, w[k * step], s);
+        float x[1];
+        if constexpr (CONV) conv_values(ar, m, k, x);
+        else x[0] = ar.xf[(size_t)m * ar.K + k];
+        s = fmaf(x[0], w[k * step], s);
     }
     return wave_sum(s);
 }
@@ -142,8 +151,9 @@ __device__ __forceinline__ void float_tile(const SplitArgs &ar, int mb, int nb, 
             for (int i = 0; i < FO; i++) {
                 const int m = min(mb + 16 * i, ar.M - 1);
                 if constexpr (CONV) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) xv[d][i][e] = k < ar.K ? conv_value(ar, m, k + e) : 0.0f;
+                    float v[4]{};
+                    if (k < ar.K) conv_values(ar, m, k, v);
+                    xv[d][i] = f32x4{v[0], v[1], v[2], v[3]};
                 } else {
                     xv[d][i] = four(ar.xf + (size_t)m * ar.K, 1, xvec, k);
                 }
@@ -209,6 +219,8 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     const size_t pitch = (size_t)ar.slices * 128;
     const size_t xpitch = EPI == SEpi::Conv ? (size_t)ar.conv_cs * 128 : pitch;
     const char *xb = ar.x + (size_t)m0 * xpitch, *wb = ar.w + (size_t)n0 * pitch;
+
+    const int mb = m0 + wm * TM + kg * FO * 16 + li;  // this lane's first row of the epilogue
 
     // Copy i of this wave moves rows 8 b .. 8 b + 7 (b = i * NW + gw) of the
     // stage; LDS granule p of a row holds global granule p ^ (row % 8), so
@@ -316,6 +328,10 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     split_wait<(ST - 1) * LD>();
     __builtin_amdgcn_s_barrier();
     fetch(0, 0);
+    int window_small[EPI == SEpi::Conv ? FO : 1];  // landed by the time the loop ends
+    if constexpr (EPI == SEpi::Conv)
+#pragma unroll
+        for (int i = 0; i < FO; i++) window_small[i] = ar.conv_small[min(mb + 16 * i, ar.M - 1)];
     // Step t: products of slice t (fragments in registers) while the
     // fragments of slice t + 1 are read; the buffer of slice t, whose reads
     // ended before this step's barrier, takes slice t + ST.  Copies past the
@@ -450,14 +466,15 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
     }
 
     // Epilogue: lane (li, lh) holds C[m][n .. n + 3], m = mb + 16 i, n = nb + 16 j.
-    const int mb = m0 + wm * TM + kg * FO * 16 + li, nb = n0 + wn * TN + 4 * lh;
+    const int nb = n0 + wn * TN + 4 * lh;
     if (n0 + wn * TN >= ar.N) return;
     const bool vec = (ar.N & 3) == 0;
     int xcode[FO], wcode[FN][4];
     float bias[FN][4], gamma[FN][4];
 #pragma unroll
     for (int i = 0; i < FO; i++)
-        xcode[i] = ar.ex ? ar.ex[EPI == SEpi::Conv ? 0 : min(mb + 16 * i, ar.M - 1)] : split_code(ar.ex_c, 0);
+        if constexpr (EPI == SEpi::Conv) xcode[i] = ar.ex[0] + split_code(-512, window_small[i]);
+        else xcode[i] = ar.ex ? ar.ex[min(mb + 16 * i, ar.M - 1)] : split_code(ar.ex_c, 0);
 #pragma unroll
     for (int j = 0; j < FN; j++)
 #pragma unroll
@@ -692,35 +709,32 @@ __global__ __launch_bounds__(WM *WN *KG * 64) void gemm_split_kernel(SplitArgs a
 // Rows of up to 1024 values stay in registers between the two passes (the
 // row is read once: 865 x 768 in 2.4 us); longer rows are read again, from
 // the cache.
-__device__ __forceinline__ int store_split4(char *row, int k, f32x4 v, int e) {
+__device__ __forceinline__ void store_split4(char *row, int k, f32x4 v, int e) {
     f16x4 hi, lo;
-    int small = 0;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         _Float16 h, l;
-        const float t = __builtin_ldexpf(v[r], -e);
-        split_f16(t, h, l);
+        split_f16(__builtin_ldexpf(v[r], -e), h, l);
         hi[r] = h;
         lo[r] = l;
-        small += split_small(v[r], t);
     }
     char *p = row + (k / 32) * 128 + (k % 32) * 2;
     *reinterpret_cast<f16x4 *>(p) = hi;
     *reinterpret_cast<f16x4 *>(p + 64) = lo;
-    return small;
 }
 
-// A wave's count of small values and its exponent to the row's code.
-__device__ __forceinline__ int wave_split_code(int e, int small) {
-    const float n = wave_sum((float)small);
-    return e == kSplitNonFinite ? kSplitNonFinite : split_code(e, (int)n);
+// The code of a row of exponent e of which each lane of a wave has found n
+// small values.
+__device__ __forceinline__ int wave_split_code(int e, int n) {
+    if (e == kSplitNonFinite) return kSplitNonFinite;
+    return split_code(e, __any(n) ? (int)wave_sum((float)n) : 0);
 }
 
 // One row of K floats to its split row, by one wave.
 __device__ __forceinline__ void split_row(const float *__restrict__ src, char *__restrict__ dst, int *__restrict__ ex,
                                           int K, int slices, int lane) {
     const int Kp = slices * 32;
-    uint32_t mx = 0;
+    uint32_t mx = 0, limit;
     int e, small = 0;
     const f32x4 zero{0.0f, 0.0f, 0.0f, 0.0f};
     if ((K & 3) == 0) {
@@ -733,28 +747,32 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
 #pragma unroll
             for (int j = 0; j < 4; j++) mx = absmax4(mx, r[j]);
             e = split_exponent(wave_umax(mx));
+            limit = small_limit(e);
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (lane + j * 64 < np4)
-                    small += store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
+            for (int j = 0; j < 4; j++) {
+                if (lane + j * 64 < np4) store_split4(dst, 4 * (lane + j * 64), e == kSplitNonFinite ? zero : r[j], e);
+                small += small_count4(r[j], limit);
+            }
         } else {
             int c = lane;
             for (; c + 192 < n4; c += 256)
                 mx = absmax4(absmax4(absmax4(absmax4(mx, src4[c]), src4[c + 64]), src4[c + 128]), src4[c + 192]);
             for (; c < n4; c += 64) mx = absmax4(mx, src4[c]);
             e = split_exponent(wave_umax(mx));
+            limit = small_limit(e);
 #pragma unroll 4
-            for (c = lane; c < np4; c += 64)
-                small += store_split4(dst, 4 * c, c < n4 && e != kSplitNonFinite ? src4[c] : zero, e);
+            for (c = lane; c < np4; c += 64) {
+                const f32x4 v = c < n4 && e != kSplitNonFinite ? src4[c] : zero;
+                small += small_count4(v, limit);
+                store_split4(dst, 4 * c, v, e);
+            }
         }
     } else {
         // Rows that are not 16-byte aligned: lane-consecutive floats, sixteen
         // loads in flight, in registers when the row has at most 1024.
         auto store1 = [&](int k, float v) {
             _Float16 h, l;
-            const float t = __builtin_ldexpf(v, -e);
-            split_f16(t, h, l);
-            small += split_small(v, t);
+            split_f16(__builtin_ldexpf(v, -e), h, l);
             _Float16 *p = reinterpret_cast<_Float16 *>(dst + (k / 32) * 128) + k % 32;
             p[0] = h;
             p[32] = l;
@@ -767,14 +785,17 @@ __device__ __forceinline__ void split_row(const float *__restrict__ src, char *_
             for (int j = 0; j < 16; j++) mx = max(mx, __float_as_uint(r[j]) & 0x7fffffffu);
         }
         e = split_exponent(wave_umax(mx));
+        limit = small_limit(e);
         for (int k0 = 0; k0 < Kp; k0 += 1024) {
             if (K > 1024) {
 #pragma unroll
                 for (int j = 0; j < 16; j++) r[j] = k0 + lane + 64 * j < K ? src[k0 + lane + 64 * j] : 0.0f;
             }
 #pragma unroll
-            for (int j = 0; j < 16; j++)
+            for (int j = 0; j < 16; j++) {
                 if (k0 + lane + 64 * j < Kp) store1(k0 + lane + 64 * j, e == kSplitNonFinite ? 0.0f : r[j]);
+                small += small_key(r[j]) < limit;
+            }
         }
     }
     const int code = wave_split_code(e, small);
@@ -903,6 +924,7 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
 #pragma unroll
     for (int w = 0; w < 16; w++) m = max(m, red[w][sc]);
     const int e = split_exponent(m), sn = n0 + sc;
+    const uint32_t limit = small_limit(e);
     int small = 0;
     for (int k0 = 0; k0 < slices * 32; k0 += 1024) {
         if (K > 1024) load(k0);
@@ -918,7 +940,8 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
                 f32x4 v;
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = e == kSplitNonFinite ? 0.0f : tile[4 * sk + j][sc];
-                small += store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
+                small += small_count4(v, limit);
+                store_split4(bs + (size_t)sn * slices * 128, ks, v, e);
             }
         }
     }
@@ -927,10 +950,12 @@ __global__ __launch_bounds__(1024) void split_operands_kernel(const float *__res
 }
 
 // Largest finite magnitude (as bits) of each chunk of n floats, with ReLU
-// applied first when relu: kConvChunks workgroups, part [kConvChunks].
+// applied first when relu: kConvChunks workgroups, part [kConvChunks].  Also
+// clears the `outs` counters that conv_split_image_kernel adds to.
 constexpr int kConvChunks = 256;
 __global__ __launch_bounds__(256) void conv_absmax_kernel(const float *__restrict__ in, uint32_t *__restrict__ part,
-                                                          size_t n, int relu) {
+                                                          size_t n, int relu, int *__restrict__ small, int outs) {
+    for (int o = blockIdx.x * 256 + threadIdx.x; o < outs; o += gridDim.x * 256) small[o] = 0;
     uint32_t mx = 0;
     auto take = [&](float v) {
         if (relu) v = fmaxf(v, 0.0f);
@@ -966,16 +991,18 @@ __global__ __launch_bounds__(256) void conv_absmax_kernel(const float *__restric
 // The CHW image [cs * 32][ih][iw] as split rows, one per pixel of the grid
 // padded by `pad` (zeros; also the rows past the grid), with one exponent:
 // grid (positions / 64, cs), a workgroup moving 64 positions of 32 channels
-// through LDS (64 consecutive pixels per load, 8 bytes per store).
+// through LDS (64 consecutive pixels per load, 8 bytes per store).  A pixel's
+// small values (about one in 60000 of N(0, 1)) are counted in at the outputs
+// whose taps read it, so that the product needs one count per output.
 __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__restrict__ in,
                                                                const uint32_t *__restrict__ part,
                                                                char *__restrict__ out, int *__restrict__ ex, int cs,
-                                                               int ih, int iw, int pad, int rows, int relu) {
+                                                               int ih, int iw, int pad, int rows, int relu,
+                                                               int *__restrict__ small, int outs, int kh, int kw) {
     __shared__ uint32_t red[4];
     __shared__ float tile[32][65];
-    uint32_t mx = wave_umax(part[threadIdx.x]);
+    const uint32_t chunk = part[threadIdx.x];
     static_assert(kConvChunks == 256, "one chunk per thread");
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
     const int wp = iw + 2 * pad, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int p = blockIdx.x * 64 + lane, y = p / wp - pad, x = p % wp - pad;
     const bool inside = p < rows && y >= 0 && y < ih && x >= 0 && x < iw;
@@ -984,6 +1011,8 @@ __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__re
     float v[8];
 #pragma unroll
     for (int c = 0; c < 8; c++) v[c] = src[c * plane];
+    const uint32_t mx = wave_umax(chunk);  // while the image's loads are in flight
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
 #pragma unroll
     for (int c = 0; c < 8; c++) {
         if (relu) v[c] = fmaxf(v[c], 0.0f);
@@ -992,9 +1021,12 @@ __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__re
     __syncthreads();
     const int e = split_exponent(max(max(red[0], red[1]), max(red[2], red[3])));
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) ex[0] = split_code(e, 0);
+    const int q0 = blockIdx.x * 64 + (threadIdx.x >> 3), c4 = 4 * (threadIdx.x & 7);
+    const uint32_t limit = small_limit(e);
+    int n[2] = {0, 0};
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-        const int pos = i * 32 + (threadIdx.x >> 3), c4 = 4 * (threadIdx.x & 7), q = blockIdx.x * 64 + pos;
+        const int pos = i * 32 + (threadIdx.x >> 3), q = q0 + i * 32;
         if (q >= rows) continue;
         f16x4 hi, lo;
 #pragma unroll
@@ -1004,11 +1036,17 @@ __global__ __launch_bounds__(256) void conv_split_image_kernel(const float *__re
             split_f16(t, h, l);
             hi[r] = h;
             lo[r] = __builtin_isfinite(t) ? l : (_Float16)0.0f;
+            n[i] += small_key(tile[c4 + r][pos]) < limit;
         }
         char *dst = out + ((size_t)q * cs + blockIdx.y) * 128 + c4 * 2;
         *reinterpret_cast<f16x4 *>(dst) = hi;
         *reinterpret_cast<f16x4 *>(dst + 64) = lo;
     }
+    if (n[0] + n[1] == 0) return;
+    for (int i = 0; i < 2; i++)
+        for (int ky = 0; ky < kh; ky++)
+            for (int kx = 0; kx < kw; kx++)
+                if (const int o = q0 + 32 * i - ky * wp - kx; n[i] && o >= 0 && o < outs) atomicAdd(small + o, n[i]);
 }
 
 // The tiles, and what a k-slice of one costs a CU in microseconds when the
@@ -1182,7 +1220,8 @@ hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *ga
 
 size_t conv_split_bytes(const SplitConv &c) {
     const size_t wp = c.iw + 2 * c.pad, rows = (c.ih + 2 * c.pad) * wp + c.kw - 1;
-    return rows * c.in_c * 4 + (kConvChunks + 1) * sizeof(int);
+    const size_t outs = (c.ih + 2 * c.pad - c.kh + 1) * wp;
+    return rows * c.in_c * 4 + (kConvChunks + 1 + outs) * sizeof(int);
 }
 
 bool conv_split_fits(const SplitConv &c) {
@@ -1216,11 +1255,12 @@ hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws) {
     const int rows = hp * wp + (int)c.kw - 1, oh = hp - (int)c.kh + 1, ow = wp - (int)c.kw + 1;
     char *img = static_cast<char *>(ws);
     uint32_t *part = reinterpret_cast<uint32_t *>(img + (size_t)rows * c.in_c * 4);
-    int *ex = reinterpret_cast<int *>(part + kConvChunks);
-    conv_absmax_kernel<<<kConvChunks, 256, 0, s>>>(c.in, part, c.in_c * c.ih * c.iw, c.relu ? 1 : 0);
+    int *ex = reinterpret_cast<int *>(part + kConvChunks), *small = ex + 1;
+    conv_absmax_kernel<<<kConvChunks, 256, 0, s>>>(c.in, part, c.in_c * c.ih * c.iw, c.relu ? 1 : 0, small, oh * wp);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     conv_split_image_kernel<<<dim3((rows + 63) / 64, cs), 256, 0, s>>>(
-        c.in, part, img, ex, cs, (int)c.ih, (int)c.iw, (int)c.pad, rows, c.relu ? 1 : 0);
+        c.in, part, img, ex, cs, (int)c.ih, (int)c.iw, (int)c.pad, rows, c.relu ? 1 : 0, small, oh * wp, (int)c.kh,
+        (int)c.kw);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     SplitArgs ar{};
     ar.x = img;
@@ -1235,6 +1275,7 @@ hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws) {
     ar.wf = c.wf;
     ar.c = c.out;
     ar.bias = c.bias;
+    ar.conv_small = small;
     ar.conv_cs = cs;
     ar.conv_kw = (int)c.kw;
     ar.conv_wp = wp;

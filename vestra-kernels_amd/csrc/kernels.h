@@ -241,9 +241,8 @@ constexpr size_t kSplitPieceFloats = (size_t)256 * 64 * 64;
 hipError_t launch_gemm_split(hipStream_t s, const SplitGemm &g);
 
 // Stride-1 convolution of a CHW image on split rows: the image is split
-// channel-last on its padded grid with one exponent for all of it (values
-// below 2^-18 of its largest are held to 2^-40 of that), then multiplied tap by
-// tap.
+// channel-last on its padded grid with one exponent for all of it, the small
+// values of each output's window are counted, then it is multiplied tap by tap.
 struct SplitConv {
     const float *in;        // [in_c][ih][iw]
     size_t in_c, ih, iw, out_c, kh, kw, pad;

@@ -59,9 +59,18 @@ __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
     return v;
 }
 
-// A value that the halves hold to less than 2^-22 of itself (v, scaled to t).
-__device__ __forceinline__ int split_small(float v, float t) {
-    return v != 0.0f && !(__builtin_fabsf(t) >= 0.125f);
+// Small values of a split row (nonzero, below 2^-3 once scaled): those whose
+// key, the magnitude's bits less one so that zero sorts above every number, is
+// below the limit of the row's exponent.
+__device__ __forceinline__ uint32_t small_key(float v) { return (__float_as_uint(v) & 0x7fffffffu) - 1u; }
+__device__ __forceinline__ uint32_t small_limit(int e) {
+    return max(__float_as_uint(__builtin_ldexpf(0.125f, e)), 1u) - 1u;
+}
+__device__ __forceinline__ int small_count4(f32x4 v, uint32_t limit) {
+    int n = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) n += small_key(v[r]) < limit;
+    return n;
 }
 
 // Running maximum of magnitudes as bit patterns (a NaN sorts above every number).
