@@ -268,6 +268,58 @@ def test_split_convolution_of_wide_ranges(rt, kind, in_c, out_c, ih, iw, k, p, r
     assert np.all(over <= 1.0), (float(over.max()), int((over > 1).sum()))
 
 
+def _wide_attention(kind, H, T, hd):
+    q, k, v = (seeded.normal(s + T, H * T * hd).reshape(H, T, hd) for s in (9860, 9870, 9880))
+    if kind == "k_row":        # a key row whose huge entry meets no query
+        q[:, :, 1] = 0.0
+        k[:, T // 2, 1] = 1e30
+    elif kind == "q_row":      # one query of another size, huge where no key has anything
+        k[:, :, 2] = 0.0
+        q[:, T // 3, 2] = -1e25
+    elif kind == "v_row":      # a huge value row that no query attends to
+        q[:, :, 0] = 30.0
+        k[:, T // 2, 0] = -300.0
+        v[:, T // 2] = 1e30
+    elif kind == "v_dims":     # value columns of very different sizes
+        v *= np.float32(10.0) ** np.linspace(-18, 18, hd, dtype=np.float32)
+    elif kind == "v_rows":     # a query that attends to a tiny value row only
+        q[:, 3:] *= 0.1
+        q[:, :3, 0] = 30.0
+        k[:, 5] *= 0.1
+        k[:, 5, 0] = 30.0
+        v[:, 5] *= np.float32(1e-12)
+    elif kind == "sink":       # a key that takes nearly all weight and has no value
+        q[:, :, 0] = 11.0
+        k[:, :, 0] = 0.0
+        k[:, 0] = 0.0
+        k[:, 0, 0] = 1.7 * np.sqrt(hd)
+        v[:, 0] = 0.0
+    elif kind == "scales":     # every row of its own size
+        for a in (q, k):
+            a *= np.exp2(-30.0 * seeded.uniform01(9890 + T, H * T)).astype(np.float32).reshape(H, T, 1)
+    return q, k, v
+
+
+@pytest.mark.parametrize("kind", ["k_row", "q_row", "v_row", "v_dims", "v_rows", "sink", "scales"])
+@pytest.mark.parametrize("H, T, hd", [(2, 130, 64), (3, 865, 64), (2, 1100, 40), (2, 300, 33)])
+def test_split_attention_of_wide_ranges(rt, kind, H, T, hd):
+    """Each output against the rounding of its own terms p |v| (as in
+    test_split_attention_vs_float64, per output): rows and columns of other
+    sizes take nothing from it."""
+    q, k, v = _wide_attention(kind, H, T, hd)
+    q64, k64, v64 = (a.astype(np.float64) for a in (q, k, v))
+    s = q64 @ k64.transpose(0, 2, 1) / np.sqrt(hd)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    terms = np.abs(q64) @ np.abs(k64).transpose(0, 2, 1) / np.sqrt(hd)
+    score = 2.0 ** -21 * np.where(p > 1e-12, terms, 0).max(-1)[:, :, None]
+    tol = 2 * (score + 2.0 ** -18 + 2.0 ** -23) + 2.0 ** -21 + T / 32 * 2.0 ** -23
+    t = [rt.upload_f32(a) for a in (q, k, v)]
+    got = rt.download_f32(rt.attention_online_f32(*t, H, T, hd)).reshape(v.shape)
+    over = np.abs(got - p @ v64) / (tol * (p @ np.abs(v64)) + 2.0 ** -148)
+    assert np.all(over <= 1.0), (float(over.max()), int((over > 1).sum()))
+
+
 # Grids of at least 128 64 x 64 tiles: ragged rows and widths, one and five
 # channel slices, 1 x 1, 3 x 3 and 5 x 5 taps with and without padding, output
 # channels that fill no tile.

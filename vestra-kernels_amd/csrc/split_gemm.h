@@ -50,13 +50,15 @@ __device__ __forceinline__ int split_exponent(uint32_t maxbits) {
     return __builtin_amdgcn_frexp_expf(__uint_as_float(maxbits)) - 15;
 }
 
+// Largest of the 64 lanes, in each of them (the steps of wave_sum).
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_umax(uint32_t v) {
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ uint32_t wave_umax(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t w = (uint32_t)__shfl_xor((int)v, o, kWave);
-        v = w > v ? w : v;
-    }
-    return v;
+    v = dpp_umax<0x140>(dpp_umax<0x141>(dpp_umax<0x4e>(dpp_umax<0xb1>(v))));
+    v = max(v, (uint32_t)__shfl_xor((int)v, 16, kWave));
+    return max(v, (uint32_t)__shfl_xor((int)v, 32, kWave));
 }
 
 // Small values of a split row (nonzero, below 2^-3 once scaled): those whose
