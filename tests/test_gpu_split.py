@@ -12,6 +12,7 @@ import math
 import numpy as np
 import pytest
 
+from block64 import block64
 from q8_compose import q8_block
 from vestra_hip import da3, seeded
 
@@ -384,3 +385,51 @@ def test_q8_block_attention_writes_q8_rows(rt, T, inf):
     xt = rt.upload_f32(x)
     rt.vit_block_run(rt.prepare_block(w, q8_0=True), xt, 1, T)
     assert np.array_equal(rt.download_f32(xt), exp, equal_nan=True)
+
+
+def _wide_block(kind):
+    w = da3.block_weights(seed=61, layerscale="uniform", ln_affine=True, qk_norm=kind.startswith("late"))
+    qkv, proj, fc1, fc2 = (w[n].reshape(s) for n, s in (("w_qkv", (768, 2304)), ("w_proj", (768, 768)),
+                                                       ("w_fc1", (768, 3072)), ("w_fc2", (3072, 768))))
+    if kind.endswith("off"):         # neurons that their bias switches off
+        w["b_fc1"][:7] = -1e8
+    elif kind.endswith("neuron"):    # a huge neuron that nothing reads
+        w["b_fc1"][11] = 1e12
+        fc2[11] = 0.0
+    elif kind.endswith("value"):     # a huge value channel that nothing reads
+        w["b_qkv"][2 * 768 + 70] = 1e12
+        proj[70] = 0.0
+    elif kind.endswith("norm"):      # a huge LayerNorm channel that nothing reads
+        w["ln1_gamma"][5], w["ln2_gamma"][9] = 1e10, 1e10
+        qkv[5] = 0.0
+        fc1[9] = 0.0
+    elif kind.endswith("weight"):    # large weights on channels that are empty
+        w["ln1_gamma"][5] = w["ln1_beta"][5] = 0.0
+        qkv[5] = 1e12
+    elif kind.endswith("scores"):    # a huge query channel against a key channel of zero
+        qkv[:, 3] *= 1e10
+        qkv[:, 768 + 3] = 0.0
+        w["b_qkv"][768 + 3] = 0.0
+    return w
+
+
+@pytest.mark.parametrize("kind", ["plain", "off", "neuron", "value", "norm", "weight", "scores", "late", "late_value",
+                                  "late_neuron"])
+def test_block_of_wide_weights_vs_float64(rt, kind):
+    """Large channels that meet zeros leave the rest of the block as it is: the
+    branches within 2e-6 of float64 (2-norm).  The split block shows 3.1e-7, and
+    the fp32 matrix instructions, which the products of huge rows are formed
+    again on, 1.0e-6 at fc2's K of 3072.  Only weights whose range the split
+    form does not hold take the other form."""
+    w = _wide_block(kind)
+    T, pos = 97, da3.positions_yx(8, 12)
+    x = seeded.normal(9965, T * 768)
+    exp = block64(x, w, T, pos)[0]
+    xt = rt.upload_f32(x)
+    blk = rt.prepare_block(w)
+    names = _launches(rt, lambda: rt.vit_block_run(blk, xt, 1, T, pos))
+    assert ("layernorm_split" in names) == (kind in ("plain", "late", "off"))
+    got = rt.download_f32(xt).astype(np.float64)
+    error = np.linalg.norm(got - exp) / np.linalg.norm(exp - x)
+    print(f"{kind}: {error:.2e}")
+    assert error <= 2e-6

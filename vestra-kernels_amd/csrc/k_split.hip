@@ -855,26 +855,35 @@ __global__ __launch_bounds__(256) void layernorm_split_kernel(const float *__res
     if (lane == 0) ex[row] = split_code(e, 0);
 }
 
-// Upper bound of |LayerNorm(x) . w_n + b_n| over every x, per row n of
-// w [N][K]: |LN| without gamma has 2-norm at most sqrt(K), so the product
-// is at most sqrt(K) ||w_n g||_2 + sum |w_n beta| + |b_n|.  One wave per row.
-__global__ __launch_bounds__(256) void ln_output_bound_kernel(const float *__restrict__ w,
-                                                              const float *__restrict__ gamma,
-                                                              const float *__restrict__ beta,
-                                                              const float *__restrict__ bias,
-                                                              float *__restrict__ bound, int N, int K) {
+// One wave per weight row; the sums in doubles, which hold the squares of every
+// float.
+__global__ __launch_bounds__(256) void weight_range_kernel(const float *__restrict__ w, const float *__restrict__ t,
+                                                           const float *__restrict__ u, WeightRange *__restrict__ out,
+                                                           int N, int K) {
     const int lane = threadIdx.x & 63;
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (n >= N) return;
-    float s2 = 0.0f, sb = 0.0f;
+    double wt = 0.0, wu = 0.0, wa = 0.0, w2 = 0.0;
+    float most = 0.0f;
     for (int k = lane; k < K; k += 64) {
-        const float v = w[(size_t)n * K + k], p = v * gamma[k];
-        s2 = fmaf(p, p, s2);
-        sb += fabsf(v * beta[k]);
+        const float v = w[(size_t)n * K + k];
+        const double a = (double)v * t[k], b = u ? (double)v * u[k] : 0.0;
+        wt += a * a;
+        wu += b;
+        wa += fabs(b);
+        w2 += (double)v * v;
+        most = fmaxf(most, fabsf(v));
     }
-    s2 = wave_sum(s2);
-    sb = wave_sum(sb);
-    if (lane == 0) bound[n] = sqrtf((float)K) * sqrtf(s2) + sb + fabsf(bias[n]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        wt += __shfl_xor(wt, o, kWave);
+        wu += __shfl_xor(wu, o, kWave);
+        wa += __shfl_xor(wa, o, kWave);
+        w2 += __shfl_xor(w2, o, kWave);
+    }
+    most = wave_max(most);
+    if (lane == 0)
+        out[n] = WeightRange{(float)__builtin_sqrt(wt), (float)wu, (float)wa, (float)__builtin_sqrt(w2), most};
 }
 
 // Both operands of a row-major product a [M][K] . b [K][N] in one launch:
@@ -1211,10 +1220,10 @@ hipError_t launch_layernorm_split(hipStream_t s, const float *in, const float *g
     return hipGetLastError();
 }
 
-hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *gamma, const float *beta,
-                                  const float *bias, float *bound, size_t n, size_t k) {
+hipError_t launch_weight_ranges(hipStream_t s, const float *w, const float *t, const float *u, WeightRange *out,
+                                size_t n, size_t k) {
     if (n == 0) return hipSuccess;
-    ln_output_bound_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(w, gamma, beta, bias, bound, (int)n, (int)k);
+    weight_range_kernel<<<(unsigned)((n + 3) / 4), 256, 0, s>>>(w, t, u, out, (int)n, (int)k);
     return hipGetLastError();
 }
 

@@ -200,9 +200,13 @@ hipError_t launch_split_operands(hipStream_t s, const float *a, void *as, int *e
 // LayerNorm of each row into split rows (cols % 32 == 0, cols <= 1024).
 hipError_t launch_layernorm_split(hipStream_t s, const float *in, const float *gamma, const float *beta,
                                   void *out, int *ex, size_t rows, size_t cols, float eps);
-// bound[n] >= |LayerNorm(x) . w_n + bias_n| for every x (w [n][k]).
-hipError_t launch_ln_output_bound(hipStream_t s, const float *w, const float *gamma, const float *beta,
-                                  const float *bias, float *bound, size_t n, size_t k);
+// Of each weight row w_n [k], with t and u of the same length: |w_n t|_2, sum w_n u,
+// sum |w_n u|, |w_n|_2 and max |w_n| (u null: zeros).
+struct WeightRange {
+    float wt, wu, wu_abs, w, most;
+};
+hipError_t launch_weight_ranges(hipStream_t s, const float *w, const float *t, const float *u, WeightRange *out,
+                                size_t n, size_t k);
 struct SplitGemm {
     const void *x;          // split rows [m][k]
     const int *ex;          // their codes, or null: exponent ex_c for all

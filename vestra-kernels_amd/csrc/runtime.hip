@@ -290,9 +290,10 @@ struct vh_linear_q8 {
 struct vh_block {
     Rt rt;
     Lin qkv, proj, fc1, fc2;
-    // f32 blocks: all four projections hold split rows, and for every input
-    // Q, K and V (after their norm and RoPE) and GELU(fc1) are at most 2^(15 +
-    // e) for these exponents, which their split rows then have.
+    // f32 blocks: all four projections hold split rows, for every input Q, K
+    // and V (after their norm and RoPE) and GELU(fc1) are at most 2^(15 + e) for
+    // these exponents, which their split rows then have, and the weights are
+    // even enough for that (ranges_hold).
     bool split = false;
     int qkv_ex[3] = {}, fc1_ex = 0;
     bool q8 = false;  // projections in Q8_0 (qqkv..qfc2) instead of f32
@@ -700,21 +701,18 @@ vh_status prepare_split_lin(RtState &s, size_t K, size_t N, const float *w, cons
     return st;
 }
 
-// Upper bounds of |LayerNorm(x) . w_n + b_n| over every x, per output n, for
-// LayerNorm parameters g, be on the device.
-vh_status ln_output_bounds(RtState &s, const Lin &L, const float *g, const float *be, std::vector<float> *h) {
-    float *bound = nullptr;
-    TRY(dalloc(s, L.N, &bound, "bound allocation"));
-    vh_status st = launch(s, "ln_output_bound", [&] {
-        return vh::launch_ln_output_bound(s.stream, L.wt, g, be, L.bias, bound, L.N, L.K);
-    });
-    h->resize(L.N);
+vh_status weight_ranges(RtState &s, const Lin &L, const float *t, const float *u, std::vector<vh::WeightRange> *out) {
+    vh::WeightRange *d = nullptr;
+    TRY(dalloc(s, L.N, &d, "weight range allocation"));
+    vh_status st =
+        launch(s, "weight_ranges", [&] { return vh::launch_weight_ranges(s.stream, L.wt, t, u, d, L.N, L.K); });
+    out->resize(L.N);
     if (!st) {
-        hipError_t he = hipMemcpyAsync(h->data(), bound, L.N * sizeof(float), hipMemcpyDeviceToHost, s.stream);
-        if (he == hipSuccess) he = hipStreamSynchronize(s.stream);
-        if (he != hipSuccess) st = fail(VH_ERR_UPLOAD, hip_msg("bound download", he));
+        hipError_t e = hipMemcpyAsync(out->data(), d, L.N * sizeof(*d), hipMemcpyDeviceToHost, s.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(s.stream);
+        if (e != hipSuccess) st = fail(VH_ERR_UPLOAD, hip_msg("weight range download", e));
     }
-    hipFreeAsync(bound, s.stream);
+    hipFreeAsync(d, s.stream);
     return st;
 }
 
@@ -733,6 +731,36 @@ bool bound_exponent(const float *v, size_t n, int *e) {
         *e = x - 15;
     }
     return *e <= 90 && *e >= -90;
+}
+
+// A block's split products have no floats to fall back on, so whether the
+// halves hold what they need is settled when its weights are prepared.  A value
+// that shares its exponent with values up to `most` is off by 2^-40 of `most`
+// (rms), which reaches output n of a projection as 2^-40 most |w_n|_2 (and the
+// weights' own as 2^-40 max |w_n| |t|_2, t the usual sizes of its inputs); the output's
+// usual size is |w_n t|_2.  Where their ratio is at most 2^14 for every n that
+// error is 2^-26 of the output, below one rounding of a float (weights of
+// N(0, 0.02^2): 2^4 to 2^6; 2^2 of the limit is for an attention that averages,
+// whose outputs are smaller than V).
+constexpr double kBlockRange = 0x1p14;
+bool ranges_hold(const std::vector<vh::WeightRange> &r, const float *bias, double most, double norm_t) {
+    for (size_t n = 0; n < r.size(); n++) {
+        if (r[n].wt == 0.0f) continue;  // every product is zero
+        const double size = std::hypot(std::hypot((double)r[n].wt, (double)r[n].wu), bias ? (double)bias[n] : 0.0);
+        if (!(most * r[n].w + norm_t * r[n].most <= kBlockRange * size)) return false;
+    }
+    return true;
+}
+
+// The sizes of a LayerNorm's outputs: at most sqrt(n) |gamma| + |beta|, usually
+// |(gamma, beta)|.
+void ln_sizes(const float *g, const float *be, size_t n, double *most, double *norm) {
+    *most = *norm = 0.0;
+    for (size_t i = 0; i < n; i++) {
+        *most = std::max(*most, std::sqrt((double)n) * std::fabs(g[i]) + std::fabs(be[i]));
+        *norm += (double)g[i] * g[i] + (double)be[i] * be[i];
+    }
+    *norm = std::sqrt(*norm);
 }
 
 // Split rows of `in` [rows][k] in the runtime's workspace, or null pointers
@@ -2415,7 +2443,9 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
         });
     }
     if (!b.split) {
-        // Weights with an inf or NaN: the fp32 matrix instructions.
+        // Weights with an inf or NaN, or of a range that the split form of the
+        // whole block does not hold: one product at a time, which looks at its
+        // own operands.
         auto norm = [&](const float *g, const float *be) {
             return launch(s, "layernorm", [&] { return vh::launch_layernorm(s.stream, x, g, be, h, M, D, eps); });
         };
@@ -2503,6 +2533,76 @@ vh_status check_block_x(const vh_tensor *x, size_t images, size_t tokens) {
 }
 }  // namespace
 
+// Whether the split form serves the f32 block b (b.split), and its exponents.
+static vh_status prepare_block_split(RtState &s, const vh_block_params &p, vh_block *b) {
+    b->split = false;
+    if (!b->qkv.sw || !b->proj.sw || !b->fc1.sw || !b->fc2.sw) return VH_OK;
+    std::vector<vh::WeightRange> r;
+    const double root = std::sqrt((double)kDim);
+    double most = 0.0, norm = 0.0;
+
+    TRY(weight_ranges(s, b->qkv, b->ln1_g, b->ln1_b, &r));
+    ln_sizes(p.ln1_gamma, p.ln1_beta, kDim, &most, &norm);
+    bool holds = ranges_hold(r, p.b_qkv, most, norm);
+    // |LayerNorm(x) . w_n + b_n| over every x: the normalised row has 2-norm
+    // sqrt(K) at most.
+    std::vector<float> bound(3 * kDim), usual(kMlp);
+    for (size_t i = 0; i < 3 * kDim; i++) bound[i] = (float)(root * r[i].wt + r[i].wu_abs + std::fabs(p.b_qkv[i]));
+    const float *nq[] = {p.q_norm_gamma, p.q_norm_beta, p.k_norm_gamma, p.k_norm_beta};
+    for (size_t i = 0; i < 2 * kDim; i++) {
+        const float *const *np = nq + 2 * (i / kDim);
+        // LayerNorm of a 64-wide row: at most sqrt(64) |gamma| + |beta|.
+        if (np[0]) bound[i] = 8.0f * fabsf(np[0][i % 64]) + fabsf(np[1][i % 64]);
+        bound[i] *= 1.4143f;  // the RoPE rotates pairs: at most sqrt(2) of the larger
+    }
+    for (int i = 0; i < 3; i++) holds = bound_exponent(bound.data() + i * kDim, kDim, &b->qkv_ex[i]) && holds;
+    if (!holds) return VH_OK;
+    const auto largest = [](const float *v, size_t n) { return (double)*std::max_element(v, v + n); };
+    // A score is off by 2^-40 of (largest |q|) (largest |k|) / 8 (rms): 2^-24 at the limit.
+    if (largest(bound.data(), kDim) * largest(bound.data() + kDim, kDim) / 8.0 > 0x1p16) return VH_OK;
+
+    // The out-projection's inputs are averages of V.
+    const auto check = [&](const Lin &L, size_t k, double at_most) -> vh_status {
+        float *t = nullptr;
+        double n2 = 0.0;
+        for (size_t i = 0; i < k; i++) n2 += (double)usual[i] * usual[i];
+        TRY(upload_array(s, usual.data(), k, &t, "input sizes"));
+        vh_status st = weight_ranges(s, L, t, nullptr, &r);
+        hipFreeAsync(t, s.stream);
+        holds = !st && ranges_hold(r, nullptr, at_most, std::sqrt(n2));
+        return st;
+    };
+    for (size_t i = 0; i < kDim; i++)
+        usual[i] = std::hypot(std::hypot(r[2 * kDim + i].wt, r[2 * kDim + i].wu), p.b_qkv[2 * kDim + i]);
+    TRY(check(b->proj, kDim, largest(bound.data() + 2 * kDim, kDim)));
+    if (!holds) return VH_OK;
+
+    TRY(weight_ranges(s, b->fc1, b->ln2_g, b->ln2_b, &r));
+    ln_sizes(p.ln2_gamma, p.ln2_beta, kDim, &most, &norm);
+    holds = ranges_hold(r, p.b_fc1, most, norm);
+    bound.resize(kMlp);
+    for (size_t i = 0; i < kMlp; i++) {
+        const double spread = root * r[i].wt, mid = (double)r[i].wu + p.b_fc1[i];
+        const double any = spread + r[i].wu_abs + std::fabs(p.b_fc1[i]);
+        // GELU(z) is at most z, and at least -0.17: a neuron that its bias
+        // switches off takes no range.  (`any` checks for inf and NaN, and
+        // covers the rounding of mid.)
+        bound[i] = any <= 1e30 ? (float)std::max(spread + mid + 1e-5 * any, 0.17) : INFINITY;
+        const double off = std::min(mid, 0.0) / std::max((double)r[i].wt, 1e-30);
+        usual[i] = (float)(std::max(mid, 0.0) + 0.4 * r[i].wt * std::exp(-0.5 * off * off));
+    }
+    holds = bound_exponent(bound.data(), kMlp, &b->fc1_ex) && holds;
+    if (!holds) return VH_OK;
+    TRY(check(b->fc2, kMlp, largest(bound.data(), kMlp)));
+    b->split = holds;
+    if (b->split)
+        for (Lin *l : {&b->qkv, &b->proj, &b->fc1, &b->fc2}) {  // no input holds an inf
+            hipFreeAsync(l->wt, s.stream);
+            l->wt = nullptr;
+        }
+    return VH_OK;
+}
+
 static vh_status block_prepare(const vh_runtime *rt, const vh_block_params *p, bool q8,
                                vh_block **out) {
     NEED(rt, "vh_block_prepare");
@@ -2539,31 +2639,7 @@ static vh_status block_prepare(const vh_runtime *rt, const vh_block_params *p, b
     if (!st) st = upload_small(s, p->ln1_beta, kDim, &b->ln1_b, "ln1 beta");
     if (!st) st = upload_small(s, p->ln2_gamma, kDim, &b->ln2_g, "ln2 gamma");
     if (!st) st = upload_small(s, p->ln2_beta, kDim, &b->ln2_b, "ln2 beta");
-    if (!st && !q8) {
-        std::vector<float> h;
-        st = ln_output_bounds(s, b->fc1, b->ln2_g, b->ln2_b, &h);
-        b->split = b->qkv.sw && b->proj.sw && b->fc1.sw && b->fc2.sw && bound_exponent(h.data(), kMlp, &b->fc1_ex);
-        if (!st) st = ln_output_bounds(s, b->qkv, b->ln1_g, b->ln1_b, &h);
-        if (!st) {
-            // The RoPE rotates pairs: at most sqrt(2) of the larger.
-            for (size_t i = 0; i < 2 * kDim; i++) h[i] *= 1.4143f;
-            if (qk_norm) {
-                // LayerNorm of a 64-wide row: at most sqrt(64) |gamma| + |beta|.
-                const float *nq[] = {p->q_norm_gamma, p->q_norm_beta, p->k_norm_gamma, p->k_norm_beta};
-                for (size_t i = 0; i < 2 * kDim; i++) {
-                    const float *const *np = nq + 2 * (i / kDim);
-                    h[i] = (8.0f * fabsf(np[0][i % 64]) + fabsf(np[1][i % 64])) * 1.4143f;
-                }
-            }
-            for (int i = 0; i < 3; i++)
-                b->split = b->split && bound_exponent(h.data() + i * kDim, kDim, &b->qkv_ex[i]);
-        }
-        if (b->split)
-            for (Lin *l : {&b->qkv, &b->proj, &b->fc1, &b->fc2}) {  // no input holds an inf
-                hipFreeAsync(l->wt, s.stream);
-                l->wt = nullptr;
-            }
-    }
+    if (!st && !q8) st = prepare_block_split(s, *p, b);
     if (qk_norm) {
         if (!st) st = upload_small(s, p->q_norm_gamma, 64, &b->qn_g, "q norm gamma");
         if (!st) st = upload_small(s, p->q_norm_beta, 64, &b->qn_b, "q norm beta");
