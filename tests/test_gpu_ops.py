@@ -298,6 +298,7 @@ def test_fc2_tail_equals_split_k(rt, monkeypatch, m):
     lin = rt.prepare_linear_f32(k, n, seeded.normal(62, k * n, 0.02), seeded.normal(63, n, 0.02), ls)
     x = seeded.normal(65, m * n)
     xt = rt.upload_f32(x)
+    monkeypatch.setenv("VESTRA_HIP_GEMM_KGROUP", "")  # the fp32 GEMM in its default form
     lin.run_residual(a, m, xt)
     tail = rt.download_f32(xt)
     monkeypatch.setenv("VESTRA_HIP_GEMM_TILE", "64x128x64x2x4x3")
@@ -306,10 +307,11 @@ def test_fc2_tail_equals_split_k(rt, monkeypatch, m):
     assert_bits_equal(tail, rt.download_f32(xs), "balanced tail against split-K 3")
 
 
-def test_gemm_balanced_tail_store_matches_float64(rt):
+def test_gemm_balanced_tail_store_matches_float64(rt, monkeypatch):
     """Store epilogue through the row-major GEMM: 336 tiles, K = 512 in two
     pieces; the fp32 error bound of test_gemm_row_major_matches_float64."""
     m, k, n = 400, 512, 3072
+    monkeypatch.setenv("VESTRA_HIP_GEMM_TAIL", "")  # the fp32 GEMM in its default form
     a = seeded.normal(51, m * k)
     b = seeded.normal(52, k * n)
     c = rt.download_f32(rt.gemm_row_major_f32(rt.upload_f32(a), rt.upload_f32(b), m, k, n))

@@ -433,3 +433,43 @@ def test_block_of_wide_weights_vs_float64(rt, kind):
     error = np.linalg.norm(got - exp) / np.linalg.norm(exp - x)
     print(f"{kind}: {error:.2e}")
     assert error <= 2e-6
+
+
+@pytest.mark.parametrize("value", ["", "0"])
+@pytest.mark.parametrize("name, asks", [("GEMM_TAIL", "gemm"), ("GEMM_KGROUP", "gemm"), ("GEMM_TILE", "gemm"),
+                                        ("GEMM_RM_DIRECT", "row_major"), ("FLASH_SPLITS", "attention"),
+                                        ("FLASH_XCD", "attention"), ("CONV_DIRECT", "conv")])
+def test_overrides_ask_for_the_fp32_kernels(rt, monkeypatch, name, asks, value):
+    """An override of the fp32 kernels, set to anything, is obeyed by every call
+    that it names: a projection, a row-major product, an attention, a
+    convolution and the whole block."""
+    if name == "FLASH_SPLITS" and value == "0":
+        value = "1"
+    m, k, n = 257, 101, 771
+    x, w = rt.upload_f32(seeded.normal(1, m * k)), seeded.normal(2, k * n)
+    wt, lin = rt.upload_f32(w), rt.prepare_linear_f32(k, n, w, seeded.normal(3, n))
+    qkv = [rt.upload_f32(seeded.normal(s, 2 * 130 * 64)) for s in (4, 5, 6)]
+    img, conv = rt.upload_f32(seeded.normal(7, 64 * 97 * 96)), rt.prepare_conv2d_f32(64, 128, 3, 3, 1, 1,
+                                                                                    seeded.normal(8, 128 * 64 * 9))
+    blk, x0 = rt.prepare_block(da3.block_weights(seed=62, layerscale="uniform")), seeded.normal(9, 97 * 768)
+
+    def block():
+        t = rt.upload_f32(x0)
+        names = _launches(rt, lambda: rt.vit_block_run(blk, t, 1, 97))
+        return names, rt.download_f32(t)
+
+    calls = {"gemm": lambda: lin.run(x, m), "row_major": lambda: rt.gemm_row_major_f32(x, wt, m, k, n),
+             "attention": lambda: rt.flash_attention_f32_da3_base(*qkv, 2, 130), "conv": lambda: conv.run(img, 97, 96)}
+    split = {c: rt.download_f32(f()) for c, f in calls.items()}
+    names, ref = block()
+    assert "layernorm_split" in names
+    monkeypatch.setenv("VESTRA_HIP_" + name, value)
+    asked = {"gemm": {"gemm", "row_major", "conv"}}.get(asks, {asks})
+    for c, f in calls.items():
+        got = rt.download_f32(f())
+        assert np.array_equal(got, split[c]) == (c not in asked), c
+        assert np.linalg.norm(got - split[c]) <= 2e-6 * np.linalg.norm(split[c]), c
+    names, got = block()
+    assert ("layernorm_split" in names) == (asks not in ("gemm", "attention"))
+    assert ("split_rows" in names) == (asks == "attention")
+    assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref)

@@ -17,6 +17,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <string>
@@ -551,15 +552,19 @@ bool grow_workspace(RtState &s, T **p, size_t *have, size_t need, bool *in_graph
     return true;
 }
 
-// VESTRA_HIP_FLASH_* choose between forms of the fp32 flash kernels (A/B
-// studies and tests, read per call): set, they ask for those kernels.
-bool fp32_flash_asked() {
-    for (const char *name : {"VESTRA_HIP_FLASH_SPLITS", "VESTRA_HIP_FLASH_STREAMS", "VESTRA_HIP_FLASH_DIRECT",
-                             "VESTRA_HIP_FLASH_FUSED", "VESTRA_HIP_FLASH_XCD"}) {
-        const char *e = std::getenv(name);
-        if (e && *e) return true;
-    }
+// Overrides that choose between forms of the fp32 kernels (A/B studies and
+// tests, read per call): set to anything, they ask for those kernels.
+bool any_set(std::initializer_list<const char *> names) {
+    for (const char *name : names)
+        if (std::getenv(name)) return true;
     return false;
+}
+bool fp32_flash_asked() {
+    return any_set({"VESTRA_HIP_FLASH_SPLITS", "VESTRA_HIP_FLASH_STREAMS", "VESTRA_HIP_FLASH_DIRECT",
+                    "VESTRA_HIP_FLASH_FUSED", "VESTRA_HIP_FLASH_XCD"});
+}
+bool fp32_gemm_asked() {
+    return any_set({"VESTRA_HIP_GEMM_TAIL", "VESTRA_HIP_GEMM_KGROUP", "VESTRA_HIP_GEMM_TILE"});
 }
 
 // Attention of bh heads of `tokens` rows of hd <= 64 floats on the f16
@@ -625,16 +630,6 @@ vh_status flash(RtState &s, const float *q, const float *k, const float *v, floa
 // representation alone costs 0.9e-7, which the fp32 ones pass at K = 32.
 constexpr size_t kSplitMinK = 64;
 bool split_k_fits(size_t m, size_t n, size_t k) { return k >= kSplitMinK && vh::split_gemm_fits(m, n, k); }
-// VESTRA_HIP_GEMM_TAIL and VESTRA_HIP_GEMM_KGROUP choose between forms of the
-// fp32 GEMM (A/B studies and tests, read per call): set, they ask for that
-// GEMM.
-bool fp32_gemm_asked() {
-    for (const char *name : {"VESTRA_HIP_GEMM_TAIL", "VESTRA_HIP_GEMM_KGROUP"}) {
-        const char *e = std::getenv(name);
-        if (e && *e) return true;
-    }
-    return false;
-}
 
 // Split rows of the weight w [n][k] for the f16 matrix cores.  Where there is
 // no memory for them *sw and *sew stay null and the fp32 kernels serve.
@@ -1274,7 +1269,8 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
     vh_tensor *t = nullptr;
     TRY(new_tensor(rt->s, mn, &t, "GEMM output allocation"));
     // Split rows of A and of B's columns, then the f16 matrix cores.
-    if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked() && vh::split_gemm_pays(m, n, k, mk + kn)) {
+    if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked() && !any_set({"VESTRA_HIP_GEMM_RM_DIRECT"}) &&
+        vh::split_gemm_pays(m, n, k, mk + kn)) {
         const size_t abytes = vh::split_bytes(m, k), bbytes = vh::split_bytes(n, k);
         char *x = nullptr;
         vh_status st = split_space(s, abytes + bbytes + (m + n) * sizeof(int), &x);
@@ -2442,7 +2438,7 @@ vh_status block_run(RtState &s, const vh_block &b, float *x, size_t images, size
                                         vh::Epi::Residual, b.qfc2.bias, b.qfc2.gamma);
         });
     }
-    if (!b.split) {
+    if (!b.split || fp32_gemm_asked() || fp32_flash_asked()) {
         // Weights with an inf or NaN, or of a range that the split form of the
         // whole block does not hold: one product at a time, which looks at its
         // own operands.
@@ -2595,11 +2591,6 @@ static vh_status prepare_block_split(RtState &s, const vh_block_params &p, vh_bl
     if (!holds) return VH_OK;
     TRY(check(b->fc2, kMlp, largest(bound.data(), kMlp)));
     b->split = holds;
-    if (b->split)
-        for (Lin *l : {&b->qkv, &b->proj, &b->fc1, &b->fc2}) {  // no input holds an inf
-            hipFreeAsync(l->wt, s.stream);
-            l->wt = nullptr;
-        }
     return VH_OK;
 }
 
