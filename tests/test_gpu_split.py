@@ -473,3 +473,12 @@ def test_overrides_ask_for_the_fp32_kernels(rt, monkeypatch, name, asks, value):
     assert ("layernorm_split" in names) == (asks not in ("gemm", "attention"))
     assert ("split_rows" in names) == (asks == "attention")
     assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("m, k, n, split", [(865, 96, 3072, False), (865, 1536, 96, False), (500, 1536, 384, False),
+                                            (865, 101, 3072, True), (865, 1536, 384, True), (500, 768, 768, True)])
+def test_projections_take_the_faster_form(rt, m, k, n, split):
+    """The shapes on both sides of the rule's lines (split_gemm_pays)."""
+    lin = rt.prepare_linear_f32(k, n, seeded.normal(1, k * n), seeded.normal(2, n))
+    x = rt.upload_f32(seeded.normal(3, m * k))
+    assert ("split_rows" in _launches(rt, lambda: lin.run(x, m))) == split

@@ -1173,20 +1173,26 @@ bool split_gemm_fits(size_t m, size_t n, size_t k) {
 
 // Splitting reads and writes four bytes per value at about 3 TB/s, in a launch
 // of 2.5 us.  The fp32 GEMM runs 64 x 64 tiles at 0.55 us per k-slice of 32,
-// the K of a grid below half the CUs in two parts at once, a partial last round
-// as K pieces (0.3 of a round), and takes twice as long where K is no
-// multiple of 32 (its masked loads).  Fitted to 12 shapes on MI355X (fp32 and
-// split, us): 16 x 768 x 768 12.7 and 8.9, 64 x 588 x 96 20.8 and 8.4, 256 x 768
-// x 768 13.0 and 10.2, 865 x 768 x 768 14.0 and 12; the fp32 GEMM keeps 300 x 96
-// x 200 (4.9 and 7.5), 3460 x 64 x 768 (8.8 and 12.6) and 3460 x 768 x 96 (13.0
-// and 16.5).  whole_tiles: the fp32 route is the channel-major one, which
-// splits no K (865 x 768 x 96 19.3 and 11).
+// the K of a grid below half the CUs in two parts at once (a long K, below a
+// quarter, in more: a third of a round), a partial last round as K pieces (0.3
+// of a round), and takes twice as long where K is no multiple of 32 (its masked
+// loads).  Both forms of 240 linears on MI355X, K = 96 to 3072, N = 96 to 3072,
+// 16 to 3460 rows (us a call, fp32 and split): 865 x 768 x 768 14.2 and 14.4,
+// 500 x 768 x 768 13.3 and 11.6, 865 x 768 x 3072 40.8 and 22.7, 865 x 1536 x 384
+// 23.4 and 18.1; the fp32 GEMM keeps K below 128 (865 x 96 x 3072 9.5 and 12.6,
+// 3460 x 96 x 3072 27.3 and 30.7: the output's bytes bound both), 865 x 1536 x 96
+// (12.1 and 15.0) and 500 x 1536 x 384 (13.9 and 17.2).  Where the rule takes
+// the split form it is at most 2 us behind (500 x 1536 x 96 11.8 and 14.0).
+// whole_tiles: the fp32 route is the channel-major one, which splits no K (865 x
+// 768 x 96 19.3 and 11).
 bool split_gemm_pays(size_t m, size_t n, size_t k, size_t split_values, bool whole_tiles) {
+    if (k < 128 && k % 32 == 0) return false;
     const int slices = (int)((k + 31) / 32);
     const float gemm_us = plan_split(m, n, slices, false, true).us;
     const float split_us = 2.5f + (float)split_values * 8.0f / 3e6f + gemm_us;
     const float tiles = (float)((m + 63) / 64) * (float)((n + 63) / 64);
     float rounds = tiles > 256.0f ? tiles / 256.0f + 0.3f : (tiles > 128.0f ? tiles / 256.0f : 0.5f);
+    if (tiles <= 64.0f && k > 1024) rounds = 0.33f;
     if (whole_tiles) rounds = ceilf(tiles / 256.0f);
     const float fp32_us = (4.0f + rounds * slices * 0.55f) * (k % 32 == 0 ? 1.0f : 2.0f);
     return split_us < fp32_us;
