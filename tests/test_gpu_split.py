@@ -177,11 +177,13 @@ def _attention64(q, k, v):
 
 
 # One key, one panel and one more (32 keys), one step and one more (128), the
-# second and third step, the one-launch split's last length (1024) and the
-# first past it, head dims that fill no granule; scores up to 3 x the usual.
+# second and third step, the one-launch split's last length (64 K floats) and the
+# first past it, head dims that fill no granule; scores up to 3 x the usual.  (At
+# head dim 64 the shapes that attn_split_pays takes.)
 @pytest.mark.parametrize("heads, tokens, hd, scale", [
-    (1, 1, 64, 1.0), (3, 32, 64, 1.0), (2, 33, 64, 1.0), (13, 128, 64, 1.0), (2, 129, 64, 3.0), (1, 257, 40, 1.0),
-    (2, 385, 7, 1.0), (1, 1024, 64, 3.0), (1, 1025, 64, 1.0), (5, 1700, 33, 1.0)])
+    (1, 1, 60, 1.0), (3, 32, 63, 1.0), (2, 33, 60, 1.0), (13, 128, 60, 1.0), (2, 129, 64, 3.0), (1, 257, 40, 1.0),
+    (2, 385, 7, 1.0), (20, 257, 64, 1.0), (13, 640, 64, 1.0), (6, 1024, 64, 3.0), (6, 1025, 64, 1.0),
+    (5, 1700, 33, 1.0)])
 def test_split_attention_vs_float64(rt, heads, tokens, hd, scale):
     """Relative to the largest |v| of the head: each weight p is off by the
     rounding of its exponent (2^-24 of up to 32, twice), the exponential (2^-23)
@@ -206,7 +208,7 @@ def test_split_attention_head_scales_and_non_finite(rt):
     """Heads of different magnitude, and heads with a NaN or an infinity,
     which fall back to floats: the NaN reaches what the float attention lets
     it reach, and no other head."""
-    H, T, hd = 5, 70, 64
+    H, T, hd = 5, 300, 64
     q, k, v = (seeded.normal(s, H * T * hd).reshape(H, T, hd) for s in (9930, 9940, 9950))
     k[1] *= np.float32(1e-20)
     v[1] *= np.float32(1e20)
@@ -302,7 +304,7 @@ def _wide_attention(kind, H, T, hd):
 
 
 @pytest.mark.parametrize("kind", ["k_row", "q_row", "v_row", "v_dims", "v_rows", "sink", "scales"])
-@pytest.mark.parametrize("H, T, hd", [(2, 130, 64), (3, 865, 64), (2, 1100, 40), (2, 300, 33)])
+@pytest.mark.parametrize("H, T, hd", [(2, 130, 64), (6, 865, 64), (2, 1100, 40), (2, 300, 33)])
 def test_split_attention_of_wide_ranges(rt, kind, H, T, hd):
     """Each output against the rounding of its own terms p |v| (as in
     test_split_attention_vs_float64, per output): rows and columns of other
@@ -365,7 +367,7 @@ def test_split_convolution_vs_float64(rt, in_c, out_c, ih, iw, k, p, relu):
     assert np.all(np.abs(got[fine] - odd[fine]) <= bound[fine])
 
 
-@pytest.mark.parametrize("T, inf", [(1, None), (65, "v"), (130, "q"), (200, None)])
+@pytest.mark.parametrize("T, inf", [(1, None), (65, "v"), (130, "q"), (200, None), (300, "v"), (560, None)])
 def test_q8_block_attention_writes_q8_rows(rt, T, inf):
     """The Q8_0 rows that the attention writes are quantize_row_q8_0 of its
     float output, bit for bit: ragged query tiles, and heads with an inf."""
@@ -482,3 +484,23 @@ def test_projections_take_the_faster_form(rt, m, k, n, split):
     lin = rt.prepare_linear_f32(k, n, seeded.normal(1, k * n), seeded.normal(2, n))
     x = rt.upload_f32(seeded.normal(3, m * k))
     assert ("split_rows" in _launches(rt, lambda: lin.run(x, m))) == split
+
+
+@pytest.mark.parametrize("H, T, split", [(12, 128, False), (12, 150, True), (48, 150, False), (12, 256, False),
+                                         (12, 300, True), (12, 500, False), (12, 560, True), (24, 420, True),
+                                         (48, 400, False), (48, 560, True), (1, 1729, False), (4, 1300, True)])
+def test_attention_takes_the_faster_form(rt, monkeypatch, H, T, split):
+    """The shapes on both sides of the rule's lines (attn_split_pays): the bits
+    are those of the fp32 kernels, asked for, or others; every entry point
+    follows the same rule."""
+    t = [rt.upload_f32(seeded.normal(s, H * T * 64)) for s in (1, 2, 3)]
+    got = rt.download_f32(rt.flash_attention_f32_da3_base(*t, H, T, False))
+    assert np.array_equal(rt.download_f32(rt.attention_online_f32(*t, H, T, 64)), got)
+    out = rt.alloc_f32(H * T * 64)
+    if 3 * H * T * 256 <= 60 << 20:  # its scratch holds the split rows
+        rt.flash_attention_f32_da3_base_into(*t, H, T, False, out)
+        assert np.array_equal(rt.download_f32(out), got)
+    monkeypatch.setenv("VESTRA_HIP_FLASH_FUSED", "")
+    asked = rt.download_f32(rt.flash_attention_f32_da3_base(*t, H, T, False))
+    assert np.array_equal(asked, got) == (not split)
+    assert np.linalg.norm(asked - got) <= 2e-6 * np.linalg.norm(got)

@@ -829,6 +829,25 @@ bool attn_split_fits(size_t bh, size_t tokens) {
            bh * ((tokens + 63) / 64) <= (size_t)INT32_MAX / 1024;
 }
 
+// From floats the split costs a launch of its own (10 us at 12 x 865), so it needs
+// enough keys to earn that, and enough workgroups that the fp32 kernels' key
+// splits no longer fill the idle CUs.  Both forms at head_dim 64 on MI355X (us a
+// call, fp32 and split): 12 x 193 9 and 14, 12 x 384 12 and 17, 12 x 505 18 and
+// 20, 24 x 384 19 and 20, 48 x 350 34 and 39, 1 x 3457 42 and 55; 12 x 600 23 and
+// 22, 12 x 865 33 and 27, 24 x 420 28 and 25, 8 x 700 22 and 23, 48 x 560 63 and
+// 52, 12 x 3457 332 and 159.  Three or five tiles of 64 keys the fp32 kernels do
+// not split evenly: 12 x 150 14 and 14, 12 x 300 20 and 16, but 48 x 150 18 and
+// 21.  Narrower heads have padding launches on that side (8 x 500 x 40 23 and 17,
+// 2 x 64 x 16 21 and 11).
+bool attn_split_pays(size_t bh, size_t tokens, size_t hd) {
+    if (hd < 64) return true;
+    const double rows = (double)bh * (double)tokens;
+    const size_t tiles = (tokens + 63) / 64;
+    if ((tiles == 3 || tiles == 5) && bh * tiles <= 128) return true;
+    if (tokens <= 512 && bh * tiles > 256) return false;
+    return rows >= 4800.0 && rows * (double)tokens >= 3.5e6;
+}
+
 size_t attn_split_bytes(size_t bh, size_t tokens) {
     return 3 * bh * tokens * 256 + 3 * bh * (kRangeChunks * sizeof(Range) + kCodes * sizeof(int));
 }

@@ -263,6 +263,9 @@ hipError_t launch_conv_split(hipStream_t s, const SplitConv &c, void *ws);
 
 // ---- attention on split rows (k_attn_split.hip) ---------------------------------
 bool attn_split_fits(size_t bh, size_t tokens);
+// Whether splitting bh heads of `tokens` float rows of hd and the split attention
+// are measured to take less time than the fp32 flash kernels.
+bool attn_split_pays(size_t bh, size_t tokens, size_t hd);
 // Workspace of launch_attn_split_f32.  With q8_qs and q8_d (head_dim 64) the
 // token-major output is written as Q8_0 blocks instead of to `out`.
 size_t attn_split_bytes(size_t bh, size_t tokens);

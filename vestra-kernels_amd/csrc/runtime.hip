@@ -573,7 +573,7 @@ vh_status try_attn_split(RtState &s, const float *q, const float *k, const float
                          size_t tokens, size_t heads, size_t hd, bool token_major, float scale, bool *done,
                          int8_t *q8_qs = nullptr, uint16_t *q8_d = nullptr) {
     *done = false;
-    if (!vh::attn_split_fits(bh, tokens) || fp32_flash_asked()) return VH_OK;
+    if (!vh::attn_split_fits(bh, tokens) || !vh::attn_split_pays(bh, tokens, hd) || fp32_flash_asked()) return VH_OK;
     const size_t need = (vh::attn_split_bytes(bh, tokens) + sizeof(float) - 1) / sizeof(float);
     if (!grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded)) return VH_OK;
     *done = true;
@@ -1580,7 +1580,7 @@ extern "C" vh_status vh_flash_attention_f32_da3_base_into(const vh_runtime *rt,
         return fail(VH_ERR_KERNEL, hip_msg(what, e));
     // The allocating entry point's choice of kernel, so the same bits; the
     // array holds the split rows of every shape accepted above.
-    if (vh::attn_split_fits(heads, tokens) && !fp32_flash_asked() &&
+    if (vh::attn_split_fits(heads, tokens) && vh::attn_split_pays(heads, tokens, 64) && !fp32_flash_asked() &&
         vh::attn_split_bytes(heads, tokens) <= kScratchBytes)
         e = vh::launch_attn_split_f32(s.stream, q->ptr, k->ptr, v->ptr, out->ptr, heads, tokens, heads, 64,
                                       token_major != 0, 0.125f, s.scratch);
