@@ -182,3 +182,21 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def test_split_products_fit_the_launch_of_their_split():
+    """Whatever shape split_gemm_fits takes, the launches that split its
+    operands (a wave per row) stay below 2^32 threads, as a launch must; a shape
+    past that goes to the fp32 GEMM."""
+    fits = getattr(vh.lib(), "_ZN2vh15split_gemm_fitsEmmm")
+    fits.restype, fits.argtypes = ctypes.c_bool, [ctypes.c_size_t] * 3
+    sizes = [1, 64, 384, 1 << 20, (1 << 25) - 64, (1 << 25) - 63, 1 << 25, 67108864, 70000000, (1 << 31) - 1, 1 << 31]
+    taken = 0
+    for m in sizes:
+        for n in sizes:
+            for k in (64, 128, 1001):
+                if not fits(m, n, k):
+                    continue
+                taken += 1
+                assert -(-m // 4) * 256 < 2 ** 32 and (-(-m // 16) + -(-n // 16)) * 1024 < 2 ** 32, (m, n, k)
+    assert taken and fits(1 << 24, 384, 128) and not fits(70000000, 384, 128)

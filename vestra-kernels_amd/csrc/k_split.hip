@@ -1160,9 +1160,13 @@ hipError_t launch_split_epi(hipStream_t s, SplitArgs ar) {
 }  // namespace
 
 bool split_gemm_fits(size_t m, size_t n, size_t k) {
+    // A wave splits a row of either operand, both in one launch: fewer than
+    // 2^32 threads.
+    constexpr size_t kMaxRows = ((size_t)1 << 25) - 64;
+    if (m > kMaxRows || n > kMaxRows) return false;
     // Row offsets inside a 256-row tile stay below 2^31 bytes, and the
     // chosen tile's grid (with or without Qkv's choice) below the launch limit.
-    if (k == 0 || k > ((size_t)1 << 21) - 32 || m > INT32_MAX || n > INT32_MAX) return false;
+    if (k == 0 || k > ((size_t)1 << 21) - 32) return false;
     if (m == 0 || n == 0) return true;
     for (bool qkv : {false, true}) {
         const SplitTile &t = kSplitTiles[plan_split(m, n, (int)((k + 31) / 32), qkv, false).tile];
