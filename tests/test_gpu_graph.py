@@ -118,3 +118,50 @@ def test_graph_keeps_its_workspace_when_a_later_run_needs_a_larger_one(rt):
     finally:
         hip.hipGraphExecDestroy(exe)
         hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("kind", ["f32", "late", "q8", "fp32_kernels", "wide"])
+def test_graph_of_a_block_outlives_larger_runs(rt, monkeypatch, kind):
+    """A captured block keeps every workspace that it was given (intermediates,
+    Q8_0 rows, attention, split-K partials, counters): after an eager run of a
+    larger size has grown them all, the replays are still right, and a size
+    that no run has prepared is refused under capture, not allocated."""
+    import vestra_hip as vh
+
+    rt = vh.Runtime(0)  # its own, whose workspaces are still small
+    hip = _hip()
+    stream = ctypes.c_void_p(rt.stream())
+    if kind == "fp32_kernels":
+        monkeypatch.setenv("VESTRA_HIP_GEMM_TILE", "64x128x64x2x4x3")
+        monkeypatch.setenv("VESTRA_HIP_FLASH_SPLITS", "4")
+    w = da3.block_weights(seed=97, layerscale="uniform", qk_norm=kind == "late")
+    if kind == "wide":  # one product at a time (the block's split form does not hold it)
+        w["b_qkv"][2 * 768 + 70] = 1e12
+        w["w_proj"].reshape(768, 768)[70] = 0.0
+    block = rt.prepare_block(w, q8_0=kind == "q8")
+    pos, more = da3.positions_yx(16, 20), da3.positions_yx(40, 40)
+    x0 = seeded.normal(9600, 321 * 768)
+    x, y = rt.upload_f32(x0), rt.upload_f32(x0)
+    rt.vit_block_run(block, y, 1, 321, pos)
+    rt.synchronize()
+    exp = rt.download_f32(y)
+    big = rt.upload_f32(seeded.normal(9601, 1601 * 768))
+    graph, exe = _capture(hip, stream, lambda: rt.vit_block_run(block, x, 1, 321, pos))
+    try:
+        def refused():
+            with pytest.raises(vh.UploadError):
+                rt.vit_block_run(block, big, 1, 1601, None)
+
+        other, other_exe = _capture(hip, stream, refused)
+        hip.hipGraphExecDestroy(other_exe)
+        hip.hipGraphDestroy(other)
+        for replay in range(3):
+            rt.vit_block_run(block, big, 1, 1601, more)
+            rt.synchronize()
+            rt.copy_segment_into_f32(x, 0, rt.upload_f32(x0), 0, x0.size)
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            assert_bits_equal(rt.download_f32(x), exp, f"replay {replay}")
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)

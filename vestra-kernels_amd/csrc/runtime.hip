@@ -127,26 +127,26 @@ bool capturing(hipStream_t stream) {
     return hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
+// A grow-only block of device memory (grow_workspace).
+struct Workspace {
+    void *p = nullptr;
+    size_t bytes = 0;
+    bool recorded = false;  // a captured graph may hold it
+};
+
 struct RtState {
     int device = 0;
     hipStream_t stream = nullptr;
     TensorPool pool;
     std::mutex mu;
     std::map<std::string, float *> rope_cache;  // host-built sin/cos tables
-    float *ws = nullptr;                        // grow-only block workspace
-    size_t ws_floats = 0;
-    float *sk = nullptr;                        // grow-only split-K partials
-    size_t sk_floats = 0;
-    float *fw = nullptr;                        // grow-only attention key-split partials
-    size_t fw_floats = 0;
-    unsigned *fcnt = nullptr;                   // and the in-kernel merge's arrival counters
-    size_t fcnt_n = 0;
-    char *aq = nullptr;                         // grow-only Q8_0 activation blocks
-    size_t aq_bytes = 0;
-    char *sx = nullptr;                         // grow-only split rows of a projection's input
-    size_t sx_bytes = 0;
-    bool fw_recorded = false, sx_recorded = false;  // fw, sx: a captured graph may hold the block
-    std::vector<void *> recorded;                   // outgrown blocks of that kind
+    Workspace ws;                               // block intermediates
+    Workspace sk;                               // split-K partials
+    Workspace fw;                               // attention split rows or key-split partials
+    Workspace fcnt;                             // and the in-kernel merge's arrival counters
+    Workspace aq;                               // Q8_0 activation blocks
+    Workspace sx;                               // split rows of a projection's input
+    std::vector<void *> recorded;               // outgrown blocks that a graph may hold
     float *tw = nullptr;                        // balanced-tail GEMM partials
     unsigned *tcnt = nullptr;                   // and arrival counters (zeroed once)
     float *scratch = nullptr;                   // this device's copy of `scratch` (below)
@@ -162,12 +162,8 @@ struct RtState {
         pool.give_back(stream);
         hipStreamSynchronize(stream);
         for (auto &kv : rope_cache) hipFree(kv.second);
-        if (ws) hipFree(ws);
-        if (sk) hipFree(sk);
-        if (fw) hipFree(fw);
-        if (fcnt) hipFree(fcnt);
-        if (aq) hipFree(aq);
-        if (sx) hipFree(sx);
+        for (Workspace *w : {&ws, &sk, &fw, &fcnt, &aq, &sx})
+            if (w->p) hipFree(w->p);
         for (void *p : recorded) hipFree(p);
         if (tw) hipFree(tw);
         if (tcnt) hipFree(tcnt);
@@ -442,48 +438,59 @@ vh_status rope_table(RtState &s, const int64_t *pos, size_t n, size_t head_dim, 
     return VH_OK;
 }
 
-vh_status workspace(RtState &s, size_t floats, float **out) {
-    if (s.ws_floats < floats) {
-        hipStreamSynchronize(s.stream);
-        if (s.ws) hipFree(s.ws);
-        s.ws = nullptr;
-        s.ws_floats = 0;
-        hipError_t e = device_malloc(s, (void **)&s.ws, floats * sizeof(float));
-        if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("block workspace allocation", e));
-        s.ws_floats = floats;
+// The workspace w grown to at least `bytes`, or null: no memory, or the stream
+// is being captured, where nothing can be allocated.  A block that a capture
+// was given may be in a graph that is yet to be replayed, so growth keeps it
+// until the runtime ends.
+void *grow_workspace(RtState &s, Workspace &w, size_t bytes) {
+    if (w.bytes >= bytes) {
+        if (capturing(s.stream)) w.recorded = true;
+        return w.p;
     }
-    *out = s.ws;
-    return VH_OK;
+    if (capturing(s.stream)) return nullptr;
+    hipStreamSynchronize(s.stream);
+    if (w.p && w.recorded) s.recorded.push_back(w.p);
+    else if (w.p) hipFree(w.p);
+    w = Workspace{};
+    if (device_malloc(s, &w.p, bytes) != hipSuccess) {
+        hipGetLastError();
+        w.p = nullptr;
+        return nullptr;
+    }
+    w.bytes = bytes;
+    return w.p;
+}
+
+vh_status no_workspace(RtState &s, const char *what) {
+    if (capturing(s.stream))
+        return fail(VH_ERR_UPLOAD, std::string(what) + ": a stream capture cannot grow it; run the size once before");
+    return fail(VH_ERR_UPLOAD, hip_msg(what, hipErrorOutOfMemory));
+}
+
+vh_status workspace(RtState &s, size_t floats, float **out) {
+    *out = static_cast<float *>(grow_workspace(s, s.ws, floats * sizeof(float)));
+    return *out ? VH_OK : no_workspace(s, "block workspace");
 }
 
 // Split-K partial tiles for the narrow (N <= 1024) projections: up to 8
-// splits of an m x n output.
+// splits of an m x n output.  Without them the GEMM keeps K whole.
 constexpr size_t kMaxSplits = 8;
-vh_status splitk_workspace(RtState &s, size_t m, size_t n, float **out, size_t *floats) {
+void splitk_workspace(RtState &s, size_t m, size_t n, float **out, size_t *floats) {
     *out = nullptr;
     *floats = 0;
-    if (n > 1024) return VH_OK;
-    const size_t need = kMaxSplits * m * n;
-    if (s.sk_floats < need) {
-        hipStreamSynchronize(s.stream);
-        if (s.sk) hipFree(s.sk);
-        s.sk = nullptr;
-        s.sk_floats = 0;
-        hipError_t e = device_malloc(s, (void **)&s.sk, need * sizeof(float));
-        if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("split-K workspace allocation", e));
-        s.sk_floats = need;
-    }
-    *out = s.sk;
-    *floats = s.sk_floats;
-    return VH_OK;
+    if (n > 1024) return;
+    *out = static_cast<float *>(grow_workspace(s, s.sk, kMaxSplits * m * n * sizeof(float)));
+    if (*out) *floats = s.sk.bytes / sizeof(float);
 }
 
 // Balanced-tail workspace of the wide GEMMs, allocated on first use.  The
 // counters are zeroed once here, on the runtime stream (so ahead of the
 // first launch that reads them, which the stream's non-blocking flag would
 // not order after a null-stream memset); every launch leaves them zero.
+// Under capture nothing is allocated: without it a grid runs whole tiles.
 vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
     if (!s.tw) {
+        if (capturing(s.stream)) return VH_OK;
         hipStreamSynchronize(s.stream);
         hipError_t e = device_malloc(s, (void **)&s.tw, vh::kTailFloats * sizeof(float));
         if (e == hipSuccess) e = hipMalloc(&s.tcnt, vh::kTailTiles * sizeof(unsigned));
@@ -504,12 +511,11 @@ vh_status tail_workspace(RtState &s, vh::GemmArgs &g) {
 }
 
 // The same room for the K pieces of a split GEMM (both run on the runtime's one
-// stream, so never at once).  Without it a grid runs whole tiles: under
-// capture nothing is allocated.
+// stream, so never at once).
 void piece_workspace(RtState &s, vh::SplitGemm &g) {
     static_assert(vh::kSplitPieceFloats <= vh::kTailFloats && vh::kTailTiles >= 256, "the tail workspace fits");
     vh::GemmArgs t{};
-    if ((!s.tw && capturing(s.stream)) || tail_workspace(s, t) != VH_OK) return;
+    if (tail_workspace(s, t) != VH_OK || !t.tail_ws) return;
     g.partial = t.tail_ws;
     g.partial_floats = t.tail_ws_floats;
     g.piece_cnt = t.tail_cnt;
@@ -523,33 +529,6 @@ bool flash_grid_fits(size_t heads, size_t tokens) {
     size_t items = 0;
     return !__builtin_mul_overflow(heads, qtiles, &items) &&
            items <= (size_t)UINT32_MAX / 256 / vh::kMaxFlashSplits;
-}
-
-// Grows the workspace *p of *have units to `need` units of `unit` bytes; false
-// where it stays too small: no memory, or the stream is being captured, where
-// nothing can be allocated.  A block that a capture was given may be in a graph
-// that is yet to be replayed, so growth keeps it until the runtime ends.
-template <typename T>
-bool grow_workspace(RtState &s, T **p, size_t *have, size_t need, bool *in_graph) {
-    if (capturing(s.stream)) {
-        if (*have >= need) *in_graph = true;
-        return *have >= need;
-    }
-    if (*have >= need) return true;
-    hipStreamSynchronize(s.stream);
-    if (*p && *in_graph) s.recorded.push_back(*p);
-    else if (*p) hipFree(*p);
-    *p = nullptr;
-    *have = 0;
-    *in_graph = false;
-    void *fresh = nullptr;
-    if (device_malloc(s, &fresh, need * sizeof(T)) != hipSuccess) {
-        hipGetLastError();
-        return false;
-    }
-    *p = static_cast<T *>(fresh);
-    *have = need;
-    return true;
 }
 
 // Overrides that choose between forms of the fp32 kernels (A/B studies and
@@ -574,11 +553,11 @@ vh_status try_attn_split(RtState &s, const float *q, const float *k, const float
                          int8_t *q8_qs = nullptr, uint16_t *q8_d = nullptr) {
     *done = false;
     if (!vh::attn_split_fits(bh, tokens) || !vh::attn_split_pays(bh, tokens, hd) || fp32_flash_asked()) return VH_OK;
-    const size_t need = (vh::attn_split_bytes(bh, tokens) + sizeof(float) - 1) / sizeof(float);
-    if (!grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded)) return VH_OK;
+    void *ws = grow_workspace(s, s.fw, vh::attn_split_bytes(bh, tokens));
+    if (!ws) return VH_OK;
     *done = true;
     return launch(s, "flash_attention", [&] {
-        return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, s.fw,
+        return vh::launch_attn_split_f32(s.stream, q, k, v, out, bh, tokens, heads, hd, token_major, scale, ws,
                                          q8_qs, q8_d);
     });
 }
@@ -596,29 +575,23 @@ vh_status flash(RtState &s, const float *q, const float *k, const float *v, floa
     // or the in-kernel merge's); without them the kernel runs unsplit.
     const size_t need =
         std::max(vh::flash_workspace_floats(bh, tokens), vh::flash_fused_workspace_floats(bh, tokens));
-    grow_workspace(s, &s.fw, &s.fw_floats, need, &s.fw_recorded);
-    // Arrival counters of the in-kernel merge, zeroed once here (outside any
-    // stream capture: the first run of a shape allocates); every run leaves
+    float *fw = static_cast<float *>(grow_workspace(s, s.fw, need * sizeof(float)));
+    // Arrival counters of the in-kernel merge, zeroed when allocated (outside
+    // any stream capture: the first run of a shape allocates); every run leaves
     // them zero.  Without them the merge runs as its own launch.
-    const size_t groups = vh::flash_query_groups(bh, tokens);
-    if (s.fcnt_n < groups) {
-        hipStreamSynchronize(s.stream);
-        if (s.fcnt) hipFree(s.fcnt);
-        s.fcnt = nullptr;
-        s.fcnt_n = 0;
-        if (hipMalloc(&s.fcnt, groups * sizeof(unsigned)) == hipSuccess &&
-            hipMemsetAsync(s.fcnt, 0, groups * sizeof(unsigned), s.stream) == hipSuccess) {
-            s.fcnt_n = groups;
-        } else {
-            hipGetLastError();
-            if (s.fcnt) hipFree(s.fcnt);
-            s.fcnt = nullptr;
-        }
+    const size_t had = s.fcnt.bytes;
+    unsigned *fcnt =
+        static_cast<unsigned *>(grow_workspace(s, s.fcnt, vh::flash_query_groups(bh, tokens) * sizeof(unsigned)));
+    if (fcnt && s.fcnt.bytes != had && hipMemsetAsync(fcnt, 0, s.fcnt.bytes, s.stream) != hipSuccess) {
+        hipGetLastError();
+        hipFree(fcnt);
+        s.fcnt = Workspace{};
+        fcnt = nullptr;
     }
+    const size_t fw_floats = fw ? s.fw.bytes / sizeof(float) : 0, fcnt_n = fcnt ? s.fcnt.bytes / sizeof(unsigned) : 0;
     return launch(s, "flash_attention", [&] {
         return vh::launch_flash_attention(s.stream, q, k, v, out, bh, tokens, heads, token_major,
-                                          s.fw, s.fw_floats, q8_qs, q8_d, quantized, scale, s.fcnt,
-                                          s.fcnt_n);
+                                          fw, fw_floats, q8_qs, q8_d, quantized, scale, fcnt, fcnt_n);
     });
 }
 
@@ -764,15 +737,11 @@ struct SplitRows {
     char *x = nullptr;
     int *ex = nullptr;
 };
-vh_status split_space(RtState &s, size_t bytes, char **out) {
-    *out = nullptr;
-    *out = grow_workspace(s, &s.sx, &s.sx_bytes, bytes, &s.sx_recorded) ? s.sx : nullptr;
-    return VH_OK;
-}
+char *split_space(RtState &s, size_t bytes) { return static_cast<char *>(grow_workspace(s, s.sx, bytes)); }
 
 vh_status split_input(RtState &s, const float *in, size_t rows, size_t k, SplitRows *out) {
     const size_t bytes = vh::split_bytes(rows, k);
-    TRY(split_space(s, bytes + rows * sizeof(int), &out->x));
+    out->x = split_space(s, bytes + rows * sizeof(int));
     if (!out->x) return VH_OK;
     out->ex = reinterpret_cast<int *>(out->x + bytes);
     return launch(s, "split_rows", [&] { return vh::launch_split_rows(s.stream, in, out->x, out->ex, rows, k); });
@@ -835,7 +804,7 @@ vh_status run_lin(RtState &s, const Lin &L, const float *in, size_t rows, vh::Ep
     g.c = c;
     g.bias = L.bias;
     g.gamma = sg.gamma;
-    TRY(splitk_workspace(s, rows, L.N, &g.ws, &g.ws_floats));
+    splitk_workspace(s, rows, L.N, &g.ws, &g.ws_floats);
     TRY(tail_workspace(s, g));
     return launch(s, name, [&] { return vh::launch_gemm(s.stream, g); });
 }
@@ -876,17 +845,10 @@ bool mul_overflows(size_t a, size_t b, size_t *out) { return __builtin_mul_overf
 vh_status q8_workspace(RtState &s, size_t rows, size_t k, int8_t **qs, uint16_t **d) {
     const size_t qbytes = (rows * k + 255) & ~size_t(255);
     const size_t need = qbytes + rows * (k / 32) * sizeof(uint16_t);
-    if (s.aq_bytes < need) {
-        hipStreamSynchronize(s.stream);
-        if (s.aq) hipFree(s.aq);
-        s.aq = nullptr;
-        s.aq_bytes = 0;
-        hipError_t e = device_malloc(s, (void **)&s.aq, need);
-        if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg("Q8_0 activation workspace allocation", e));
-        s.aq_bytes = need;
-    }
-    *qs = reinterpret_cast<int8_t *>(s.aq);
-    *d = reinterpret_cast<uint16_t *>(s.aq + qbytes);
+    char *aq = static_cast<char *>(grow_workspace(s, s.aq, need));
+    if (!aq) return no_workspace(s, "Q8_0 activation workspace");
+    *qs = reinterpret_cast<int8_t *>(aq);
+    *d = reinterpret_cast<uint16_t *>(aq + qbytes);
     return VH_OK;
 }
 
@@ -1272,9 +1234,9 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
     if (mn && split_k_fits(m, n, k) && !fp32_gemm_asked() && !any_set({"VESTRA_HIP_GEMM_RM_DIRECT"}) &&
         vh::split_gemm_pays(m, n, k, mk + kn)) {
         const size_t abytes = vh::split_bytes(m, k), bbytes = vh::split_bytes(n, k);
-        char *x = nullptr;
-        vh_status st = split_space(s, abytes + bbytes + (m + n) * sizeof(int), &x);
-        if (!st && x) {
+        vh_status st = VH_OK;
+        char *x = split_space(s, abytes + bbytes + (m + n) * sizeof(int));
+        if (x) {
             vh::SplitGemm g{};
             char *w = x + abytes;
             int *ex = reinterpret_cast<int *>(w + bbytes), *ew = ex + m;
@@ -2753,7 +2715,7 @@ vh_status gemm_nt(RtState &s, const float *a, const float *bt, const float *bias
     g.epi = vh::Epi::Store;
     g.c = c;
     g.bias = bias;
-    TRY(splitk_workspace(s, rows, cols, &g.ws, &g.ws_floats));
+    splitk_workspace(s, rows, cols, &g.ws, &g.ws_floats);
     TRY(tail_workspace(s, g));
     return launch(s, name, [&] { return vh::launch_gemm(s.stream, g); });
 }
@@ -2778,8 +2740,7 @@ vh_status conv_run(RtState &s, const vh_conv2d &c, const float *in, size_t ih, s
         const vh::SplitConv sc{in,     c.in_c, ih,   iw,    c.out_c, c.kh, c.kw,
                                c.pad,  relu,   c.sw, c.sew, c.w,     c.bias, out};
         if (vh::conv_split_fits(sc)) {
-            char *ws = nullptr;
-            TRY(split_space(s, vh::conv_split_bytes(sc), &ws));
+            char *ws = split_space(s, vh::conv_split_bytes(sc));
             if (ws) return launch(s, "conv_gemm", [&] { return vh::launch_conv_split(s.stream, sc, ws); });
         }
     }
