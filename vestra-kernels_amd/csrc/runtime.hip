@@ -15,16 +15,17 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <map>
 #include <memory>
-#include <initializer_list>
 #include <mutex>
 #include <new>
+#include <set>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "kernels.h"
+#include "tensor_pool.h"
 
 #define NEED(p, what) \
     do {              \
@@ -78,53 +79,21 @@ struct ProfileRec {
     hipEvent_t a, b;
 };
 
-// Device blocks of freed tensors, kept for the next tensor of the same size:
-// hipMallocAsync and hipFreeAsync cost a call about 10 us of host time between
-// them on MI355X (vh_linear_run at 16 x 768 x 768 18.3 us a call, 8.7 with
-// the pool), a lookup here none that shows.  A block only ever serves its runtime's one stream, whose
-// order makes the reuse safe exactly as hipFreeAsync's would; the blocks held
-// are bounded (larger ones, and those past the bound, go back at once), are
-// given back when an allocation fails and when the runtime ends, and are left
-// alone while the stream is captured, where allocations become the graph's.
-struct TensorPool {
-    static constexpr size_t kMaxBlock = (size_t)128 << 20, kMaxHeld = (size_t)512 << 20, kGrain = 512;
-    std::mutex mu;  // tensors may be freed from any host thread
-    std::unordered_map<size_t, std::vector<void *>> blocks;
-    size_t held = 0;
-    static size_t rounded(size_t bytes) { return (bytes + kGrain - 1) / kGrain * kGrain; }
-    void *take(size_t bytes) {
-        std::lock_guard<std::mutex> lock(mu);
-        auto it = blocks.find(bytes);
-        if (it == blocks.end() || it->second.empty()) return nullptr;
-        void *p = it->second.back();
-        it->second.pop_back();
-        held -= bytes;
-        return p;
-    }
-    bool keep(void *p, size_t bytes) noexcept {
-        if (bytes > kMaxBlock) return false;
-        std::lock_guard<std::mutex> lock(mu);
-        if (held + bytes > kMaxHeld) return false;
-        try {
-            blocks[bytes].push_back(p);
-        } catch (...) {
-            return false;
-        }
-        held += bytes;
-        return true;
-    }
-    void give_back(hipStream_t stream) {
-        std::lock_guard<std::mutex> lock(mu);
-        for (auto &kv : blocks)
-            for (void *p : kv.second) hipFreeAsync(p, stream);
-        blocks.clear();
-        held = 0;
-    }
-};
-
 bool capturing(hipStream_t stream) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
+// The runtimes of the process, so that one whose allocation fails gets the
+// blocks that the others of its device have kept.
+struct RtState;
+struct RuntimeList {
+    std::mutex mu;
+    std::set<RtState *> live;
+};
+RuntimeList &runtimes() {
+    static auto *list = new RuntimeList;  // outlives every runtime
+    return *list;
 }
 
 // A grow-only block of device memory (grow_workspace).
@@ -137,7 +106,9 @@ struct Workspace {
 struct RtState {
     int device = 0;
     hipStream_t stream = nullptr;
-    TensorPool pool;
+    // Freed tensors' blocks; left alone while the stream is captured, where
+    // allocations become the graph's.
+    vh::TensorPool pool;
     std::mutex mu;
     std::map<std::string, float *> rope_cache;  // host-built sin/cos tables
     Workspace ws;                               // block intermediates
@@ -156,10 +127,18 @@ struct RtState {
     std::map<std::string, std::pair<unsigned long long, double>> totals;
     hipEvent_t t0 = nullptr, t1 = nullptr;
 
+    void give_back() {
+        pool.give_back([this](void *p) { hipFreeAsync(p, stream); });
+    }
+
     ~RtState() {
         if (!stream) return;
+        {
+            std::lock_guard<std::mutex> lock(runtimes().mu);
+            runtimes().live.erase(this);
+        }
         hipSetDevice(device);
-        pool.give_back(stream);
+        give_back();
         hipStreamSynchronize(stream);
         for (auto &kv : rope_cache) hipFree(kv.second);
         for (Workspace *w : {&ws, &sk, &fw, &fcnt, &aq, &sx})
@@ -178,14 +157,30 @@ struct RtState {
     }
 };
 
-// Device memory of the runtime's own, with the tensor pool's blocks given back
-// if it takes them.
+// After an allocation of s has failed: the tensor blocks that the runtimes of its
+// device hold go back (not of another one that is being captured, whose graph
+// the frees would become part of), and what the stream-ordered pool keeps with
+// them.
+void give_back_all(RtState &s) {
+    hipGetLastError();
+    {
+        std::lock_guard<std::mutex> lock(runtimes().mu);
+        for (RtState *r : runtimes().live) {
+            if (r->device != s.device || capturing(r->stream)) continue;
+            r->give_back();
+            hipStreamSynchronize(r->stream);
+        }
+    }
+    hipMemPool_t pool = nullptr;
+    if (hipDeviceGetDefaultMemPool(&pool, s.device) == hipSuccess && pool) hipMemPoolTrimTo(pool, 0);
+    hipGetLastError();
+}
+
+// Device memory of the runtime's own.
 hipError_t device_malloc(RtState &s, void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipSuccess) return e;
-    hipGetLastError();
-    s.pool.give_back(s.stream);
-    hipStreamSynchronize(s.stream);
+    give_back_all(s);
     e = hipMalloc(p, bytes);
     if (e != hipSuccess) *p = nullptr;
     return e;
@@ -206,9 +201,11 @@ struct vh_tensor {
     size_t block = 0;  // bytes of the block, a TensorPool size; 0: a captured allocation
     ~vh_tensor() {
         if (!ptr || !rt) return;
-        if (block && !capturing(rt->stream) && rt->pool.keep(ptr, block)) return;
-        hipSetDevice(rt->device);
-        hipFreeAsync(ptr, rt->stream);
+        const auto release = [this](void *p) {
+            hipSetDevice(rt->device);
+            hipFreeAsync(p, rt->stream);
+        };
+        if (!block || capturing(rt->stream) || !rt->pool.keep(ptr, block, release)) release(ptr);
     }
 };
 
@@ -323,8 +320,7 @@ vh_status dalloc(RtState &s, size_t count, T **out, const char *what) {
     void *p = nullptr;
     hipError_t e = hipMallocAsync(&p, bytes, s.stream);
     if (e != hipSuccess && !capturing(s.stream)) {
-        hipGetLastError();
-        s.pool.give_back(s.stream);
+        give_back_all(s);
         e = hipMallocAsync(&p, bytes, s.stream);
     }
     if (e != hipSuccess) return fail(VH_ERR_UPLOAD, hip_msg(what, e));
@@ -354,14 +350,13 @@ vh_status upload_array(RtState &s, const float *host, size_t n, float **out, con
 vh_status new_tensor(const Rt &rt, size_t len, vh_tensor **out, const char *what) {
     vh_tensor *t = new (std::nothrow) vh_tensor;
     if (!t) return fail(VH_ERR_UPLOAD, std::string(what) + ": host allocation failed");
-    const size_t bytes = len <= (SIZE_MAX >> 3) ? TensorPool::rounded((len ? len : 1) * sizeof(float)) : SIZE_MAX;
+    const size_t bytes = len <= (SIZE_MAX >> 3) ? vh::TensorPool::rounded((len ? len : 1) * sizeof(float)) : SIZE_MAX;
     const bool captured = capturing(rt->stream);
     void *p = captured ? nullptr : rt->pool.take(bytes);
     if (!p) {
         hipError_t e = hipMallocAsync(&p, bytes, rt->stream);
         if (e != hipSuccess && !captured) {
-            hipGetLastError();
-            rt->pool.give_back(rt->stream);
+            give_back_all(*rt);
             p = nullptr;
             e = hipMallocAsync(&p, bytes, rt->stream);
         }
@@ -1013,6 +1008,10 @@ extern "C" vh_status vh_runtime_new(size_t device, vh_runtime **out) {
     }
     vh_runtime *rt = new vh_runtime;
     rt->s = s;
+    {
+        std::lock_guard<std::mutex> lock(runtimes().mu);
+        runtimes().live.insert(s.get());
+    }
     *out = rt;
     return VH_OK;
     GUARD_END
