@@ -873,3 +873,15 @@ def test_quantize_bit_exact_over_a_float32_sweep(rt):
         exp = O.quantize_rows_q8_0(x, rows, k)
         ok = got.view(np.uint8).reshape(-1, 34) == np.asarray(exp).view(np.uint8).reshape(-1, 34)
         assert ok.all(), (start, np.nonzero(~ok.all(1))[0][:4])
+
+
+def test_a_failed_allocation_leaves_no_error_to_the_next_call(rt):
+    """More than the device holds is refused, and the call after it is not."""
+    x = seeded.normal(9800, 3 * 768)
+    g, b = np.ones(768, np.float32), np.zeros(768, np.float32)
+    t, gt, bt = rt.upload_f32(x), rt.upload_f32(g), rt.upload_f32(b)
+    with pytest.raises(vh.UploadError):
+        rt.alloc_f32(1 << 45)
+    got = rt.download_f32(rt.layernorm_f32(t, gt, bt, 3, 768, 1e-6))
+    assert_bits_equal(got, rt.download_f32(rt.layernorm_f32(t, gt, bt, 3, 768, 1e-6)))
+    assert max_rel(got, O.layernorm(x, 3, 768, g, b, 1e-6)) <= 1e-5

@@ -70,7 +70,10 @@ vh_status null_arg(const char *what) {
     return fail(VH_ERR_INVALID_ARGUMENT, std::string(what) + ": null handle or pointer");
 }
 
+// Of a failed HIP call.  The error is also left as the thread's last one, which
+// the next launch's own check would take for its own: cleared.
 std::string hip_msg(const char *what, hipError_t e) {
+    hipGetLastError();
     return std::string(what) + ": " + hipGetErrorName(e) + " (" + hipGetErrorString(e) + ")";
 }
 
