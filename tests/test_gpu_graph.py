@@ -165,3 +165,58 @@ def test_graph_of_a_block_outlives_larger_runs(rt, monkeypatch, kind):
     finally:
         hip.hipGraphExecDestroy(exe)
         hip.hipGraphDestroy(graph)
+
+
+def test_a_failed_allocation_takes_back_what_other_runtimes_hold(rt):
+    """The blocks that another runtime of the device has kept go back to the
+    device; a capture that its thread has begun meanwhile is not disturbed (no
+    free becomes part of its graph, and the blocks it uses stay)."""
+    import vestra_hip as vh
+
+    hip = _hip()
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    other = vh.Runtime(0)
+    stream = ctypes.c_void_p(other.stream())
+
+    def fill():
+        for t in [other.alloc_f32((16 << 20) + 1024 * i) for i in range(4)]:
+            t.free()
+        other.synchronize()
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    def refused():
+        with pytest.raises(vh.UploadError):
+            rt.alloc_f32(1 << 45)
+
+    fill()
+    before = free_bytes()
+    refused()
+    assert free_bytes() >= before + 4 * (64 << 20)
+
+    lin = other.prepare_linear_f32(256, 256, seeded.normal(9700, 256 * 256, 0.05), seeded.normal(9701, 256))
+    x, r0 = other.upload_f32(seeded.normal(9702, 300 * 256)), seeded.normal(9703, 300 * 256)
+    res = other.upload_f32(r0)
+    lin.run_residual(x, 300, res)
+    exp = other.download_f32(res)
+    res = other.upload_f32(r0)
+    fill()
+
+    def run():
+        lin.run_residual(x, 300, res)
+        refused()
+
+    graph, exe = _capture(hip, stream, run)
+    try:
+        for replay in range(3):
+            fill()
+            other.copy_segment_into_f32(res, 0, other.upload_f32(r0), 0, r0.size)
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            assert_bits_equal(other.download_f32(res), exp, f"replay {replay}")
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)

@@ -48,7 +48,11 @@ int main() {
         CHECK(keep(600, 4096) && keep(1000 + i, 32 * mb + 512 * i));
         CHECK(pool.take(4096) == (void *)600);
     }
-    pool.give_back(release);
+    // All of them, or, where they may still be in use, none.
+    const size_t held = pool.held(), before = freed.size();
+    pool.give_back([] { return false; }, release);
+    CHECK(held > 0 && pool.held() == held && freed.size() == before);
+    pool.give_back([] { return true; }, release);
     CHECK(pool.held() == 0 && !pool.take(16 * mb + 512 * 99) && freed.count(199) && freed.count(1099));
 
     // Freed from several threads.
@@ -61,7 +65,7 @@ int main() {
                     shared.keep((void *)(uintptr_t)(1 + t), 512 * (1 + i % 7), [](void *) { std::exit(2); });
         });
     for (auto &t : threads) t.join();
-    shared.give_back([](void *) {});
+    shared.give_back([] { return true; }, [](void *) {});
     CHECK(shared.held() == 0);
     return 0;
 }

@@ -131,7 +131,7 @@ struct RtState {
     hipEvent_t t0 = nullptr, t1 = nullptr;
 
     void give_back() {
-        pool.give_back([this](void *p) { hipFreeAsync(p, stream); });
+        pool.give_back([] { return true; }, [this](void *p) { hipFreeAsync(p, stream); });
     }
 
     ~RtState() {
@@ -161,19 +161,25 @@ struct RtState {
 };
 
 // After an allocation of s has failed: the tensor blocks that the runtimes of its
-// device hold go back (not of another one that is being captured, whose graph
-// the frees would become part of), and what the stream-ordered pool keeps with
-// them.
+// device hold go back, and what the stream-ordered pool keeps with them.  A
+// runtime that is being captured keeps its blocks.  Another thread may begin a
+// capture of its runtime at any moment, and a free on that stream would become
+// part of the graph: its work is waited for, and the blocks, which nothing
+// uses any more, are freed on the stream of s.  (A capture that begins during
+// that wait ends with an error.)
 void give_back_all(RtState &s) {
     hipGetLastError();
+    s.give_back();
     {
         std::lock_guard<std::mutex> lock(runtimes().mu);
         for (RtState *r : runtimes().live) {
-            if (r->device != s.device || capturing(r->stream)) continue;
-            r->give_back();
-            hipStreamSynchronize(r->stream);
+            if (r == &s || r->device != s.device) continue;
+            r->pool.give_back(
+                [&] { return !capturing(r->stream) && hipStreamSynchronize(r->stream) == hipSuccess; },
+                [&](void *p) { hipFreeAsync(p, s.stream); });
         }
     }
+    hipStreamSynchronize(s.stream);
     hipMemPool_t pool = nullptr;
     if (hipDeviceGetDefaultMemPool(&pool, s.device) == hipSuccess && pool) hipMemPoolTrimTo(pool, 0);
     hipGetLastError();

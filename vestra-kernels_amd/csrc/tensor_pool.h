@@ -65,9 +65,11 @@ public:
         return true;
     }
 
-    template <class Release>
-    void give_back(Release release) {
+    // Releases every block, if ready() says so once no more can be taken.
+    template <class Ready, class Release>
+    void give_back(Ready ready, Release release) {
         std::lock_guard<std::mutex> lock(mu_);
+        if (blocks_.empty() || !ready()) return;
         for (const Block &b : blocks_) release(b.p);
         blocks_.clear();
         by_size_.clear();
