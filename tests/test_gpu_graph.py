@@ -167,6 +167,60 @@ def test_graph_of_a_block_outlives_larger_runs(rt, monkeypatch, kind):
         hip.hipGraphDestroy(graph)
 
 
+def _free_bytes(hip):
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_a_failed_allocation_takes_back_the_split_rows(rt):
+    """The workspace of the largest projection that a runtime has run goes back
+    where an allocation needs it, unless a graph holds it; later calls get a
+    new one."""
+    import vestra_hip as vh
+
+    rt = vh.Runtime(0)
+    hip = _hip()
+    stream = ctypes.c_void_p(rt.stream())
+    m, k, n = 200000, 389, 128  # 333 MB of split rows
+    lin = rt.prepare_linear_f32(k, n, seeded.normal(9750, k * n, 0.05), seeded.normal(9751, n))
+    x, r0 = rt.upload_f32(seeded.normal(9752, 4096 * k)), seeded.normal(9753, 4096 * n)
+    big, acc, res = rt.alloc_f32(m * k), rt.alloc_f32(m * n), rt.upload_f32(r0)
+    for i in range(0, m, 4096):
+        rows = min(4096, m - i)
+        rt.copy_segment_into_f32(big, i * k, x, 0, rows * k)
+        rt.copy_segment_into_f32(acc, i * n, res, 0, rows * n)
+
+    def refused():
+        with pytest.raises(vh.UploadError):
+            rt.alloc_f32(1 << 45)
+
+    lin.run_residual(x, 4096, res)
+    exp = rt.download_f32(res)
+    refused()
+    before = _free_bytes(hip)
+    lin.run_residual(big, m, acc)
+    rt.synchronize()
+    assert _free_bytes(hip) <= before - m * k * 4
+    refused()
+    assert _free_bytes(hip) >= before - (16 << 20)  # (but for small first-use workspaces)
+    res = rt.upload_f32(r0)
+    lin.run_residual(x, 4096, res)
+    assert_bits_equal(rt.download_f32(res), exp, "after it went back")
+    graph, exe = _capture(hip, stream, lambda: lin.run_residual(x, 4096, res))
+    try:
+        for replay in range(3):
+            refused()
+            rt.copy_segment_into_f32(res, 0, rt.upload_f32(r0), 0, r0.size)
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            assert_bits_equal(rt.download_f32(res), exp, f"replay {replay}")
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+
+
 def test_a_failed_allocation_takes_back_what_other_runtimes_hold(rt):
     """The blocks that another runtime of the device has kept go back to the
     device; a capture that its thread has begun meanwhile is not disturbed (no
@@ -174,7 +228,6 @@ def test_a_failed_allocation_takes_back_what_other_runtimes_hold(rt):
     import vestra_hip as vh
 
     hip = _hip()
-    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
     other = vh.Runtime(0)
     stream = ctypes.c_void_p(other.stream())
 
@@ -183,19 +236,14 @@ def test_a_failed_allocation_takes_back_what_other_runtimes_hold(rt):
             t.free()
         other.synchronize()
 
-    def free_bytes():
-        free, total = ctypes.c_size_t(), ctypes.c_size_t()
-        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-        return free.value
-
     def refused():
         with pytest.raises(vh.UploadError):
             rt.alloc_f32(1 << 45)
 
     fill()
-    before = free_bytes()
+    before = _free_bytes(hip)
     refused()
-    assert free_bytes() >= before + 4 * (64 << 20)
+    assert _free_bytes(hip) >= before + 4 * (64 << 20)
 
     lin = other.prepare_linear_f32(256, 256, seeded.normal(9700, 256 * 256, 0.05), seeded.normal(9701, 256))
     x, r0 = other.upload_f32(seeded.normal(9702, 300 * 256)), seeded.normal(9703, 300 * 256)

@@ -161,8 +161,9 @@ struct RtState {
 };
 
 // After an allocation of s has failed: the tensor blocks that the runtimes of its
-// device hold go back, and what the stream-ordered pool keeps with them.  A
-// runtime that is being captured keeps its blocks.  Another thread may begin a
+// device hold go back, what the stream-ordered pool keeps with them, and the split
+// rows of s (as large as its largest call's, and taken after every other
+// allocation of a call, so that none is using them here).  A runtime that is being captured keeps its blocks.  Another thread may begin a
 // capture of its runtime at any moment, and a free on that stream would become
 // part of the graph: its work is waited for, and the blocks, which nothing
 // uses any more, are freed on the stream of s.  (A capture that begins during
@@ -180,6 +181,10 @@ void give_back_all(RtState &s) {
         }
     }
     hipStreamSynchronize(s.stream);
+    if (s.sx.p && !s.sx.recorded) {
+        hipFree(s.sx.p);
+        s.sx = Workspace{};
+    }
     hipMemPool_t pool = nullptr;
     if (hipDeviceGetDefaultMemPool(&pool, s.device) == hipSuccess && pool) hipMemPoolTrimTo(pool, 0);
     hipGetLastError();
@@ -782,12 +787,12 @@ vh_status try_split(RtState &s, const Lin &L, vh::SplitGemm g, const char *name,
     if (!L.sw || g.m == 0 || !split_k_fits(g.m, g.n, g.k) || fp32_gemm_asked() ||
         !vh::split_gemm_pays(g.m, g.n, g.k, g.m * g.k, g.chw))
         return VH_OK;
+    piece_workspace(s, g);
     SplitRows x;
     TRY(split_input(s, g.xf, g.m, g.k, &x));
     if (!x.x) return VH_OK;
     g.x = x.x;
     g.ex = x.ex;
-    piece_workspace(s, g);
     *done = true;
     return launch(s, name, [&] { return vh::launch_gemm_split(s.stream, g); });
 }
@@ -1243,9 +1248,10 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
         vh::split_gemm_pays(m, n, k, mk + kn)) {
         const size_t abytes = vh::split_bytes(m, k), bbytes = vh::split_bytes(n, k);
         vh_status st = VH_OK;
+        vh::SplitGemm g{};
+        piece_workspace(s, g);
         char *x = split_space(s, abytes + bbytes + (m + n) * sizeof(int));
         if (x) {
-            vh::SplitGemm g{};
             char *w = x + abytes;
             int *ex = reinterpret_cast<int *>(w + bbytes), *ew = ex + m;
             g.x = x;
@@ -1260,7 +1266,6 @@ extern "C" vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor
             g.k = k;
             g.epi = vh::Epi::Store;
             g.c = t->ptr;
-            piece_workspace(s, g);
             st = launch(s, "split_operands", [&] {
                 return vh::launch_split_operands(s.stream, a->ptr, x, ex, m, b->ptr, w, ew, k, n);
             });
