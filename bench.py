@@ -1,8 +1,8 @@
 #!/usr/bin/env python3
 """DA3-BASE ViT block benchmark on one MI355X.
 
-Metric (BASELINE.json): "DA3-BASE ViT block us @504x336 (865 tok); GEMM/attn %
-fp32-MFMA peak".  A step is one full encoder block (BASELINE config 3) over a
+Metric: "DA3-BASE ViT block us @504x336 (865 tok); GEMM/attn %
+fp32-MFMA peak".  A step is one full encoder block over a
 synthetic 865-token image already resident in HBM, as seven kernels on the
 runtime's stream: LayerNorm 1 to split rows; QKV+RoPE; flash attention;
 out-projection+LayerScale+residual; LayerNorm 2 to split rows; fc1+GELU;
@@ -20,8 +20,8 @@ per block from idle and 164.5 us after 50-400 ms of blocks; half a second of
 idling brings the 189 us back).  Both passes therefore run twice: from the
 idle GPU right after preparation (`cold_start`), then after CLOCK_SETTLE_MS
 of untimed blocks (`value`, `kernels`, `roofline`).  The secondary sections
-follow (Q8_0 block, elementwise kernels, DPT head, BASELINE configs 4, 1, 2
-and 5).  The CPU baselines
+follow (Q8_0 block, elementwise kernels, DPT head, the Q8_0 GEMM, attention and
+projections standalone, the 12-layer encoder).  The CPU baselines
 are the oracle's restatement of the crate's AVX-512 kernels (block, each
 projection, flash attention, VNNI Q8_0 GEMM, the Q8_0 block and the 12-layer
 encoder), timed on this host with 16 threads and with every core of the
@@ -191,7 +191,7 @@ def log(msg: str) -> None:
 
 
 class BlockBench:
-    """One DA3-BASE block at 865 tokens (BASELINE config 3 weights and
+    """One DA3-BASE block at 865 tokens (seeded weights and
     input), prepared once so that its timing passes have no host work
     between them and the GPU work before them."""
 
@@ -272,8 +272,7 @@ class BlockBench:
         return out
 
 
-# BASELINE config 5 (4 x 865 tokens, one 3457-token image) and the north
-# star's own target, one 504 x 336 image (865 tokens).
+# 4 x 865 tokens, one 3457-token image and one 504 x 336 image (865 tokens).
 ENCODER_CASES = (("encoder_12x_4x865", 4, 24, 36), ("encoder_12x_1x3457", 1, 48, 72),
                  ("encoder_12x_1x865", 1, 24, 36))
 ENCODER_LAYERS = 12
@@ -311,9 +310,9 @@ ENCODER_MIN_MS = 20.0
 
 
 def gpu_encoder() -> dict:
-    """the 12-layer DA3-BASE encoder (independent seeded
+    """The 12-layer DA3-BASE encoder (independent seeded
     layers) at 4 images x 865 tokens and at one 1008 x 672 image (3457
-    tokens), and the north star's one 504 x 336 image (865 tokens), whole
+    tokens), and at one 504 x 336 image (865 tokens), whole
     encoder between two HIP events, with its algorithmic FLOPs as a
     fraction of the fp32-MFMA peak.  Each case first runs untimed passes
     for CLOCK_SETTLE_MS, as the block does: the host work between cases
@@ -364,7 +363,7 @@ def gpu_encoder() -> dict:
 
 
 def gpu_q8_0(steps: int) -> dict:
-    """fc1-shaped Q8_0 path.  X [865, 768] ~ N(0,1)
+    """The fc1-shaped Q8_0 path.  X [865, 768] ~ N(0,1)
     quantised on the device each step, W [768, 3072] ~ N(0, 0.02^2)
     quantised along K at load time, C = X_q . W_q [865, 3072] f32."""
     import vestra_hip as vh
@@ -615,13 +614,13 @@ def gpu_dpt(reps: int = 20) -> dict:
     return out
 
 
-# BASELINE config 2 shapes (K, N) per launch, and the config-1 attention.
+# Projection shapes (K, N) per launch, and the attention.
 PROJ_SHAPES = {"gemm_qkv_rope": (D, 3 * D), "gemm_proj_residual": (D, D),
                "gemm_fc1_gelu": (D, F), "gemm_fc2_residual": (F, D)}
 
 
 def config2_weights(name: str):
-    """BASELINE config 2 inputs of one projection: X ~ N(0,1) [T, K],
+    """Inputs of one projection: X ~ N(0,1) [T, K],
     W ~ N(0, 0.02^2) [K, N] row-major, b ~ N(0, 0.01^2) [N]."""
     from vestra_hip import seeded
 
@@ -632,16 +631,16 @@ def config2_weights(name: str):
 
 
 def config1_qkv():
-    """BASELINE config 1 inputs: Q, K, V ~ N(0,1), [12, 865, 64] each."""
+    """Attention inputs: Q, K, V ~ N(0,1), [12, 865, 64] each."""
     from vestra_hip import seeded
 
     return tuple(seeded.normal(1 + i, H * T * HD) for i in range(3))
 
 
 def gpu_configs(reps: int = 20) -> dict:
-    """BASELINE configs 1 and 2 standalone, each on its own stated inputs:
-    the config-1 attention (token-major output [865, 768]) and the four
-    config-2 projections with bias (vh_linear_run: the split of the input rows
+    """Attention and projections standalone, each on its own inputs:
+    the attention (token-major output [865, 768]) and the four
+    projections with bias (vh_linear_run: the split of the input rows
     and one GEMM launch with the bias epilogue).  Each case first runs for CLOCK_SETTLE_MS untimed (the
     preparation between cases idles the GPU and its clock drops), then
     `reps` launches each between its own pair of HIP events (`us`, the
@@ -719,7 +718,7 @@ def cpu_median_us(fn, min_runs: int = 10, budget_s: float = 2.0, max_runs: int =
 
 def cpu_kernels() -> dict:
     """Per-kernel CPU baselines: the oracle's restatements of the crate's
-    AVX-512 kernels on BASELINE config 1/2/4 inputs -- qkv_avx512_column_split
+    AVX-512 kernels on the standalone inputs -- qkv_avx512_column_split
     (36 panels), linear_bias_scale_avx512_rows<6> for out-proj and fc2 (145
     row tiles), linear_avx512_column_split_rows<6> for fc1 (48 panels), the
     QT8 flash attention (12 x 109 query tiles), each at 16 threads and at

@@ -1,5 +1,5 @@
-"""Float64 transcription of the DA3-BASE pre-LN ViT block (BASELINE config
-3), the exact result of the block on float32 inputs and weights: LN -> QKV
+"""Float64 transcription of the DA3-BASE pre-LN ViT block, the
+exact result of the block on float32 inputs and weights: LN -> QKV
 (+bias) -> [late blocks: LayerNorm of each 64-wide Q/K head row] -> 2-D RoPE
 on Q, K -> softmax(QK^T/8)V -> out-proj (+bias) * LayerScale + residual ->
 LN -> fc1 (+bias) -> exact-erf GELU -> fc2 (+bias) * LayerScale + residual.

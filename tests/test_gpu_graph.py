@@ -167,6 +167,39 @@ def test_graph_of_a_block_outlives_larger_runs(rt, monkeypatch, kind):
         hip.hipGraphDestroy(graph)
 
 
+def test_graph_of_a_projection_that_no_run_has_prepared(rt):
+    """Without a workspace for its split rows a captured projection takes the
+    fp32 GEMM: the replays are right, and the same every time."""
+    import vestra_hip as vh
+
+    rt = vh.Runtime(0)  # its own, without workspaces
+    hip = _hip()
+    stream = ctypes.c_void_p(rt.stream())
+    m, k, n = 500, 770, 768
+    w = seeded.normal(9650, k * n, 0.02)
+    lin = rt.prepare_linear_f32(k, n, w, np.zeros(n, np.float32))
+    x, r0 = seeded.normal(9651, m * k), seeded.normal(9652, m * n)
+    xt, res = rt.upload_f32(x), rt.upload_f32(r0)
+    graph, exe = _capture(hip, stream, lambda: lin.run_residual(xt, m, res))
+    try:
+        got = []
+        for replay in range(3):
+            rt.copy_segment_into_f32(res, 0, rt.upload_f32(r0), 0, r0.size)
+            assert hip.hipGraphLaunch(exe, stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            got.append(rt.download_f32(res))
+            res2 = rt.upload_f32(r0)
+            lin.run_residual(xt, m, res2)  # eagerly, on split rows, between the replays
+        exp = r0 + (x.reshape(m, k).astype(np.float64) @ w.reshape(k, n)).reshape(-1)
+        for g in got:
+            assert_bits_equal(g, got[0])
+            assert np.linalg.norm(g - exp) <= 1e-6 * np.linalg.norm(exp)
+        assert (rt.download_f32(res2) != got[0]).any()
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+
+
 def _free_bytes(hip):
     hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
     free, total = ctypes.c_size_t(), ctypes.c_size_t()

@@ -202,8 +202,8 @@ def test_gemm_row_major_b_in_place_equals_transposed_copy(rt, monkeypatch, m, k,
     assert_bits_equal(outs[0], outs[1], f"row-major GEMM {m}x{k}x{n}: B in place vs transposed")
 
 
-# M = 865 is one 504x336 image; 3460 = the batch of 4 (BASELINE config 5a) and
-# 3457 = one 1008x672 image (config 5b).  Past M = 1024 the GEMM takes other
+# M = 865 is one 504x336 image; 3460 = the batch of 4 and
+# 3457 = one 1008x672 image.  Past M = 1024 the GEMM takes other
 # tiles, an XCD-ordered tile walk and other split-K choices, so those paths
 # are compared with the oracle at those sizes too.
 PROJ_M = [865, 3460, 3457]
@@ -488,7 +488,7 @@ def test_flash_da3_production_shape_vs_oracle(rt):
 
 
 def test_flash_config1_normal_inputs_token_major(rt):
-    """BASELINE config 1: Q, K, V ~ N(0,1), 12 heads x 865 x 64, out [865, 768]."""
+    """Q, K, V ~ N(0,1), 12 heads x 865 x 64, out [865, 768]."""
     H, T = 12, 865
     n = H * T * 64
     q, k, v = seeded.normal(1, n), seeded.normal(2, n), seeded.normal(3, n)
@@ -668,7 +668,7 @@ def test_q8_0_upload_download_every_int8_value(rt):
 @pytest.mark.parametrize("m,n,k", [(865, 3072, 768), (8, 8, 64), (5, 17, 96), (64, 96, 3072),
                                    (33, 70, 1056), (1024, 1920, 2112), (1024, 1920, 1120)])
 def test_gemm_q8_0_bit_exact(rt, m, n, k):
-    """BASELINE config 4 (fc1 weights N(0, 0.02^2), activations N(0,1) quantised
+    """The Q8_0 GEMM at fc1 ( weights N(0, 0.02^2), activations N(0,1) quantised
     on the device), the tests/q8_0_dot_matches_f32.rs shape, and the scale
     chunking and prefetch grouping: the 32x32 tile with 96 blocks in one
     chunk (3072) and an odd block count (1056: one block per prefetch

@@ -1,5 +1,5 @@
 """Pins the oracle's DA3-BASE block composition against an independent
-float64 transcription of the pre-LN ViT block (BASELINE config 3): LN ->
+float64 transcription of the pre-LN ViT block: LN ->
 QKV (+bias) -> [late blocks: LayerNorm of each 64-wide Q/K head row] ->
 2-D RoPE on Q, K -> softmax(QK^T/8)V -> out-proj (+bias) * LayerScale +
 residual -> LN -> fc1 (+bias) -> exact-erf GELU -> fc2 (+bias) * LayerScale
