@@ -3,9 +3,9 @@
 //
 // Q, K and V are split rows [bh][tokens] of 256 bytes (two slices of 32
 // dims, hi then lo), each tensor with one exponent per head or one for all.
-// A workgroup of eight waves owns QG * 32 queries of one head; QG groups of
-// waves each take 32 of the queries and KS = 8 / QG key streams share the
-// keys: of every step's 128 keys stream s takes PK = 128 / KS.  K and V
+// A workgroup of eight waves owns 64 queries of one head; QG = 2 groups of
+// waves each take 32 of the queries and KS = 4 key streams share the keys: of
+// every step's 128 keys stream s takes PK = 32.  K and V
 // panels are copied straight into LDS, one step ahead of their use.  Per
 // panel a wave computes
 //     S^T[key][query] = K . Q^T
@@ -58,6 +58,9 @@ namespace {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kPBits = 5.0f;    // P is held as 2^kPBits p
 constexpr float kMaxSlack = 8.0f; // scores may pass the running maximum by this (base 2)
+
+constexpr int QG = 2, KS = 8 / QG;          // query groups and key streams of a workgroup
+constexpr int PK = 128 / KS, KT = PK / 16;  // keys of a stream and step, and their tiles of 16
 
 // Codes per head and tensor, one from each workgroup that split its rows: the
 // exponent, and whether that workgroup has seen a small value.
@@ -161,7 +164,6 @@ __device__ __forceinline__ float max_row16(float v) {
 // O^T += V^T . P^T as there, 4 dims or keys to an instruction: lane (li, lh)
 // holds dims 16 c + 4 lh + e of its row, and the key 4 lh + r of instruction
 // r of P . V.
-template <int PK>
 __device__ __forceinline__ void float_pass(const AttnArgs &fa, size_t off, int qw, int stream, int lane,
                                            f32x4 (&o)[4][2], float (&m)[2], float (&l)[2]) {
     const int li = lane & 15, lh = lane >> 4, T = fa.T, hd = fa.hd;
@@ -248,9 +250,8 @@ __device__ __forceinline__ void float_pass(const AttnArgs &fa, size_t off, int q
     }
 }
 
-template <int QG, AOut OUT>
+template <AOut OUT>
 __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
-    constexpr int KS = 8 / QG, PK = 128 / KS, KT = PK / 16;
     constexpr int HALF = 128 * 256;  // bytes of a step's K (or V) panels
     extern __shared__ __attribute__((aligned(16))) char smem_c[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -389,7 +390,6 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
         }
         // Kept off zero and infinity: a masked score (-inf) stays -inf.
         const float scale = fminf(fmaxf(__builtin_ldexpf(fa.scale_log2, e_score), 0x1p-126f), 0x1p127f);
-        static_assert(KT == 2, "32 keys per stream and step");
         f32x4 s0[KT][2], s1[KT][2];
         read_k(0);
         score_round(I0{}, s0);
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(512, 2) void attn_split_kernel(AttnArgs fa) {
     }
     if constexpr (OUT != AOut::Split) {
         if (floats) {
-            float_pass<PK>(fa, off, q0 + qg * 32, stream, lane, o, m, l);
+            float_pass(fa, off, q0 + qg * 32, stream, lane, o, m, l);
             merge();
             ev = 0;
         }
@@ -801,22 +801,17 @@ __global__ __launch_bounds__(NT) void attn_split_rows_kernel(const float *__rest
     }
 }
 
-template <int QG, AOut OUT>
+template <AOut OUT>
 hipError_t run_attn(hipStream_t s, AttnArgs fa) {
     constexpr size_t lds = 4 * 128 * 256;  // two steps of K and of V panels
     static_assert(lds >= 8 * 8 * 64 * 16 + 8 * 64 * 16 + 8 * 2 * 16 * 4 + 4, "the merge fits the panels' LDS");
-    auto kernel = attn_split_kernel<QG, OUT>;
+    auto kernel = attn_split_kernel<OUT>;
     static std::atomic<uint64_t> configured{0};
     if (hipError_t e = ensure_dynamic_lds(kernel, lds, configured); e != hipSuccess) return e;
     fa.qtiles = (fa.T + QG * 32 - 1) / (QG * 32);
     const int total = fa.bh * fa.qtiles;
     kernel<<<(unsigned)((total + 7) / 8 * 8), 512, lds, s>>>(fa);
     return hipGetLastError();
-}
-
-template <AOut OUT>
-hipError_t dispatch_attn(hipStream_t s, const AttnArgs &fa) {
-    return run_attn<2, OUT>(s, fa);
 }
 
 constexpr int kRangeChunks = 16;
@@ -896,7 +891,7 @@ hipError_t launch_attn_split_f32(hipStream_t s, const float *q, const float *k, 
     fa.token_major = token_major ? 1 : 0;
     fa.q8_qs = q8_qs;
     fa.q8_d = q8_d;
-    return q8_qs ? dispatch_attn<AOut::Q8>(s, fa) : dispatch_attn<AOut::F32>(s, fa);
+    return q8_qs ? run_attn<AOut::Q8>(s, fa) : run_attn<AOut::F32>(s, fa);
 }
 
 hipError_t launch_attn_split(hipStream_t s, const SplitQkv &p, void *out_split, size_t bh, size_t tokens,
@@ -916,7 +911,7 @@ hipError_t launch_attn_split(hipStream_t s, const SplitQkv &p, void *out_split, 
     fa.hd = 64;
     fa.scale_log2 = 0.125f * kLog2e;
     fa.out_split = static_cast<char *>(out_split);
-    return dispatch_attn<AOut::Split>(s, fa);
+    return run_attn<AOut::Split>(s, fa);
 }
 
 }  // namespace vh

@@ -1892,8 +1892,7 @@ extern "C" vh_status vh_linear_run_chw(const vh_linear *linear, const vh_tensor 
         sg.chw = true;
         st = try_split(s, L, sg, "gemm_bias_chw", &done);
     }
-    if (done) {
-    } else if (!st && !L.gamma && L.K % 32 == 0 && rows <= (size_t)INT32_MAX) {
+    if (!st && !done && !L.gamma && L.K % 32 == 0 && rows <= (size_t)INT32_MAX) {
         // The transposed product in one GEMM: the weight rows [N][K] as A and
         // the input rows as Bt, stored channel-major with the bias per
         // channel by the implicit convolution's epilogue (a 1 x 1 tap over
@@ -1912,7 +1911,7 @@ extern "C" vh_status vh_linear_run_chw(const vh_linear *linear, const vh_tensor 
         g.conv_wp = rows;
         g.conv_ow = rows;
         st = launch(s, "gemm_bias_chw", [&] { return vh::launch_gemm(s.stream, g); });
-    } else if (!st) {
+    } else if (!st && !done) {
         float *tmp = nullptr;
         st = dalloc(s, len, &tmp, "GEMM output allocation");
         if (!st) st = run_lin(s, L, input->ptr, rows, vh::Epi::Store, tmp, "gemm_bias_scale");
