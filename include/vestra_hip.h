@@ -101,9 +101,13 @@ vh_status vh_add_f32_in_place(const vh_runtime *rt, vh_tensor *destination,
 
 /* ---- GEMM and epilogues --------------------------------------------------- */
 /* src/cuda.rs:661-704 gemm_row_major_f32: C[m,n] = A[m,k] x B[k,n], row-major.
- * Replaces cublasSgemm: f32 in and out, on split rows and the f16 matrix
- * cores where that is faster (closer to the exact product than the fp32
- * matrix instructions), else on those. */
+ * Replaces cublasSgemm: f32 in and out, on split rows (each float as two
+ * halves) and the f16 matrix cores where that is faster, else on the fp32
+ * matrix instructions.  On operands of like magnitude the split form is closer
+ * to the exact product than those (about half their 2-norm error); an output
+ * that the range of its row or column may have cost bits is formed again from
+ * the floats.  The same holds for the prepared linears, the convolutions and
+ * the attention below. */
 vh_status vh_gemm_row_major_f32(const vh_runtime *rt, const vh_tensor *a, const vh_tensor *b,
                                 size_t m, size_t k, size_t n, vh_tensor **out);
 /* src/cuda.rs:708-742 bias_scale_f32_in_place: v = (v + bias[c]) * gamma[c]. */
@@ -132,7 +136,8 @@ vh_status vh_attention_online_f32(const vh_runtime *rt, const vh_tensor *q, cons
                                   const vh_tensor *v, size_t heads, size_t tokens,
                                   size_t head_dim, vh_tensor **out);
 /* flash_attention_f32_da3_base (src/lib.rs:82-91, src/specialized.rs:730-765):
- * head_dim 64, scale 1/8, online softmax, split products.  Any token count is
+ * head_dim 64, scale 1/8, online softmax, split products where they are
+ * faster.  Any token count is
  * accepted (the reference's tokens % 865 gate is a CPU-kernel limit).
  * token_major = 0 writes head-major [heads,tokens,64]; 1 writes token-major
  * [tokens, heads*64] (the fused hnd_to_token of src/cuda.rs:984-1036). */

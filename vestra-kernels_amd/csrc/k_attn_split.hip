@@ -38,7 +38,7 @@
 //
 // Error against float64 at 12 x 865 x 64, N(0, 1): 2.5e-7, against 4.3e-7 of the
 // fp32 matrix instructions.  Time on split rows (kernel trace): 12 x 865 18 us
-// against 28 (fp32 matrix instructions), 48 x 865 54 against 100, 12 x 3457
+// against 28 (fp32 matrix instructions), 48 x 865 53 against 100, 12 x 3457
 // 157 against 343.  Products alone would take a third of that: the softmax's
 // VALU work and the products share the SIMD's issue (a product holds it
 // for 8 of its 16 cycles, measured), and taking out the copies, the LDS reads or

@@ -2744,9 +2744,9 @@ vh_status conv_run(RtState &s, const vh_conv2d &c, const float *in, size_t ih, s
     float *xh = nullptr, *col = nullptr, *tmp = nullptr;
     vh_status st = VH_OK;
     const char *direct_env = std::getenv("VESTRA_HIP_CONV_DIRECT");
-    // On split rows and the f16 matrix cores: three launches, but 3 to 4 times
-    // the fp32 form's rate (128 -> 128 on 96 x 144: 21 + 6.5 + 3.9 us
-    // against 69).  VESTRA_HIP_CONV_DIRECT and the GEMM overrides ask for the
+    // On split rows and the f16 matrix cores: three launches, but 2 to 3 times
+    // the fp32 form's rate (128 -> 128 on 96 x 144, kernel trace: 18.4 + 6.0 +
+    // 4.4 us against 50).  VESTRA_HIP_CONV_DIRECT and the GEMM overrides ask for the
     // fp32 forms.
     if (c.sw && !direct_env && !fp32_gemm_asked()) {
         const vh::SplitConv sc{in,     c.in_c, ih,   iw,    c.out_c, c.kh, c.kw,
